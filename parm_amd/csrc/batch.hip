@@ -264,7 +264,7 @@ __global__ __launch_bounds__(kBlock) void k_batch_skin(int nsys, BatchArrays A,
 // The systems to rebuild at the end of a step are those whose skin flag is
 // set (or all, when forced).  k_batch_worklist turns the flags into a list
 // (system ids in ascending order, count first) and counts each listed
-// system's slices of kBuildSlice atoms (exclusive prefix in wslice).  Then
+// system's build slices (exclusive prefix in wslice).  Then
 // two launches on fixed grids, so the launch shapes do not depend on how
 // many systems rebuild (the step stays graph-capturable) and no workgroup is
 // started for a system that keeps its list:
@@ -272,21 +272,21 @@ __global__ __launch_bounds__(kBlock) void k_batch_skin(int nsys, BatchArrays A,
 //                  keys, a stable counting sort of the system's atoms by
 //                  cell in LDS, the cell starts, sorted copies of the
 //                  positions and diameters, xref = x;
-//   k_batch_build  one workgroup of kBuildSlice threads per slice of a
-//                  listed system, a thread per atom: the exact list build
-//                  over the periodic 27-cell stencil (candidates in cell
-//                  order, then sorted order: deterministic), four candidates
-//                  in flight per thread.  A large system's build is spread
-//                  over many workgroups.
+//   k_batch_build  one workgroup per slice of a listed system's atoms,
+//                  several lanes per atom: the exact list build over the
+//                  stencil rows of the periodic cell grid
+//                  (candidates in row order, then sorted order:
+//                  deterministic).  A large system's build is spread over
+//                  many workgroups.
 // With `alt` (the positions one step ahead), |alt - xref| is recomputed for
 // the next skin test.
 constexpr int kBatchMaxCells = kBatchMaxCellsPerSystem;
 constexpr int kSortThreads = 1024;
 constexpr int kWorklistThreads = 1024;
-constexpr int kBuildSlice = 256;
+constexpr int kBuildThreads = 256;
 
 __global__ __launch_bounds__(kWorklistThreads) void k_batch_worklist(
-    int nsys, const uint32_t *__restrict__ flags, int force,
+    int nsys, const uint32_t *__restrict__ flags, int force, int slice,
     const BatchGeom *__restrict__ geom, int32_t *__restrict__ work,
     int32_t *__restrict__ wslice) {
     __shared__ int wsum[kWorklistThreads / kWave][2];
@@ -298,7 +298,7 @@ __global__ __launch_bounds__(kWorklistThreads) void k_batch_worklist(
         const int s = s0 + q;
         if (s < nsys && (force || flags[s] != 0u)) {
             loc++;
-            lsl += (geom[s].n + kBuildSlice - 1) / kBuildSlice;
+            lsl += (geom[s].n + slice - 1) / slice;
         }
     }
     const int lane = t % kWave, w = t / kWave;
@@ -331,7 +331,7 @@ __global__ __launch_bounds__(kWorklistThreads) void k_batch_worklist(
             work[1 + pos] = s;
             wslice[pos] = psl;
             pos++;
-            psl += (geom[s].n + kBuildSlice - 1) / kBuildSlice;
+            psl += (geom[s].n + slice - 1) / slice;
         }
     }
     if (t == 0) {
@@ -466,8 +466,16 @@ __global__ __launch_bounds__(kSortThreads) void k_batch_sort(
                        flags, which, nent, hist);
 }
 
-template <int D>
-__global__ __launch_bounds__(kBuildSlice) void k_batch_build(
+// G lanes per atom, U candidates per lane and round.  The build is bound by
+// the latency of its chain of dependent loads (cell bounds, then candidates),
+// not by arithmetic: at a step a few dozen systems rebuild.  A stencil row of
+// three x-adjacent cells is one contiguous range (two where it wraps), so an
+// atom takes 9 rows, not 27 cells; the group's lanes load all rows' bounds
+// together and test G * U candidates per round.  48 liquids of 300 - 1000 atoms:
+// 179 us per launch with one thread per atom, a step 210 -> 69 us; 1024
+// packings of 64 - 4096 (4 x 2 lanes): 200 steps 85.1 -> 80.0 ms.
+template <int D, int G, int U>
+__global__ __launch_bounds__(kBuildThreads) void k_batch_build(
     BatchArrays A, const typename PosStore<D>::T *__restrict__ alt, double skin,
     int type_bits, int tpa, int cap, int npad, uint32_t *__restrict__ nbr,
     int32_t *__restrict__ ncount, const int32_t *__restrict__ keys,
@@ -475,10 +483,15 @@ __global__ __launch_bounds__(kBuildSlice) void k_batch_build(
     const typename PosStore<D>::T *__restrict__ xs, const double *__restrict__ dsort,
     unsigned long long *__restrict__ nent, uint32_t *__restrict__ gflag,
     const int32_t *__restrict__ work, const int32_t *__restrict__ wslice) {
-    __shared__ unsigned long long red[kBuildSlice / kWave];
+    constexpr int kSlice = kBuildThreads / G;  // atoms per slice
+    constexpr int RPL = (9 + G - 1) / G;       // rows whose bounds a lane loads
+    __shared__ unsigned long long red[kBuildThreads / kWave];
     const int count = work[0];
     const int total = wslice[count];
     const int t = threadIdx.x;
+    const int sub = t % G, lane = t % kWave;
+    const int gbase = lane - sub;  // first lane of this atom's group
+    const unsigned long long below = (1ull << sub) - 1ull;
     for (int gs = blockIdx.x; gs < total; gs += gridDim.x) {
         // the listed system holding slice gs: the last q with wslice[q] <= gs
         int lo = 0, hi = count;
@@ -490,51 +503,81 @@ __global__ __launch_bounds__(kBuildSlice) void k_batch_build(
                 hi = mid;
         }
         const int s = work[1 + lo];
-        const BatchGeom G = A.geom[s];
-        const int off = G.off, n = G.n, nc0 = G.grid.nc[0], nc1 = G.grid.nc[1],
-                  nc2 = G.grid.nc[2];
-        const int u = (gs - wslice[lo]) * kBuildSlice + t;
+        const BatchGeom G_ = A.geom[s];
+        const int off = G_.off, n = G_.n, nc0 = G_.grid.nc[0], nc1 = G_.grid.nc[1],
+                  nc2 = G_.grid.nc[2];
+        const int u = (gs - wslice[lo]) * kSlice + t / G;
         unsigned long long mycnt = 0;
         if (u < n) {
-            const int lo0 = nc0 >= 3 ? -1 : 0, lo1 = (D >= 2 && nc1 >= 3) ? -1 : 0,
-                      lo2 = (D == 3 && nc2 >= 3) ? -1 : 0;
             const int i = cellidx[off + u];
             const Vec<D> xi = PosStore<D>::load(xs[off + u]);
             const double di = dsort[off + u];
             int key = keys[i];
-            int ci[3] = {0, 0, 0};
-            ci[0] = key % nc0;
+            const int c0 = key % nc0;
             key /= nc0;
-            if (D >= 2) {
-                ci[1] = key % nc1;
-                key /= nc1;
+            const int c1 = D >= 2 ? key % nc1 : 0;
+            const int c2 = D == 3 ? key / nc1 : 0;
+            const int ny = (D >= 2 && nc1 >= 3) ? 3 : 1, nz = (D == 3 && nc2 >= 3) ? 3 : 1;
+            const int nrows = ny * nz;
+            // the row's x cells as at most two contiguous cell ranges
+            int xa0 = 0, xb0 = 0, xa1 = 0, xb1 = -1;
+            if (nc0 >= 3) {
+                xa0 = c0 > 0 ? c0 - 1 : 0;
+                xb0 = c0 < nc0 - 1 ? c0 + 1 : c0;
+                if (c0 == 0) xa1 = xb1 = nc0 - 1;
+                if (c0 == nc0 - 1) xa1 = xb1 = 0;
             }
-            if (D == 3) ci[2] = key % nc2;
+            // lane sub loads the bounds of rows sub, sub + G, ...
+            int bnd[RPL][4];
+#pragma unroll
+            for (int q = 0; q < RPL; q++) {
+                const int r = sub + q * G;
+                bnd[q][0] = bnd[q][1] = bnd[q][2] = bnd[q][3] = 0;
+                if (r < nrows) {
+                    int q1 = c1 + (ny == 3 ? r % 3 - 1 : 0), q2 = c2 + (nz == 3 ? r / ny - 1 : 0);
+                    q1 = q1 < 0 ? q1 + nc1 : (q1 >= nc1 ? q1 - nc1 : q1);
+                    q2 = q2 < 0 ? q2 + nc2 : (q2 >= nc2 ? q2 - nc2 : q2);
+                    const int row = G_.cell_off + (D == 3 ? q2 * nc1 + q1 : q1) * nc0;
+                    bnd[q][0] = cstart[row + xa0];
+                    bnd[q][1] = cstart[row + xb0 + 1];
+                    if (xb1 >= 0) {
+                        bnd[q][2] = cstart[row + xa1];
+                        bnd[q][3] = cstart[row + xb1 + 1];
+                    }
+                }
+            }
             int cnt = 0;
-            for (int oz = lo2; oz <= -lo2; oz++)
-                for (int oy = lo1; oy <= -lo1; oy++)
-                    for (int ox = lo0; ox <= -lo0; ox++) {
-                        int q0 = ci[0] + ox, q1 = ci[1] + oy, q2 = ci[2] + oz;
-                        q0 = q0 < 0 ? q0 + nc0 : (q0 >= nc0 ? q0 - nc0 : q0);
-                        q1 = q1 < 0 ? q1 + nc1 : (q1 >= nc1 ? q1 - nc1 : q1);
-                        q2 = q2 < 0 ? q2 + nc2 : (q2 >= nc2 ? q2 - nc2 : q2);
-                        const int cc = (D == 3 ? (q2 * nc1 + q1) * nc0 : q1 * nc0) + q0;
-                        const int s0 = cstart[G.cell_off + cc] - off;
-                        const int s1 = cstart[G.cell_off + cc + 1] - off;
-                        for (int v0 = s0; v0 < s1; v0 += 4) {
-                            // four candidates' loads in flight together
-                            Vec<D> xj[4];
-                            double dj[4];
+            for (int r = 0; r < nrows; r++) {
+                const int owner = gbase + (r % G);
+                int rb[4];
 #pragma unroll
-                            for (int q = 0; q < 4; q++) {
-                                const int v = v0 + q < s1 ? v0 + q : s0;
-                                xj[q] = PosStore<D>::load(xs[off + v]);
-                                dj[q] = dsort[off + v];
-                            }
+                for (int k = 0; k < 4; k++) {
+                    int v = bnd[0][k];
 #pragma unroll
-                            for (int q = 0; q < 4; q++) {
-                                const int v = v0 + q;
-                                if (v >= s1 || v == u) continue;
+                    for (int q = 1; q < RPL; q++) v = r / G == q ? bnd[q][k] : v;
+                    rb[k] = __shfl(v, owner);
+                }
+#pragma unroll
+                for (int h = 0; h < 2; h++) {
+                    const int a = rb[2 * h], b = rb[2 * h + 1];
+                    for (int base = a; base < b; base += G * U) {
+                        // the round's loads in flight together; a slot past
+                        // the range reads the atom's own (and is not tested)
+                        Vec<D> xj[U];
+                        double dj[U];
+#pragma unroll
+                        for (int q = 0; q < U; q++) {
+                            const int v = base + q * G + sub;
+                            const int vv = v < b ? v : off + u;
+                            xj[q] = PosStore<D>::load(xs[vv]);
+                            dj[q] = dsort[vv];
+                        }
+#pragma unroll
+                        for (int q = 0; q < U; q++) {
+                            if (base + q * G >= b) break;  // uniform over the group
+                            const int v = base + q * G + sub;
+                            bool pass = false;
+                            if (v < b && v != off + u) {
                                 // minimum image by rint: equal to the
                                 // reference's remainder up to rounding far
                                 // inside the 1e-6 band, where the reference's
@@ -543,35 +586,41 @@ __global__ __launch_bounds__(kBuildSlice) void k_batch_build(
 #pragma unroll
                                 for (int k = 0; k < D; k++) {
                                     double dk = xi.c[k] - xj[q].c[k];
-                                    dk -= G.box.L[k] * rint(dk * G.box.invL[k]);
+                                    dk -= G_.box.L[k] * rint(dk * G_.box.invL[k]);
                                     d2 = fma(dk, dk, d2);
                                 }
                                 const double cut = (di + dj[q]) / 2 + skin;
-                                const double c2 = cut * cut;
-                                const bool pass =
-                                    d2 < c2 * (1.0 - 1e-6) ||
-                                    (d2 <= c2 * (1.0 + 1e-6) &&
-                                     in_list<D>(xi, xj[q], di, dj[q], G.box, skin));
-                                if (pass) {
-                                    if (cnt < cap) {
-                                        const int j = cellidx[off + v];
-                                        nbr[untiled_entry(cnt, i, tpa, npad)] =
-                                            ((uint32_t)j << type_bits) | (uint32_t)A.type[j];
-                                    }
-                                    cnt++;
+                                const double c2c = cut * cut;
+                                pass = d2 < c2c * (1.0 - 1e-6) ||
+                                       (d2 <= c2c * (1.0 + 1e-6) &&
+                                        in_list<D>(xi, xj[q], di, dj[q], G_.box, skin));
+                            }
+                            const unsigned long long m =
+                                (__ballot(pass) >> gbase) & ((1ull << G) - 1ull);
+                            if (pass) {
+                                const int w = cnt + __popcll(m & below);
+                                if (w < cap) {
+                                    const int j = cellidx[v];
+                                    nbr[untiled_entry(w, i, tpa, npad)] =
+                                        ((uint32_t)j << type_bits) | (uint32_t)A.type[j];
                                 }
                             }
+                            cnt += __popcll(m);
                         }
                     }
-            ncount[i] = cnt < cap ? cnt : cap;
-            if (cnt > cap) atomicOr(gflag, kFlagOverflow);
-            mycnt = (unsigned long long)cnt;
-            if (alt) {
-                const Vec<D> xa = PosStore<D>::load(alt[i]);
-                Vec<D> dd;
+                }
+            }
+            if (sub == 0) {
+                ncount[i] = cnt < cap ? cnt : cap;
+                if (cnt > cap) atomicOr(gflag, kFlagOverflow);
+                mycnt = (unsigned long long)cnt;
+                if (alt) {
+                    const Vec<D> xa = PosStore<D>::load(alt[i]);
+                    Vec<D> dd;
 #pragma unroll
-                for (int d = 0; d < D; d++) dd.c[d] = xa.c[d] - xi.c[d];
-                A.disp[i] = sqrt(sqnorm<D>(dd));
+                    for (int d = 0; d < D; d++) dd.c[d] = xa.c[d] - xi.c[d];
+                    A.disp[i] = sqrt(sqnorm<D>(dd));
+                }
             }
         }
         unsigned long long sum = mycnt;
@@ -581,7 +630,7 @@ __global__ __launch_bounds__(kBuildSlice) void k_batch_build(
         __syncthreads();
         if (t == 0) {
             unsigned long long tot = 0;
-            for (int q = 0; q < kBuildSlice / kWave; q++) tot += red[q];
+            for (int q = 0; q < kBuildThreads / kWave; q++) tot += red[q];
             atomicAdd(&nent[s], tot);
         }
         __syncthreads();
@@ -760,6 +809,15 @@ hipError_t launch_batch_skin(int nsys, const BatchArrays &A, double skin, uint32
     return hipGetLastError();
 }
 
+// Build lanes per atom and candidates per lane and round: a dense system (a
+// liquid: ~50 atoms in a stencil row) 8 x 4, a sparse one (packed spheres: ~8)
+// 4 x 2, whose round is a row (200 steps of 1024 packings: 80.0 ms, 87.1 ms with
+// 8 x 4; one thread per atom 85.1 ms).  The caller's line between them, 20
+// atoms to a row of three cells, lies where a row is two to three sparse
+// rounds and over half a dense one.
+constexpr int kBuildLanes = 8, kBuildAhead = 4;
+constexpr int kBuildLanesSparse = 4, kBuildAheadSparse = 2;
+
 hipError_t launch_batch_rebuild(int ndim, int nsys, const BatchArrays &A, const void *pos,
                                 const void *alt, int force, int count_rebuild, double skin,
                                 int type_bits, int tpa, int cap, int npad, uint32_t *nbr,
@@ -767,28 +825,32 @@ hipError_t launch_batch_rebuild(int ndim, int nsys, const BatchArrays &A, const 
                                 int32_t *cstart, void *xs, double *dsort, uint32_t *flags,
                                 uint32_t *which, unsigned long long *nent, uint32_t *gflag,
                                 int32_t *work, int32_t *wslice, int sort_grid, int build_grid,
-                                hipStream_t s) {
+                                bool sparse, hipStream_t s) {
     if (nsys <= 0) return hipSuccess;
+    // (see k_batch_build)
+    const int lanes = sparse ? kBuildLanesSparse : kBuildLanes;
     hipLaunchKernelGGL(k_batch_worklist, dim3(1), dim3(kWorklistThreads), 0, s, nsys, flags,
-                       force, A.geom, work, wslice);
+                       force, kBuildThreads / lanes, A.geom, work, wslice);
     const int gs = sort_grid < nsys ? sort_grid : nsys;
+#define PARM_BB(DD, PT, GG, UU)                                                               \
+    hipLaunchKernelGGL((k_batch_build<DD, GG, UU>), dim3(build_grid), dim3(kBuildThreads), 0, \
+                       s, A, (const PT *)alt, skin, type_bits, tpa, cap, npad, nbr, ncount,   \
+                       keys, cellidx, cstart, (const PT *)xs, dsort, nent, gflag, work, wslice)
+#define PARM_BR(DD, PT)                                                                       \
+    hipLaunchKernelGGL(k_batch_sort<DD>, dim3(gs), dim3(kSortThreads), 0, s, A,               \
+                       (const PT *)pos, count_rebuild, keys, cellidx, cstart, (PT *)xs,       \
+                       dsort, flags, which, nent, work);                                      \
+    if (sparse)                                                                               \
+        PARM_BB(DD, PT, kBuildLanesSparse, kBuildAheadSparse);                                \
+    else                                                                                      \
+        PARM_BB(DD, PT, kBuildLanes, kBuildAhead)
     if (ndim == 3) {
-        hipLaunchKernelGGL(k_batch_sort<3>, dim3(gs), dim3(kSortThreads), 0, s, A,
-                           (const double4 *)pos, count_rebuild, keys, cellidx, cstart,
-                           (double4 *)xs, dsort, flags, which, nent, work);
-        hipLaunchKernelGGL(k_batch_build<3>, dim3(build_grid), dim3(kBuildSlice), 0, s, A,
-                           (const double4 *)alt, skin, type_bits, tpa, cap, npad, nbr, ncount,
-                           keys, cellidx, cstart, (const double4 *)xs, dsort, nent, gflag,
-                           work, wslice);
+        PARM_BR(3, double4);
     } else {
-        hipLaunchKernelGGL(k_batch_sort<2>, dim3(gs), dim3(kSortThreads), 0, s, A,
-                           (const double2 *)pos, count_rebuild, keys, cellidx, cstart,
-                           (double2 *)xs, dsort, flags, which, nent, work);
-        hipLaunchKernelGGL(k_batch_build<2>, dim3(build_grid), dim3(kBuildSlice), 0, s, A,
-                           (const double2 *)alt, skin, type_bits, tpa, cap, npad, nbr, ncount,
-                           keys, cellidx, cstart, (const double2 *)xs, dsort, nent, gflag,
-                           work, wslice);
+        PARM_BR(2, double2);
     }
+#undef PARM_BR
+#undef PARM_BB
     return hipGetLastError();
 }
 

@@ -287,7 +287,8 @@ int brebuild(parm_batch *b, bool force, bool count, const void *pos,
                                 count ? 1 : 0, b->skin, b->type_bits, b->tpa, b->cap,
                                 b->npad, b->nbr, b->ncount, b->keys, b->cellidx, b->cstart,
                                 b->xs, b->dsort, b->flags, b->which, b->nent, b->gflag,
-                                b->work, b->wslice, b->sort_grid, b->build_grid, b->stream));
+                                b->work, b->wslice, b->sort_grid, b->build_grid,
+                                b->ntot * 3.0 <= 20.0 * b->total_cells, b->stream));
     return PARM_OK;
 }
 

@@ -274,7 +274,8 @@ hipError_t launch_batch_skin(int nsys, const BatchArrays &A, double skin, uint32
 // Rebuilds the systems whose skin flag is set (all with force): worklist,
 // sort, then the list build spread over slices of the listed systems.
 // work: nsys + 1 ints (count, then system ids); wslice: nsys + 1 ints (each
-// listed system's first build slice, then the total).  nent: per system the
+// listed system's first build slice, then the total).  sparse: few atoms per
+// stencil row (the build's lanes per atom).  nent: per system the
 // list entries of its last build (twice its pairs).
 hipError_t launch_batch_rebuild(int ndim, int nsys, const BatchArrays &A, const void *pos,
                                 const void *alt, int force, int count_rebuild, double skin,
@@ -283,7 +284,7 @@ hipError_t launch_batch_rebuild(int ndim, int nsys, const BatchArrays &A, const 
                                 int32_t *cstart, void *xs, double *dsort, uint32_t *flags,
                                 uint32_t *which, unsigned long long *nent, uint32_t *gflag,
                                 int32_t *work, int32_t *wslice, int sort_grid, int build_grid,
-                                hipStream_t s);
+                                bool sparse, hipStream_t s);
 hipError_t launch_batch_sys_sums(int nsys, const BatchArrays &A, const double *eatom,
                                  double *out, hipStream_t s);
 constexpr int kBatchMaxCellsPerSystem = 4096;
