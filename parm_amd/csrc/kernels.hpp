@@ -211,11 +211,15 @@ hipError_t launch_force(int ndim, int precision, int stage, bool energy,
 // (dimension, precision, pair kind, one pair type or several; no pair kind
 // yet gets the largest staging).
 size_t tiled_force_lds(int ndim, int prec, int kind, bool single, int smax);
-// Tiled force launch (step_tiled.hip); same contract as launch_force.
-hipError_t launch_force_tiled(int ndim, int precision, int stage, bool energy,
-                              const AtomArrays &A, const ListView &Lv, const PairView &P,
-                              const Box &box, const StepCoef &c, const ReduceBuf &R,
-                              hipStream_t s);
+// The force launches of one dimension, pair kind and precision: over the
+// untiled list (force.hip) and the tiled one (step_tiled.hip).
+template <int D, int KIND, int PREC>
+void force_part(int stage, bool energy, const AtomArrays &A, const ListView &Lv,
+                const PairView &P, const Box &box, const StepCoef &c, const ReduceBuf &R,
+                hipStream_t s);
+template <int D, int KIND, int PREC>
+void force_tiled_part(int stage, const AtomArrays &A, const ListView &Lv, const PairView &P,
+                      const Box &box, const StepCoef &c, const ReduceBuf &R, hipStream_t s);
 // k_finalize over nparts workgroup partials.
 hipError_t launch_finalize_rt(bool sums, bool skin, int nparts, const ReduceBuf &R,
                               hipStream_t s);
@@ -263,6 +267,11 @@ struct BatchArrays {
     const BatchGeom *geom; // per system
 };
 
+// The batched force launches of one dimension, pair kind and precision
+// (batch_force.hip).
+template <int D, int KIND, int PREC>
+void batch_force_part(int stage, bool energy, const BatchArrays &A, const ListView &Lv,
+                      const PairView &P, const StepCoef &c, double *eatom, hipStream_t s);
 hipError_t launch_batch_force(int ndim, int precision, int stage, bool energy,
                               const BatchArrays &A, const ListView &Lv, const PairView &P,
                               const StepCoef &c, double *eatom, hipStream_t s);

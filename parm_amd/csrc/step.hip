@@ -1,22 +1,12 @@
-// step.hip -- pair forces over the device Verlet list, fused with the
-// velocity-Verlet / damped-Verlet update and the skin test.
+// step.hip -- the per-atom step kernels (drift, skin test, observables, state
+// transfers), the reductions of workgroup partials, and the dispatch of the
+// force launches (force.hip, step_tiled.hip).
 //
 // Reference behaviour restated (paths relative to the reference root):
-//   NListed<A,P>::set_forces / energy / pressure / stress
-//                                   src/interaction.hpp:2153-2291
-//   LJAttractRepulsePair::forces/energy  src/interaction.hpp:1270-1298
-//   RepulsionPair::forces/energy         src/interaction.hpp:1538-1556
 //   Collection::set_forces               src/collection.cpp:159-179
 //   CollectionVerlet::timestep           src/collection.cpp:442-469
 //   CollectionDamped::timestep           src/collection.cpp:356-381
 //   NeighborList::update_list skin test  src/trackers.cpp:23-53
-//
-// The device list is a FULL list (each pair appears in both atoms' rows), so
-// each thread gathers the force on its own atom without atomics and in a
-// fixed order.  The per-pair force from j on i uses r = diff(x_i, x_j); the
-// visit from j computes -r bit for bit, so the two visits are exact negatives
-// and only the summation order differs from the reference's half-list
-// scatter.  Energies, virials and contact counts are halved.
 #include <algorithm>
 
 #include "common.hpp"
@@ -213,94 +203,6 @@ static void launch_finalize(int nparts, const ReduceBuf &R, hipStream_t s) {
     hipLaunchKernelGGL((k_finalize<SUMS, SKIN>), dim3(1), dim3(kFinal), 0, s, nparts, R);
 }
 
-// TPA lanes share one atom: lane `sub` visits list entries sub, sub + TPA, ...
-// The list is stored in groups of TPA entries per atom (entry q of slot i at
-// ((q / TPA) * npad + i) * TPA + q % TPA), so the 64 lanes of a wave read
-// 64 consecutive words per step of the loop.  Two entries per lane are in
-// flight at a time (both list words, then both position gathers) to hide
-// memory latency.  The TPA partial forces are summed with a fixed butterfly,
-// so the result is deterministic.
-template <int D, int KIND, int PREC, bool SINGLE, bool HARM, int STAGE, bool ENERGY,
-          int TPA>
-__global__ __launch_bounds__(kBlock) void k_force(AtomArrays A, ListView Lv,
-                                                  PairView P, Box box, StepCoef c,
-                                                  ReduceBuf R) {
-    using PT = typename PosStore<D>::T;
-    const int gt = xcd_block(blockIdx.x, gridDim.x) * kBlock + threadIdx.x;
-    const int i = gt / TPA;
-    const int sub = gt % TPA;
-    const bool act = i < A.n;
-    PairAcc acc;
-    double fi[D];
-    float f32[D];
-#pragma unroll
-    for (int k = 0; k < D; k++) {
-        fi[k] = 0.0;
-        f32[k] = 0.0f;
-    }
-
-    const PT *pos = static_cast<const PT *>(A.pos_in);
-    Vec<D> xi;
-    if (act) xi = PosStore<D>::load(pos[i]);
-    // the integrator inputs of the atom, loaded now to arrive during the
-    // pair loop (lane sub == 0 applies the stage)
-    AtomIn<D> ain;
-    if (act && sub == 0) atom_load<D, STAGE, false>(A, i, ain);
-    const bool member = act && A.rank[i] >= 0;
-    if (member && Lv.built) {
-        // lane sub's entries m = 0 .. nl-1 sit at (m * npad + i) * TPA + sub
-        const int nl = Lv.lcount[(size_t)i * TPA + sub];
-        const size_t stride = (size_t)Lv.npad * TPA;
-        const uint32_t *nb = Lv.nbr + (size_t)i * TPA + sub;
-        const int tb = Lv.type_bits;
-        const uint32_t tmask = (1u << tb) - 1u;
-        const PairParam *row = P.tab;
-        PairParam p0;
-        if (SINGLE)
-            p0 = P.p0;
-        else
-            row = P.tab + (size_t)A.type[i] * P.ntypes;
-        int m = 0;
-        size_t off = 0;
-        for (; m + 1 < nl; m += 2, off += 2 * stride) {
-            const uint32_t e0 = nb[off];
-            const uint32_t e1 = nb[off + stride];
-            const PT pj0 = pos[e0 >> tb];
-            const PT pj1 = pos[e1 >> tb];
-            const Vec<D> r0 = diff<D>(xi, PosStore<D>::load(pj0), box);
-            visit<D, KIND, PREC, ENERGY, HARM>(SINGLE ? p0 : row[e0 & tmask], r0, fi,
-                                               f32, acc);
-            const Vec<D> r1 = diff<D>(xi, PosStore<D>::load(pj1), box);
-            visit<D, KIND, PREC, ENERGY, HARM>(SINGLE ? p0 : row[e1 & tmask], r1, fi,
-                                               f32, acc);
-        }
-        if (m < nl) {
-            const uint32_t e0 = nb[off];
-            const Vec<D> r0 = diff<D>(xi, PosStore<D>::load(pos[e0 >> tb]), box);
-            visit<D, KIND, PREC, ENERGY, HARM>(SINGLE ? p0 : row[e0 & tmask], r0, fi,
-                                               f32, acc);
-        }
-    }
-    if (PREC != kFP64) {
-#pragma unroll
-        for (int k = 0; k < D; k++) fi[k] = (double)f32[k];
-    }
-    // sum the TPA partial forces of the atom (all lanes take part)
-#pragma unroll
-    for (int o = 1; o < TPA; o <<= 1) {
-#pragma unroll
-        for (int k = 0; k < D; k++) fi[k] += __shfl_xor(fi[k], o);
-    }
-
-    Top2 top;
-    double nonfinite = 0.0;
-    if (act && sub == 0) {
-        ain.x = xi;
-        atom_store<D, STAGE>(A, i, fi, ain, c, top, nonfinite);
-    }
-    group_partials<D, STAGE, ENERGY, kBlock / kWave>(acc, top, nonfinite, R);
-}
-
 // Standalone first half of a step (drift + half kick) and skin test.
 template <int D, bool DAMPED>
 __global__ __launch_bounds__(kBlock) void k_drift(AtomArrays A, StepCoef c,
@@ -434,114 +336,6 @@ __global__ __launch_bounds__(kBlock) void k_download(AtomArrays A, int what,
 int reduce_blocks(int n) { return n <= 0 ? 1 : (n + kBlock - 1) / kBlock; }
 int force_blocks(int n, int tpa) { return reduce_blocks(n * tpa); }
 
-template <int D, int KIND, int PREC, bool SINGLE, bool HARM, int STAGE, int TPA>
-static void launch_force_tt(bool energy, const AtomArrays &A, const ListView &Lv,
-                            const PairView &P, const Box &box, const StepCoef &c,
-                            const ReduceBuf &R, hipStream_t s) {
-    constexpr bool DRIFT =
-        (STAGE == kStageVerletKickDrift || STAGE == kStageDampedKickDrift);
-    // energies are accumulated by the sums stage only
-    constexpr bool ENERGY = STAGE == kStageSums;
-    (void)energy;
-    const int nb = force_blocks(A.n, TPA);
-    dim3 g(nb), b(kBlock);
-    hipLaunchKernelGGL((k_force<D, KIND, PREC, SINGLE, HARM, STAGE, ENERGY, TPA>), g, b, 0,
-                       s, A, Lv, P, box, c, R);
-    if (R.done) (void)hipEventRecord(R.done, s);
-    if (ENERGY || DRIFT) launch_finalize<ENERGY, DRIFT>(nb, R, s);
-}
-
-template <int D, int KIND, int PREC, bool SINGLE, bool HARM, int STAGE>
-static void launch_force_t(bool energy, const AtomArrays &A, const ListView &Lv,
-                           const PairView &P, const Box &box, const StepCoef &c,
-                           const ReduceBuf &R, hipStream_t s) {
-    switch (Lv.tpa) {
-    case 1:
-        launch_force_tt<D, KIND, PREC, SINGLE, HARM, STAGE, 1>(energy, A, Lv, P, box, c,
-                                                               R, s);
-        break;
-    case 2:
-        launch_force_tt<D, KIND, PREC, SINGLE, HARM, STAGE, 2>(energy, A, Lv, P, box, c,
-                                                               R, s);
-        break;
-    case 8:
-        launch_force_tt<D, KIND, PREC, SINGLE, HARM, STAGE, 8>(energy, A, Lv, P, box, c,
-                                                               R, s);
-        break;
-    default:
-        launch_force_tt<D, KIND, PREC, SINGLE, HARM, STAGE, 4>(energy, A, Lv, P, box, c,
-                                                               R, s);
-        break;
-    }
-}
-
-template <int D, int KIND, int PREC, bool SINGLE, bool HARM>
-static void launch_force_s(int stage, bool energy, const AtomArrays &A,
-                           const ListView &Lv, const PairView &P, const Box &box,
-                           const StepCoef &c, const ReduceBuf &R, hipStream_t s) {
-    switch (stage) {
-#define PARM_STAGE(S)                                                          \
-    case S:                                                                    \
-        launch_force_t<D, KIND, PREC, SINGLE, HARM, S>(energy, A, Lv, P, box,  \
-                                                       c, R, s);               \
-        break;
-        PARM_STAGE(kStageForceOnly)
-        PARM_STAGE(kStageForceA)
-        PARM_STAGE(kStageVerletKick)
-        PARM_STAGE(kStageVerletKickDrift)
-        PARM_STAGE(kStageDampedKick)
-        PARM_STAGE(kStageDampedKickDrift)
-        PARM_STAGE(kStageSums)
-        PARM_STAGE(kStageForceAdd)
-#undef PARM_STAGE
-    }
-}
-
-template <int D, int KIND, int PREC>
-static void launch_force_k(int stage, bool energy, const AtomArrays &A,
-                           const ListView &Lv, const PairView &P, const Box &box,
-                           const StepCoef &c, const ReduceBuf &R, hipStream_t s) {
-    if constexpr (KIND == kPairRepulsion) {
-        if (P.harmonic) {
-            if (P.single)
-                launch_force_s<D, KIND, PREC, true, true>(stage, energy, A, Lv, P, box,
-                                                          c, R, s);
-            else
-                launch_force_s<D, KIND, PREC, false, true>(stage, energy, A, Lv, P, box,
-                                                           c, R, s);
-            return;
-        }
-    }
-    {
-        if (P.single)
-            launch_force_s<D, KIND, PREC, true, false>(stage, energy, A, Lv, P, box,
-                                                       c, R, s);
-        else
-            launch_force_s<D, KIND, PREC, false, false>(stage, energy, A, Lv, P, box,
-                                                        c, R, s);
-    }
-}
-
-template <int D>
-static void launch_force_d(int precision, int stage, bool energy, const AtomArrays &A,
-                           const ListView &Lv, const PairView &P, const Box &box,
-                           const StepCoef &c, const ReduceBuf &R, hipStream_t s) {
-    if (P.kind == kPairRepulsion) {
-        if (precision == kFP64)
-            launch_force_k<D, kPairRepulsion, kFP64>(stage, energy, A, Lv, P, box, c,
-                                                     R, s);
-        else
-            launch_force_k<D, kPairRepulsion, kMixed>(stage, energy, A, Lv, P, box,
-                                                      c, R, s);
-    } else {
-        if (precision == kFP64)
-            launch_force_k<D, kPairLJ, kFP64>(stage, energy, A, Lv, P, box, c, R, s);
-        else
-            launch_force_k<D, kPairLJ, kMixed>(stage, energy, A, Lv, P, box, c, R,
-                                               s);
-    }
-}
-
 hipError_t launch_finalize_rt(bool sums, bool skin, int nparts, const ReduceBuf &R,
                               hipStream_t s) {
     if (sums && skin)
@@ -553,18 +347,51 @@ hipError_t launch_finalize_rt(bool sums, bool skin, int nparts, const ReduceBuf 
     return hipGetLastError();
 }
 
+size_t tiled_force_lds(int ndim, int prec, int kind, bool single, int smax) {
+    const bool raw = prec == kFP64 && kind == kPairRepulsion;
+    const bool rel32 = prec != kFP64 && kind == kPairLJ;
+    if (raw) return (size_t)smax * sizeof(double4);
+    if (single && kind != kPairNone)
+        return (size_t)smax * ndim * (rel32 ? sizeof(float) : sizeof(double));
+    if (rel32) return (size_t)smax * (sizeof(float4) + sizeof(int32_t));
+    return (size_t)smax * (sizeof(double4) + sizeof(int32_t));
+}
+
+// F(D, KIND, PREC) for the runtime dimension, pair kind and precision.
+#define PARM_DISPATCH(F)                                                          \
+    do {                                                                          \
+        const bool rep = P.kind == kPairRepulsion, dbl = precision == kFP64;      \
+        if (ndim == 3) {                                                          \
+            if (rep) {                                                            \
+                if (dbl) F(3, kPairRepulsion, kFP64); else F(3, kPairRepulsion, kMixed); \
+            } else {                                                              \
+                if (dbl) F(3, kPairLJ, kFP64); else F(3, kPairLJ, kMixed);        \
+            }                                                                     \
+        } else {                                                                  \
+            if (rep) {                                                            \
+                if (dbl) F(2, kPairRepulsion, kFP64); else F(2, kPairRepulsion, kMixed); \
+            } else {                                                              \
+                if (dbl) F(2, kPairLJ, kFP64); else F(2, kPairLJ, kMixed);        \
+            }                                                                     \
+        }                                                                         \
+    } while (0)
+
 hipError_t launch_force(int ndim, int precision, int stage, bool energy,
                         const AtomArrays &A, const ListView &Lv, const PairView &P,
                         const Box &box, const StepCoef &c, const ReduceBuf &R,
                         hipStream_t s) {
     if (energy != (stage == kStageSums)) return hipErrorInvalidValue;
     if (A.n <= 0) return hipSuccess;
-    if (Lv.tiled && Lv.built)
-        return launch_force_tiled(ndim, precision, stage, energy, A, Lv, P, box, c, R, s);
-    if (ndim == 3)
-        launch_force_d<3>(precision, stage, energy, A, Lv, P, box, c, R, s);
-    else
-        launch_force_d<2>(precision, stage, energy, A, Lv, P, box, c, R, s);
+    if (Lv.tiled && Lv.built) {
+        if (Lv.ntiles <= 0) return hipSuccess;
+#define PARM_F(D, K, Q) force_tiled_part<D, K, Q>(stage, A, Lv, P, box, c, R, s)
+        PARM_DISPATCH(PARM_F);
+#undef PARM_F
+    } else {
+#define PARM_F(D, K, Q) force_part<D, K, Q>(stage, energy, A, Lv, P, box, c, R, s)
+        PARM_DISPATCH(PARM_F);
+#undef PARM_F
+    }
     return hipGetLastError();
 }
 

@@ -544,16 +544,6 @@ __global__ __launch_bounds__(kWave *TPA) void k_force_tiled(AtomArrays A, ListVi
 }
 
 // ======================================================== host launchers
-size_t tiled_force_lds(int ndim, int prec, int kind, bool single, int smax) {
-    const bool raw = prec == kFP64 && kind == kPairRepulsion;
-    const bool rel32 = prec != kFP64 && kind == kPairLJ;
-    if (raw) return (size_t)smax * sizeof(double4);
-    if (single && kind != kPairNone)
-        return (size_t)smax * ndim * (rel32 ? sizeof(float) : sizeof(double));
-    if (rel32) return (size_t)smax * (sizeof(float4) + sizeof(int32_t));
-    return (size_t)smax * (sizeof(double4) + sizeof(int32_t));
-}
-
 namespace {
 
 template <int D, int KIND, int PREC, bool SINGLE, bool HARM, int STAGE, int TPA>
@@ -626,36 +616,17 @@ void tiled_k(int stage, const AtomArrays &A, const ListView &Lv, const PairView 
         tiled_s<D, KIND, PREC, false, false>(stage, A, Lv, P, box, c, R, s);
 }
 
-template <int D>
-void tiled_d(int precision, int stage, const AtomArrays &A, const ListView &Lv,
-             const PairView &P, const Box &box, const StepCoef &c, const ReduceBuf &R,
-             hipStream_t s) {
-    if (P.kind == kPairRepulsion) {
-        if (precision == kFP64)
-            tiled_k<D, kPairRepulsion, kFP64>(stage, A, Lv, P, box, c, R, s);
-        else
-            tiled_k<D, kPairRepulsion, kMixed>(stage, A, Lv, P, box, c, R, s);
-    } else {
-        if (precision == kFP64)
-            tiled_k<D, kPairLJ, kFP64>(stage, A, Lv, P, box, c, R, s);
-        else
-            tiled_k<D, kPairLJ, kMixed>(stage, A, Lv, P, box, c, R, s);
-    }
-}
-
 }  // namespace
 
-hipError_t launch_force_tiled(int ndim, int precision, int stage, bool energy,
-                              const AtomArrays &A, const ListView &Lv, const PairView &P,
-                              const Box &box, const StepCoef &c, const ReduceBuf &R,
-                              hipStream_t s) {
-    if (energy != (stage == kStageSums)) return hipErrorInvalidValue;
-    if (A.n <= 0 || Lv.ntiles <= 0) return hipSuccess;
-    if (ndim == 3)
-        tiled_d<3>(precision, stage, A, Lv, P, box, c, R, s);
-    else
-        tiled_d<2>(precision, stage, A, Lv, P, box, c, R, s);
-    return hipGetLastError();
+// One dimension, pair kind and precision per object file (PARM_PART, set by
+// the Makefile), so that the instantiations compile side by side.
+template <int D, int KIND, int PREC>
+void force_tiled_part(int stage, const AtomArrays &A, const ListView &Lv, const PairView &P,
+                      const Box &box, const StepCoef &c, const ReduceBuf &R, hipStream_t s) {
+    tiled_k<D, KIND, PREC>(stage, A, Lv, P, box, c, R, s);
 }
+template void force_tiled_part<PARM_PART_D, PARM_PART_KIND, PARM_PART_PREC>(
+    int, const AtomArrays &, const ListView &, const PairView &, const Box &, const StepCoef &,
+    const ReduceBuf &, hipStream_t);
 
 }  // namespace parm
