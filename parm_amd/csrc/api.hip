@@ -79,10 +79,13 @@ void dfree(T *&p) {
 }  // namespace
 
 constexpr int kFlagRing = 4;
-// flag words: [0, kFlagRing) step ring, then the list-build overflow flag, a
+// flag words: [0, kFlagRing) the step loop's skin tests (by step number), then the list-build overflow flag, a
 // scratch word for reductions that raise no flag, and the on-demand skin test
 // dynamic LDS of one tiled build workgroup, at most (the stencil's atoms)
 constexpr size_t kTiledLdsMax = 56 * 1024;
+// run-ahead of the step loop (step_runahead)
+constexpr int kRunAhead = 2, kRunAheadAtoms = 1 << 15;
+static_assert(kRunAhead + 1 < kFlagRing, "a flag word is not reused while a launch may read it");
 constexpr int kSlotBuild = kFlagRing + 1, kSlotScratch = kFlagRing + 2,
               kSlotSkin = kFlagRing + 3;
 
@@ -164,8 +167,8 @@ struct parm_system {
     uint32_t *hflag = nullptr;      // pinned mirror, written by the kernels
     uint32_t *hflag_dev = nullptr;  // its device-side address
     double *hout = nullptr;         // pinned mirror of out
-    hipEvent_t ev_flag = nullptr;
-    hipEvent_t ev_ring[kFlagRing] = {};
+    double *part2 = nullptr;        // the step loop's skin partials alternate: part, part2
+    uint32_t step_seq = 0;          // sequence number of the last step flag asked for
 
     // asynchronous snapshots for output: a ring of device staging buffers
     // and pinned host copies, filled on the system's stream and copied to the
@@ -634,7 +637,7 @@ int update_list(parm_system *s, bool force, int *rebuilt) {
     if (rebuilt) *rebuilt = 0;
     if (!s->list_cfg) return fail(PARM_E_STATE, "neighbour list not configured");
     if (!force && !s->ignorechanged) {
-        PARM_HIP(launch_skin(s->ndim, s->arrays(), s->redbuf(kSlotSkin), s->stream));
+        PARM_HIP(launch_skin(s->ndim, s->arrays(), s->redbuf(kSlotSkin), true, s->stream));
         uint32_t fl = 0;
         PARM_CHECK(read_flag(s, kSlotSkin, &fl));
         if (fl & kFlagNonFinite)
@@ -798,24 +801,55 @@ int autotune(parm_system *s, int stage, const StepCoef &c) {
     return PARM_OK;
 }
 
-// Records the ring event of flag slot q: the launch just queued stores the
-// slot in the pinned mirror (an empty system launches nothing: the slot is
-// cleared here).
-int post_flag(parm_system *s, int slot) {
-    if (s->n == 0) s->hflag[slot] = 0;
-    PARM_HIP(hipEventRecord(s->ev_ring[slot], s->stream));
-    return PARM_OK;
+// Waits for the pinned word that a step launch's reduction stores for
+// sequence number seq (24 bits of it above the flag bits); *flag = its flags.
+// The stream's state is asked for now and then, so the wait ends also when
+// the device reports an error or the stream drains without the word.
+int wait_step_flag(parm_system *s, int slot, uint32_t seq, uint32_t *flag) {
+    const volatile uint32_t *w = s->hflag + slot;
+    const uint32_t want = seq & (0xffffffffu >> kFlagBits);
+    bool drained = false;
+    for (;;) {
+        for (int k = 0; k < 1 << 14; k++) {
+            const uint32_t v = *w;
+            if ((v >> kFlagBits) == want) {
+                *flag = v & ((1u << kFlagBits) - 1u);
+                return PARM_OK;
+            }
+            __builtin_ia32_pause();
+        }
+        if (drained) return fail(PARM_E_DEVICE, "a step's skin test did not report");
+        const hipError_t e = hipStreamQuery(s->stream);
+        if (e == hipSuccess)
+            drained = true;  // one more look: the word was stored before the drain
+        else if (e != hipErrorNotReady)
+            return fail(PARM_E_DEVICE, std::string("step loop: ") + hipGetErrorString(e));
+    }
 }
+
+// Step launches queued beyond the oldest one whose flag the host waits for.
+// Small systems: a launch takes a few microseconds, less than a flag's trip to
+// the host and the launch that answers it, so the queue has to run ahead.
+// Large ones: the flag arrives early in a launch that has long to run, and a
+// launch queued in vain (its workgroups start and stop) would cost more than
+// it hides.  Depth 1 / 2 / 3 / 4, us for 200 - 60 steps: 1000 atoms 2437 / 2388 /
+// 2398 / 2407, 2003 disks 4644 / 4298 / 4320 / 4446, 20,011 spheres 4984 / 4843
+// / 4802 / 4941, 48,611 atoms 2146 / 2157 / 2172 / 2177, 1M atoms 12324 / 12451
+// / 12600 / 12664.
+int step_runahead(const parm_system *s) { return s->n <= kRunAheadAtoms ? kRunAhead : 1; }
 
 // nsteps x timestep() of CollectionVerlet / CollectionDamped, fused.
 //
 // The reference step is: drift (first loop), set_forces, kick (second loop),
 // update_trackers (skin test -> maybe rebuild).  Here one kernel per step does
 // the force + kick of step q AND the drift of step q+1 into the alternate
-// position buffer, plus the skin test of those drifted positions.  The list
-// decision for the end of step q needs the skin test of x_{q+1}, which the
-// previous kernel produced: the host waits for that flag while the current
-// kernel runs.  A rebuild at x_{q+1} permutes both position buffers and
+// position buffer, and leaves the skin-test partials of those drifted
+// positions.  Launch q reduces the partials of x_{q+1}, left by launch q - 1,
+// and raises flag q from them: the list decision for the end of step q, which
+// has to be carried out before the forces of step q+1.  Launch q+1 reads flag
+// q on the device and does nothing when it is set, so the host queues launches
+// before it knows the flags; when flag q is set it starts again from launch
+// q+1 after the rebuild at x_{q+1}, which permutes both position buffers and
 // re-tests x_{q+2} against the new reference positions.  The last step runs
 // force + kick only, so the state returned is at a full step.
 int run_steps(parm_system *s, bool damped, const StepCoef &c, int64_t nsteps) {
@@ -825,48 +859,92 @@ int run_steps(parm_system *s, bool damped, const StepCoef &c, int64_t nsteps) {
     const int kick_drift = damped ? kStageDampedKickDrift : kStageVerletKickDrift;
     if (nsteps >= 16) PARM_CHECK(autotune(s, kick_drift, c));
     hipStream_t st = s->stream;
+    // partials of x_{q+1} (written by launch q - 1) in buffer q & 1
+    double *pbuf[2] = {s->part, s->part2};
+    int npart[2] = {reduce_blocks(s->n), 0};
     // first half of step 0
-    PARM_HIP(launch_drift(s->ndim, kick, s->arrays(), c, s->redbuf(0), st));
-    PARM_CHECK(post_flag(s, 0));
+    {
+        ReduceBuf R = s->redbuf(kSlotScratch);
+        R.part = pbuf[0];
+        PARM_HIP(launch_drift(s->ndim, kick, s->arrays(), c, R, st));
+    }
+    if (s->n == 0) {
+        // no launches and no flags: only a pending forced update
+        if (s->ignorechanged) PARM_CHECK(rebuild(s));
+        return PARM_OK;
+    }
+    // launch q reads x_{q+1} from xb[q & 1] and writes x_{q+2} to the other
+    void *xb[2] = {s->pos, s->pos_alt};
+    uint32_t seq[kFlagRing];
+    size_t nprof[kFlagRing];  // step events recorded once launch q was queued
+    const int ahead = step_runahead(s);
+    int64_t queued = 0;
+    bool gated = false;  // launch `queued` checks the flag before it
     for (int64_t q = 0; q < nsteps; q++) {
-        const bool last = (q == nsteps - 1);
-        const int slot = (int)(q % kFlagRing), next = (int)((q + 1) % kFlagRing);
-        if (!last) {
-            {
+        // queue launches up to q + ahead (none past q while a forced rebuild
+        // is due at its end)
+        while (queued < nsteps && queued < q + ahead && !(s->ignorechanged && queued > q)) {
+            const bool last = (queued == nsteps - 1);
+            const int cur = (int)(queued & 1), slot = (int)(queued % kFlagRing);
+            AtomArrays A = s->arrays();
+            A.pos_in = xb[cur];
+            A.pos_out = last ? xb[cur] : xb[1 - cur];
+            ReduceBuf R = s->redbuf(kSlotScratch);
+            R.part = pbuf[1 - cur];
+            R.g.prev = pbuf[cur];
+            R.g.nprev = npart[cur];
+            R.g.gate = gated ? s->dflag + (queued + kFlagRing - 1) % kFlagRing : nullptr;
+            R.g.flag = s->dflag + slot;
+            R.g.hflag = s->hflag_dev + slot;
+            R.g.seq = seq[slot] = ++s->step_seq;
+            const ListView Lv = s->listview();
+            if (!last) {
                 ProfScope ps(s, &s->prof_step, s->prof_seq++ % s->prof_every == 0);
-                ReduceBuf R = s->redbuf(next);
                 R.done = ps.end();
-                PARM_HIP(launch_force(s->ndim, s->prec, kick_drift, false,
-                                      s->arrays(true), s->listview(), s->pairview(),
+                PARM_HIP(launch_force(s->ndim, s->prec, kick_drift, false, A, Lv,
+                                      s->pairview(), s->box, c, R, st));
+                npart[1 - cur] = force_partials(s->n, Lv);
+            } else {
+                PARM_HIP(launch_force(s->ndim, s->prec, kick, false, A, Lv, s->pairview(),
                                       s->box, c, R, st));
             }
-            PARM_CHECK(post_flag(s, next));
-        } else {
-            PARM_HIP(launch_force(s->ndim, s->prec, kick, false, s->arrays(),
-                                  s->listview(), s->pairview(), s->box, c,
-                                  s->redbuf(kSlotScratch), st));
+            nprof[slot] = s->prof_step.size();
+            gated = true;
+            queued++;
         }
         // update_trackers at the end of step q: skin test of x_{q+1}
-        PARM_HIP(hipEventSynchronize(s->ev_ring[slot]));
-        const uint32_t fl = *(volatile uint32_t *)(s->hflag + slot);
+        const bool last = (q == nsteps - 1);
+        const int cur = (int)(q & 1), slot = (int)(q % kFlagRing);
+        uint32_t fl = 0;
+        PARM_CHECK(wait_step_flag(s, slot, seq[slot], &fl));
+        s->pos = xb[cur];
+        s->pos_alt = xb[1 - cur];
         if (fl & kFlagNonFinite)
             return fail(PARM_E_NONFINITE,
                         "position became non-finite at step " + std::to_string(q));
         if ((fl & kFlagRebuild) || s->ignorechanged) {
+            // the launches queued past q did nothing: queue them again
+            s->prof_seq -= std::max<int64_t>(0, std::min(queued, nsteps - 1) - (q + 1));
+            s->prof_step.resize(nprof[slot]);
+            queued = q + 1;
+            gated = false;
             {
                 ProfScope ps(s, &s->prof_rebuild);
                 // before the last step's end the next launch rewrites a and
                 // f before anything reads them: they need no permutation
                 PARM_CHECK(rebuild(s, last));
             }
+            xb[cur] = s->pos;
+            xb[1 - cur] = s->pos_alt;
             if (!last) {
                 AtomArrays A = s->arrays();
                 A.pos_in = s->pos_alt;
-                PARM_HIP(launch_skin(s->ndim, A, s->redbuf(next), st));
-                PARM_CHECK(post_flag(s, next));
+                ReduceBuf R = s->redbuf(kSlotScratch);
+                R.part = pbuf[1 - cur];
+                PARM_HIP(launch_skin(s->ndim, A, R, false, st));
+                npart[1 - cur] = reduce_blocks(s->n);
             }
         }
-        if (!last) std::swap(s->pos, s->pos_alt);
     }
     return PARM_OK;
 }
@@ -954,6 +1032,7 @@ void destroy(parm_system *s) {
     dfree(s->ex_off);
     dfree(s->ex_part);
     dfree(s->part);
+    dfree(s->part2);
     dfree(s->out);
     dfree(s->fcnt);
     dfree(s->fgpart);
@@ -971,9 +1050,6 @@ void destroy(parm_system *s) {
         (void)hipStreamSynchronize(s->out_stream);
         (void)hipStreamDestroy(s->out_stream);
     }
-    if (s->ev_flag) (void)hipEventDestroy(s->ev_flag);
-    for (hipEvent_t &e : s->ev_ring)
-        if (e) (void)hipEventDestroy(e);
     for (hipEvent_t e : s->ev_pool) (void)hipEventDestroy(e);
     if (s->stream) (void)hipStreamDestroy(s->stream);
     delete s;
@@ -1116,11 +1192,6 @@ int parm_system_create(int ndim, int precision, int64_t natoms, const double *ma
                                             : (size_t)0);
     if (hipStreamCreateWithFlags(&s->stream, hipStreamNonBlocking) != hipSuccess)
         return bail(fail(PARM_E_DEVICE, "stream creation failed"));
-    if (hipEventCreateWithFlags(&s->ev_flag, hipEventDisableTiming) != hipSuccess)
-        return bail(fail(PARM_E_DEVICE, "event creation failed"));
-    for (hipEvent_t &e : s->ev_ring)
-        if (hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess)
-            return bail(fail(PARM_E_DEVICE, "event creation failed"));
     const size_t n = (size_t)std::max(1, s->n);
     if ((rc = dalloc((char **)&s->pos, n * s->pos_bytes)) ||
         (rc = dalloc((char **)&s->pos_alt, n * s->pos_bytes)) ||
@@ -1147,6 +1218,7 @@ int parm_system_create(int ndim, int precision, int64_t natoms, const double *ma
         (rc = dalloc(&s->stats, 2)) ||
         (rc = dalloc(&s->bpart, 2 * (size_t)build_blocks((int)n))) ||
         (rc = dalloc(&s->part, (size_t)kRedWidth * force_blocks((int)n, 8))) ||
+        (rc = dalloc(&s->part2, (size_t)kRedWidth * force_blocks((int)n, 8))) ||
         (rc = dalloc(&s->out, kRedWidth)) || (rc = dalloc(&s->fcnt, 1)) ||
         (rc = dalloc(&s->fgpart, 3 * kFinBlocks)) ||
         (rc = dalloc(&s->dflag, 2 * kFlagRing + 4)) || (rc = dalloc(&s->tinfo, 4)))

@@ -307,6 +307,8 @@ enum : uint32_t {
     kFlagNonFinite = 2u,    // a displacement was NaN/Inf
     kFlagOverflow = 4u,     // neighbour capacity exceeded during a build
     kFlagReplan = 8u,       // a speculative tiled build met a tile its bounds do not fit
+    kFlagStopped = 16u,     // a step launch that an earlier test's flag stopped
 };
+constexpr int kFlagBits = 8;  // flag bits of a host word; a sequence number above them
 
 }  // namespace parm

@@ -36,7 +36,17 @@ __global__ __launch_bounds__(kBlock) void k_force(AtomArrays A, ListView Lv,
                                                   PairView P, Box box, StepCoef c,
                                                   ReduceBuf R) {
     using PT = typename PosStore<D>::T;
-    const int gt = xcd_block(blockIdx.x, gridDim.x) * kBlock + threadIdx.x;
+    constexpr bool STEP = STAGE == kStageVerletKickDrift || STAGE == kStageDampedKickDrift ||
+                          STAGE == kStageVerletKick || STAGE == kStageDampedKick;
+    // a step launch's first workgroup reduces the previous launch's skin test
+    const int extra = STEP && R.g.nprev > 0 ? 1 : 0;
+    if (STEP && extra && blockIdx.x == 0) {
+        reduce_prev<kBlock / kWave>(R);
+        return;
+    }
+    if (STEP && step_stopped(R.g)) return;
+    const int blk = (int)blockIdx.x - extra;
+    const int gt = xcd_block(blk, (int)gridDim.x - extra) * kBlock + threadIdx.x;
     const int i = gt / TPA;
     const int sub = gt % TPA;
     const bool act = i < A.n;
@@ -108,7 +118,7 @@ __global__ __launch_bounds__(kBlock) void k_force(AtomArrays A, ListView Lv,
         ain.x = xi;
         atom_store<D, STAGE>(A, i, fi, ain, c, top, nonfinite);
     }
-    group_partials<D, STAGE, ENERGY, kBlock / kWave>(acc, top, nonfinite, R);
+    group_partials<D, STAGE, ENERGY, kBlock / kWave>(acc, top, nonfinite, R, blk);
 }
 
 template <int D, int KIND, int PREC, bool SINGLE, bool HARM, int STAGE, int TPA>
@@ -121,11 +131,12 @@ static void launch_force_tt(bool energy, const AtomArrays &A, const ListView &Lv
     constexpr bool ENERGY = STAGE == kStageSums;
     (void)energy;
     const int nb = force_blocks(A.n, TPA);
-    dim3 g(nb), b(kBlock);
+    constexpr bool STEP = DRIFT || STAGE == kStageVerletKick || STAGE == kStageDampedKick;
+    dim3 g(nb + (STEP && R.g.nprev > 0 ? 1 : 0)), b(kBlock);
     hipLaunchKernelGGL((k_force<D, KIND, PREC, SINGLE, HARM, STAGE, ENERGY, TPA>), g, b, 0,
                        s, A, Lv, P, box, c, R);
     if (R.done) (void)hipEventRecord(R.done, s);
-    if (ENERGY || DRIFT) (void)launch_finalize_rt(ENERGY, DRIFT, nb, R, s);
+    if (ENERGY) (void)launch_finalize_rt(true, false, nb, R, s);
 }
 
 template <int D, int KIND, int PREC, bool SINGLE, bool HARM, int STAGE>

@@ -187,6 +187,18 @@ struct StepCoef {
     double k0, k1, k2, k3, k4;
 };
 
+// The skin test of the launch before, reduced inside a step launch (one extra
+// workgroup) and the test before that, which may have stopped the run: see
+// step_gate / reduce_prev in stepcore.hpp.
+struct StepGate {
+    const double *prev;           // the previous launch's skin partials (fields as ReduceBuf::part)
+    int nprev;                    // their number (0: no reduction in this launch)
+    const uint32_t *gate;         // or null: flag word of the test one launch earlier
+    uint32_t *flag;               // device flag word of this reduction's test
+    uint32_t *hflag;              // device-visible pinned word: (seq << kFlagBits) | flags
+    uint32_t seq;
+};
+
 // Reduction scratch: one partial per workgroup, reduced by k_finalize.
 struct ReduceBuf {
     double *part;                 // kRedWidth fields x pstride workgroups
@@ -199,10 +211,13 @@ struct ReduceBuf {
                                   // after the force kernel, before its k_finalize (timing)
     uint32_t *cnt;                // or null: the skin-test reduction over several
     double *gpart;                // workgroups (counter, kFinBlocks x 3 results)
+    StepGate g;
 };
 constexpr int kFinBlocks = 32;    // workgroups of the multi-workgroup skin reduction
 constexpr int kRedWidth = 16;     // U, W, S[9], contacts, overlaps, top1, top2, nonfinite
 
+// A kick + drift stage leaves its skin-test partials (force_partials of them)
+// to the next step launch, whose ReduceBuf::g names them.
 hipError_t launch_force(int ndim, int precision, int stage, bool energy,
                         const AtomArrays &A, const ListView &Lv, const PairView &P,
                         const Box &box, const StepCoef &c, const ReduceBuf &R,
@@ -223,9 +238,11 @@ void force_tiled_part(int stage, const AtomArrays &A, const ListView &Lv, const 
 // k_finalize over nparts workgroup partials.
 hipError_t launch_finalize_rt(bool sums, bool skin, int nparts, const ReduceBuf &R,
                               hipStream_t s);
+// The drift leaves its skin-test partials (reduce_blocks(n) of them) to the
+// next step launch; launch_skin with finalize == false does the same.
 hipError_t launch_drift(int ndim, int stage, const AtomArrays &A, const StepCoef &c,
                         const ReduceBuf &R, hipStream_t s);
-hipError_t launch_skin(int ndim, const AtomArrays &A, const ReduceBuf &R,
+hipError_t launch_skin(int ndim, const AtomArrays &A, const ReduceBuf &R, bool finalize,
                        hipStream_t s);
 // Atom observables: mode 0 -> out[0] = K(originv), out[1..D] = momentum,
 // out[4] = mass ; mode 1 -> out[0] = sum |f|, out[13] = max |f|.
@@ -240,6 +257,7 @@ hipError_t launch_download(int ndim, int what, const AtomArrays &A,
                            const int32_t *orig, double *dst, hipStream_t s);
 int reduce_blocks(int n);
 int force_blocks(int n, int tpa);  // workgroups of a force launch (also partials)
+int force_partials(int n, const ListView &Lv);  // partials of a launch over this list
 
 // ---------------------------------------------------------------- batch.hip
 // Geometry of one system of a batch.

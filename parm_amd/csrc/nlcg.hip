@@ -116,7 +116,7 @@ __global__ __launch_bounds__(kBlock) void k_nlcg_vec(AtomArrays A, double beta, 
             v[4] = dotv<D>(w, w);
         }
     }
-    block_partial<true, false, kBlock / kWave>(v, Top2{}, R);
+    block_partial<true, false, kBlock / kWave>(v, Top2{}, R, blockIdx.x);
 }
 
 hipError_t launch_nlcg_stepx(int ndim, const AtomArrays &A, const double *lfac, double dx,

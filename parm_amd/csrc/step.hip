@@ -231,7 +231,7 @@ __global__ __launch_bounds__(kBlock) void k_drift(AtomArrays A, StepCoef c,
 #pragma unroll
     for (int k = 0; k < kRedWidth; k++) v[k] = 0.0;
     v[kNonFinite] = nonfinite;
-    block_partial<false, true, kBlock / kWave>(v, top, R);
+    block_partial<false, true, kBlock / kWave>(v, top, R, blockIdx.x);
 }
 
 // Skin test only (after a rebuild, or for update_list(false) on demand).
@@ -249,7 +249,7 @@ __global__ __launch_bounds__(kBlock) void k_skin(AtomArrays A, ReduceBuf R) {
 #pragma unroll
     for (int k = 0; k < kRedWidth; k++) v[k] = 0.0;
     v[kNonFinite] = nonfinite;
-    block_partial<false, true, kBlock / kWave>(v, top, R);
+    block_partial<false, true, kBlock / kWave>(v, top, R, blockIdx.x);
 }
 
 // Atom-wise observables (AtomGroup::kinetic_energy / momentum / mass,
@@ -290,7 +290,7 @@ __global__ __launch_bounds__(kBlock) void k_atom_sums(AtomArrays A, Vec<D> ov,
             top.add(fn);
         }
     }
-    block_partial<true, MODE == 1, kBlock / kWave>(v, top, R);
+    block_partial<true, MODE == 1, kBlock / kWave>(v, top, R, blockIdx.x);
 }
 
 template <int D>
@@ -335,6 +335,9 @@ __global__ __launch_bounds__(kBlock) void k_download(AtomArrays A, int what,
 // ======================================================== host launchers
 int reduce_blocks(int n) { return n <= 0 ? 1 : (n + kBlock - 1) / kBlock; }
 int force_blocks(int n, int tpa) { return reduce_blocks(n * tpa); }
+int force_partials(int n, const ListView &Lv) {
+    return Lv.tiled && Lv.built ? Lv.ntiles : force_blocks(n, Lv.tpa);
+}
 
 hipError_t launch_finalize_rt(bool sums, bool skin, int nparts, const ReduceBuf &R,
                               hipStream_t s) {
@@ -411,7 +414,6 @@ hipError_t launch_drift(int ndim, int stage, const AtomArrays &A, const StepCoef
         else
             hipLaunchKernelGGL((k_drift<2, false>), g, b, 0, s, A, c, R);
     }
-    launch_finalize<false, true>((int)g.x, R, s);
     return hipGetLastError();
 }
 
@@ -464,7 +466,7 @@ hipError_t launch_download(int ndim, int what, const AtomArrays &A,
     return hipGetLastError();
 }
 
-hipError_t launch_skin(int ndim, const AtomArrays &A, const ReduceBuf &R,
+hipError_t launch_skin(int ndim, const AtomArrays &A, const ReduceBuf &R, bool finalize,
                        hipStream_t s) {
     if (A.n <= 0) return hipSuccess;
     dim3 g(reduce_blocks(A.n)), b(kBlock);
@@ -472,7 +474,7 @@ hipError_t launch_skin(int ndim, const AtomArrays &A, const ReduceBuf &R,
         hipLaunchKernelGGL((k_skin<3>), g, b, 0, s, A, R);
     else
         hipLaunchKernelGGL((k_skin<2>), g, b, 0, s, A, R);
-    launch_finalize<false, true>((int)g.x, R, s);
+    if (finalize) launch_finalize<false, true>((int)g.x, R, s);
     return hipGetLastError();
 }
 

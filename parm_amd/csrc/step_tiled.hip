@@ -143,7 +143,17 @@ __global__ __launch_bounds__(kWave *TPA) void k_force_tiled(AtomArrays A, ListVi
     int32_t *stj = REL32 ? reinterpret_cast<int32_t *>(st32 + Lv.smax)
                          : reinterpret_cast<int32_t *>(st64 + Lv.smax);
 
-    const int t = xcd_block(blockIdx.x, gridDim.x);
+    constexpr bool STEP = STAGE == kStageVerletKickDrift || STAGE == kStageDampedKickDrift ||
+                          STAGE == kStageVerletKick || STAGE == kStageDampedKick;
+    // a step launch's first workgroup reduces the previous launch's skin test
+    const int extra = STEP && R.g.nprev > 0 ? 1 : 0;
+    if (STEP && extra && blockIdx.x == 0) {
+        reduce_prev<TPA>(R);
+        return;
+    }
+    if (STEP && step_stopped(R.g)) return;
+    const int blk = (int)blockIdx.x - extra;
+    const int t = xcd_block(blk, (int)gridDim.x - extra);
     if (threadIdx.x < kRunSlots) runs[threadIdx.x] = run_entry(Lv.truns, t, threadIdx.x);
     if (threadIdx.x == 0) hdr = Lv.tiles[t];
     __syncthreads();
@@ -540,7 +550,7 @@ __global__ __launch_bounds__(kWave *TPA) void k_force_tiled(AtomArrays A, ListVi
             atom_store<D, STAGE>(A, a0 + (int)threadIdx.x, fa, ain, c, top, nonfinite);
         }
     }
-    group_partials<D, STAGE, ENERGY, TPA, true>(acc, top, nonfinite, R);
+    group_partials<D, STAGE, ENERGY, TPA, true>(acc, top, nonfinite, R, blk);
 }
 
 // ======================================================== host launchers
@@ -553,10 +563,12 @@ void tiled_tt(const AtomArrays &A, const ListView &Lv, const PairView &P, const 
         (STAGE == kStageVerletKickDrift || STAGE == kStageDampedKickDrift);
     constexpr bool ENERGY = STAGE == kStageSums;
     const size_t lds = tiled_force_lds(D, PREC, KIND, SINGLE, Lv.smax);
+    constexpr bool STEP = DRIFT || STAGE == kStageVerletKick || STAGE == kStageDampedKick;
+    const int nb = Lv.ntiles + (STEP && R.g.nprev > 0 ? 1 : 0);
     hipLaunchKernelGGL((k_force_tiled<D, KIND, PREC, SINGLE, HARM, STAGE, TPA>),
-                       dim3(Lv.ntiles), dim3(kWave * TPA), lds, s, A, Lv, P, box, c, R);
+                       dim3(nb), dim3(kWave * TPA), lds, s, A, Lv, P, box, c, R);
     if (R.done) (void)hipEventRecord(R.done, s);
-    if (ENERGY || DRIFT) (void)launch_finalize_rt(ENERGY, DRIFT, Lv.ntiles, R, s);
+    if (ENERGY) (void)launch_finalize_rt(true, false, Lv.ntiles, R, s);
 }
 
 template <int D, int KIND, int PREC, bool SINGLE, bool HARM, int STAGE>

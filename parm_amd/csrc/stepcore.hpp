@@ -20,7 +20,8 @@ namespace parm {
 // A kernel that reduces (sums of energy / virial / stress / counts, and the
 // skin test's top-2 and non-finite count) writes one partial per workgroup
 // with plain stores; k_finalize, launched right after it on the same stream,
-// reduces the partials in a fixed order.  (A last-workgroup reduction inside
+// reduces the partials in a fixed order (the step loop's skin test: the next
+// step launch, below).  (A last-workgroup reduction inside
 // the launch would need a device-scope release per workgroup, which on a
 // multi-XCD part writes back the XCD's L2: far dearer than one more launch.)  No fences or contended atomics are
 // needed inside the hot kernel, and the result does not depend on scheduling.
@@ -42,7 +43,7 @@ __device__ __forceinline__ uint32_t skin_flag(const Top2 &tt, double nft, double
 // are the neutral ones and skip their wavefront reduction).
 template <bool SUMS, bool SKIN, int NW, bool SKIN_W0 = false>
 __device__ __forceinline__ void block_partial(double (&v)[kRedWidth], Top2 t,
-                                              const ReduceBuf &R) {
+                                              const ReduceBuf &R, int block) {
     __shared__ double sh[NW][kRedWidth];
     const int lane = threadIdx.x % kWave, w = threadIdx.x / kWave;
     if (SUMS) {
@@ -67,7 +68,7 @@ __device__ __forceinline__ void block_partial(double (&v)[kRedWidth], Top2 t,
     __syncthreads();
     const int k = threadIdx.x;
     // field-major partials: field k of workgroup b at part[k * pstride + b]
-    double *dst = R.part + blockIdx.x;
+    double *dst = R.part + block;
     const size_t ps = (size_t)R.pstride;
     if (SUMS && k < kTop1) {
         double p = 0.0;
@@ -188,11 +189,70 @@ __device__ __forceinline__ void atom_store(const AtomArrays &A, int i, const dou
     for (int k = 0; k < D; k++) A.v[k][i] = v[k];
 }
 
+// ------------------------------------------- the step loop's skin test
+// The skin test of step q's positions decides whether the list is rebuilt
+// before step q + 2's forces: a whole launch lies between.  So the partials
+// that one step launch leaves are reduced inside the next one, by one extra
+// workgroup (the first), beside the pair work, instead of by a launch of its
+// own between the two; and the launch after that reads the resulting flag
+// word (`gate`) itself and does nothing when it says stop, so the host may
+// queue step launches before it has seen the flags of the earlier ones.  A
+// stopped launch passes the stop on in its own flag word (kFlagStopped) and
+// tells the host nothing; the host takes up from the launch that raised the
+// flag.  As a launch of its own with the host deciding in between, the test
+// took 4.0 us and 9.6 us of idle GPU per step at 1000 atoms (6.9 and 5.8 us
+// at 1M): 200 steps of 1000 atoms 3718 -> 2388 us, 60 of 48,611 2653 -> 2146
+// us, 50 of 1M 12.77 -> 12.31 ms.
+__device__ __forceinline__ bool step_stopped(const StepGate &g) {
+    return g.gate && (*g.gate & (kFlagRebuild | kFlagNonFinite | kFlagStopped)) != 0u;
+}
+
+template <int NW>
+__device__ void reduce_prev(const ReduceBuf &R) {
+    __shared__ double fin[NW][3];
+    const StepGate &g = R.g;
+    const size_t ps = (size_t)R.pstride;
+    const int tid = threadIdx.x, lane = tid % kWave, w = tid / kWave;
+    const bool stopped = step_stopped(g);
+    Top2 t;
+    double nf = 0.0;
+#pragma unroll 4
+    for (int b = tid; b < g.nprev; b += NW * kWave) {
+        Top2 o;
+        o.a = g.prev[kTop1 * ps + b];
+        o.b = g.prev[kTop2 * ps + b];
+        t.merge(o);
+        nf += g.prev[kNonFinite * ps + b];
+    }
+    t = wave_top2(t);
+    nf = wave_count(nf);
+    if (lane == 0) {
+        fin[w][0] = t.a;
+        fin[w][1] = t.b;
+        fin[w][2] = nf;
+    }
+    __syncthreads();
+    if (tid == 0) {
+        for (int q = 1; q < NW; q++) {
+            Top2 o;
+            o.a = fin[q][0];
+            o.b = fin[q][1];
+            t.merge(o);
+            nf += fin[q][2];
+        }
+        const uint32_t fl = stopped ? (uint32_t)kFlagStopped : skin_flag(t, nf, R.skin);
+        *g.flag = fl;
+        if (!stopped)
+            __hip_atomic_store(g.hflag, (g.seq << kFlagBits) | fl, __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+}
+
 // This workgroup's reduction partials (all threads call it).  SKIN_W0: the
 // stage's writes (and so the skin test) were done by the first wavefront.
 template <int D, int STAGE, bool ENERGY, int NW, bool SKIN_W0 = false>
 __device__ __forceinline__ void group_partials(const PairAcc &acc, Top2 top, double nonfinite,
-                                               const ReduceBuf &R) {
+                                               const ReduceBuf &R, int block) {
     constexpr bool DRIFT =
         (STAGE == kStageVerletKickDrift || STAGE == kStageDampedKickDrift);
     if (ENERGY || DRIFT) {
@@ -208,7 +268,7 @@ __device__ __forceinline__ void group_partials(const PairAcc &acc, Top2 top, dou
             v[kSumOverlaps] = acc.overlaps;
         }
         v[kNonFinite] = nonfinite;
-        block_partial<ENERGY, DRIFT, NW, SKIN_W0>(v, top, R);
+        block_partial<ENERGY, DRIFT, NW, SKIN_W0>(v, top, R, block);
     }
 }
 

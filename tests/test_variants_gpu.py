@@ -33,3 +33,59 @@ def test_batch_build_slice_edges(ndim, lj):
         fr, lr = r.pairs()
         assert np.array_equal(fd, fr) and np.array_equal(ld, lr), (s, sizes[s])
     b.close()
+
+
+# the step loop queues launches ahead of the flags that may stop them: rebuilds
+# at every step, at none, and on both sides of the run-ahead's size limit
+@pytest.mark.parametrize("n,skin,steps", [(1, 0.3, 3), (300, 0.0, 1), (300, 0.0, 2),
+                                          (300, 1e-3, 7), (1000, 0.05, 40),
+                                          (33000, 0.02, 6)])
+@pytest.mark.parametrize("damped", [False, True])
+def test_step_loop_rebuild_schedule(n, skin, steps, damped):
+    _device_or_fail()
+    print(f"step loop n={n} skin={skin} steps={steps} damped={damped}", flush=True)
+    x, L = S.jittered_lattice(n, 0.7, 3, seed=n) if n > 1 else (np.zeros((1, 3)), np.full(3, 9.0))
+    v = S.gaussian_velocities(n, 3, 1.0, seed=n) if n > 1 else np.ones((1, 3))
+    p = S.lj_params(n)
+    t = O.PairTable(O.LJ_ATTRACT_REPULSE, p["eps"], p["sigma"], p["third"], p["types"])
+    r = O.System(np.ones(n), L, t, p["diam"], skin, ndim=3, brute=False)
+    s = capi.System(3, np.ones(n))
+    s.set_box(L)
+    s.nlist_set(skin, p["diam"])
+    s.set_lj(p["eps"], p["sigma"], p["third"], p["types"])
+    for q in (r, s):
+        q.set_state(x=x, v=v, a=np.zeros_like(x))
+        q.initialize()
+    s.profile_enable(True)
+    for _ in range(2):
+        if damped:
+            r.damped(0.002, 0.3, steps)
+            s.damped(0.002, 0.3, steps)
+        else:
+            r.verlet(0.002, steps)
+            s.verlet(0.002, steps)
+    assert s.which() == r.which()
+    assert s.profile_read()["step_launches"] == 2 * (steps - 1)
+    xr, vr = r.state()[:2]
+    xd, vd = s.state()[:2]
+    assert np.abs(xd - xr).max() <= 1e-11 * max(1.0, np.abs(xr).max())
+    assert np.abs(vd - vr).max() <= 1e-9 * max(1.0, np.abs(vr).max())
+    s.close()
+
+
+def test_step_loop_stops_at_nonfinite():
+    _device_or_fail()
+    n = 2000
+    x, L = S.jittered_lattice(n, 0.7, 3, seed=4)
+    s = capi.System(3, np.ones(n))
+    s.set_box(L)
+    s.nlist_set(0.3, np.full(n, 2.5))
+    s.set_lj([[1.0]], [1.0], [2.5], np.zeros(n, np.int32))
+    v = np.zeros_like(x)
+    v[17, 1] = np.inf
+    s.set_state(x=x, v=v, a=np.zeros_like(x))
+    s.initialize()
+    with pytest.raises(capi.ParmError) as e:
+        s.verlet(0.002, 8)
+    assert e.value.code == capi.E_NONFINITE and "step 0" in str(e.value)
+    s.close()
