@@ -83,6 +83,7 @@ constexpr int kFlagRing = 4;
 // scratch word for reductions that raise no flag, and the on-demand skin test
 // dynamic LDS of one tiled build workgroup, at most (the stencil's atoms)
 constexpr size_t kTiledLdsMax = 56 * 1024;
+constexpr int kMixedUntiledAtoms = 1 << 15;  // autotune
 // run-ahead of the step loop (step_runahead)
 constexpr int kRunAhead = 2, kRunAheadAtoms = 1 << 15;
 static_assert(kRunAhead + 1 < kFlagRing, "a flag word is not reused while a launch may read it");
@@ -416,7 +417,7 @@ int launch_tile_plan(parm_system *s) {
 // list build's staging is smaller: a plan the build accepts can still need
 // the untiled force layout).
 bool tiled_force_fits(const parm_system *s) {
-    return tiled_force_lds(s->ndim, s->prec, s->pair_kind, s->single != 0, s->smax) <=
+    return tiled_force_lds(s->ndim, s->prec, s->pair_kind, s->ntypes, s->smax) <=
            s->lds_max;
 }
 
@@ -724,7 +725,12 @@ int autotune(parm_system *s, int stage, const StepCoef &c) {
     std::vector<std::pair<int, int>> cands;  // (tiled, tpa)
     std::vector<int> layouts;
     const bool tiled_ok = s->tile_ok && tiled_force_fits(s);
-    if (tiled_ok && s->layout_pref != 2) layouts.push_back(1);
+    // (mixed-precision LJ: the tiled list's FP32 offsets cost precision, the
+    // error of a 10,007-atom trajectory is 4.6e-7 against 1e-7 untiled, and
+    // at such sizes gain nothing: 1685 against 1706 us per 100 steps)
+    const bool coarse = s->prec == kMixed && s->pair_kind == kPairLJ && s->layout_pref == 0 &&
+                        s->n <= kMixedUntiledAtoms;
+    if (tiled_ok && s->layout_pref != 2 && !coarse) layouts.push_back(1);
     if (s->layout_pref != 1 || !tiled_ok) layouts.push_back(0);
     for (int lay : layouts) {
         if (s->tpa_fixed) {

@@ -44,7 +44,6 @@ __global__ __launch_bounds__(kBlock) void k_force(AtomArrays A, ListView Lv,
         reduce_prev<kBlock / kWave>(R);
         return;
     }
-    if (STEP && step_stopped(R.g)) return;
     const int blk = (int)blockIdx.x - extra;
     const int gt = xcd_block(blk, (int)gridDim.x - extra) * kBlock + threadIdx.x;
     const int i = gt / TPA;
@@ -67,6 +66,8 @@ __global__ __launch_bounds__(kBlock) void k_force(AtomArrays A, ListView Lv,
     AtomIn<D> ain;
     if (act && sub == 0) atom_load<D, STAGE, false>(A, i, ain);
     const bool member = act && A.rank[i] >= 0;
+    // (the gate word arrives with the atom's own data)
+    if (STEP && step_stopped(R.g)) return;
     if (member && Lv.built) {
         // lane sub's entries m = 0 .. nl-1 sit at (m * npad + i) * TPA + sub
         const int nl = Lv.lcount[(size_t)i * TPA + sub];

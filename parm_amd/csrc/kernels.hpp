@@ -223,9 +223,9 @@ hipError_t launch_force(int ndim, int precision, int stage, bool energy,
                         const Box &box, const StepCoef &c, const ReduceBuf &R,
                         hipStream_t s);
 // Dynamic LDS of the tiled force kernel for a stencil of smax staged slots
-// (dimension, precision, pair kind, one pair type or several; no pair kind
-// yet gets the largest staging).
-size_t tiled_force_lds(int ndim, int prec, int kind, bool single, int smax);
+// (dimension, precision, pair kind, pair types; no pair kind yet gets the
+// largest staging).
+size_t tiled_force_lds(int ndim, int prec, int kind, int ntypes, int smax);
 // The force launches of one dimension, pair kind and precision: over the
 // untiled list (force.hip) and the tiled one (step_tiled.hip).
 template <int D, int KIND, int PREC>

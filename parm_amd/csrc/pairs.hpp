@@ -35,6 +35,25 @@ __device__ __forceinline__ double lj64_fs(const PairParam &pp, double d2, double
     return fmagR * idsq;
 }
 
+// The force factor alone, for the branch-free pair loops: 6 (sigma / r)^6
+// products instead of 7, rsix (p6 rsix - p6) with one rounding where lj64_fs
+// has two (p6 rsix, rsix - 1), so no further from the exact value.  d2 =
+// far_unless's stand-in gives exactly 0: rsix underflows.
+__device__ __forceinline__ double lj64_force(double sig2, double p6, double d2) {
+    const double idsq = rcp64_1(d2);
+    const double ir = sig2 * idsq;
+    const double rsix = ir * ir * ir;
+    return fma(p6, rsix, -p6) * rsix * idsq;
+}
+
+// d2, or (out of range) d2 with its upper word replaced: about 2^497, whose
+// force factor is 0.  One 32-bit select instead of two on the factor.
+__device__ __forceinline__ double far_unless(bool in, double d2) {
+    const unsigned long long u = (unsigned long long)__double_as_longlong(d2);
+    const unsigned hi = in ? (unsigned)(u >> 32) : 0x5f000000u;
+    return __longlong_as_double((long long)(((unsigned long long)hi << 32) | (unsigned)u));
+}
+
 // The same in FP32 (mixed precision).
 __device__ __forceinline__ float lj32_fs(const PairParam &pp, float d2, float &rsix,
                                          float &fmagR) {

@@ -350,13 +350,17 @@ hipError_t launch_finalize_rt(bool sums, bool skin, int nparts, const ReduceBuf 
     return hipGetLastError();
 }
 
-size_t tiled_force_lds(int ndim, int prec, int kind, bool single, int smax) {
+size_t tiled_force_lds(int ndim, int prec, int kind, int ntypes, int smax) {
     const bool raw = prec == kFP64 && kind == kPairRepulsion;
-    const bool rel32 = prec != kFP64 && kind == kPairLJ;
     if (raw) return (size_t)smax * sizeof(double4);
-    if (single && kind != kPairNone)
-        return (size_t)smax * ndim * (rel32 ? sizeof(float) : sizeof(double));
-    if (rel32) return (size_t)smax * (sizeof(float4) + sizeof(int32_t));
+    if (kind == kPairLJ) {
+        // (lj_slots_bytes in step_tiled.hip) + table + type bytes
+        const size_t real = prec == kFP64 ? sizeof(double) : sizeof(float);
+        size_t b = ((size_t)(smax + 1) * ndim * real + 15) & ~(size_t)15;
+        if (ntypes > 1) b += (size_t)ntypes * ntypes * 4 * real + (size_t)smax + 1;
+        return b;
+    }
+    if (ntypes == 1 && kind != kPairNone) return (size_t)smax * ndim * sizeof(double);
     return (size_t)smax * (sizeof(double4) + sizeof(int32_t));
 }
 

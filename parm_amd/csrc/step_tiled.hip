@@ -16,13 +16,15 @@
 //         reference's minimum image diff(x_i, x_j), so every pair force is
 //         the untiled kernel's bit for bit.
 //   REL64 (FP64 LJ, mixed repulsion): the FP64 minimum-image offset of each
-//         atom from the tile's first atom.  A pair displacement is the
+//         atom from the tile's middle atom.  A pair displacement is the
 //         difference of two offsets (both in [-L/2, L/2], so one fold gives
 //         the minimum image; when every offset of the tile is under L/4 the
 //         difference already is, and the fold is skipped).  It differs from
 //         diff(x_i, x_j) only by rounding (~1e-16 relative); the LJ in/out
 //         decision within 1e-14 of the cutoff is taken on the exact d2, so the
 //         set of interacting pairs is the reference's.
+//         With several types a slot's type is a byte of its own and the pair
+//         parameters are a table in LDS.
 //   REL32 (mixed LJ): the same offsets rounded to FP32 and differenced in
 //         FP32 (half the LDS traffic; the rounding of offsets of a few sigma
 //         costs ~1e-6 sigma in r).  Repulsion does not use it: its force
@@ -115,10 +117,36 @@ __device__ __forceinline__ Vec<D> offset_folded(const Vec<D> &x, const Vec<D> &o
 }
 
 // List words per lane read ahead of the pair loop (two entries a word), and
-// the entries the one-type LJ loop evaluates side by side.
+// the entries the LJ loop evaluates side by side.
 constexpr int kChunkWords = 4;
 constexpr int kGroup = 4;
 static_assert(kChunkWords % (kGroup / 2) == 0, "groups tile a chunk");
+
+// One row of the LJ pair table in LDS (several types).
+template <int PREC>
+struct LjRow;
+template <>
+struct LjRow<kFP64> {
+    double sig2, p6, lo, hi;
+    __device__ static LjRow make(const PairParam &p) {
+        return LjRow{p.sig2, p.p6, p.lim_lo, p.lim_hi};
+    }
+};
+template <>
+struct LjRow<kMixed> {
+    float sig2, p6, lo, hi;
+    __device__ static LjRow make(const PairParam &p) {
+        return LjRow{p.sig2_f, p.p6_f, p.lim_f * 0.99999f, p.lim_f * 1.00001f};
+    }
+};
+
+// Dynamic LDS of the LJ staging, in this order: smax + 1 slots of D offsets
+// (the last one a stand-in for entries past a lane's count: see the pair
+// loop), then with several types the pair table and a type byte per slot.
+template <int D, int PREC>
+__host__ __device__ constexpr size_t lj_slots_bytes(int smax) {
+    return (((size_t)(smax + 1) * D * (PREC == kFP64 ? 8 : 4)) + 15) & ~(size_t)15;
+}
 
 template <int D, int KIND, int PREC, bool SINGLE, bool HARM, int STAGE, int TPA>
 __global__ __launch_bounds__(kWave *TPA) void k_force_tiled(AtomArrays A, ListView Lv,
@@ -128,11 +156,14 @@ __global__ __launch_bounds__(kWave *TPA) void k_force_tiled(AtomArrays A, ListVi
     constexpr bool ENERGY = STAGE == kStageSums;
     constexpr bool RAW = PREC == kFP64 && KIND != kPairLJ;
     constexpr bool REL32 = PREC != kFP64 && KIND == kPairLJ;
-    // COMPACT (one pair type, offsets staged): a slot is the D offsets only
-    // (FP64: 8 D bytes, FP32: 4 D bytes), no type, no atom index (the rare
+    // COMPACT (LJ, or one pair type, offsets staged): a slot is the D offsets
+    // only (FP64: 8 D bytes, FP32: 4 D bytes), no atom index (the rare
     // exact-d2 path finds the atom from the runs): less LDS per workgroup,
-    // more workgroups per CU.
-    constexpr bool COMPACT = SINGLE && !RAW;
+    // more workgroups per CU.  LJ with several types keeps a type byte per
+    // slot beside them.
+    constexpr bool LJ = KIND == kPairLJ;
+    constexpr bool COMPACT = LJ || (SINGLE && !RAW);
+    using Real = typename std::conditional<REL32, float, double>::type;
     constexpr int NT = kWave * TPA;
     extern __shared__ double4 st64[];
     __shared__ int2 runs[kRunSlots];  // run_entry form (tiles.hpp)
@@ -140,6 +171,10 @@ __global__ __launch_bounds__(kWave *TPA) void k_force_tiled(AtomArrays A, ListVi
     float4 *st32 = reinterpret_cast<float4 *>(st64);
     double *stc64 = reinterpret_cast<double *>(st64);
     float *stc32 = reinterpret_cast<float *>(st64);
+    Real *stc = reinterpret_cast<Real *>(st64);
+    LjRow<PREC> *ljtab = reinterpret_cast<LjRow<PREC> *>(reinterpret_cast<char *>(st64) +
+                                                         lj_slots_bytes<D, PREC>(Lv.smax));
+    uint8_t *ljtype = reinterpret_cast<uint8_t *>(ljtab + (size_t)P.ntypes * P.ntypes);
     int32_t *stj = REL32 ? reinterpret_cast<int32_t *>(st32 + Lv.smax)
                          : reinterpret_cast<int32_t *>(st64 + Lv.smax);
 
@@ -151,11 +186,12 @@ __global__ __launch_bounds__(kWave *TPA) void k_force_tiled(AtomArrays A, ListVi
         reduce_prev<TPA>(R);
         return;
     }
-    if (STEP && step_stopped(R.g)) return;
     const int blk = (int)blockIdx.x - extra;
     const int t = xcd_block(blk, (int)gridDim.x - extra);
     if (threadIdx.x < kRunSlots) runs[threadIdx.x] = run_entry(Lv.truns, t, threadIdx.x);
     if (threadIdx.x == 0) hdr = Lv.tiles[t];
+    // (the gate word arrives with the header)
+    if (STEP && step_stopped(R.g)) return;
     __syncthreads();
     const int a0 = hdr.x, tcnt = hdr.y;
     const int S = hdr.z >= 0 ? hdr.w : 0;
@@ -192,9 +228,20 @@ __global__ __launch_bounds__(kWave *TPA) void k_force_tiled(AtomArrays A, ListVi
                 if (q < Lv.wcap) cur[q] = wp[(size_t)q * wstride];
         }
     }
-    // the tile origin: loaded now, folded once the stencil's loads are issued
+    if constexpr (LJ) {
+        // the stand-in slot: far outside any cutoff (not folded: see `group`)
+        if (threadIdx.x < D) stc[(size_t)Lv.smax * D + threadIdx.x] = (Real)(REL32 ? 1e18 : 1e150);
+        if constexpr (!SINGLE) {
+            if (threadIdx.x == 0) ljtype[Lv.smax] = 0;
+            for (int q = threadIdx.x; q < P.ntypes * P.ntypes; q += NT)
+                ljtab[q] = LjRow<PREC>::make(P.tab[q]);
+        }
+    }
+    // the tile origin, its middle atom (offsets half as large, and rounded
+    // half as far in FP32, as from the first one): loaded now, folded once
+    // the stencil's loads are issued
     PT xo_raw{};
-    if (!RAW && S > 0) xo_raw = pos[a0];
+    if (!RAW && S > 0) xo_raw = pos[a0 + (tcnt >> 1)];
     Vec<D> xo;
 #pragma unroll
     for (int k = 0; k < D; k++) xo.c[k] = 0.0;
@@ -252,6 +299,7 @@ __global__ __launch_bounds__(kWave *TPA) void k_force_tiled(AtomArrays A, ListVi
                 else
                     stc64[s * D + k] = v.c[k];
             }
+            if constexpr (LJ && !SINGLE) ljtype[s] = (uint8_t)tj;
         } else if (REL32) {
             float4 q;
             q.x = (float)v.c[0];
@@ -335,6 +383,7 @@ __global__ __launch_bounds__(kWave *TPA) void k_force_tiled(AtomArrays A, ListVi
                 if constexpr (COMPACT) {
 #pragma unroll
                     for (int k = 0; k < D; k++) qc[k] = stc32[s * D + k];
+                    if constexpr (!SINGLE) tj = ljtype[s];
                 } else {
                     const float4 q = st32[s];
                     qc[0] = q.x;
@@ -357,6 +406,7 @@ __global__ __launch_bounds__(kWave *TPA) void k_force_tiled(AtomArrays A, ListVi
                 if constexpr (COMPACT) {
 #pragma unroll
                     for (int k = 0; k < D; k++) qc[k] = stc64[s * D + k];
+                    if constexpr (LJ && !SINGLE) tj = ljtype[s];
                 } else {
                     const double4 q = st64[s];
                     qc[0] = q.x;
@@ -384,115 +434,152 @@ __global__ __launch_bounds__(kWave *TPA) void k_force_tiled(AtomArrays A, ListVi
                 }
             }
         };
-        // kGroup entries (kGroup / 2 words) of the one-type LJ list at once,
-        // branch-free but for the in/out decision within a hair of the
-        // cutoff: their staged offsets read together, their force factors
-        // evaluated side by side, then added in list order (an entry outside
-        // the cutoff, or past the lane's count, adds 0 * r, which leaves the
-        // sum as it is; a slot past the count reads slot 0, which holds a
-        // staged offset whenever any entry exists).
-        auto group = [&](const uint32_t *wd, int e, auto fold_c) {
+        // kGroup entries (kGroup / 2 words) of the LJ list at once, with no
+        // branch but one, uniform over the wavefront, for a pair within a
+        // hair of the cutoff.  An entry out of range adds 0 * r.  The words
+        // hold valid slots throughout: the stand-in slot smax takes the place
+        // of the entries past a lane's count; it lies far outside the cutoff
+        // unless the displacement is folded, where it is told by its number.
+        //
+        // The loop is bound by VALU issue (an FP64 instruction is 4 cycles of
+        // a SIMD) and, below four waves a SIMD, by the ~25 cycles of each
+        // compare-and-select and of each branch: 25 VALU instructions per
+        // entry.  One-type FP64 at 1M atoms 186 -> 179 us per launch against
+        // a form that decided each near-cutoff entry in place (four mask
+        // merges and a jump per group); two types at 48,611 atoms 25.3 ->
+        // 21.7 us against one entry at a time with parameters from memory
+        // (untiled: 24.6 us).
+        const int ti = SINGLE ? 0 : (int)A.type[i] * P.ntypes;
+        auto displacement = [&](auto fold_c, Real (&r)[D]) {  // staged offset -> r
             constexpr bool FOLD = decltype(fold_c)::value;
-            int sl[kGroup];
-            bool ok[kGroup], in[kGroup], band[kGroup];
 #pragma unroll
-            for (int g = 0; g < kGroup; g++) {
-                const uint32_t w = wd[g >> 1];
-                ok[g] = e + g < nlane;
-                sl[g] = ok[g] ? (int)((g & 1) ? (w >> 16) : (w & 0xffffu)) : 0;
-            }
-            if constexpr (PREC == kFP64) {
-                double r[kGroup][D], fs[kGroup];
-#pragma unroll
-                for (int g = 0; g < kGroup; g++) {
-#pragma unroll
-                    for (int k = 0; k < D; k++) {
-                        double d = ri64.c[k] - stc64[sl[g] * D + k];
-                        if (FOLD)
-                            d = d > box.halfL[k] ? d - box.L[k]
-                                                 : (d < -box.halfL[k] ? d + box.L[k] : d);
-                        r[g][k] = d;
-                    }
-                    double d2 = r[g][0] * r[g][0];
-#pragma unroll
-                    for (int k = 1; k < D; k++) d2 = fma(r[g][k], r[g][k], d2);
-                    const bool lo = d2 < p0.lim_lo;
-                    band[g] = ok[g] && !lo && !(d2 > p0.lim_hi);
-                    in[g] = ok[g] && lo;
-                    double rsix, fmagR;
-                    fs[g] = lj64_fs(p0, d2, rsix, fmagR);
-                }
-                bool anyband = false;
-#pragma unroll
-                for (int g = 0; g < kGroup; g++) anyband |= band[g];
-                if (anyband) {
-#pragma unroll
-                    for (int g = 0; g < kGroup; g++)
-                        if (band[g]) in[g] = !(exact_d2(sl[g]) / p0.sig2 > p0.cut2);
-                }
-#pragma unroll
-                for (int g = 0; g < kGroup; g++) {
-                    const double m = in[g] ? fs[g] : 0.0;
-#pragma unroll
-                    for (int k = 0; k < D; k++) fi[k] = fma(m, r[g][k], fi[k]);
-                }
-            } else {
-                float r[kGroup][D], fs[kGroup];
-#pragma unroll
-                for (int g = 0; g < kGroup; g++) {
-#pragma unroll
-                    for (int k = 0; k < D; k++) {
-                        float d = ri[k] - stc32[sl[g] * D + k];
-                        if (FOLD) d = d > hLf[k] ? d - Lf[k] : (d < -hLf[k] ? d + Lf[k] : d);
-                        r[g][k] = d;
-                    }
-                    float d2 = r[g][0] * r[g][0];
-#pragma unroll
-                    for (int k = 1; k < D; k++) d2 = fmaf(r[g][k], r[g][k], d2);
-                    const bool lo = !(d2 > p0.lim_f * 0.99999f);
-                    band[g] = ok[g] && !lo && !(d2 > p0.lim_f * 1.00001f);
-                    in[g] = ok[g] && lo;
-                    float rsix, fmagR;
-                    fs[g] = lj32_fs(p0, d2, rsix, fmagR);
-                }
-                bool anyband = false;
-#pragma unroll
-                for (int g = 0; g < kGroup; g++) anyband |= band[g];
-                if (anyband) {
-#pragma unroll
-                    for (int g = 0; g < kGroup; g++) {
-                        if (band[g]) {
-                            const double d2d = exact_d2(sl[g]);
-                            in[g] = d2d < p0.lim_lo ||
-                                    (!(d2d > p0.lim_hi) && !(d2d / p0.sig2 > p0.cut2));
-                        }
-                    }
-                }
-#pragma unroll
-                for (int g = 0; g < kGroup; g++) {
-                    const float m = in[g] ? fs[g] : 0.0f;
-#pragma unroll
-                    for (int k = 0; k < D; k++) f32[k] = fmaf(m, r[g][k], f32[k]);
+            for (int k = 0; k < D; k++) {
+                if constexpr (REL32) {
+                    float d = ri[k] - r[k];
+                    if (FOLD) d = fmaf(-Lf[k], rintf(d * (float)box.invL[k]), d);
+                    r[k] = d;
+                } else {
+                    double d = ri64.c[k] - r[k];
+                    if (FOLD) d = fma(-box.L[k], rint(d * box.invL[k]), d);
+                    r[k] = d;
                 }
             }
         };
-        // two entries per 32-bit word; for the one-type LJ forms the lane's
-        // words stream from memory kChunkWords at a time, each chunk loaded
-        // while the one before it is evaluated (the first was loaded before
-        // the staging)
+        auto sq = [&](const Real (&r)[D]) {
+            Real d2 = r[0] * r[0];
+#pragma unroll
+            for (int k = 1; k < D; k++) d2 = fma(r[k], r[k], d2);
+            return d2;
+        };
+        auto ljrow = [&](int s) {
+            if constexpr (SINGLE)
+                return LjRow<PREC>::make(p0);
+            else
+                return ljtab[ti + ljtype[s]];
+        };
+        auto ljfs = [&](const LjRow<PREC> &q, Real d2) {
+            if constexpr (PREC == kFP64) {
+                return lj64_force(q.sig2, q.p6, d2);
+            } else {
+                const float idsq = __builtin_amdgcn_rcpf(d2);
+                const float ir = q.sig2 * idsq;
+                const float rsix = ir * ir * ir;
+                return q.p6 * rsix * (rsix - 1.0f) * idsq;
+            }
+        };
+        auto addf = [&](Real m, const Real (&r)[D]) {
+#pragma unroll
+            for (int k = 0; k < D; k++) {
+                if constexpr (PREC == kFP64)
+                    fi[k] = fma(m, r[k], fi[k]);
+                else
+                    f32[k] = fmaf(m, r[k], f32[k]);
+            }
+        };
+        auto group = [&](uint32_t wa, uint32_t wb, auto fold_c) {
+            constexpr bool FOLD = decltype(fold_c)::value;
+            const int sl[kGroup] = {(int)(wa & 0xffffu), (int)(wa >> 16), (int)(wb & 0xffffu),
+                                    (int)(wb >> 16)};
+            Real r[kGroup][D], fs[kGroup];
+            unsigned long long band = 0;
+            // the group's slots are read together, before any is used
+#pragma unroll
+            for (int g = 0; g < kGroup; g++)
+#pragma unroll
+                for (int k = 0; k < D; k++) r[g][k] = stc[sl[g] * D + k];
+#pragma unroll
+            for (int g = 0; g < kGroup; g++) {
+                displacement(fold_c, r[g]);
+                const LjRow<PREC> q = ljrow(sl[g]);
+                const Real d2 = sq(r[g]);
+                bool in = d2 < q.lo, near = d2 <= q.hi;
+                if (FOLD) {
+                    in = in && sl[g] != Lv.smax;
+                    near = near && sl[g] != Lv.smax;
+                }
+                band |= __ballot(near) & ~__ballot(in);
+                if constexpr (PREC == kFP64) {
+                    fs[g] = ljfs(q, far_unless(in, d2));
+                } else {
+                    const float m = ljfs(q, d2);
+                    fs[g] = in ? m : 0.0f;
+                }
+            }
+#pragma unroll
+            for (int g = 0; g < kGroup; g++) addf(fs[g], r[g]);
+            if (band) {
+                // pairs near the cutoff: the reference's decision, on its d2
+#pragma unroll 1
+                for (int g = 0; g < kGroup; g++) {
+                    const uint32_t w = g < 2 ? wa : wb;
+                    const int s = (g & 1) ? (int)(w >> 16) : (int)(w & 0xffffu);
+                    Real rr[D];
+#pragma unroll
+                    for (int k = 0; k < D; k++) rr[k] = stc[s * D + k];
+                    displacement(fold_c, rr);
+                    const LjRow<PREC> q = ljrow(s);
+                    const Real d2 = sq(rr);
+                    if (s != Lv.smax && !(d2 < q.lo) && d2 <= q.hi) {
+                        const int j = slot_atom(runs, s);
+                        const PairParam &pp = SINGLE ? p0 : P.tab[ti + (SINGLE ? 0 : ljtype[s])];
+                        const double d2x = sqnorm<D>(diff<D>(xi, PosStore<D>::load(pos[j]), box));
+                        if (d2x < pp.lim_lo || (!(d2x > pp.lim_hi) && !(d2x / pp.sig2 > pp.cut2)))
+                            addf(ljfs(q, d2), rr);
+                    }
+                }
+            }
+        };
+        // two entries per 32-bit word; for the LJ forms the lane's words
+        // stream from memory kChunkWords at a time, each chunk loaded while
+        // the one before it is evaluated (the first was loaded before the
+        // staging); the loop runs for the wavefront's longest lane
         auto loop = [&](auto fold_c) {
-            if constexpr (COMPACT && !ENERGY && KIND == kPairLJ) {
+            if constexpr (LJ && !ENERGY) {
+                const uint32_t none = (uint32_t)Lv.smax * 0x10001u;
+                // word w of the lane with the entries past the count replaced
+                auto fix = [&](uint32_t v, int w) {
+                    const int left = nlane - 2 * w;
+                    v = left == 1 ? (v & 0xffffu) | (none & 0xffff0000u) : v;
+                    return left > 0 ? v : none;
+                };
                 const int nw = (nlane + 1) >> 1;
-                for (int w0 = 0; w0 < nw; w0 += kChunkWords) {
+                for (int w0 = 0; __ballot(w0 < nw) != 0ull; w0 += kChunkWords) {
                     uint32_t nxt[kChunkWords];
 #pragma unroll
                     for (int q = 0; q < kChunkWords; q++) {
                         const int w = w0 + kChunkWords + q;
-                        nxt[q] = w < nw ? wp[(size_t)w * wstride] : 0u;
+                        nxt[q] = none;
+                        if (__ballot(w < nw) != 0ull) nxt[q] = wp[(size_t)w * wstride];
+                    }
+                    // (wave-uniform: most chunks are full in every lane)
+                    if (__ballot(2 * (w0 + kChunkWords) > nlane) != 0ull) {
+#pragma unroll
+                        for (int q = 0; q < kChunkWords; q++) cur[q] = fix(cur[q], w0 + q);
                     }
 #pragma unroll
                     for (int q = 0; q < kChunkWords; q += kGroup / 2)
-                        if (2 * (w0 + q) < nlane) group(cur + q, 2 * (w0 + q), fold_c);
+                        if (__ballot(2 * (w0 + q) < nlane) != 0ull)
+                            group(cur[q], cur[q + 1], fold_c);
 #pragma unroll
                     for (int q = 0; q < kChunkWords; q++) cur[q] = nxt[q];
                 }
@@ -562,7 +649,7 @@ void tiled_tt(const AtomArrays &A, const ListView &Lv, const PairView &P, const 
     constexpr bool DRIFT =
         (STAGE == kStageVerletKickDrift || STAGE == kStageDampedKickDrift);
     constexpr bool ENERGY = STAGE == kStageSums;
-    const size_t lds = tiled_force_lds(D, PREC, KIND, SINGLE, Lv.smax);
+    const size_t lds = tiled_force_lds(D, PREC, KIND, P.ntypes, Lv.smax);
     constexpr bool STEP = DRIFT || STAGE == kStageVerletKick || STAGE == kStageDampedKick;
     const int nb = Lv.ntiles + (STEP && R.g.nprev > 0 ? 1 : 0);
     hipLaunchKernelGGL((k_force_tiled<D, KIND, PREC, SINGLE, HARM, STAGE, TPA>),

@@ -89,3 +89,39 @@ def test_step_loop_stops_at_nonfinite():
         s.verlet(0.002, 8)
     assert e.value.code == capi.E_NONFINITE and "step 0" in str(e.value)
     s.close()
+
+
+# the tiled LJ pair loop: several types (table and type bytes in LDS), counts
+# that are no multiple of a group, folded (small box) and plain offsets, and
+# pairs at the cutoff itself
+@pytest.mark.parametrize("tpa", [1, 4, 8])
+@pytest.mark.parametrize("ntypes", [1, 3, 16])
+@pytest.mark.parametrize("n", [65, 500, 6000])
+def test_tiled_lj_group_edges(monkeypatch, tpa, ntypes, n):
+    _device_or_fail()
+    print(f"tiled lj tpa={tpa} ntypes={ntypes} n={n}", flush=True)
+    monkeypatch.setenv("PARM_TPA", str(tpa))
+    monkeypatch.setenv("PARM_TILED", "1")
+    x, L = S.jittered_lattice(n, 0.75, 3, seed=n + ntypes)
+    rng = np.random.default_rng(ntypes)
+    types = rng.integers(0, ntypes, n).astype(np.int32)
+    eps = rng.uniform(0.5, 1.5, (ntypes, ntypes))
+    eps = (eps + eps.T) / 2
+    sigma = rng.uniform(0.8, 1.0, ntypes)
+    cut = rng.uniform(1.5, 2.2, ntypes)
+    # pairs of atoms exactly at their cutoff along x (inside: d2 / sig2 > cut2 is false)
+    if ntypes == 1:
+        x[1] = x[0] + [sigma[0] * cut[0], 0, 0]
+    diam = (sigma * cut)[types]
+    t = O.PairTable(O.LJ_ATTRACT_REPULSE, eps, sigma, cut, types)
+    s = capi.System(3, np.ones(n))
+    s.set_box(L)
+    s.nlist_set(0.3, diam)
+    s.set_lj(eps, sigma, cut, types)
+    s.set_state(x=x)
+    s.update_list(True)
+    s.set_forces(False)
+    assert s.list_info()["tiled"]
+    first, last = O.nlist(x, L, diam, 0.3)
+    S.assert_fp64_forces(s.forces(), O.forces(x, L, t, first, last), x, L, t, first, last)
+    s.close()
