@@ -83,7 +83,7 @@ constexpr int kFlagRing = 4;
 // scratch word for reductions that raise no flag, and the on-demand skin test
 // dynamic LDS of one tiled build workgroup, at most (the stencil's atoms)
 constexpr size_t kTiledLdsMax = 56 * 1024;
-constexpr int kMixedUntiledAtoms = 1 << 15;  // autotune
+constexpr int kMixedUntiledAtoms = 1 << 15, kMixedRepulsionFixed = 100000;  // autotune
 // run-ahead of the step loop (step_runahead)
 constexpr int kRunAhead = 2, kRunAheadAtoms = 1 << 15;
 static_assert(kRunAhead + 1 < kFlagRing, "a flag word is not reused while a launch may read it");
@@ -738,6 +738,17 @@ int autotune(parm_system *s, int stage, const StepCoef &c) {
         } else {
             for (int tpa : {1, 2, 4, 8}) cands.emplace_back(lay, tpa);
         }
+    }
+    // Mixed-precision repulsion of many atoms: only the candidates that add
+    // an atom's pair forces in the same order (one lane untiled keeps a lane
+    // pair's two sums: force.hip).  They are the fastest there and race within
+    // a few per cent, so the pick differs from run to run, and a relaxation
+    // from random positions amplifies another order of the FP32 sums (1e-3 in
+    // single velocities after 200 steps of 262,144 disks).
+    if (s->prec == kMixed && s->pair_kind == kPairRepulsion && s->n >= kMixedRepulsionFixed &&
+        s->layout_pref == 0 && !s->tpa_fixed) {
+        cands = {{0, 1}, {0, 2}};
+        if (tiled_ok) cands.emplace_back(1, 2);
     }
     if (cands.size() <= 1) {
         if (!cands.empty() && (cands[0].first != (int)s->tiled || cands[0].second != s->tpa)) {

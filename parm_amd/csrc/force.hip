@@ -51,11 +51,15 @@ __global__ __launch_bounds__(kBlock) void k_force(AtomArrays A, ListView Lv,
     const bool act = i < A.n;
     PairAcc acc;
     double fi[D];
-    float f32[D];
+    // (mixed) the FP32 sums of the even and the odd entries: one lane adds up
+    // as two lanes do, so the result does not depend on which of them the
+    // autotuner takes
+    constexpr bool PAIRSUM = PREC != kFP64 && TPA == 1;
+    float f32[D], f32o[D];
 #pragma unroll
     for (int k = 0; k < D; k++) {
         fi[k] = 0.0;
-        f32[k] = 0.0f;
+        f32[k] = f32o[k] = 0.0f;
     }
 
     const PT *pos = static_cast<const PT *>(A.pos_in);
@@ -93,7 +97,7 @@ __global__ __launch_bounds__(kBlock) void k_force(AtomArrays A, ListView Lv,
                                                f32, acc);
             const Vec<D> r1 = diff<D>(xi, PosStore<D>::load(pj1), box);
             visit<D, KIND, PREC, ENERGY, HARM>(SINGLE ? p0 : row[e1 & tmask], r1, fi,
-                                               f32, acc);
+                                               PAIRSUM ? f32o : f32, acc);
         }
         if (m < nl) {
             const uint32_t e0 = nb[off];
@@ -104,7 +108,8 @@ __global__ __launch_bounds__(kBlock) void k_force(AtomArrays A, ListView Lv,
     }
     if (PREC != kFP64) {
 #pragma unroll
-        for (int k = 0; k < D; k++) fi[k] = (double)f32[k];
+        for (int k = 0; k < D; k++)
+            fi[k] = PAIRSUM ? (double)f32[k] + (double)f32o[k] : (double)f32[k];
     }
     // sum the TPA partial forces of the atom (all lanes take part)
 #pragma unroll
