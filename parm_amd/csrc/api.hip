@@ -143,6 +143,9 @@ struct parm_system {
     uint32_t *keys = nullptr, *tkeys = nullptr, *hist = nullptr;
     int32_t *vals = nullptr, *tvals = nullptr, *cstart = nullptr;
     int cstart_cap = 0;
+    uint32_t *ccount = nullptr, *ctotal = nullptr;  // counted ordering (launch_cell_order)
+    bool ccount_clear = false;                      // ccount is all zero
+    uint32_t build_seq = 0;                         // number of the last build report asked for
     unsigned long long *stats = nullptr, *bpart = nullptr;
 
     // NeighborList::ignore: excluded pairs as sorted keys (hi << 32 | lo) of
@@ -349,16 +352,16 @@ int initial_capacity(const parm_system *s) {
     return std::max(16, (int)cap);
 }
 
-// Permute every per-slot array by perm (new slot i <- old slot perm[i]).
-// Every per-slot array into the new slot order, in one launch: the position
+// Every per-slot array into the new slot order (vals: the sorted old slots, or
+// with `counted` each cell's atoms as launch_cell_order left them), in one launch: the position
 // buffers (the alternate one holds the next step's drifted positions inside
 // a fused step loop; xref is free to take one of them, the list build
 // rewrites it), the ndim components of v, a, f, the masses and diameters,
 // and the type / original index / member rank.  Each lands in its spare,
 // which then becomes the column.  keep_af = false leaves a and f in the old
 // order: for a rebuild inside the step loop whose next launch writes both
-// before anything reads them.
-int permute_all(parm_system *s, const int32_t *perm, bool keep_af = true) {
+// before anything reads them.  skin: see launch_cell_permute.
+int permute_all(parm_system *s, bool keep_af, bool counted, const ReduceBuf *skin) {
     PermuteSet P{};
     P.pos_src[0] = s->pos;
     P.pos_dst[0] = s->xref;
@@ -384,7 +387,11 @@ int permute_all(parm_system *s, const int32_t *perm, bool keep_af = true) {
         P.i_dst[c] = s->spare_i[c];
     }
     P.ni = kPermI;
-    PARM_HIP(launch_permute(s->ndim, s->n, perm, P, s->stream));
+    if (counted)
+        PARM_HIP(launch_cell_permute(s->ndim, s->n, s->vals, s->tkeys, s->cstart, s->grid,
+                                     s->box, s->keys, s->xwrap, P, skin, s->stream));
+    else
+        PARM_HIP(launch_permute(s->ndim, s->n, s->vals, P, s->stream));
     std::swap(s->pos, s->xref);
     std::swap(s->pos_alt, s->pos_spare);
     for (int c = 0; c < nd; c++) std::swap(*dcols[c], s->spare_d[c]);
@@ -441,6 +448,7 @@ int plan_tiles(parm_system *s) {
         accept_tiles(s, 0, 0, 0);
         return PARM_OK;
     }
+    PARM_HIP(launch_tile_extremes(s->tiles, s->tinfo, s->stream));
     PARM_HIP(hipMemcpyAsync(s->htinfo, s->tinfo, 3 * sizeof(int), hipMemcpyDeviceToHost,
                             s->stream));
     PARM_HIP(hipStreamSynchronize(s->stream));
@@ -450,7 +458,7 @@ int plan_tiles(parm_system *s) {
 
 // Builds the list at positions `at` (the current ones, or xref for a
 // relayout) in the layout chosen by accept_tiles.
-int build_list(parm_system *s, const void *at) {
+int build_list(parm_system *s, const void *at, bool wrapped) {
     PARM_CHECK(check_lane_counts(s));
     hipStream_t st = s->stream;
     if (s->tile_ok) {
@@ -461,22 +469,39 @@ int build_list(parm_system *s, const void *at) {
                                     s->cstart, s->grid, s->box, s->skin, s->dmax, s->tpa,
                                     s->cap, s->npad, !s->tiled, s->nbr, s->ncount, s->lcount,
                                     s->xref, s->bpart, s->stats, s->dflag + kSlotBuild,
-                                    nullptr, s->dmin == s->dmax, s->exview(), s->hrep_dev,
-                                    st));
+                                    nullptr, s->dmin == s->dmax, s->exview(), wrapped,
+                                    s->hrep_dev, ++s->build_seq, st));
     } else {
         PARM_HIP(launch_build_list(s->ndim, s->n, at, s->xwrap, s->rank, s->diam, s->type,
                                    s->keys, s->cstart, s->grid, s->box, s->skin, s->dmax,
                                    s->type_bits, s->tpa, s->cap, s->npad, s->nbr, s->ncount,
                                    s->lcount, s->xref, s->bpart, s->stats, s->dflag + kSlotBuild,
-                                   s->exview(), s->hrep_dev, st));
+                                   s->exview(), wrapped, s->hrep_dev, ++s->build_seq, st));
     }
     return PARM_OK;
 }
 
-// The report of the build just queued, once the stream has finished.
+// The report of the build just queued, as soon as its last launch has stored
+// it (its number last): a poll of the pinned word answers sooner than a wait
+// for the stream.  The stream's state is asked for now and then, so the poll
+// ends also when the device reports an error or drains without a report.
 int read_report(parm_system *s, BuildReport *r) {
-    PARM_HIP(hipStreamSynchronize(s->stream));
     const volatile BuildReport *h = s->hrep;
+    bool drained = false;
+    for (;;) {
+        bool there = false;
+        for (int k = 0; k < 1 << 14 && !there; k++) {
+            there = __atomic_load_n(&s->hrep->seq, __ATOMIC_ACQUIRE) == s->build_seq;
+            if (!there) __builtin_ia32_pause();
+        }
+        if (there) break;
+        if (drained) return fail(PARM_E_DEVICE, "a list build did not report");
+        const hipError_t e = hipStreamQuery(s->stream);
+        if (e == hipSuccess)
+            drained = true;  // one more look
+        else if (e != hipErrorNotReady)
+            return fail(PARM_E_DEVICE, std::string("list build: ") + hipGetErrorString(e));
+    }
     r->sum = h->sum;
     r->max = h->max;
     r->ntiles = h->ntiles;
@@ -489,9 +514,9 @@ int read_report(parm_system *s, BuildReport *r) {
 // build_list until the list fits: the capacity a layout needs is the
 // fullest lane's count times the lanes per atom, so it can grow on a rebuild
 // and on a change of lanes per atom alike.  Sets npairs.
-int build_checked(parm_system *s, const void *at) {
+int build_checked(parm_system *s, const void *at, bool wrapped = false) {
     for (int attempt = 0; attempt < 4; attempt++) {
-        PARM_CHECK(build_list(s, at));
+        PARM_CHECK(build_list(s, at, wrapped));
         BuildReport r{};
         if (s->n == 0) {
             s->npairs = 0;
@@ -513,7 +538,7 @@ int build_checked(parm_system *s, const void *at) {
 // tile capacity as its grid.  The report then carries the plan: when the
 // plan fits the bounds (and the list its capacity) the build stands;
 // otherwise the plan is accepted as read and the list built again.
-int build_speculative(parm_system *s) {
+int build_speculative(parm_system *s, bool wrapped) {
     PARM_CHECK(check_lane_counts(s));
     const int pstride = force_blocks(std::max(s->n, 1), 8);
     const int grid = std::min(s->tiles_cap, pstride);
@@ -530,7 +555,7 @@ int build_speculative(parm_system *s) {
                                 s->box, s->skin, s->dmax, s->tpa, s->cap, s->npad, !tiled,
                                 s->nbr, s->ncount, s->lcount, s->xref, s->bpart, s->stats,
                                 s->dflag + kSlotBuild, s->tinfo, s->dmin == s->dmax,
-                                s->exview(), s->hrep_dev, s->stream));
+                                s->exview(), wrapped, s->hrep_dev, ++s->build_seq, s->stream));
     BuildReport r{};
     PARM_CHECK(read_report(s, &r));
     accept_tiles(s, r.ntiles, r.smax, r.bad);
@@ -542,7 +567,7 @@ int build_speculative(parm_system *s) {
         return PARM_OK;
     }
     if (fits) PARM_CHECK(ensure_list_capacity(s, (int)(r.max + r.max / 8 + 8)));
-    return build_checked(s, s->pos);
+    return build_checked(s, s->pos, wrapped);
 }
 
 // The exclusion CSR of s->excl on the device: for every atom (original
@@ -589,7 +614,9 @@ int upload_exclusions(parm_system *s) {
 
 // NeighborList::update_list's rebuild branch (src/trackers.cpp:55-69):
 // lastlocs = x, then the full pair list from the predicate.
-int rebuild(parm_system *s, bool keep_af = true) {
+// skin (inside a step loop): where the skin test of pos_alt against the new
+// reference positions leaves its partials.
+int rebuild(parm_system *s, bool keep_af = true, const ReduceBuf *skin = nullptr) {
     if (!s->list_cfg) return fail(PARM_E_STATE, "neighbour list not configured");
     PARM_CHECK(upload_exclusions(s));
     hipStream_t st = s->stream;
@@ -597,28 +624,49 @@ int rebuild(parm_system *s, bool keep_af = true) {
     make_grid(s);
     if (s->grid.ncell + 1 > s->cstart_cap) {
         dfree(s->cstart);
+        dfree(s->ccount);
+        dfree(s->ctotal);
         s->cstart_cap = s->grid.ncell + 1;
         PARM_CHECK(dalloc(&s->cstart, (size_t)s->cstart_cap));
+        PARM_CHECK(dalloc(&s->ccount, (size_t)s->cstart_cap));
+        PARM_CHECK(dalloc(&s->ctotal, (size_t)scan_tiles(s->cstart_cap)));
+        s->ccount_clear = false;
     }
     // from here on the previous list no longer matches the atom order
     s->built = false;
-    if (n > 0) {
-        PARM_HIP(launch_cell_keys(s->ndim, n, s->pos, s->rank, s->grid, s->keys, s->vals,
-                                  st));
-        int bits = 1;
-        while ((1u << bits) <= (uint32_t)s->grid.ncell && bits < 32) bits++;
-        PARM_HIP(radix_sort(n, bits, s->keys, s->vals, s->tkeys, s->tvals, s->hist, st));
-        PARM_CHECK(permute_all(s, s->vals, keep_af));
+    const bool counted = n > 0 && s->nmem == n;
+    if (counted) {
+        if (!s->ccount_clear)
+            PARM_HIP(hipMemsetAsync(s->ccount, 0, sizeof(uint32_t) * s->cstart_cap, st));
+        s->ccount_clear = false;
+        PARM_HIP(launch_cell_order(s->ndim, n, s->pos, s->grid, s->box, s->tkeys, s->tvals,
+                                   s->ccount, s->ctotal, s->cstart, s->vals, s->tinfo, st));
+        s->ccount_clear = true;
+        PARM_CHECK(permute_all(s, keep_af, true, skin));
+    } else {
+        if (n > 0) {
+            PARM_HIP(launch_cell_keys(s->ndim, n, s->pos, s->rank, s->grid, s->keys, s->vals,
+                                      s->tinfo, st));
+            int bits = 1;
+            while ((1u << bits) <= (uint32_t)s->grid.ncell && bits < 32) bits++;
+            PARM_HIP(radix_sort(n, bits, s->keys, s->vals, s->tkeys, s->tvals, s->hist, st));
+            PARM_CHECK(permute_all(s, keep_af, false, nullptr));
+        }
+        PARM_HIP(launch_cell_bounds(n, s->grid.ncell, s->keys, s->cstart, st));
     }
-    PARM_HIP(launch_cell_bounds(n, s->grid.ncell, s->keys, s->cstart, st));
     if (s->cap == 0) PARM_CHECK(ensure_list_capacity(s, initial_capacity(s)));
     PARM_CHECK(launch_tile_plan(s));
     if (n > 0 && s->spec_smax > 0) {
-        PARM_CHECK(build_speculative(s));
+        PARM_CHECK(build_speculative(s, counted));
     } else {
         PARM_CHECK(plan_tiles(s));
-        PARM_CHECK(build_checked(s, s->pos));
+        PARM_CHECK(build_checked(s, s->pos, counted));
         s->spec_smax = s->tile_ok ? s->smax : 0;
+    }
+    if (skin && !counted) {
+        AtomArrays A = s->arrays();
+        A.pos_in = s->pos_alt;
+        PARM_HIP(launch_skin(s->ndim, A, *skin, false, st));
     }
     s->built = true;
     s->which++;
@@ -949,18 +997,13 @@ int run_steps(parm_system *s, bool damped, const StepCoef &c, int64_t nsteps) {
                 ProfScope ps(s, &s->prof_rebuild);
                 // before the last step's end the next launch rewrites a and
                 // f before anything reads them: they need no permutation
-                PARM_CHECK(rebuild(s, last));
+                ReduceBuf R = s->redbuf(kSlotScratch);
+                R.part = pbuf[1 - cur];
+                PARM_CHECK(rebuild(s, last, last ? nullptr : &R));
             }
             xb[cur] = s->pos;
             xb[1 - cur] = s->pos_alt;
-            if (!last) {
-                AtomArrays A = s->arrays();
-                A.pos_in = s->pos_alt;
-                ReduceBuf R = s->redbuf(kSlotScratch);
-                R.part = pbuf[1 - cur];
-                PARM_HIP(launch_skin(s->ndim, A, R, false, st));
-                npart[1 - cur] = reduce_blocks(s->n);
-            }
+            npart[1 - cur] = reduce_blocks(s->n);
         }
     }
     return PARM_OK;
@@ -1039,6 +1082,8 @@ void destroy(parm_system *s) {
     dfree(s->vals);
     dfree(s->tvals);
     dfree(s->cstart);
+    dfree(s->ccount);
+    dfree(s->ctotal);
     dfree(s->tiles);
     dfree(s->truns);
     dfree(s->tinfo);
@@ -1266,6 +1311,7 @@ int parm_system_create(int ndim, int precision, int64_t natoms, const double *ma
     (void)hipMemsetAsync(s->dflag, 0, (2 * kFlagRing + 4) * sizeof(uint32_t), st);
     (void)hipMemsetAsync(s->fcnt, 0, sizeof(uint32_t), st);
     for (int k = 0; k < 2 * kFlagRing + 4; k++) s->hflag[k] = 0;
+    s->hrep->seq = 0;
     hipLaunchKernelGGL(k_iota, dim3(nb), dim3(256), 0, st, (int)n, s->orig);
     hipLaunchKernelGGL(k_fill_i32, dim3(nb), dim3(256), 0, st, (int)n, s->rank, -1);
     if (hipGetLastError() != hipSuccess || hipStreamSynchronize(st) != hipSuccess)

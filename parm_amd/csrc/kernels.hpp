@@ -22,7 +22,7 @@ struct CellGrid {
 // ---------------------------------------------------------------- nlist.hip
 int radix_blocks(int n);
 hipError_t launch_cell_keys(int ndim, int n, const void *pos, const int32_t *rank,
-                            const CellGrid &g, uint32_t *keys, int32_t *vals,
+                            const CellGrid &g, uint32_t *keys, int32_t *vals, int *info,
                             hipStream_t s);
 hipError_t radix_sort(int n, int bits, uint32_t *&keys, int32_t *&vals,
                       uint32_t *&tmp_keys, int32_t *&tmp_vals, uint32_t *hist,
@@ -43,6 +43,22 @@ struct PermuteSet {
 };
 hipError_t launch_permute(int ndim, int n, const int32_t *perm, const PermuteSet &P,
                           hipStream_t s);
+// Order by cell of a system whose atoms are all list members: the cells'
+// starts (cstart, ncell + 1) and atoms in arrival order (slot), then every
+// column into the stable order, the sorted keys, the wrapped positions and,
+// with skin, the partials (reduce_blocks(n)) of the skin test of pos_src[1]
+// against pos_src[0].  ukeys, arrival: n words of scratch; count: ncell words,
+// zero before and after; total: scan_tiles(ncell) words.
+int scan_tiles(int ncell);
+struct ReduceBuf;
+hipError_t launch_cell_order(int ndim, int n, const void *pos, const CellGrid &g,
+                             const Box &box, uint32_t *ukeys, int32_t *arrival,
+                             uint32_t *count, uint32_t *total, int32_t *cstart, int32_t *slot,
+                             int *info, hipStream_t s);
+hipError_t launch_cell_permute(int ndim, int n, const int32_t *slot, const uint32_t *ukeys,
+                               const int32_t *cstart, const CellGrid &g, const Box &box,
+                               uint32_t *keys, void *xw, const PermuteSet &P,
+                               const ReduceBuf *skin, hipStream_t s);
 hipError_t launch_cell_bounds(int n, int ncell, const uint32_t *keys, int32_t *start,
                               hipStream_t s);
 // Outcome of one list build, stored by the build's last launch in pinned
@@ -53,6 +69,7 @@ struct BuildReport {
     unsigned long long sum, max;
     int ntiles, smax, bad;
     uint32_t flag;
+    uint32_t seq;  // the launch's number, stored last
 };
 
 // NeighborList::ignore exclusions (src/trackers.hpp:190-193): excluded
@@ -67,8 +84,9 @@ struct ExclView {
 };
 
 // Builds the full list (and xref = pos); stats[0] = sum of counts, stats[1] =
-// max count; part holds 2 * build_blocks(n) scratch words.  report: a
-// device-visible pinned BuildReport, or null.
+// max count; part holds 2 * build_blocks(n) scratch words.  wrapped: xw
+// already holds the wrapped positions.  report: a device-visible pinned
+// BuildReport, or null.
 int build_blocks(int n);
 hipError_t launch_build_list(int ndim, int n, const void *pos, void *xw,
                              const int32_t *rank, const double *diam, const int32_t *type,
@@ -77,15 +95,18 @@ hipError_t launch_build_list(int ndim, int n, const void *pos, void *xw,
                              int type_bits, int tpa, int cap, int npad, uint32_t *nbr,
                              int32_t *ncount, uint16_t *lcount, void *xref,
                              unsigned long long *part, unsigned long long *stats,
-                             uint32_t *flag, const ExclView &ex, BuildReport *report,
-                             hipStream_t s);
+                             uint32_t *flag, const ExclView &ex, bool wrapped,
+                             BuildReport *report, uint32_t seq, hipStream_t s);
 
-// Tiled layout (tiles.hpp).  launch_tiles fills tiles (cap_tiles records)
-// and info[0] = tiles, info[1] = largest staged stencil, info[2] != 0 when the
-// layout does not apply.
+// Tiled layout (tiles.hpp).  launch_tiles fills tiles (cap_tiles records) and,
+// info having been cleared by the ordering launches, info[0] = tiles and
+// info[2] != 0 when they exceed cap_tiles.
 hipError_t launch_tiles(int ndim, int n, const CellGrid &g, const uint32_t *keys,
                         const int32_t *cstart, int cap_tiles, int4 *tiles, int2 *truns,
                         int *info, hipStream_t s);
+// info[1] = largest stencil, info[2] |= one does not fit (launch_tiles leaves
+// info[1] alone; a speculative build's report carries both by itself).
+hipError_t launch_tile_extremes(const int4 *tiles, int *info, hipStream_t s);
 size_t tiled_build_lds(int smax);
 // spec == null: ntiles and smax are the plan's.  spec == the plan's info
 // (launch_tiles, not yet read by the host): ntiles and smax are bounds;
@@ -100,8 +121,8 @@ hipError_t launch_build_tiled(int ndim, int n, int ntiles, int smax, const int4 
                               int npad, bool out32, void *nbr, int32_t *ncount,
                               uint16_t *lcount, void *xref, unsigned long long *part,
                               unsigned long long *stats, uint32_t *flag, const int *spec,
-                              int uni, const ExclView &ex, BuildReport *report,
-                              hipStream_t s);
+                              int uni, const ExclView &ex, bool wrapped,
+                              BuildReport *report, uint32_t seq, hipStream_t s);
 hipError_t launch_tiled_to_global(int ndim, int ntiles, const int4 *tiles,
                                   const uint32_t *keys, const int32_t *cstart,
                                   const CellGrid &g, const uint16_t *nb16,

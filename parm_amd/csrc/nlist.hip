@@ -8,16 +8,26 @@
 // sort of the atoms by cell.  The sort also renumbers the device slots, so
 // atoms that are close in space are close in memory for the force gathers.
 //
-// Pipeline (one rebuild):
+// Pipeline (one rebuild), every atom a list member:
+//   k_cell_count     cell of each atom, counted; the atom's arrival number
+//   k_cell_scan      counts -> first slot of each cell (two launches when
+//                    there are many cells)
+//   k_cell_scatter   the atoms of each cell, in arrival order
+//   k_cell_permute   every per-slot array into the new order (each atom's place
+//                    in its cell from the number of the cell's atoms with a
+//                    smaller old slot: the stable order), the wrapped copies
+//                    and, inside a step loop, the skin test of the positions
+//                    one step ahead
+//   k_build_list<D>  full (both directions) list, ELL layout nbr[k*npad + i]
+// With non-members (sorted last) the order comes from a radix sort instead:
 //   k_cell_keys      key = cell of each member, ncell for non-members
 //   radix passes     k_radix_hist -> k_radix_scan -> k_radix_scatter (8 bits)
 //   k_permute        every per-slot array permuted into the new order
 //   k_cell_bounds    first slot of each cell
-//   k_build_list<D>  full (both directions) list, ELL layout nbr[k*npad + i]
 //
 // Tiled layout (tiles.hpp), used when every tile's stencil fits in LDS:
-//   k_tile_rows      rows of cells -> tiles of <= kTileAtoms atoms
-//   k_tile_sizes<D>  staged slots of each tile, their maximum
+//   k_tile_plan<D>   rows of cells -> tiles of <= kTileAtoms atoms, their
+//                    stencil runs and staged slots
 //   k_build_tiled<D> the tile's stencil staged in LDS, the same predicate
 //                    evaluated from LDS, 16-bit staged-slot entries
 #include <algorithm>
@@ -26,17 +36,84 @@
 
 #include "common.hpp"
 #include "kernels.hpp"
+#include "stepcore.hpp"
 #include "tiles.hpp"
 
 namespace parm {
 
 // ------------------------------------------------------------ cell keys
+// Cell of x, and x wrapped into [0, L) per component with the same floor.
+template <int D>
+__device__ __forceinline__ uint32_t cell_of(const Vec<D> &x, const CellGrid &g, const Box &box,
+                                            Vec<D> &w) {
+    uint32_t key = 0;
+#pragma unroll
+    for (int k = D - 1; k >= 0; k--) {
+        double s = x.c[k] * g.invL[k];
+        s -= floor(s);
+        w.c[k] = s * box.L[k];
+        int c = (int)(s * (double)g.nc[k]);
+        c = c < 0 ? 0 : (c >= g.nc[k] ? g.nc[k] - 1 : c);
+        key = key * (uint32_t)g.nc[k] + (uint32_t)c;
+    }
+    return key;
+}
+
+// ---------------------------------------------------- order by cell, counted
+// A rebuild is a chain of short launches, bound by their number and latency
+// more than by bytes: counting atoms per cell and placing each by its cell's
+// start takes 5 launches where a radix sort of the cell keys takes 8 (16-bit
+// keys) or 11, and the cell starts come with it.  The atomic counters give
+// arrival numbers in no fixed order; k_cell_permute restores the stable one.
+// With the tile plan in one launch, the wrapped copies and the skin re-test
+// inside the permutation, and the host polling the build's report, a rebuild
+// takes 7 launches where it took 14 to 18: 200 steps of 2,003 disks (a rebuild
+// every 6 steps) 4.22 -> 3.01 ms, 150 of 20,011 spheres 4.75 -> 3.28, 200 of
+// 262,144 disks 7.91 -> 6.04, 50 of 1M atoms 11.46 -> 11.34.
+template <int D>
+__global__ __launch_bounds__(kBlock) void k_cell_count(
+    int n, const typename PosStore<D>::T *__restrict__ pos, CellGrid g, Box box,
+    uint32_t *__restrict__ key, int32_t *__restrict__ arrival, uint32_t *__restrict__ count,
+    int *__restrict__ info) {
+    const int i = blockIdx.x * kBlock + threadIdx.x;
+    if (i < 3) info[i] = 0;  // the tile plan's totals (k_tile_plan)
+    const bool act = i < n;
+    uint32_t c = 0xffffffffu;
+    if (act) {
+        Vec<D> w;
+        c = cell_of<D>(PosStore<D>::load(pos[i]), g, box, w);
+        key[i] = c;
+    }
+    // neighbouring slots mostly share a cell (the order of the last rebuild):
+    // each run of equal cells in the wavefront adds its length once, not one
+    // by one to the same counter (78 -> 9 us at 1M atoms, 18 to a cell)
+    const int lane = threadIdx.x % kWave;
+    const uint32_t before = __shfl_up(c, 1);
+    const unsigned long long heads = __ballot(lane == 0 || before != c);
+    const unsigned long long upto = heads & (~0ull >> (kWave - 1 - lane));
+    const int head = kWave - 1 - __builtin_clzll(upto);
+    const unsigned long long after = head < kWave - 1 ? heads & (~0ull << (head + 1)) : 0ull;
+    const int end = after ? __builtin_ctzll(after) : kWave;
+    uint32_t at = 0;
+    if (act && lane == head) at = atomicAdd(count + c, (uint32_t)(end - head));
+    at = __shfl(at, head);
+    if (act) arrival[i] = (int32_t)at + lane - head;
+}
+
+__global__ __launch_bounds__(kBlock) void k_cell_scatter(
+    int n, const uint32_t *__restrict__ key, const int32_t *__restrict__ arrival,
+    const int32_t *__restrict__ cstart, int32_t *__restrict__ slot) {
+    const int i = blockIdx.x * kBlock + threadIdx.x;
+    if (i < n) slot[cstart[key[i]] + arrival[i]] = i;
+}
+
 template <int D>
 __global__ __launch_bounds__(kBlock) void k_cell_keys(
     int n, const typename PosStore<D>::T *__restrict__ pos,
     const int32_t *__restrict__ rank, CellGrid g, uint32_t *__restrict__ keys,
-    int32_t *__restrict__ vals) {
+    int32_t *__restrict__ vals, int *__restrict__ info) {
     int i = blockIdx.x * kBlock + threadIdx.x;
+    if (i < 3) info[i] = 0;  // the tile plan's totals (k_tile_plan)
     if (i >= n) return;
     vals[i] = i;
     if (rank[i] < 0) {
@@ -213,6 +290,119 @@ __global__ __launch_bounds__(kBlock) void k_permute(int n, const int32_t *__rest
 #pragma unroll
     for (int c = 0; c < kPermI; c++)
         if (c < P.ni) P.i_dst[c][i] = q[c];
+}
+
+// Exclusive scan of the ncell counts into cstart (cstart[ncell] = n), the
+// counts cleared for the next rebuild.  A workgroup takes kScanTile cells; the
+// sum before them is that of the smaller tiles' totals (k_cell_total) or, for
+// a single tile, zero.
+constexpr int kScanThreads = 1024, kScanPer = 4;
+constexpr int kScanTile = kScanThreads * kScanPer;
+
+__global__ __launch_bounds__(kScanThreads) void k_cell_total(int ncell,
+                                                             const uint32_t *__restrict__ count,
+                                                             uint32_t *__restrict__ total) {
+    uint32_t v = 0;
+#pragma unroll
+    for (int q = 0; q < kScanPer; q++) {
+        const int c = blockIdx.x * kScanTile + q * kScanThreads + threadIdx.x;
+        if (c < ncell) v += count[c];
+    }
+    uint32_t t = 0;
+    (void)block_excl_scan_u32<kScanThreads>(v, t);
+    if (threadIdx.x == 0) total[blockIdx.x] = t;
+}
+
+__global__ __launch_bounds__(kScanThreads) void k_cell_scan(int ncell, int n,
+                                                            uint32_t *__restrict__ count,
+                                                            const uint32_t *__restrict__ total,
+                                                            int32_t *__restrict__ cstart) {
+    uint32_t before = 0;
+    if (blockIdx.x > 0) {
+        uint32_t v = 0;
+        for (int b = threadIdx.x; b < (int)blockIdx.x; b += kScanThreads) v += total[b];
+        (void)block_excl_scan_u32<kScanThreads>(v, before);
+    }
+    const int c0 = blockIdx.x * kScanTile + (int)threadIdx.x * kScanPer;
+    uint32_t v[kScanPer], sum = 0, all = 0;
+#pragma unroll
+    for (int q = 0; q < kScanPer; q++) {
+        v[q] = c0 + q < ncell ? count[c0 + q] : 0u;
+        sum += v[q];
+    }
+    uint32_t run = before + block_excl_scan_u32<kScanThreads>(sum, all);
+#pragma unroll
+    for (int q = 0; q < kScanPer; q++) {
+        if (c0 + q < ncell) {
+            cstart[c0 + q] = (int32_t)run;
+            count[c0 + q] = 0u;
+        }
+        run += v[q];
+    }
+    if (blockIdx.x == 0 && threadIdx.x == 0) cstart[ncell] = n;
+}
+
+// Thread p takes the atom i at place p of its cell's arrival order to its
+// place in the stable order: the cell's start plus the number of the cell's
+// atoms from smaller old slots (a cell's atoms are few, and the list build
+// tests each against 27 cells of them).  SKIN: pos_src[1] holds the positions
+// one step ahead, whose skin test against the new reference positions (this
+// rebuild's) leaves its partials in R.
+template <int D, bool SKIN>
+__global__ __launch_bounds__(kBlock) void k_cell_permute(
+    int n, const int32_t *__restrict__ slot, const uint32_t *__restrict__ key,
+    const int32_t *__restrict__ cstart, CellGrid g, Box box, uint32_t *__restrict__ keys,
+    typename PosStore<D>::T *__restrict__ xw, PermuteSet P, ReduceBuf R) {
+    using PT = typename PosStore<D>::T;
+    const int p = blockIdx.x * kBlock + threadIdx.x;
+    Top2 top;
+    double nonfinite = 0.0;
+    if (p < n) {
+        const int i = slot[p];
+        const uint32_t c = key[i];
+        // every load first, then every store: the gathers are in flight together
+        const PT x0 = static_cast<const PT *>(P.pos_src[0])[i];
+        const PT x1 = static_cast<const PT *>(P.pos_src[1])[i];
+        double d[kPermD];
+        int32_t q[kPermI];
+#pragma unroll
+        for (int k = 0; k < kPermD; k++)
+            if (k < P.nd) d[k] = P.d_src[k][i];
+#pragma unroll
+        for (int k = 0; k < kPermI; k++)
+            if (k < P.ni) q[k] = P.i_src[k][i];
+        const int s0 = cstart[c], s1 = cstart[c + 1];
+        int to = s0;
+        for (int k = s0; k < s1; k++) to += slot[k] < i ? 1 : 0;
+        Vec<D> w;
+        (void)cell_of<D>(PosStore<D>::load(x0), g, box, w);
+        keys[to] = c;
+        xw[to] = PosStore<D>::make(w);
+        static_cast<PT *>(P.pos_dst[0])[to] = x0;
+        static_cast<PT *>(P.pos_dst[1])[to] = x1;
+#pragma unroll
+        for (int k = 0; k < kPermD; k++)
+            if (k < P.nd) P.d_dst[k][to] = d[k];
+#pragma unroll
+        for (int k = 0; k < kPermI; k++)
+            if (k < P.ni) P.i_dst[k][to] = q[k];
+        if (SKIN) {
+            const Vec<D> xa = PosStore<D>::load(x1), xr = PosStore<D>::load(x0);
+            Vec<D> dd;
+#pragma unroll
+            for (int k = 0; k < D; k++) dd.c[k] = xa.c[k] - xr.c[k];
+            const double dist = sqrt(sqnorm<D>(dd));
+            top.add(dist);
+            if (!isfinite(dist)) nonfinite += 1.0;
+        }
+    }
+    if (SKIN) {
+        double v[kRedWidth];
+#pragma unroll
+        for (int k = 0; k < kRedWidth; k++) v[k] = 0.0;
+        v[kNonFinite] = nonfinite;
+        block_partial<false, true, kBlock / kWave>(v, top, R, blockIdx.x);
+    }
 }
 
 // ---------------------------------------------------------- cell bounds
@@ -460,135 +650,150 @@ __global__ __launch_bounds__(kBlock) void k_build_list(
 }
 
 // ------------------------------------------------------------ row tiles
-// One workgroup of 1024 threads.  Row r (cells r*nc0 .. r*nc0 + nc0 - 1)
-// holds atoms cstart[r*nc0] .. cstart[(r+1)*nc0]; it is cut into
-// ceil(n_r / kTileAtoms) tiles in order.  Non-members (slots from
-// cstart[ncell] on) get tail tiles.  info[0] = number of tiles (0 and
-// info[2] |= 1 if they exceed cap_tiles).
-constexpr int kTileScan = 1024;
+// Row r (cells r*nc0 .. r*nc0 + nc0 - 1) holds atoms cstart[r*nc0] ..
+// cstart[(r+1)*nc0]; it is cut into ceil(n_r / kTileAtoms) tiles in order.
+// Non-members (slots from cstart[ncell] on) get tail tiles.  info[0] = number
+// of tiles, info[2] != 0: they exceed cap_tiles (info is cleared before).  A
+// tile whose stencil is wider than kTileWMax cells or holds more than
+// kTileMaxSlots atoms has S = -1 (tile_extremes finds them); the system then
+// uses the untiled layout.
+//
+// One launch: a workgroup takes `per` rows (the last one the tail too) and
+// counts the tiles of the rows before them itself, a few loads per thread;
+// kPlanLanes lanes work out one tile's runs together, one run each.  The chain
+// of dependent loads bounds it, so a workgroup takes one row until there are
+// more than kPlanGroups of them (1,521 rows at 1M atoms: eight rows each 32
+// us, one 10 us; as two launches, one workgroup laying out the rows and a
+// thread per tile, 26 us).
+constexpr int kPlanMaxRows = 64, kPlanGroups = 2048, kPlanLanes = 32;
+static_assert(kPlanLanes >= kTileRuns, "a lane per run");
 
-__device__ __forceinline__ int block_excl_scan(int v, int &total) {
-    __shared__ int wsum[kTileScan / kWave];
-    const int lane = threadIdx.x % kWave, w = threadIdx.x / kWave;
-    int incl = v;
-#pragma unroll
-    for (int o = 1; o < kWave; o <<= 1) {
-        const int y = __shfl_up(incl, o);
-        if (lane >= o) incl += y;
-    }
-    if (lane == kWave - 1) wsum[w] = incl;
-    __syncthreads();
-    int before = 0;
-    total = 0;
-    for (int q = 0; q < kTileScan / kWave; q++) {
-        const int ws = wsum[q];
-        if (q < w) before += ws;
-        total += ws;
-    }
-    __syncthreads();
-    return before + incl - v;
+__device__ __forceinline__ int row_tiles(const int32_t *cstart, int r, int nc0) {
+    return (cstart[(r + 1) * nc0] - cstart[r * nc0] + kTileAtoms - 1) / kTileAtoms;
 }
 
-__global__ __launch_bounds__(kTileScan) void k_tile_rows(
-    int n, int nrows, int nc0, int ncell, const int32_t *__restrict__ cstart,
-    int cap_tiles, TileRec *__restrict__ tiles, int *__restrict__ info) {
-    int base = 0;
-    for (int r0 = 0; r0 < nrows; r0 += kTileScan) {
-        const int r = r0 + (int)threadIdx.x;
-        int a = 0, cnt = 0, nt = 0;
-        if (r < nrows) {
-            a = cstart[r * nc0];
-            cnt = cstart[(r + 1) * nc0] - a;
-            nt = (cnt + kTileAtoms - 1) / kTileAtoms;
-        }
-        int total = 0;
-        const int off = base + block_excl_scan(nt, total);
-        for (int q = 0; q < nt; q++) {
-            const int idx = off + q;
-            if (idx < cap_tiles)
-                tiles[idx] = TileRec{a + q * kTileAtoms,
-                                     min(kTileAtoms, cnt - q * kTileAtoms), r, 0};
-        }
-        base += total;
-    }
-    const int m0 = cstart[ncell];
-    const int ntail = (n - m0 + kTileAtoms - 1) / kTileAtoms;
-    for (int q = (int)threadIdx.x; q < ntail; q += kTileScan) {
-        const int idx = base + q;
-        if (idx < cap_tiles)
-            tiles[idx] = TileRec{m0 + q * kTileAtoms, min(kTileAtoms, n - m0 - q * kTileAtoms),
-                                 -1, 0};
-    }
-    if (threadIdx.x == 0) {
-        const int nt = base + ntail;
-        info[0] = nt <= cap_tiles ? nt : 0;
-        info[1] = 0;
-        info[2] = nt <= cap_tiles ? 0 : 1;
-    }
-}
-
-// One thread per tile: stencil width and staged slots.  A tile whose stencil
-// is wider than kTileWMax cells or holds more than kTileMaxSlots atoms marks
-// info[2]; the system then uses the untiled layout.
 template <int D>
-__global__ __launch_bounds__(kBlock) void k_tile_sizes(int cap_tiles, CellGrid g,
-                                                       const uint32_t *__restrict__ keys,
-                                                       const int32_t *__restrict__ cstart,
-                                                       TileRec *__restrict__ tiles,
-                                                       int2 *__restrict__ truns,
-                                                       int *__restrict__ info) {
-    const int t = blockIdx.x * kBlock + threadIdx.x;
-    const int nt = info[0];
-    int S = 0, bad = 0;
-    if (t < nt && t < cap_tiles) {
-        TileRec T = tiles[t];
-        int2 *runs = truns + (size_t)t * kTileRuns;
-        int nr = 0;
-        if (T.z >= 0 && T.y > 0) {
-            int xa = (int)(keys[T.x] % (uint32_t)g.nc[0]);
-            const int xb = (int)(keys[T.x + T.y - 1] % (uint32_t)g.nc[0]);
+__global__ __launch_bounds__(kBlock) void k_tile_plan(
+    int n, int nrows, int per, CellGrid g, const uint32_t *__restrict__ keys,
+    const int32_t *__restrict__ cstart, int cap_tiles, TileRec *__restrict__ tiles,
+    int2 *__restrict__ truns, int *__restrict__ info) {
+    __shared__ int first[kPlanMaxRows + 2];  // first tile of each row, relative
+    const int nc0 = g.nc[0];
+    const int r0 = blockIdx.x * per, r1 = min(nrows, r0 + per);
+    const bool lastb = blockIdx.x == gridDim.x - 1;
+    uint32_t v = 0, base = 0;
+    for (int r = threadIdx.x; r < r0; r += kBlock) v += (uint32_t)row_tiles(cstart, r, nc0);
+    (void)block_excl_scan_u32<kBlock>(v, base);
+    const int m0 = cstart[g.ncell];
+    const int ntail = lastb ? (n - m0 + kTileAtoms - 1) / kTileAtoms : 0;
+    if ((int)threadIdx.x < per)
+        first[threadIdx.x] =
+            r0 + (int)threadIdx.x < r1 ? row_tiles(cstart, r0 + (int)threadIdx.x, nc0) : 0;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        int t = 0;
+        for (int q = 0; q < per; q++) {
+            const int c = first[q];
+            first[q] = t;
+            t += c;
+        }
+        first[per] = t;
+        first[per + 1] = t + ntail;
+        if (lastb) {
+            const int nt = (int)base + t + ntail;
+            info[0] = nt <= cap_tiles ? nt : 0;
+            if (nt > cap_tiles) info[2] = 1;
+        }
+    }
+    __syncthreads();
+    const int rowt = first[per], all = first[per + 1];
+    const int lane = threadIdx.x % kPlanLanes;
+    for (int q = threadIdx.x / kPlanLanes; q < all; q += kBlock / kPlanLanes) {
+        const int idx = (int)base + q;
+        if (idx >= cap_tiles) break;
+        TileRec T;
+        int g0 = 0, len = 0, wide = 0;
+        if (q < rowt) {
+            int r = r0;
+            while (first[r - r0 + 1] <= q) r++;
+            const int a = cstart[r * nc0], cnt = cstart[(r + 1) * nc0] - a;
+            const int at = (q - first[r - r0]) * kTileAtoms;
+            T = TileRec{a + at, min(kTileAtoms, cnt - at), r, 0};
+            int xa = (int)(keys[T.x] % (uint32_t)nc0);
+            const int xb = (int)(keys[T.x + T.y - 1] % (uint32_t)nc0);
             int W = 0;
             const int xfull = stencil_x(g, xa, xb, W);
-            if (W > kTileWMax) {
-                bad = 1;
-            } else {
-                const int cy = D >= 2 ? T.z % g.nc[1] : 0;
-                const int cz = D == 3 ? T.z / g.nc[1] : 0;
-                const int NR = stencil_ny<D>(g) * stencil_nz<D>(g);
-                // per stencil row: the cells before / after the wrap along x
-                const int ustar = stencil_ustar(g, xa, W, xfull);
-                for (int k = 0; k < NR; k++) {
-                    for (int h = 0; h < 2; h++) {
-                        const int u0 = h == 0 ? 0 : ustar, u1 = h == 0 ? ustar : W;
-                        int g0 = 0, len = 0;
-                        if (u1 > u0) {
-                            int img[3];
-                            const int c0 = stencil_cell<D>(g, cy, cz, xa, k, u0, img);
-                            const int c1 = stencil_cell<D>(g, cy, cz, xa, k, u1 - 1, img);
-                            g0 = cstart[c0];
-                            len = cstart[c1 + 1] - g0;
-                        }
-                        runs[nr++] = int2{g0, S};
-                        S += len;
-                    }
-                }
-                if (S > kTileMaxSlots) bad = 1;
+            wide = W > kTileWMax ? 1 : 0;
+            // run lane: stencil row lane / 2, the cells before (even) or from
+            // (odd) the wrap along x
+            const int ustar = stencil_ustar(g, xa, W, xfull);
+            const int u0 = (lane & 1) ? ustar : 0, u1 = (lane & 1) ? W : ustar;
+            if (lane / 2 < stencil_ny<D>(g) * stencil_nz<D>(g) && u1 > u0) {
+                const int cy = D >= 2 ? r % g.nc[1] : 0, cz = D == 3 ? r / g.nc[1] : 0;
+                int img[3];
+                const int c0 = stencil_cell<D>(g, cy, cz, xa, lane / 2, u0, img);
+                const int c1 = stencil_cell<D>(g, cy, cz, xa, lane / 2, u1 - 1, img);
+                g0 = cstart[c0];
+                len = cstart[c1 + 1] - g0;
             }
+        } else {
+            const int at = (q - rowt) * kTileAtoms;
+            T = TileRec{m0 + at, min(kTileAtoms, n - m0 - at), -1, 0};
         }
-        for (; nr < kTileRuns; nr++) runs[nr] = int2{0, S};
-        T.w = bad ? -1 : S;
-        tiles[t] = T;
+        int incl = len;
+#pragma unroll
+        for (int o = 1; o < kPlanLanes; o <<= 1) {
+            const int y = __shfl_up(incl, o, kPlanLanes);
+            if (lane >= o) incl += y;
+        }
+        const int S = __shfl(incl, kPlanLanes - 1, kPlanLanes);
+        const int b = (wide || S > kTileMaxSlots) ? 1 : 0;
+        // a tile whose stencil is too wide keeps no runs
+        if (lane < kTileRuns)
+            truns[(size_t)idx * kTileRuns + lane] = wide ? int2{0, 0} : int2{g0, incl - len};
+        T.w = b ? -1 : S;
+        if (lane == 0) tiles[idx] = T;
     }
-    // one atomic per wavefront
-    int smax = bad ? 0 : S;
+}
+
+// Largest staged stencil over the plan's tiles, and whether any does not fit
+// (one workgroup; the tiles' atomics on one word took 76 us at 1M atoms).
+constexpr int kStatsThreads = 1024;
+
+__device__ __forceinline__ void tile_extremes(const TileRec *__restrict__ tiles, int nt,
+                                              int &smax, int &bad) {
+    __shared__ int red[kStatsThreads / kWave][2];
+    smax = 0;
+    bad = 0;
+#pragma unroll 4
+    for (int t = threadIdx.x; t < nt; t += kStatsThreads) {
+        const int S = tiles[t].w;
+        smax = max(smax, S);
+        bad |= S < 0 ? 1 : 0;
+    }
 #pragma unroll
     for (int o = kWave / 2; o > 0; o >>= 1) {
         smax = max(smax, __shfl_xor(smax, o));
         bad |= __shfl_xor(bad, o);
     }
     if (threadIdx.x % kWave == 0) {
-        if (smax > 0) atomicMax(info + 1, smax);
-        if (bad) atomicOr(info + 2, 1);
+        red[threadIdx.x / kWave][0] = smax;
+        red[threadIdx.x / kWave][1] = bad;
+    }
+    __syncthreads();
+    for (int q = 0; q < kStatsThreads / kWave; q++) {
+        smax = max(smax, red[q][0]);
+        bad |= red[q][1];
+    }
+}
+
+__global__ __launch_bounds__(kStatsThreads) void k_tile_extremes(
+    const TileRec *__restrict__ tiles, int *__restrict__ info) {
+    int smax, bad;
+    tile_extremes(tiles, info[0], smax, bad);
+    if (threadIdx.x == 0) {
+        info[1] = smax;
+        info[2] |= bad;
     }
 }
 
@@ -1058,13 +1263,14 @@ __global__ __launch_bounds__(kBlock) void k_wrap(int n,
     xw[i] = PosStore<D>::make(x);
 }
 
-constexpr int kStatsThreads = 1024;
-
 __global__ __launch_bounds__(kStatsThreads) void k_build_stats(
     int nparts, const unsigned long long *__restrict__ part,
     unsigned long long *__restrict__ stats, uint32_t *__restrict__ flag,
-    const int *__restrict__ info, BuildReport *report) {
+    const TileRec *__restrict__ tiles, const int *__restrict__ info, BuildReport *report,
+    uint32_t seq) {
     __shared__ unsigned long long red[kStatsThreads / kWave][2];
+    int smax = 0, bad = 0;
+    if (info) tile_extremes(tiles, info[0], smax, bad);
     unsigned long long sum = 0, mx = 0;
 #pragma unroll 4
     for (int b = threadIdx.x; b < nparts; b += kStatsThreads) {
@@ -1099,10 +1305,11 @@ __global__ __launch_bounds__(kStatsThreads) void k_build_stats(
             __hip_atomic_store(&report->flag, fl, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
             __hip_atomic_store(&report->ntiles, info ? info[0] : 0, __ATOMIC_RELAXED,
                                __HIP_MEMORY_SCOPE_SYSTEM);
-            __hip_atomic_store(&report->smax, info ? info[1] : 0, __ATOMIC_RELAXED,
+            __hip_atomic_store(&report->smax, smax, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+            __hip_atomic_store(&report->bad, info ? info[2] | bad : 0, __ATOMIC_RELAXED,
                                __HIP_MEMORY_SCOPE_SYSTEM);
-            __hip_atomic_store(&report->bad, info ? info[2] : 0, __ATOMIC_RELAXED,
-                               __HIP_MEMORY_SCOPE_SYSTEM);
+            // the host polls this word: it says that the others are there
+            __hip_atomic_store(&report->seq, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
         }
     }
 }
@@ -1111,15 +1318,61 @@ __global__ __launch_bounds__(kStatsThreads) void k_build_stats(
 static inline int nblk(long n) { return (int)((n + kBlock - 1) / kBlock); }
 
 hipError_t launch_cell_keys(int ndim, int n, const void *pos, const int32_t *rank,
-                            const CellGrid &g, uint32_t *keys, int32_t *vals,
+                            const CellGrid &g, uint32_t *keys, int32_t *vals, int *info,
                             hipStream_t s) {
     if (n <= 0) return hipSuccess;
     if (ndim == 3)
         hipLaunchKernelGGL(k_cell_keys<3>, dim3(nblk(n)), dim3(kBlock), 0, s, n,
-                           (const double4 *)pos, rank, g, keys, vals);
+                           (const double4 *)pos, rank, g, keys, vals, info);
     else
         hipLaunchKernelGGL(k_cell_keys<2>, dim3(nblk(n)), dim3(kBlock), 0, s, n,
-                           (const double2 *)pos, rank, g, keys, vals);
+                           (const double2 *)pos, rank, g, keys, vals, info);
+    return hipGetLastError();
+}
+
+int scan_tiles(int ncell) { return (ncell + kScanTile - 1) / kScanTile; }
+
+hipError_t launch_cell_order(int ndim, int n, const void *pos, const CellGrid &g,
+                             const Box &box, uint32_t *ukeys, int32_t *arrival,
+                             uint32_t *count, uint32_t *total, int32_t *cstart, int32_t *slot,
+                             int *info, hipStream_t s) {
+    if (ndim == 3)
+        hipLaunchKernelGGL(k_cell_count<3>, dim3(nblk(n)), dim3(kBlock), 0, s, n,
+                           (const double4 *)pos, g, box, ukeys, arrival, count, info);
+    else
+        hipLaunchKernelGGL(k_cell_count<2>, dim3(nblk(n)), dim3(kBlock), 0, s, n,
+                           (const double2 *)pos, g, box, ukeys, arrival, count, info);
+    const int nt = scan_tiles(g.ncell);
+    if (nt > 1)
+        hipLaunchKernelGGL(k_cell_total, dim3(nt), dim3(kScanThreads), 0, s, g.ncell, count,
+                           total);
+    hipLaunchKernelGGL(k_cell_scan, dim3(nt), dim3(kScanThreads), 0, s, g.ncell, n, count, total,
+                       cstart);
+    hipLaunchKernelGGL(k_cell_scatter, dim3(nblk(n)), dim3(kBlock), 0, s, n, ukeys, arrival,
+                       cstart, slot);
+    return hipGetLastError();
+}
+
+hipError_t launch_cell_permute(int ndim, int n, const int32_t *slot, const uint32_t *ukeys,
+                               const int32_t *cstart, const CellGrid &g, const Box &box,
+                               uint32_t *keys, void *xw, const PermuteSet &P,
+                               const ReduceBuf *skin, hipStream_t s) {
+    const ReduceBuf R = skin ? *skin : ReduceBuf{};
+#define PARM_CP(DD, PT, SK)                                                                   \
+    hipLaunchKernelGGL((k_cell_permute<DD, SK>), dim3(nblk(n)), dim3(kBlock), 0, s, n, slot, \
+                       ukeys, cstart, g, box, keys, (PT *)xw, P, R)
+    if (ndim == 3) {
+        if (skin)
+            PARM_CP(3, double4, true);
+        else
+            PARM_CP(3, double4, false);
+    } else {
+        if (skin)
+            PARM_CP(2, double2, true);
+        else
+            PARM_CP(2, double2, false);
+    }
+#undef PARM_CP
     return hipGetLastError();
 }
 
@@ -1196,44 +1449,50 @@ hipError_t launch_build_list(int ndim, int n, const void *pos, void *xw,
                              int type_bits, int tpa, int cap, int npad, uint32_t *nbr,
                              int32_t *ncount, uint16_t *lcount, void *xref,
                              unsigned long long *part, unsigned long long *stats,
-                             uint32_t *flag, const ExclView &ex, BuildReport *report,
-                             hipStream_t s) {
+                             uint32_t *flag, const ExclView &ex, bool wrapped,
+                             BuildReport *report, uint32_t seq, hipStream_t s) {
     if (n <= 0) return hipSuccess;
     const int nb = build_blocks(n);
     if (ndim == 3) {
-        hipLaunchKernelGGL(k_wrap<3>, dim3(nblk(n)), dim3(kBlock), 0, s, n,
+        if (!wrapped)
+            hipLaunchKernelGGL(k_wrap<3>, dim3(nblk(n)), dim3(kBlock), 0, s, n,
                            (const double4 *)pos, g, box, (double4 *)xw);
         hipLaunchKernelGGL((k_build_list<3, kBuildLanes, kBuildUnroll>), dim3(nb), dim3(kBlock), 0, s,
                            n, (const double4 *)pos, (const double4 *)xw, rank, diam, type,
                            keys, cstart, g, box, skin, dmax, type_bits, tpa, cap, npad,
                            nbr, ncount, lcount, (double4 *)xref, part, flag, ex);
     } else {
-        hipLaunchKernelGGL(k_wrap<2>, dim3(nblk(n)), dim3(kBlock), 0, s, n,
-                           (const double2 *)pos, g, box, (double2 *)xw);
+        if (!wrapped)
+            hipLaunchKernelGGL(k_wrap<2>, dim3(nblk(n)), dim3(kBlock), 0, s, n,
+                               (const double2 *)pos, g, box, (double2 *)xw);
         hipLaunchKernelGGL((k_build_list<2, kBuildLanes, kBuildUnroll>), dim3(nb), dim3(kBlock), 0, s,
                            n, (const double2 *)pos, (const double2 *)xw, rank, diam, type,
                            keys, cstart, g, box, skin, dmax, type_bits, tpa, cap, npad,
                            nbr, ncount, lcount, (double2 *)xref, part, flag, ex);
     }
     hipLaunchKernelGGL(k_build_stats, dim3(1), dim3(kStatsThreads), 0, s, nb, part, stats,
-                       flag, (const int *)nullptr, report);
+                       flag, (const TileRec *)nullptr, (const int *)nullptr, report, seq);
     return hipGetLastError();
 }
 
 // ------------------------------------------------------ tiled launchers
+hipError_t launch_tile_extremes(const TileRec *tiles, int *info, hipStream_t s) {
+    hipLaunchKernelGGL(k_tile_extremes, dim3(1), dim3(kStatsThreads), 0, s, tiles, info);
+    return hipGetLastError();
+}
+
 hipError_t launch_tiles(int ndim, int n, const CellGrid &g, const uint32_t *keys,
                         const int32_t *cstart, int cap_tiles, TileRec *tiles, int2 *truns,
                         int *info, hipStream_t s) {
     const int nrows = g.ncell / g.nc[0];
-    hipLaunchKernelGGL(k_tile_rows, dim3(1), dim3(kTileScan), 0, s, n, nrows, g.nc[0],
-                       g.ncell, cstart, cap_tiles, tiles, info);
-    const int nb = (cap_tiles + kBlock - 1) / kBlock;
+    const int per = std::min(kPlanMaxRows, std::max(1, nrows / kPlanGroups));
+    const int nb = (nrows + per - 1) / per;
     if (ndim == 3)
-        hipLaunchKernelGGL(k_tile_sizes<3>, dim3(nb), dim3(kBlock), 0, s, cap_tiles, g, keys,
-                           cstart, tiles, truns, info);
+        hipLaunchKernelGGL(k_tile_plan<3>, dim3(nb), dim3(kBlock), 0, s, n, nrows, per, g, keys,
+                           cstart, cap_tiles, tiles, truns, info);
     else
-        hipLaunchKernelGGL(k_tile_sizes<2>, dim3(nb), dim3(kBlock), 0, s, cap_tiles, g, keys,
-                           cstart, tiles, truns, info);
+        hipLaunchKernelGGL(k_tile_plan<2>, dim3(nb), dim3(kBlock), 0, s, n, nrows, per, g, keys,
+                           cstart, cap_tiles, tiles, truns, info);
     return hipGetLastError();
 }
 
@@ -1257,8 +1516,8 @@ hipError_t launch_build_tiled(int ndim, int n, int ntiles, int smax, const TileR
                               int npad, bool out32, void *nbr, int32_t *ncount,
                               uint16_t *lcount, void *xref, unsigned long long *part,
                               unsigned long long *stats, uint32_t *flag, const int *spec,
-                              int uni, const ExclView &ex, BuildReport *report,
-                              hipStream_t s) {
+                              int uni, const ExclView &ex, bool wrapped,
+                              BuildReport *report, uint32_t seq, hipStream_t s) {
     if (n <= 0 || ntiles <= 0) return hipSuccess;
     const size_t slot = (size_t)(uni ? ndim : ndim + 1) * sizeof(float);
     const size_t lds = (size_t)(smax + kBuildPad) * slot +
@@ -1289,16 +1548,18 @@ hipError_t launch_build_tiled(int ndim, int n, int ntiles, int smax, const TileR
         PARM_BT_S(DD, PT, O32, false) \
     }
     if (ndim == 3) {
-        hipLaunchKernelGGL(k_wrap<3>, dim3(nblk(n)), dim3(kBlock), 0, s, n,
-                           (const double4 *)pos, g, box, (double4 *)xw);
+        if (!wrapped)
+            hipLaunchKernelGGL(k_wrap<3>, dim3(nblk(n)), dim3(kBlock), 0, s, n,
+                               (const double4 *)pos, g, box, (double4 *)xw);
         if (out32) {
             PARM_BT_U(3, double4, true)
         } else {
             PARM_BT_U(3, double4, false)
         }
     } else {
-        hipLaunchKernelGGL(k_wrap<2>, dim3(nblk(n)), dim3(kBlock), 0, s, n,
-                           (const double2 *)pos, g, box, (double2 *)xw);
+        if (!wrapped)
+            hipLaunchKernelGGL(k_wrap<2>, dim3(nblk(n)), dim3(kBlock), 0, s, n,
+                               (const double2 *)pos, g, box, (double2 *)xw);
         if (out32) {
             PARM_BT_U(2, double2, true)
         } else {
@@ -1309,7 +1570,7 @@ hipError_t launch_build_tiled(int ndim, int n, int ntiles, int smax, const TileR
 #undef PARM_BT_S
 #undef PARM_BT
     hipLaunchKernelGGL(k_build_stats, dim3(1), dim3(kStatsThreads), 0, s, ntiles, part, stats,
-                       flag, spec, report);
+                       flag, tiles, spec, report, seq);
     return hipGetLastError();
 }
 

@@ -125,3 +125,36 @@ def test_tiled_lj_group_edges(monkeypatch, tpa, ntypes, n):
     first, last = O.nlist(x, L, diam, 0.3)
     S.assert_fp64_forces(s.forces(), O.forces(x, L, t, first, last), x, L, t, first, last)
     s.close()
+
+
+# the counted order and the tile plan: one and several scan tiles of cells,
+# several rows to a plan workgroup, crowded cells, empty rows, and a rebuild on
+# top of the order of the one before
+@pytest.mark.parametrize("n,ndim,edge,clustered", [
+    (1, 3, 9.0, False), (2, 2, 9.0, False), (63, 3, 4.0, False), (65, 2, 12.0, True),
+    (1500, 3, 40.0, False), (1500, 3, 40.0, True), (3000, 2, 150.0, False),
+    (70000, 3, 84.0, False)])
+def test_counted_order_and_tile_plan(n, ndim, edge, clustered):
+    _device_or_fail()
+    print(f"counted order n={n} ndim={ndim} edge={edge} clustered={clustered}", flush=True)
+    rng = np.random.default_rng(n + ndim)
+    L = np.full(ndim, edge)
+    x = rng.uniform(0, edge / (6 if clustered else 1), (n, ndim))
+    x += rng.integers(-2, 3, (n, ndim)) * edge
+    diam = rng.uniform(0.8, 1.0, n)
+    s = capi.System(ndim, np.ones(n))
+    s.set_box(L)
+    s.nlist_set(0.3, diam)
+    t = O.PairTable(O.REPULSION, [1.0], [1.0], [2.0], np.zeros(n, np.int32))
+    r = O.System(np.ones(n), L, t, diam, 0.3, ndim=ndim, brute=False)
+    for _ in range(2):
+        s.set_state(x=x)
+        r.set_state(x=x)
+        s.update_list(True)
+        r.update_list(True)
+        fd, ld = s.pairs()
+        fr, lr = r.pairs()
+        assert np.array_equal(fd, fr) and np.array_equal(ld, lr)
+        assert np.array_equal(s.positions(), x)
+        x = x + rng.normal(scale=0.4, size=x.shape)
+    s.close()
