@@ -170,7 +170,8 @@ struct parm_system {
     uint32_t *dflag = nullptr;      // flag words (see kSlot*)
     uint32_t *hflag = nullptr;      // pinned mirror, written by the kernels
     uint32_t *hflag_dev = nullptr;  // its device-side address
-    double *hout = nullptr;         // pinned mirror of out
+    SumRec *hrec = nullptr, *hrec_dev = nullptr;  // pinned records of the sums
+    unsigned long long sum_seq = 0;               // number of the last sums asked for
     double *part2 = nullptr;        // the step loop's skin partials alternate: part, part2
     uint32_t step_seq = 0;          // sequence number of the last step flag asked for
 
@@ -481,27 +482,45 @@ int build_list(parm_system *s, const void *at, bool wrapped) {
     return PARM_OK;
 }
 
-// The report of the build just queued, as soon as its last launch has stored
-// it (its number last): a poll of the pinned word answers sooner than a wait
-// for the stream.  The stream's state is asked for now and then, so the poll
-// ends also when the device reports an error or drains without a report.
-int read_report(parm_system *s, BuildReport *r) {
-    const volatile BuildReport *h = s->hrep;
+// Polls pinned memory until there() says that what the launches queued last
+// store has come: sooner than a wait for the stream answers.  The stream's
+// state is asked for now and then, so the poll ends also when the device
+// reports an error or the stream drains without it.
+template <typename There>
+int poll_pinned(parm_system *s, const char *what, const There &there) {
     bool drained = false;
     for (;;) {
-        bool there = false;
-        for (int k = 0; k < 1 << 14 && !there; k++) {
-            there = __atomic_load_n(&s->hrep->seq, __ATOMIC_ACQUIRE) == s->build_seq;
-            if (!there) __builtin_ia32_pause();
+        for (int k = 0; k < 1 << 14; k++) {
+            if (there()) return PARM_OK;
+            __builtin_ia32_pause();
         }
-        if (there) break;
-        if (drained) return fail(PARM_E_DEVICE, "a list build did not report");
+        if (drained) return fail(PARM_E_DEVICE, std::string(what) + " did not report");
         const hipError_t e = hipStreamQuery(s->stream);
         if (e == hipSuccess)
-            drained = true;  // one more look
+            drained = true;  // one more look: it was stored before the drain
         else if (e != hipErrorNotReady)
-            return fail(PARM_E_DEVICE, std::string("list build: ") + hipGetErrorString(e));
+            return fail(PARM_E_DEVICE, std::string(what) + ": " + hipGetErrorString(e));
     }
+}
+
+// The flags of a skin test: its pinned word holds the test's number (24 bits of
+// it) above the flag bits.
+int wait_flag(parm_system *s, int slot, uint32_t seq, uint32_t *flag) {
+    const volatile uint32_t *w = s->hflag + slot;
+    const uint32_t want = seq & (0xffffffffu >> kFlagBits);
+    return poll_pinned(s, "a skin test", [&]() {
+        const uint32_t v = *w;
+        *flag = v & ((1u << kFlagBits) - 1u);
+        return (v >> kFlagBits) == want;
+    });
+}
+
+// The report of the build just queued.
+int read_report(parm_system *s, BuildReport *r) {
+    PARM_CHECK(poll_pinned(s, "a list build", [&]() {
+        return __atomic_load_n(&s->hrep->seq, __ATOMIC_ACQUIRE) == s->build_seq;
+    }));
+    const volatile BuildReport *h = s->hrep;
     r->sum = h->sum;
     r->max = h->max;
     r->ntiles = h->ntiles;
@@ -674,21 +693,15 @@ int rebuild(parm_system *s, bool keep_af = true, const ReduceBuf *skin = nullptr
     return PARM_OK;
 }
 
-// Flag slot idx once the stream has finished: the skin-test launches store
-// it in the pinned mirror themselves (nothing ran for an empty system).
-int read_flag(parm_system *s, int idx, uint32_t *flag) {
-    PARM_HIP(hipStreamSynchronize(s->stream));
-    *flag = s->n > 0 ? *(volatile uint32_t *)(s->hflag + idx) : 0u;
-    return PARM_OK;
-}
-
 int update_list(parm_system *s, bool force, int *rebuilt) {
     if (rebuilt) *rebuilt = 0;
     if (!s->list_cfg) return fail(PARM_E_STATE, "neighbour list not configured");
     if (!force && !s->ignorechanged) {
-        PARM_HIP(launch_skin(s->ndim, s->arrays(), s->redbuf(kSlotSkin), true, s->stream));
+        ReduceBuf R = s->redbuf(kSlotSkin);
+        R.g.seq = ++s->step_seq;
+        PARM_HIP(launch_skin(s->ndim, s->arrays(), R, true, s->stream));
         uint32_t fl = 0;
-        PARM_CHECK(read_flag(s, kSlotSkin, &fl));
+        if (s->n > 0) PARM_CHECK(wait_flag(s, kSlotSkin, R.g.seq, &fl));
         if (fl & kFlagNonFinite)
             return fail(PARM_E_NONFINITE, "non-finite position in skin test");
         if (!(fl & kFlagRebuild)) return PARM_OK;
@@ -866,32 +879,6 @@ int autotune(parm_system *s, int stage, const StepCoef &c) {
     return PARM_OK;
 }
 
-// Waits for the pinned word that a step launch's reduction stores for
-// sequence number seq (24 bits of it above the flag bits); *flag = its flags.
-// The stream's state is asked for now and then, so the wait ends also when
-// the device reports an error or the stream drains without the word.
-int wait_step_flag(parm_system *s, int slot, uint32_t seq, uint32_t *flag) {
-    const volatile uint32_t *w = s->hflag + slot;
-    const uint32_t want = seq & (0xffffffffu >> kFlagBits);
-    bool drained = false;
-    for (;;) {
-        for (int k = 0; k < 1 << 14; k++) {
-            const uint32_t v = *w;
-            if ((v >> kFlagBits) == want) {
-                *flag = v & ((1u << kFlagBits) - 1u);
-                return PARM_OK;
-            }
-            __builtin_ia32_pause();
-        }
-        if (drained) return fail(PARM_E_DEVICE, "a step's skin test did not report");
-        const hipError_t e = hipStreamQuery(s->stream);
-        if (e == hipSuccess)
-            drained = true;  // one more look: the word was stored before the drain
-        else if (e != hipErrorNotReady)
-            return fail(PARM_E_DEVICE, std::string("step loop: ") + hipGetErrorString(e));
-    }
-}
-
 // Step launches queued beyond the oldest one whose flag the host waits for.
 // Small systems: a launch takes a few microseconds, less than a flag's trip to
 // the host and the launch that answers it, so the queue has to run ahead.
@@ -981,7 +968,7 @@ int run_steps(parm_system *s, bool damped, const StepCoef &c, int64_t nsteps) {
         const bool last = (q == nsteps - 1);
         const int cur = (int)(q & 1), slot = (int)(q % kFlagRing);
         uint32_t fl = 0;
-        PARM_CHECK(wait_step_flag(s, slot, seq[slot], &fl));
+        PARM_CHECK(wait_flag(s, slot, seq[slot], &fl));
         s->pos = xb[cur];
         s->pos_alt = xb[1 - cur];
         if (fl & kFlagNonFinite)
@@ -1039,17 +1026,29 @@ int upload_scalar(parm_system *s, const T *host, T *dst) {
     return PARM_OK;
 }
 
-// The reduction results of the launch just queued.  An empty system queues
-// no reduction: its sums are exactly zero (the device buffer is not read).
-int read_out(parm_system *s) {
-    if (s->n == 0) {
-        for (int k = 0; k < kRedWidth; k++) s->hout[k] = 0.0;
-        return PARM_OK;
-    }
-    PARM_HIP(hipMemcpyAsync(s->hout, s->out, sizeof(double) * kRedWidth,
-                            hipMemcpyDeviceToHost, s->stream));
-    PARM_HIP(hipStreamSynchronize(s->stream));
-    return PARM_OK;
+// Reduction scratch of a launch whose sums the host reads (read_sums).
+ReduceBuf sumbuf(parm_system *s) {
+    ReduceBuf R = s->redbuf(kSlotScratch);
+    R.rec = s->hrec_dev;
+    R.rseq = ++s->sum_seq;
+    return R;
+}
+
+// The sums of the launch just queued with sumbuf (fields 0 .. kRedWidth - 4,
+// with top the top-2 fields too).  An empty system queues no reduction: its
+// sums are exactly zero.
+int read_sums(parm_system *s, double (&out)[kRedWidth], bool top = false) {
+    for (double &v : out) v = 0.0;
+    if (s->n == 0) return PARM_OK;
+    const int nf = top ? kRedWidth : kRedWidth - 3;
+    int k = 0;  // fields seen so far
+    return poll_pinned(s, "a reduction", [&]() {
+        while (k < nf && __atomic_load_n(&s->hrec[k].seq, __ATOMIC_ACQUIRE) == s->sum_seq) {
+            out[k] = *(const volatile double *)&s->hrec[k].v;
+            k++;
+        }
+        return k == nf;
+    });
 }
 
 void destroy(parm_system *s) {
@@ -1101,7 +1100,7 @@ void destroy(parm_system *s) {
     dfree(s->dflag);
     if (s->hflag) (void)hipHostFree(s->hflag);
     if (s->hrep) (void)hipHostFree(s->hrep);
-    if (s->hout) (void)hipHostFree(s->hout);
+    if (s->hrec) (void)hipHostFree(s->hrec);
     for (parm_system::Snap &q : s->snap) {
         dfree(q.dev);
         if (q.host) (void)hipHostFree(q.host);
@@ -1291,7 +1290,9 @@ int parm_system_create(int ndim, int precision, int64_t natoms, const double *ma
         hipHostMalloc((void **)&s->hrep, sizeof(BuildReport),
                       hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess ||
         hipHostGetDevicePointer((void **)&s->hrep_dev, s->hrep, 0) != hipSuccess ||
-        hipHostMalloc((void **)&s->hout, kRedWidth * sizeof(double), 0) != hipSuccess ||
+        hipHostMalloc((void **)&s->hrec, kRedWidth * sizeof(SumRec),
+                      hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess ||
+        hipHostGetDevicePointer((void **)&s->hrec_dev, s->hrec, 0) != hipSuccess ||
         hipHostMalloc((void **)&s->htinfo, 4 * sizeof(int), 0) != hipSuccess)
         return bail(fail(PARM_E_NOMEM, "pinned host allocation failed"));
     hipStream_t st = s->stream;
@@ -1312,6 +1313,7 @@ int parm_system_create(int ndim, int precision, int64_t natoms, const double *ma
     (void)hipMemsetAsync(s->fcnt, 0, sizeof(uint32_t), st);
     for (int k = 0; k < 2 * kFlagRing + 4; k++) s->hflag[k] = 0;
     s->hrep->seq = 0;
+    for (int k = 0; k < kRedWidth; k++) s->hrec[k].seq = 0;
     hipLaunchKernelGGL(k_iota, dim3(nb), dim3(256), 0, st, (int)n, s->orig);
     hipLaunchKernelGGL(k_fill_i32, dim3(nb), dim3(256), 0, st, (int)n, s->rank, -1);
     if (hipGetLastError() != hipSuccess || hipStreamSynchronize(st) != hipSuccess)
@@ -1615,9 +1617,9 @@ int parm_pair_sums(parm_system *s, double *U, double *W, double *S, uint64_t *co
     PARM_CHECK(set_device(s));
     StepCoef c{};
     PARM_HIP(launch_force(s->ndim, s->prec, kStageSums, true, s->arrays(), s->listview(),
-                          s->pairview(), s->box, c, s->redbuf(kSlotScratch), s->stream));
-    PARM_CHECK(read_out(s));
-    const double *o = s->hout;
+                          s->pairview(), s->box, c, sumbuf(s), s->stream));
+    double o[kRedWidth];
+    PARM_CHECK(read_sums(s, o));
     if (U) *U = o[0];
     if (W) *W = o[1];
     if (S)
@@ -1707,36 +1709,36 @@ int parm_pair_sums_noalloc(parm_system *s, double *out) {
 int parm_kinetic_energy(parm_system *s, const double *originv, double *K) {
     PARM_CHECK(check_sys(s));
     PARM_CHECK(set_device(s));
-    ReduceBuf R = s->redbuf(kSlotScratch);
-    R.skin = INFINITY;
+    ReduceBuf R = sumbuf(s);
     PARM_HIP(launch_atom_sums(s->ndim, 0, s->arrays(), originv, R, s->stream));
-    PARM_CHECK(read_out(s));
-    if (K) *K = s->hout[0];
+    double o[kRedWidth];
+    PARM_CHECK(read_sums(s, o));
+    if (K) *K = o[0];
     return PARM_OK;
 }
 
 int parm_momentum(parm_system *s, double *p, double *mass) {
     PARM_CHECK(check_sys(s));
     PARM_CHECK(set_device(s));
-    ReduceBuf R = s->redbuf(kSlotScratch);
-    R.skin = INFINITY;
+    ReduceBuf R = sumbuf(s);
     PARM_HIP(launch_atom_sums(s->ndim, 0, s->arrays(), nullptr, R, s->stream));
-    PARM_CHECK(read_out(s));
+    double o[kRedWidth];
+    PARM_CHECK(read_sums(s, o));
     if (p)
-        for (int k = 0; k < s->ndim; k++) p[k] = s->hout[1 + k];
-    if (mass) *mass = s->hout[4];
+        for (int k = 0; k < s->ndim; k++) p[k] = o[1 + k];
+    if (mass) *mass = o[4];
     return PARM_OK;
 }
 
 int parm_force_stats(parm_system *s, double *fmax, double *fmean) {
     PARM_CHECK(check_sys(s));
     PARM_CHECK(set_device(s));
-    ReduceBuf R = s->redbuf(kSlotScratch);
-    R.skin = INFINITY;
+    ReduceBuf R = sumbuf(s);
     PARM_HIP(launch_atom_sums(s->ndim, 1, s->arrays(), nullptr, R, s->stream));
-    PARM_CHECK(read_out(s));
-    if (fmax) *fmax = s->hout[13];
-    if (fmean) *fmean = s->n > 0 ? s->hout[0] / s->n : 0.0;
+    double o[kRedWidth];
+    PARM_CHECK(read_sums(s, o, true));
+    if (fmax) *fmax = o[13];
+    if (fmean) *fmean = s->n > 0 ? o[0] / s->n : 0.0;
     return PARM_OK;
 }
 
@@ -1993,6 +1995,8 @@ struct parm_nlcg {
     // tracking
     double alpha = 0, beta = 0, betaused = 0, dxsum = 0, alphavmax = 0, maxdV = 0;
     unsigned sec = 0;
+    // the sums (nlcg.hpp) of the last force launch
+    double sums[kRedWidth] = {};
 };
 
 namespace {
@@ -2008,15 +2012,16 @@ double length_squared(const parm_system *s) {
     return s->ndim == 3 ? std::pow(box_V(s), 2.0 / 3.0) : box_V(s);
 }
 
-// One vector pass (assignment op, then the sums), read back.
-int nlcg_pass(parm_nlcg *c, int op, double beta, double lfac_all, double out[5]) {
+// One vector pass: the assignment op, then, with out, the sums read back.
+int nlcg_pass(parm_nlcg *c, int op, double beta, double lfac_all, double *out) {
     parm_system *s = c->s;
     const double lf[3] = {lfac_all, lfac_all, lfac_all};
-    ReduceBuf R = s->redbuf(kSlotScratch);
-    PARM_HIP(launch_nlcg_vec(s->ndim, op, s->arrays(), beta, lf, R, s->stream));
+    const ReduceBuf R = out ? sumbuf(s) : s->redbuf(kSlotScratch);
+    PARM_HIP(launch_nlcg_vec(s->ndim, op, s->arrays(), beta, lf, out != nullptr, R, s->stream));
     if (!out) return PARM_OK;
-    PARM_CHECK(read_out(s));
-    for (int q = 0; q < 5; q++) out[q] = s->hout[q];
+    double o[kRedWidth];
+    PARM_CHECK(read_sums(s, o));
+    for (int q = 0; q < 5; q++) out[q] = o[q];
     return PARM_OK;
 }
 
@@ -2039,30 +2044,20 @@ int nlcg_stepx(parm_nlcg *c, double dx) {
     return apply_box(s, L);
 }
 
-// Collection::set_forces_get_pressure(false) (src/collection.cpp:181-208):
-// f = pair forces, a = 0 for fixed atoms; returns sum r.f.
-int forces_get_pressure(parm_system *s, double *W) {
-    PARM_CHECK(set_forces(s, false));
-    double zero[3] = {1.0, 1.0, 1.0};
-    ReduceBuf R = s->redbuf(kSlotScratch);
-    PARM_HIP(launch_nlcg_vec(s->ndim, kNlcgFixedA0, s->arrays(), 0.0, zero, R, s->stream));
-    StepCoef cf{};
-    PARM_HIP(launch_force(s->ndim, s->prec, kStageSums, true, s->arrays(), s->listview(),
-                          s->pairview(), s->box, cf, s->redbuf(kSlotScratch), s->stream));
-    PARM_CHECK(read_out(s));
-    *W = s->hout[1];
-    return PARM_OK;
-}
-
 // CollectionNLCG::set_forces(constraints_and_a, setV) (src/collection.cpp:
-// 537-569).
+// 537-569); with setV its pair forces and pressure are
+// Collection::set_forces_get_pressure(false) (:181-208: f, a = 0 for fixed
+// atoms, sum r.f), one launch that also gives the point's dot products, kept
+// in c->sums.
 int nlcg_set_forces(parm_nlcg *c, bool constraints_and_a, bool setV) {
     parm_system *s = c->s;
     const double V = box_V(s);
     if (setV) {
-        double interacP = 0;
-        PARM_CHECK(forces_get_pressure(s, &interacP));
-        c->fl = ((interacP / s->ndim) - (c->P0 * V)) / c->kappa;
+        StepCoef cf{};
+        PARM_HIP(launch_force(s->ndim, s->prec, kStageNlcg, false, s->arrays(), s->listview(),
+                              s->pairview(), s->box, cf, sumbuf(s), s->stream));
+        PARM_CHECK(read_sums(s, c->sums));
+        c->fl = ((c->sums[kNlcgW] / s->ndim) - (c->P0 * V)) / c->kappa;
         if (constraints_and_a) {
             c->al = c->fl;
             c->vl = c->fl;
@@ -2078,15 +2073,16 @@ int nlcg_set_forces(parm_nlcg *c, bool constraints_and_a, bool setV) {
     return PARM_OK;
 }
 
-// fdotv / vdotv / fdota (src/collection.cpp:650-683) from one pass.
-int nlcg_dots(parm_nlcg *c, double *fdota, double *fdotv, double *vdotv) {
-    double o[5];
-    PARM_CHECK(nlcg_pass(c, kNlcgDots, 0.0, 1.0, o));
-    const double l2 = length_squared(c->s);
-    if (fdota) *fdota = o[kNlcgFA] / l2 + c->fl * c->al;
-    if (fdotv) *fdotv = o[kNlcgFV] / l2 + c->fl * c->vl;
-    if (vdotv) *vdotv = o[kNlcgVV] / l2 + c->vl * c->vl;
-    return PARM_OK;
+// fdota / fdotv / vdotv (src/collection.cpp:650-683) at the point of the last
+// nlcg_set_forces(c, false, true).
+double fdota(const parm_nlcg *c) {
+    return c->sums[kNlcgFA] / length_squared(c->s) + c->fl * c->al;
+}
+double fdotv(const parm_nlcg *c) {
+    return c->sums[kNlcgFV] / length_squared(c->s) + c->fl * c->vl;
+}
+double vdotv(const parm_nlcg *c) {
+    return c->sums[kNlcgVV] / length_squared(c->s) + c->vl * c->vl;
 }
 
 int nlcg_update_trackers(parm_nlcg *c) { return update_list(c->s, false, nullptr); }
@@ -2095,17 +2091,15 @@ int nlcg_update_trackers(parm_nlcg *c) { return update_list(c->s, false, nullptr
 int nlcg_timestep(parm_nlcg *c) {
     PARM_CHECK(nlcg_stepx(c, c->dt));
     PARM_CHECK(nlcg_set_forces(c, false, true));
-    double fv = 0;
-    PARM_CHECK(nlcg_dots(c, nullptr, &fv, nullptr));
-    double eta0 = -fv;  // slope at x0 - dt
+    double eta0 = -fdotv(c);  // slope at x0 - dt
     double eta;
     PARM_CHECK(nlcg_stepx(c, -c->dt));
     PARM_CHECK(nlcg_update_trackers(c));
     c->alpha = -c->dt;
     PARM_CHECK(nlcg_set_forces(c, false, true));
     c->dxsum = 0;
-    double vdv = 0;
-    PARM_CHECK(nlcg_dots(c, nullptr, &fv, &vdv));
+    double fv = fdotv(c);
+    const double vdv = vdotv(c);
     const int d = c->s->ndim;
     // secant steps along v until the slope along v is small
     for (c->sec = 0; c->sec < c->secmax; c->sec++) {
@@ -2142,17 +2136,14 @@ int nlcg_timestep(parm_nlcg *c) {
             break;
         }
         // the next iteration's slope (the reference's fdotv at its top)
-        PARM_CHECK(nlcg_dots(c, nullptr, &fv, nullptr));
+        fv = fdotv(c);
     }
     c->alphavmax = std::sqrt(c->alpha * c->alpha * vdv);
     const double Kold = c->Knew;
-    double Kmid = 0;
-    PARM_CHECK(nlcg_dots(c, &Kmid, nullptr, nullptr));
-    // a = f, al = fl, Knew = fdota
-    double o[5];
-    PARM_CHECK(nlcg_pass(c, kNlcgAssignA, 0.0, 1.0, o));
+    const double Kmid = fdota(c);
+    // a = f (with v below), al = fl, Knew = fdota, which is f.f now
     c->al = c->fl;
-    c->Knew = o[kNlcgFA] / length_squared(c->s) + c->fl * c->al;
+    c->Knew = c->sums[kNlcgFF] / length_squared(c->s) + c->fl * c->al;
     c->beta = (c->Knew - Kmid) / Kold;
     c->betaused = c->beta;
     c->k++;
@@ -2163,7 +2154,7 @@ int nlcg_timestep(parm_nlcg *c) {
     } else if (c->betaused > 1) {
         c->betaused = 1;
     }
-    PARM_CHECK(nlcg_pass(c, kNlcgAssignV, c->betaused, 1.0, nullptr));
+    PARM_CHECK(nlcg_pass(c, kNlcgConjugate, c->betaused, 1.0, nullptr));
     c->vl = c->al + c->betaused * c->vl;
     return PARM_OK;
 }

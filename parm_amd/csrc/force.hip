@@ -119,12 +119,12 @@ __global__ __launch_bounds__(kBlock) void k_force(AtomArrays A, ListView Lv,
     }
 
     Top2 top;
-    double nonfinite = 0.0;
+    double nonfinite = 0.0, dots[4] = {0.0, 0.0, 0.0, 0.0};
     if (act && sub == 0) {
         ain.x = xi;
-        atom_store<D, STAGE>(A, i, fi, ain, c, top, nonfinite);
+        atom_store<D, STAGE>(A, i, fi, ain, c, top, nonfinite, dots);
     }
-    group_partials<D, STAGE, ENERGY, kBlock / kWave>(acc, top, nonfinite, R, blk);
+    group_partials<D, STAGE, ENERGY, kBlock / kWave>(acc, top, nonfinite, dots, R, blk);
 }
 
 template <int D, int KIND, int PREC, bool SINGLE, bool HARM, int STAGE, int TPA>
@@ -133,8 +133,8 @@ static void launch_force_tt(bool energy, const AtomArrays &A, const ListView &Lv
                             const ReduceBuf &R, hipStream_t s) {
     constexpr bool DRIFT =
         (STAGE == kStageVerletKickDrift || STAGE == kStageDampedKickDrift);
-    // energies are accumulated by the sums stage only
-    constexpr bool ENERGY = STAGE == kStageSums;
+    // energies and virials are accumulated by these stages only
+    constexpr bool ENERGY = STAGE == kStageSums || STAGE == kStageNlcg;
     (void)energy;
     const int nb = force_blocks(A.n, TPA);
     constexpr bool STEP = DRIFT || STAGE == kStageVerletKick || STAGE == kStageDampedKick;
@@ -142,7 +142,7 @@ static void launch_force_tt(bool energy, const AtomArrays &A, const ListView &Lv
     hipLaunchKernelGGL((k_force<D, KIND, PREC, SINGLE, HARM, STAGE, ENERGY, TPA>), g, b, 0,
                        s, A, Lv, P, box, c, R);
     if (R.done) (void)hipEventRecord(R.done, s);
-    if (ENERGY) (void)launch_finalize_rt(true, false, nb, R, s);
+    if (ENERGY) (void)launch_finalize_sums(false, nb, R, s);
 }
 
 template <int D, int KIND, int PREC, bool SINGLE, bool HARM, int STAGE>
@@ -187,6 +187,7 @@ static void launch_force_s(int stage, bool energy, const AtomArrays &A,
         PARM_STAGE(kStageDampedKickDrift)
         PARM_STAGE(kStageSums)
         PARM_STAGE(kStageForceAdd)
+        PARM_STAGE(kStageNlcg)
 #undef PARM_STAGE
     }
 }

@@ -201,6 +201,7 @@ enum Stage : int {
     kStageDampedKickDrift = 5,
     kStageSums = 6,        // energy / virial / stress only, nothing written
     kStageForceAdd = 7,    // NListed::set_forces: f += pair forces
+    kStageNlcg = 8,        // f, a = 0 for fixed atoms, and the sums of nlcg.hpp
 };
 
 struct StepCoef {
@@ -220,7 +221,15 @@ struct StepGate {
     uint32_t seq;
 };
 
-// Reduction scratch: one partial per workgroup, reduced by k_finalize.
+// A reduced sum as the host reads it, in pinned memory: the value, then the
+// number of the reduction that stored it.
+struct SumRec {
+    double v;
+    unsigned long long seq;
+};
+
+// Reduction scratch: one partial per workgroup, reduced by k_finalize_sums (and
+// k_finalize, k_finalize_skin for a skin test on demand).
 struct ReduceBuf {
     double *part;                 // kRedWidth fields x pstride workgroups
     int pstride;                  // field stride (>= workgroups of any launch)
@@ -233,6 +242,8 @@ struct ReduceBuf {
     uint32_t *cnt;                // or null: the skin-test reduction over several
     double *gpart;                // workgroups (counter, kFinBlocks x 3 results)
     StepGate g;
+    SumRec *rec;                  // or null: device-visible pinned records of the sums
+    unsigned long long rseq;      // and their number
 };
 constexpr int kFinBlocks = 32;    // workgroups of the multi-workgroup skin reduction
 constexpr int kRedWidth = 16;     // U, W, S[9], contacts, overlaps, top1, top2, nonfinite
@@ -256,9 +267,8 @@ void force_part(int stage, bool energy, const AtomArrays &A, const ListView &Lv,
 template <int D, int KIND, int PREC>
 void force_tiled_part(int stage, const AtomArrays &A, const ListView &Lv, const PairView &P,
                       const Box &box, const StepCoef &c, const ReduceBuf &R, hipStream_t s);
-// k_finalize over nparts workgroup partials.
-hipError_t launch_finalize_rt(bool sums, bool skin, int nparts, const ReduceBuf &R,
-                              hipStream_t s);
+// The sums over nparts workgroup partials (and with top the top-2 fields).
+hipError_t launch_finalize_sums(bool top, int nparts, const ReduceBuf &R, hipStream_t s);
 // The drift leaves its skin-test partials (reduce_blocks(n) of them) to the
 // next step launch; launch_skin with finalize == false does the same.
 hipError_t launch_drift(int ndim, int stage, const AtomArrays &A, const StepCoef &c,

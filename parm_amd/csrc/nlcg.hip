@@ -5,8 +5,11 @@
 // The minimiser's scalar control flow (secant line search, Polak-Ribiere
 // beta, restarts) stays on the host: each of its steps needs one of these
 // O(N) passes over the device state, reduced with the deterministic
-// compensated partial sums the force kernels use (stepcore.hpp), so a step
-// costs a few launches and one read of four doubles.
+// compensated partial sums the force kernels use (stepcore.hpp).  The sums of
+// a line-search point (virial, f.f, f.a, f.v, v.v) come out of its force
+// launch (kStageNlcg): a point costs the move of the atoms, that launch, its
+// reduction and one answer to the host (four launches more and two copies before:
+// 10 iterations of 4,001 spheres 4.56 -> 1.58 ms).
 //
 // Reference behaviour restated (paths relative to the reference root):
 //   CollectionNLCG::stepx           src/collection.cpp:608-625
@@ -40,15 +43,6 @@ __global__ __launch_bounds__(kBlock) void k_nlcg_stepx(AtomArrays A, Vec<D> lfac
     pos[i] = PosStore<D>::make(x);
 }
 
-// Dot products in the reference's Eigen order for one atom.
-template <int D>
-__device__ __forceinline__ double dotv(const double (&p)[D], const double (&q)[D]) {
-    if constexpr (D == 3)
-        return (p[0] * q[0] + p[1] * q[1]) + p[2] * q[2];
-    else
-        return p[0] * q[0] + p[1] * q[1];
-}
-
 // One pass: the assignment `op` (NlcgOp), then, for atoms with a finite
 // positive mass, the partial sums f.f, f.a, f.v, v.v (fields 0..3) and
 // |v + x lfac|^2 (field 4).
@@ -75,25 +69,18 @@ __global__ __launch_bounds__(kBlock) void k_nlcg_vec(AtomArrays A, double beta, 
 #pragma unroll
             for (int k = 0; k < D; k++) a[k] = vv[k] = fixed ? 0.0 : f[k];
             wa = wv = true;
-        } else if (OP == kNlcgAssignA) {  // a = f
+        } else if (OP == kNlcgConjugate) {  // a = f, v = a + v * beta
 #pragma unroll
-            for (int k = 0; k < D; k++) a[k] = fixed ? 0.0 : f[k];
-            wa = true;
-        } else if (OP == kNlcgAssignV) {  // v = a + v * beta
-#pragma unroll
-            for (int k = 0; k < D; k++) vv[k] = fixed ? 0.0 : a[k] + vv[k] * beta;
-            wv = true;
+            for (int k = 0; k < D; k++) {
+                a[k] = fixed ? 0.0 : f[k];
+                vv[k] = fixed ? 0.0 : a[k] + vv[k] * beta;
+            }
+            wa = wv = true;
         } else if (OP == kNlcgDescend) {  // v = a = f (fixed atoms untouched)
             if (!fixed) {
 #pragma unroll
                 for (int k = 0; k < D; k++) a[k] = vv[k] = f[k];
                 wa = wv = true;
-            }
-        } else if (OP == kNlcgFixedA0) {  // a = 0 for fixed atoms
-            if (fixed) {
-#pragma unroll
-                for (int k = 0; k < D; k++) a[k] = 0.0;
-                wa = true;
             }
         }
         if (wa) {
@@ -144,31 +131,25 @@ static void nlcg_vec_d(int op, const AtomArrays &A, double beta, const Vec<D> &l
         case kNlcgAssignAV:
             hipLaunchKernelGGL((k_nlcg_vec<D, kNlcgAssignAV>), g, b, 0, s, A, beta, l, R);
             break;
-        case kNlcgAssignA:
-            hipLaunchKernelGGL((k_nlcg_vec<D, kNlcgAssignA>), g, b, 0, s, A, beta, l, R);
-            break;
-        case kNlcgAssignV:
-            hipLaunchKernelGGL((k_nlcg_vec<D, kNlcgAssignV>), g, b, 0, s, A, beta, l, R);
-            break;
-        case kNlcgDescend:
-            hipLaunchKernelGGL((k_nlcg_vec<D, kNlcgDescend>), g, b, 0, s, A, beta, l, R);
+        case kNlcgConjugate:
+            hipLaunchKernelGGL((k_nlcg_vec<D, kNlcgConjugate>), g, b, 0, s, A, beta, l, R);
             break;
         default:
-            hipLaunchKernelGGL((k_nlcg_vec<D, kNlcgFixedA0>), g, b, 0, s, A, beta, l, R);
+            hipLaunchKernelGGL((k_nlcg_vec<D, kNlcgDescend>), g, b, 0, s, A, beta, l, R);
             break;
     }
 }
 
 hipError_t launch_nlcg_vec(int ndim, int op, const AtomArrays &A, double beta,
-                           const double *lfac, const ReduceBuf &R, hipStream_t s) {
+                           const double *lfac, bool sums, const ReduceBuf &R, hipStream_t s) {
     if (A.n <= 0) return hipSuccess;
     if (ndim == 3)
         nlcg_vec_d<3>(op, A, beta, Vec<3>{{lfac[0], lfac[1], lfac[2]}}, R, s);
     else
         nlcg_vec_d<2>(op, A, beta, Vec<2>{{lfac[0], lfac[1]}}, R, s);
     hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    return launch_finalize_rt(true, false, reduce_blocks(A.n), R, s);
+    if (e != hipSuccess || !sums) return e;
+    return launch_finalize_sums(false, reduce_blocks(A.n), R, s);
 }
 
 }  // namespace parm

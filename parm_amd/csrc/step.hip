@@ -16,93 +16,132 @@
 
 namespace parm {
 
-// One workgroup of kFinal threads: thread t reduces partials t, t + kFinal,
-// ... of each field (Neumaier; the loads of a field are coalesced across the
-// workgroup), then a fixed butterfly per wave and a fixed combine over waves
-// (compensated two-sum), so the result is deterministic.
+// Sums: one workgroup per field (the last one, with TOP, takes the top-2 and
+// non-finite fields), so a field's partials are read by 256 threads on a CU of
+// their own: thread t adds partials t, t + 256, ... (Neumaier), then a fixed
+// butterfly per wave and a fixed combine over waves (compensated two-sum), so
+// the result is deterministic.  Each result goes to device memory and, for the
+// host, to a pinned record whose number says that it is there: the host polls
+// the records.  Latency bounds it: one workgroup of 1024 threads over all
+// fields took 17 us for 16 as for 16,384 partials, and the copy of the
+// results and the wait for the stream another 35.  6 frames of 100,003 atoms
+// (two reductions each) 1.84 -> 1.66 ms.
+constexpr int kFinSumThreads = 256;
+
+__device__ __forceinline__ void put_sum(const ReduceBuf &R, int k, double v) {
+    R.out[k] = v;
+    if (R.rec) {
+        __hip_atomic_store(&R.rec[k].v, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        __hip_atomic_store(&R.rec[k].seq, R.rseq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+}
+
+template <bool TOP>
+__global__ __launch_bounds__(kFinSumThreads) void k_finalize_sums(int nparts, ReduceBuf R) {
+    constexpr int NW = kFinSumThreads / kWave;
+    const int tid = threadIdx.x, lane = tid % kWave, w = tid / kWave;
+    const int k = blockIdx.x;
+    const size_t ps = (size_t)R.pstride;
+    __shared__ double fin[NW][3];
+    if (TOP && k == kTop1) {
+        Top2 t;
+        double nf = 0.0;
+#pragma unroll 4
+        for (int b = tid; b < nparts; b += kFinSumThreads) {
+            Top2 o;
+            o.a = R.part[kTop1 * ps + b];
+            o.b = R.part[kTop2 * ps + b];
+            t.merge(o);
+            nf += R.part[kNonFinite * ps + b];
+        }
+        t = wave_top2(t);
+        nf = wave_count(nf);
+        if (lane == 0) {
+            fin[w][0] = t.a;
+            fin[w][1] = t.b;
+            fin[w][2] = nf;
+        }
+        __syncthreads();
+        if (tid == 0) {
+            for (int q = 1; q < NW; q++) {
+                Top2 o;
+                o.a = fin[q][0];
+                o.b = fin[q][1];
+                t.merge(o);
+                nf += fin[q][2];
+            }
+            put_sum(R, kTop1, t.a);
+            put_sum(R, kTop2, t.b);
+            put_sum(R, kNonFinite, nf);
+        }
+        return;
+    }
+    KSum q;
+    const double *p = R.part + k * ps;
+#pragma unroll 8
+    for (int b = tid; b < nparts; b += kFinSumThreads) q.add(p[b]);
+    CSum c{q.s, q.c};
+#pragma unroll
+    for (int off = kWave / 2; off > 0; off >>= 1)
+        c = csum_merge(c, CSum{__shfl_xor(c.s, off), __shfl_xor(c.c, off)});
+    if (lane == 0) {
+        fin[w][0] = c.s;
+        fin[w][1] = c.c;
+    }
+    __syncthreads();
+    if (tid == 0) {
+        for (int v = 1; v < NW; v++) c = csum_merge(c, CSum{fin[v][0], fin[v][1]});
+        put_sum(R, k, c.s + c.c);
+    }
+}
+
+// The skin test on demand: one workgroup over the partials, the flag stored in
+// device memory and, with its number, in the pinned word the host polls.
 constexpr int kFinal = 1024;
 
-template <bool SUMS, bool SKIN>
 __global__ __launch_bounds__(kFinal) void k_finalize(int nparts, ReduceBuf R) {
     const int tid = threadIdx.x;
     const int lane = tid % kWave, w = tid / kWave;
     constexpr int NW = kFinal / kWave;
     const size_t ps = (size_t)R.pstride;
-    if constexpr (SUMS) {
-        CSum cs[kTop1];
-#pragma unroll 4
-        for (int b = tid; b < nparts; b += kFinal) {
-#pragma unroll
-            for (int k = 0; k < kTop1; k++) {
-                KSum q{cs[k].s, cs[k].c};
-                q.add(R.part[k * ps + b]);
-                cs[k] = CSum{q.s, q.c};
-            }
-        }
-#pragma unroll
-        for (int off = kWave / 2; off > 0; off >>= 1) {
-#pragma unroll
-            for (int k = 0; k < kTop1; k++) {
-                CSum o{__shfl_xor(cs[k].s, off), __shfl_xor(cs[k].c, off)};
-                cs[k] = csum_merge(cs[k], o);
-            }
-        }
-        __shared__ double fin[NW][2 * kTop1];
-        if (lane == 0) {
-#pragma unroll
-            for (int k = 0; k < kTop1; k++) {
-                fin[w][2 * k] = cs[k].s;
-                fin[w][2 * k + 1] = cs[k].c;
-            }
-        }
-        __syncthreads();
-        if (tid < kTop1) {
-            CSum tot;
-            for (int q = 0; q < NW; q++)
-                tot = csum_merge(tot, CSum{fin[q][2 * tid], fin[q][2 * tid + 1]});
-            R.out[tid] = tot.s + tot.c;
-        }
-    }
-    if constexpr (SKIN) {
-        Top2 bt;
-        double nf = 0.0;
-        // deep unroll: a partial array of ~10^4 workgroups is read in one or
-        // two rounds of loads in flight
+    Top2 bt;
+    double nf = 0.0;
+    // deep unroll: a partial array of ~10^4 workgroups is read in one or
+    // two rounds of loads in flight
 #pragma unroll 16
-        for (int b = tid; b < nparts; b += kFinal) {
+    for (int b = tid; b < nparts; b += kFinal) {
+        Top2 o;
+        o.a = R.part[kTop1 * ps + b];
+        o.b = R.part[kTop2 * ps + b];
+        bt.merge(o);
+        nf += R.part[kNonFinite * ps + b];
+    }
+    bt = wave_top2(bt);
+    nf = wave_count(nf);
+    __shared__ double fin2[NW][3];
+    if (lane == 0) {
+        fin2[w][0] = bt.a;
+        fin2[w][1] = bt.b;
+        fin2[w][2] = nf;
+    }
+    __syncthreads();
+    if (tid == 0) {
+        Top2 tt;
+        double nft = 0.0;
+        for (int q = 0; q < NW; q++) {
             Top2 o;
-            o.a = R.part[kTop1 * ps + b];
-            o.b = R.part[kTop2 * ps + b];
-            bt.merge(o);
-            nf += R.part[kNonFinite * ps + b];
+            o.a = fin2[q][0];
+            o.b = fin2[q][1];
+            tt.merge(o);
+            nft += fin2[q][2];
         }
-        bt = wave_top2(bt);
-        nf = wave_count(nf);
-        __shared__ double fin2[NW][3];
-        if (lane == 0) {
-            fin2[w][0] = bt.a;
-            fin2[w][1] = bt.b;
-            fin2[w][2] = nf;
-        }
-        __syncthreads();
-        if (tid == 0) {
-            Top2 tt;
-            double nft = 0.0;
-            for (int q = 0; q < NW; q++) {
-                Top2 o;
-                o.a = fin2[q][0];
-                o.b = fin2[q][1];
-                tt.merge(o);
-                nft += fin2[q][2];
-            }
-            R.out[kTop1] = tt.a;
-            R.out[kTop2] = tt.b;
-            R.out[kNonFinite] = nft;
-            const uint32_t fl = skin_flag(tt, nft, R.skin);
-            *R.flag = fl;
-            if (R.hflag)
-                __hip_atomic_store(R.hflag, fl, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-        }
+        R.out[kTop1] = tt.a;
+        R.out[kTop2] = tt.b;
+        R.out[kNonFinite] = nft;
+        const uint32_t fl = skin_flag(tt, nft, R.skin);
+        *R.flag = fl;
+        __hip_atomic_store(R.hflag, (R.g.seq << kFlagBits) | fl, __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_SYSTEM);
     }
 }
 
@@ -183,8 +222,8 @@ __global__ __launch_bounds__(kFinThreads) void k_finalize_skin(int nparts, Reduc
         R.out[kNonFinite] = nu;
         const uint32_t fl = skin_flag(u, nu, R.skin);
         *R.flag = fl;
-        if (R.hflag)
-            __hip_atomic_store(R.hflag, fl, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        __hip_atomic_store(R.hflag, (R.g.seq << kFlagBits) | fl, __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_SYSTEM);
     }
 }
 
@@ -193,14 +232,23 @@ __global__ __launch_bounds__(kFinThreads) void k_finalize_skin(int nparts, Reduc
 // step at 1000 atoms, +4 % at 32,768; -1.6 % at 1M atoms, 16,384 partials)
 constexpr int kFinMultiMin = 8 * kFinal;
 
-template <bool SUMS, bool SKIN>
 static void launch_finalize(int nparts, const ReduceBuf &R, hipStream_t s) {
-    if (!SUMS && SKIN && R.cnt && R.gpart && nparts >= kFinMultiMin) {
+    if (R.cnt && R.gpart && nparts >= kFinMultiMin) {
         const int G = std::max(1, std::min(kFinBlocks, (nparts + kFinThreads - 1) / kFinThreads));
         hipLaunchKernelGGL(k_finalize_skin, dim3(G), dim3(kFinThreads), 0, s, nparts, R);
         return;
     }
-    hipLaunchKernelGGL((k_finalize<SUMS, SKIN>), dim3(1), dim3(kFinal), 0, s, nparts, R);
+    hipLaunchKernelGGL(k_finalize, dim3(1), dim3(kFinal), 0, s, nparts, R);
+}
+
+hipError_t launch_finalize_sums(bool top, int nparts, const ReduceBuf &R, hipStream_t s) {
+    if (top)
+        hipLaunchKernelGGL(k_finalize_sums<true>, dim3(kTop1 + 1), dim3(kFinSumThreads), 0, s,
+                           nparts, R);
+    else
+        hipLaunchKernelGGL(k_finalize_sums<false>, dim3(kTop1), dim3(kFinSumThreads), 0, s,
+                           nparts, R);
+    return hipGetLastError();
 }
 
 // Standalone first half of a step (drift + half kick) and skin test.
@@ -339,17 +387,6 @@ int force_partials(int n, const ListView &Lv) {
     return Lv.tiled && Lv.built ? Lv.ntiles : force_blocks(n, Lv.tpa);
 }
 
-hipError_t launch_finalize_rt(bool sums, bool skin, int nparts, const ReduceBuf &R,
-                              hipStream_t s) {
-    if (sums && skin)
-        launch_finalize<true, true>(nparts, R, s);
-    else if (sums)
-        launch_finalize<true, false>(nparts, R, s);
-    else if (skin)
-        launch_finalize<false, true>(nparts, R, s);
-    return hipGetLastError();
-}
-
 size_t tiled_force_lds(int ndim, int prec, int kind, int ntypes, int smax) {
     const bool raw = prec == kFP64 && kind == kPairRepulsion;
     if (raw) return (size_t)smax * sizeof(double4);
@@ -441,11 +478,7 @@ hipError_t launch_atom_sums(int ndim, int mode, const AtomArrays &A,
         else
             hipLaunchKernelGGL((k_atom_sums<2, 1>), g, b, 0, s, A, ov, R);
     }
-    if (mode == 0)
-        launch_finalize<true, false>((int)g.x, R, s);
-    else
-        launch_finalize<true, true>((int)g.x, R, s);
-    return hipGetLastError();
+    return launch_finalize_sums(mode != 0, (int)g.x, R, s);
 }
 
 hipError_t launch_upload(int ndim, int what, const AtomArrays &A, const int32_t *orig,
@@ -478,7 +511,7 @@ hipError_t launch_skin(int ndim, const AtomArrays &A, const ReduceBuf &R, bool f
         hipLaunchKernelGGL((k_skin<3>), g, b, 0, s, A, R);
     else
         hipLaunchKernelGGL((k_skin<2>), g, b, 0, s, A, R);
-    if (finalize) launch_finalize<false, true>((int)g.x, R, s);
+    if (finalize) launch_finalize((int)g.x, R, s);
     return hipGetLastError();
 }
 

@@ -159,7 +159,7 @@ __global__ __launch_bounds__(kWave *TPA) void k_force_tiled(AtomArrays A, ListVi
                                                             PairView P, Box box, StepCoef c,
                                                             ReduceBuf R) {
     using PT = typename PosStore<D>::T;
-    constexpr bool ENERGY = STAGE == kStageSums;
+    constexpr bool ENERGY = STAGE == kStageSums || STAGE == kStageNlcg;
     constexpr bool RAW = PREC == kFP64 && KIND != kPairLJ;
     constexpr bool REL32 = PREC != kFP64 && KIND == kPairLJ;
     // COMPACT (LJ, or one pair type, offsets staged): a slot is the D offsets
@@ -665,7 +665,7 @@ __global__ __launch_bounds__(kWave *TPA) void k_force_tiled(AtomArrays A, ListVi
     // wavefront, one lane per atom (64 consecutive atoms: coalesced), with
     // the summed forces passed through LDS.
     Top2 top;
-    double nonfinite = 0.0;
+    double nonfinite = 0.0, dots[4] = {0.0, 0.0, 0.0, 0.0};
     if (STAGE != kStageSums) {
         __shared__ double fsum[D][kTileAtoms];
         if (act && sub == 0) {
@@ -677,10 +677,11 @@ __global__ __launch_bounds__(kWave *TPA) void k_force_tiled(AtomArrays A, ListVi
             double fa[D];
 #pragma unroll
             for (int k = 0; k < D; k++) fa[k] = fsum[k][threadIdx.x];
-            atom_store<D, STAGE>(A, a0 + (int)threadIdx.x, fa, ain, c, top, nonfinite);
+            atom_store<D, STAGE>(A, a0 + (int)threadIdx.x, fa, ain, c, top, nonfinite,
+                                 dots);
         }
     }
-    group_partials<D, STAGE, ENERGY, TPA, true>(acc, top, nonfinite, R, blk);
+    group_partials<D, STAGE, ENERGY, TPA, true>(acc, top, nonfinite, dots, R, blk);
 }
 
 // ======================================================== host launchers
@@ -691,14 +692,14 @@ void tiled_tt(const AtomArrays &A, const ListView &Lv, const PairView &P, const 
               const StepCoef &c, const ReduceBuf &R, hipStream_t s) {
     constexpr bool DRIFT =
         (STAGE == kStageVerletKickDrift || STAGE == kStageDampedKickDrift);
-    constexpr bool ENERGY = STAGE == kStageSums;
+    constexpr bool ENERGY = STAGE == kStageSums || STAGE == kStageNlcg;
     const size_t lds = tiled_force_lds(D, PREC, KIND, P.ntypes, Lv.smax);
     constexpr bool STEP = DRIFT || STAGE == kStageVerletKick || STAGE == kStageDampedKick;
     const int nb = Lv.ntiles + (STEP && R.g.nprev > 0 ? 1 : 0);
     hipLaunchKernelGGL((k_force_tiled<D, KIND, PREC, SINGLE, HARM, STAGE, TPA>),
                        dim3(nb), dim3(kWave * TPA), lds, s, A, Lv, P, box, c, R);
     if (R.done) (void)hipEventRecord(R.done, s);
-    if (ENERGY) (void)launch_finalize_rt(true, false, Lv.ntiles, R, s);
+    if (ENERGY) (void)launch_finalize_sums(false, Lv.ntiles, R, s);
 }
 
 template <int D, int KIND, int PREC, bool SINGLE, bool HARM, int STAGE>
@@ -736,6 +737,7 @@ void tiled_s(int stage, const AtomArrays &A, const ListView &Lv, const PairView 
         PARM_TSTAGE(kStageDampedKickDrift)
         PARM_TSTAGE(kStageSums)
         PARM_TSTAGE(kStageForceAdd)
+        PARM_TSTAGE(kStageNlcg)
 #undef PARM_TSTAGE
     }
 }

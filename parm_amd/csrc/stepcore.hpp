@@ -19,9 +19,9 @@ namespace parm {
 // ------------------------------------------------------ reductions
 // A kernel that reduces (sums of energy / virial / stress / counts, and the
 // skin test's top-2 and non-finite count) writes one partial per workgroup
-// with plain stores; k_finalize, launched right after it on the same stream,
-// reduces the partials in a fixed order (the step loop's skin test: the next
-// step launch, below).  (A last-workgroup reduction inside
+// with plain stores; k_finalize_sums, launched right after it on the same
+// stream, reduces the partials in a fixed order (the step loop's skin test: the
+// next step launch, below).  (A last-workgroup reduction inside
 // the launch would need a device-scope release per workgroup, which on a
 // multi-XCD part writes back the XCD's L2: far dearer than one more launch.)  No fences or contended atomics are
 // needed inside the hot kernel, and the result does not depend on scheduling.
@@ -108,10 +108,19 @@ __device__ __forceinline__ void skin_atom(const Vec<D> &x, const void *xref, int
 template <int D>
 struct AtomIn {
     double m;
-    double v[D];
+    double v[D], a[D];  // a: kStageNlcg only
     Vec<D> x, xref;
     bool member;
 };
+
+// Dot products in the reference's Eigen order for one atom.
+template <int D>
+__device__ __forceinline__ double dotv(const double (&p)[D], const double (&q)[D]) {
+    if constexpr (D == 3)
+        return (p[0] * q[0] + p[1] * q[1]) + p[2] * q[2];
+    else
+        return p[0] * q[0] + p[1] * q[1];
+}
 
 template <int D, int STAGE, bool LOADX = true>
 __device__ __forceinline__ void atom_load(const AtomArrays &A, int i, AtomIn<D> &in) {
@@ -124,6 +133,10 @@ __device__ __forceinline__ void atom_load(const AtomArrays &A, int i, AtomIn<D> 
 #pragma unroll
         for (int k = 0; k < D; k++) in.v[k] = A.v[k][i];
     }
+    if (STAGE == kStageNlcg) {
+#pragma unroll
+        for (int k = 0; k < D; k++) in.a[k] = A.a[k][i];
+    }
     if (DRIFT) {
         if (LOADX) in.x = PosStore<D>::load(static_cast<const PT *>(A.pos_in)[i]);
         in.member = A.rank[i] >= 0;
@@ -132,11 +145,12 @@ __device__ __forceinline__ void atom_load(const AtomArrays &A, int i, AtomIn<D> 
 }
 
 // The stage's writes for atom i with total pair force fi and inputs `in`;
-// the skin test of the drifted position feeds top / nonfinite.
+// the skin test of the drifted position feeds top / nonfinite, the minimiser's
+// dot products (f.f, f.a, f.v, v.v) go to dots.
 template <int D, int STAGE>
 __device__ __forceinline__ void atom_store(const AtomArrays &A, int i, const double (&fi)[D],
                                            const AtomIn<D> &in, const StepCoef &c, Top2 &top,
-                                           double &nonfinite) {
+                                           double &nonfinite, double (&dots)[4]) {
     using PT = typename PosStore<D>::T;
     constexpr bool DRIFT =
         (STAGE == kStageVerletKickDrift || STAGE == kStageDampedKickDrift);
@@ -157,6 +171,18 @@ __device__ __forceinline__ void atom_store(const AtomArrays &A, int i, const dou
     }
     if (STAGE == kStageForceOnly || STAGE == kStageForceAdd) return;
     const bool fixed = is_fixed(in.m);
+    if constexpr (STAGE == kStageNlcg) {
+        if (fixed) {
+#pragma unroll
+            for (int k = 0; k < D; k++) A.a[k][i] = 0.0;
+        } else {
+            dots[0] = dotv<D>(fi, fi);
+            dots[1] = dotv<D>(fi, in.a);
+            dots[2] = dotv<D>(fi, in.v);
+            dots[3] = dotv<D>(in.v, in.v);
+        }
+        return;
+    }
     double a[D];
 #pragma unroll
     for (int k = 0; k < D; k++) a[k] = fixed ? 0.0 : fi[k] / in.m;
@@ -252,14 +278,20 @@ __device__ void reduce_prev(const ReduceBuf &R) {
 // stage's writes (and so the skin test) were done by the first wavefront.
 template <int D, int STAGE, bool ENERGY, int NW, bool SKIN_W0 = false>
 __device__ __forceinline__ void group_partials(const PairAcc &acc, Top2 top, double nonfinite,
-                                               const ReduceBuf &R, int block) {
+                                               const double (&dots)[4], const ReduceBuf &R,
+                                               int block) {
     constexpr bool DRIFT =
         (STAGE == kStageVerletKickDrift || STAGE == kStageDampedKickDrift);
     if (ENERGY || DRIFT) {
         double v[kRedWidth];
 #pragma unroll
         for (int k = 0; k < kRedWidth; k++) v[k] = 0.0;
-        if (ENERGY) {
+        if (STAGE == kStageNlcg) {
+            // (fields as in nlcg.hpp)
+#pragma unroll
+            for (int k = 0; k < 4; k++) v[k] = dots[k];
+            v[5] = 0.5 * acc.w;
+        } else if (ENERGY) {
             v[kSumU] = 0.5 * acc.e;
             v[kSumW] = 0.5 * acc.w;
 #pragma unroll

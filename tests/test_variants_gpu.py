@@ -158,3 +158,37 @@ def test_counted_order_and_tile_plan(n, ndim, edge, clustered):
         assert np.array_equal(s.positions(), x)
         x = x + rng.normal(scale=0.4, size=x.shape)
     s.close()
+
+
+# the minimiser's sums out of the force launch: fixed atoms (no dot products,
+# a = 0), both list layouts, workgroup edges
+@pytest.mark.parametrize("tiled", ["0", "1"])
+@pytest.mark.parametrize("ndim,n", [(2, 63), (3, 257), (2, 900), (3, 2000)])
+def test_nlcg_point_sums(monkeypatch, tiled, ndim, n):
+    _device_or_fail()
+    print(f"nlcg sums tiled={tiled} ndim={ndim} n={n}", flush=True)
+    monkeypatch.setenv("PARM_TILED", tiled)
+    p = B.packings([n], 0.6, ndim, seed=n)[0]
+    m = np.ones(n)
+    m[::7] = np.inf
+    x, L = p["x"], [p["L"]] * ndim
+    t = O.PairTable(O.REPULSION, B.REP["eps"], B.REP["sigma"], B.REP["third"], p["types"])
+    r = O.System(m, L, t, p["sig"], 0.3, ndim=ndim)
+    s = capi.System(ndim, m)
+    s.set_box(L)
+    s.nlist_set(0.3, p["sig"])
+    s.set_repulsion(B.REP["eps"], B.REP["sigma"], B.REP["third"], p["types"])
+    for q in (r, s):
+        q.set_state(x=x, v=np.zeros_like(x), a=np.ones_like(x))
+    c, cr = capi.NLCG(s, 0.1, 1e-2), O.NLCG(r, 0.1, 1e-2)
+    for q in (c, cr):
+        q.set_limits(stepmax=1e-2)
+        q.timestep(4)
+    d, dr = c.info(), cr.info()
+    assert d["sec"] == dr["sec"] and d["k"] == dr["k"]
+    for key in ("alpha", "dxsum", "vl", "fl", "al", "Knew", "beta"):
+        assert abs(d[key] - dr[key]) <= 1e-9 * (abs(dr[key]) + 1e-12), key
+    for a, b in zip(s.state(), r.state()):
+        assert np.abs(a - b).max() <= 1e-9 * max(1.0, np.abs(b).max())
+    c.close()
+    s.close()
