@@ -9,23 +9,26 @@
 // steps can be captured in a HIP graph.
 //
 // Per step:  k_batch_force    forces + kick (+ next drift, |x - xref| per atom)
-//            k_batch_worklist the systems whose skin flag is set, as a list
 //            k_batch_sort     a fixed grid taking the listed systems in turn:
 //                             cell sort in LDS, sorted copies, xref = x
 //            k_batch_build    a fixed grid over slices of the listed
-//                             systems: the exact list build, a thread per atom
-//            k_batch_skin     one wavefront per system: top-2 of |x - xref|
-//                             -> the system's flag for the next rebuild
+//                             systems: the exact list build
+//            k_batch_skin     top-2 of |x - xref| per system -> the list of
+//                             systems for the next rebuild
+// parm_batch_initialize orders every system's slots by cell (k_batch_reorder).
 #include "common.hpp"
 #include "kernels.hpp"
 #include "pairs.hpp"
 
 namespace parm {
 
-// First half of a step (drift + half kick) and |x - xref|.
+// First half of a step (drift + half kick) and |x - xref|; empties the skin
+// test's worklist.
 template <int D, bool DAMPED>
-__global__ __launch_bounds__(kBlock) void k_batch_drift(BatchArrays A, StepCoef c) {
+__global__ __launch_bounds__(kBlock) void k_batch_drift(BatchArrays A, StepCoef c,
+                                                        unsigned long long *wl) {
     using PT = typename PosStore<D>::T;
+    if (blockIdx.x == 0 && threadIdx.x == 0) *wl = 0ull;
     const int i = blockIdx.x * kBlock + threadIdx.x;
     if (i >= A.ntot) return;
     PT *pos = static_cast<PT *>(A.pos_out);
@@ -48,10 +51,13 @@ __global__ __launch_bounds__(kBlock) void k_batch_drift(BatchArrays A, StepCoef 
     A.disp[i] = sqrt(sqnorm<D>(d));
 }
 
-// |x - xref| for every atom (update_list(false) outside a step).
+// |x - xref| for every atom (update_list(false) outside a step); empties the
+// skin test's worklist.
 template <int D>
-__global__ __launch_bounds__(kBlock) void k_batch_disp(BatchArrays A) {
+__global__ __launch_bounds__(kBlock) void k_batch_disp(BatchArrays A,
+                                                       unsigned long long *wl) {
     using PT = typename PosStore<D>::T;
+    if (blockIdx.x == 0 && threadIdx.x == 0) *wl = 0ull;
     const int i = blockIdx.x * kBlock + threadIdx.x;
     if (i >= A.ntot) return;
     const Vec<D> x = PosStore<D>::load(static_cast<const PT *>(A.pos_in)[i]);
@@ -63,44 +69,78 @@ __global__ __launch_bounds__(kBlock) void k_batch_disp(BatchArrays A) {
 }
 
 // ------------------------------------------------------------ skin test
-// One wavefront per system: the reference's rule (src/trackers.cpp:23-53),
-// rebuild iff the two largest displacements sum to >= skin, checked only
-// once something moved.  The flag is overwritten, never accumulated.
-__global__ __launch_bounds__(kBlock) void k_batch_skin(int nsys, BatchArrays A,
-                                                       double skin,
-                                                       uint32_t *__restrict__ flags,
+// The reference's rule (src/trackers.cpp:23-53) per system: rebuild iff the
+// two largest displacements sum to >= skin, checked only once something
+// moved.  A system that rebuilds puts itself on the worklist: one 64-bit add
+// on `wl` returns its place (high word) and its first build slice (low word),
+// so the list's slice offsets ascend with its places, whatever the order the
+// systems arrive in (their rebuilds are independent).
+// W wavefronts per system, each thread kSkinAhead loads at a time: the pass is
+// bound by the latency of its loads, not their 8 bytes per atom.  1024 systems
+// of 64 - 4096 atoms: SKIN_MEASURED
+constexpr int kSkinAhead = 4;
+
+template <int W>
+__global__ __launch_bounds__(kBlock) void k_batch_skin(int nsys, BatchArrays A, double skin,
+                                                       int slice,
+                                                       unsigned long long *__restrict__ wl,
+                                                       int32_t *__restrict__ work,
+                                                       int32_t *__restrict__ wslice,
                                                        uint32_t *__restrict__ gflag) {
-    const int s = blockIdx.x * (kBlock / kWave) + threadIdx.x / kWave;
-    const int lane = threadIdx.x % kWave;
-    if (s >= nsys) return;
-    const int off = A.geom[s].off, n = A.geom[s].n;
-    Top2 t;
+    constexpr int kPer = kBlock / kWave / W;  // systems per workgroup
+    constexpr int NT = W * kWave;
+    __shared__ double red[kBlock / kWave][2];
+    const int s = blockIdx.x * kPer + threadIdx.x / NT;
+    const int t = threadIdx.x % NT, lane = threadIdx.x % kWave, w = threadIdx.x / kWave;
+    const int off = s < nsys ? A.geom[s].off : 0, n = s < nsys ? A.geom[s].n : 0;
+    Top2 m;
     bool bad = false;
-    for (int k = lane; k < n; k += kWave) {
-        const double d = A.disp[off + k];
-        t.add(d);
-        bad |= !isfinite(d);
+    for (int k = t; k < n; k += NT * kSkinAhead) {
+        double d[kSkinAhead];
+#pragma unroll
+        for (int q = 0; q < kSkinAhead; q++)
+            d[q] = k + q * NT < n ? A.disp[off + k + q * NT] : 0.0;
+#pragma unroll
+        for (int q = 0; q < kSkinAhead; q++) {
+            m.add(d[q]);
+            bad |= !isfinite(d[q]);
+        }
     }
-    t = wave_top2(t);
-    const unsigned long long anybad = __ballot(bad);
-    if (lane == 0) {
-        flags[s] = (t.a > 0 && t.b + t.a >= skin) ? 1u : 0u;
-        if (anybad) atomicOr(gflag, kFlagNonFinite);
+    m = wave_top2(m);
+    if (__ballot(bad) != 0ull && lane == 0) atomicOr(gflag, kFlagNonFinite);
+    if (W > 1) {
+        if (lane == 0) {
+            red[w][0] = m.a;
+            red[w][1] = m.b;
+        }
+        __syncthreads();
+        if (t == 0) {
+#pragma unroll
+            for (int q = 1; q < W; q++) {
+                m.add(red[w + q][0]);
+                m.add(red[w + q][1]);
+            }
+        }
+    }
+    if (t == 0 && s < nsys && m.a > 0 && m.b + m.a >= skin) {
+        const unsigned long long at =
+            atomicAdd(wl, (1ull << 32) | (unsigned long long)((n + slice - 1) / slice));
+        work[at >> 32] = s;
+        wslice[at >> 32] = (int32_t)(at & 0xffffffffull);
     }
 }
 
 // -------------------------------------------------------------- rebuild
-// The systems to rebuild at the end of a step are those whose skin flag is
-// set (or all, when forced).  k_batch_worklist turns the flags into a list
-// (system ids in ascending order, count first) and counts each listed
-// system's build slices (exclusive prefix in wslice).  Then
-// two launches on fixed grids, so the launch shapes do not depend on how
-// many systems rebuild (the step stays graph-capturable) and no workgroup is
-// started for a system that keeps its list:
+// The systems to rebuild at the end of a step are those on the worklist of
+// the skin test (or all, listed by k_batch_all): wl holds their count (high
+// word) and their build slices (low word), work the systems, wslice the first
+// slice of each.  Two launches on fixed grids, so the launch shapes do not
+// depend on how many systems rebuild (the step stays graph-capturable) and no
+// workgroup is started for a system that keeps its list:
 //   k_batch_sort   one workgroup of kSortThreads per listed system: cell
 //                  keys, a stable counting sort of the system's atoms by
 //                  cell in LDS, the cell starts, sorted copies of the
-//                  positions and diameters, xref = x;
+//                  positions, diameters, keys and list words, xref = x;
 //   k_batch_build  one workgroup per slice of a listed system's atoms,
 //                  several lanes per atom: the exact list build over the
 //                  stencil rows of the periodic cell grid
@@ -111,102 +151,142 @@ __global__ __launch_bounds__(kBlock) void k_batch_skin(int nsys, BatchArrays A,
 // the next skin test.
 constexpr int kBatchMaxCells = kBatchMaxCellsPerSystem;
 constexpr int kSortThreads = 1024;
-constexpr int kWorklistThreads = 1024;
+constexpr int kAllThreads = 1024;
 constexpr int kBuildThreads = 256;
 
-__global__ __launch_bounds__(kWorklistThreads) void k_batch_worklist(
-    int nsys, const uint32_t *__restrict__ flags, int force, int slice,
-    const BatchGeom *__restrict__ geom, int32_t *__restrict__ work,
+// Every system on the worklist, in order.
+__global__ __launch_bounds__(kAllThreads) void k_batch_all(
+    int nsys, int slice, const BatchGeom *__restrict__ geom,
+    unsigned long long *__restrict__ wl, int32_t *__restrict__ work,
     int32_t *__restrict__ wslice) {
-    __shared__ int wsum[kWorklistThreads / kWave][2];
+    __shared__ int wsum[kAllThreads / kWave];
     const int t = threadIdx.x;
-    const int per = (nsys + kWorklistThreads - 1) / kWorklistThreads;
+    const int per = (nsys + kAllThreads - 1) / kAllThreads;
     const int s0 = t * per;
-    int loc = 0, lsl = 0;
-    for (int q = 0; q < per; q++) {
-        const int s = s0 + q;
-        if (s < nsys && (force || flags[s] != 0u)) {
-            loc++;
-            lsl += (geom[s].n + slice - 1) / slice;
-        }
-    }
+    int loc = 0;
+    for (int q = 0; q < per; q++)
+        if (s0 + q < nsys) loc += (geom[s0 + q].n + slice - 1) / slice;
     const int lane = t % kWave, w = t / kWave;
-    int incl = loc, isl = lsl;
+    int incl = loc;
 #pragma unroll
     for (int o = 1; o < kWave; o <<= 1) {
-        const int y = __shfl_up(incl, o), z = __shfl_up(isl, o);
-        if (lane >= o) {
-            incl += y;
-            isl += z;
-        }
+        const int y = __shfl_up(incl, o);
+        if (lane >= o) incl += y;
     }
-    if (lane == kWave - 1) {
-        wsum[w][0] = incl;
-        wsum[w][1] = isl;
-    }
+    if (lane == kWave - 1) wsum[w] = incl;
     __syncthreads();
-    int pos = incl - loc, psl = isl - lsl, tot = 0, totsl = 0;
-    for (int q = 0; q < kWorklistThreads / kWave; q++) {
-        if (q < w) {
-            pos += wsum[q][0];
-            psl += wsum[q][1];
-        }
-        tot += wsum[q][0];
-        totsl += wsum[q][1];
+    int run = incl - loc, tot = 0;
+    for (int q = 0; q < kAllThreads / kWave; q++) {
+        if (q < w) run += wsum[q];
+        tot += wsum[q];
     }
     for (int q = 0; q < per; q++) {
         const int s = s0 + q;
-        if (s < nsys && (force || flags[s] != 0u)) {
-            work[1 + pos] = s;
-            wslice[pos] = psl;
-            pos++;
-            psl += (geom[s].n + slice - 1) / slice;
+        if (s < nsys) {
+            work[s] = s;
+            wslice[s] = run;
+            run += (geom[s].n + slice - 1) / slice;
         }
     }
-    if (t == 0) {
-        work[0] = tot;
-        wslice[tot] = totsl;
-    }
+    if (t == 0) *wl = ((unsigned long long)nsys << 32) | (unsigned long long)tot;
 }
 
+// A system of up to kSortKeep atoms per thread, no cell of it with more than
+// kRankMax atoms, is sorted from registers: one load of the positions, each
+// atom's arrival on its cell's counter, then its rank among the cell's atoms
+// by their indices (so the order is the stable one).  The general form
+// reloads the positions per chunk and takes its ranks from ballots, the
+// wavefronts in turn: 16 barriers per chunk.  SORT_MEASURED
+constexpr int kSortKeep = 4;
+constexpr int kRankMax = 64;
+
 template <int D>
-__device__ __forceinline__ void sort_system(
-    const int s, const BatchArrays &A, const typename PosStore<D>::T *__restrict__ pos,
-    int count_rebuild, int32_t *__restrict__ keys, int32_t *__restrict__ cellidx,
-    int32_t *__restrict__ cstart, typename PosStore<D>::T *__restrict__ xs,
-    double *__restrict__ dsort, uint32_t *__restrict__ flags, uint32_t *__restrict__ which,
-    unsigned long long *__restrict__ nent, int *hist) {
+__device__ __forceinline__ int batch_key(const Vec<D> &x, const BatchGeom &G) {
+    int key = 0;
+#pragma unroll
+    for (int d = D - 1; d >= 0; d--) {
+        double sv = x.c[d] * G.grid.invL[d];
+        sv -= floor(sv);
+        int cd = (int)(sv * (double)G.grid.nc[d]);
+        cd = cd < 0 ? 0 : (cd >= G.grid.nc[d] ? G.grid.nc[d] - 1 : cd);
+        key = key * G.grid.nc[d] + cd;
+    }
+    return key;
+}
+
+// The per-slot outputs of the sort.
+template <int D>
+struct SortOut {
+    int32_t *keys;     // cell of each sorted slot
+    uint32_t *ent;     // list word of its atom: (index << type_bits) | type
+    int32_t *cstart;
+    typename PosStore<D>::T *xs;
+    double *dsort;
+};
+
+template <int D>
+__device__ __forceinline__ void sort_system(const int s, const BatchArrays &A,
+                                            const typename PosStore<D>::T *__restrict__ pos,
+                                            int count_rebuild, int type_bits,
+                                            const SortOut<D> &S, uint32_t *__restrict__ which,
+                                            unsigned long long *__restrict__ nent, int *hist,
+                                            int *slots) {
     using PT = typename PosStore<D>::T;
     constexpr int NT = kSortThreads;
     const BatchGeom G = A.geom[s];
     const int off = G.off, n = G.n, ncell = G.grid.ncell;
     const int t = threadIdx.x;
+    const bool keep = n <= kSortKeep * NT;
+    PT *const xref = static_cast<PT *>(A.xref_w);
+    PT xk[kSortKeep];
+    double dk[kSortKeep];
+    int32_t tk[kSortKeep];
+    int kk[kSortKeep], ak[kSortKeep];  // key, arrival on the cell's counter
+#pragma unroll
+    for (int q = 0; q < kSortKeep; q++) {
+        const int k = t + q * NT;
+        if (keep && k < n) {
+            xk[q] = pos[off + k];
+            dk[q] = A.diam[off + k];
+            tk[q] = A.type[off + k];
+        }
+    }
     for (int c = t; c < ncell; c += NT) hist[c] = 0;
     __syncthreads();
     // keys and counts
-    for (int k = t; k < n; k += NT) {
-        const Vec<D> x = PosStore<D>::load(pos[off + k]);
-        int key = 0;
+    if (keep) {
 #pragma unroll
-        for (int d = D - 1; d >= 0; d--) {
-            double sv = x.c[d] * G.grid.invL[d];
-            sv -= floor(sv);
-            int cd = (int)(sv * (double)G.grid.nc[d]);
-            cd = cd < 0 ? 0 : (cd >= G.grid.nc[d] ? G.grid.nc[d] - 1 : cd);
-            key = key * G.grid.nc[d] + cd;
+        for (int q = 0; q < kSortKeep; q++) {
+            const int k = t + q * NT;
+            kk[q] = ak[q] = 0;
+            if (k < n) {
+                kk[q] = batch_key<D>(PosStore<D>::load(xk[q]), G);
+                ak[q] = atomicAdd(&hist[kk[q]], 1);
+                xref[off + k] = xk[q];
+            }
         }
-        keys[off + k] = key;
-        atomicAdd(&hist[key], 1);
+    } else {
+        for (int k = t; k < n; k += NT) {
+            const PT x = pos[off + k];
+            atomicAdd(&hist[batch_key<D>(PosStore<D>::load(x), G)], 1);
+            xref[off + k] = x;
+        }
     }
     __syncthreads();
     // exclusive scan of the counts: each thread sums a run of kScanPer
     // cells, a block scan of the run sums, then each thread writes its run
+    int crowd = 0;
     {
         constexpr int kScanPer = kBatchMaxCells / NT;
         __shared__ int wsum[NT / kWave];
         const int c0 = t * kScanPer;
         int loc = 0;
-        for (int q = 0; q < kScanPer; q++) loc += (c0 + q < ncell) ? hist[c0 + q] : 0;
+#pragma unroll
+        for (int q = 0; q < kScanPer; q++) {
+            const int h = c0 + q < ncell ? hist[c0 + q] : 0;
+            crowd |= h > kRankMax;
+            loc += h;
+        }
         const int lane = t % kWave, w = t / kWave;
         int incl = loc;
 #pragma unroll
@@ -215,28 +295,52 @@ __device__ __forceinline__ void sort_system(
             if (lane >= o) incl += y;
         }
         if (lane == kWave - 1) wsum[w] = incl;
-        __syncthreads();
+        crowd = __syncthreads_or(crowd);
         int run = incl - loc;
         for (int q = 0; q < w; q++) run += wsum[q];
-        __syncthreads();
+#pragma unroll
         for (int q = 0; q < kScanPer; q++) {
             const int c = c0 + q;
             if (c < ncell) {
                 const int h = hist[c];
-                cstart[G.cell_off + c] = off + run;
+                S.cstart[G.cell_off + c] = off + run;
                 hist[c] = run;
                 run += h;
             }
         }
-        if (t == 0) cstart[G.cell_off + ncell] = off + n;
+        if (t == 0) {
+            S.cstart[G.cell_off + ncell] = off + n;
+            hist[ncell] = n;
+        }
     }
     __syncthreads();
-    // stable scatter, one chunk of NT atoms at a time: within a wavefront the
-    // rank among equal keys comes from ballots over the key bits; the
-    // wavefronts of the chunk then take their turn, in order, on the cell
-    // counters (the wavefront's reads of hist[key] precede, in its program
-    // order, the update by its last lane of that key)
-    {
+    auto place = [&](int slot, int k, int key, const PT &x, double d, int32_t type) {
+        S.xs[off + slot] = x;
+        S.dsort[off + slot] = d;
+        S.keys[off + slot] = key;
+        S.ent[off + slot] = ((uint32_t)(off + k) << type_bits) | (uint32_t)type;
+    };
+    if (keep && !crowd) {
+#pragma unroll
+        for (int q = 0; q < kSortKeep; q++)
+            if (t + q * NT < n) slots[hist[kk[q]] + ak[q]] = t + q * NT;
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < kSortKeep; q++) {
+            const int k = t + q * NT;
+            if (k < n) {
+                const int a = hist[kk[q]], b = hist[kk[q] + 1];
+                int r = a;
+                for (int e = a; e < b; e++) r += slots[e] < k;
+                place(r, k, kk[q], xk[q], dk[q], tk[q]);
+            }
+        }
+    } else {
+        // stable scatter, one chunk of NT atoms at a time: within a wavefront
+        // the rank among equal keys comes from ballots over the key bits; the
+        // wavefronts of the chunk then take their turn, in order, on the cell
+        // counters (the wavefront's reads of hist[key] precede, in its program
+        // order, the update by its last lane of that key)
         constexpr int kKeyBits = 12;
         static_assert(kBatchMaxCells <= (1 << kKeyBits), "cell keys fit the ballot match");
         const int lane = t % kWave, wv = t / kWave;
@@ -244,7 +348,15 @@ __device__ __forceinline__ void sort_system(
         for (int base = 0; base < n; base += NT) {
             const int k = base + t;
             const bool valid = k < n;
-            const int key = valid ? keys[off + k] : 0;
+            PT x{};
+            double d = 0.0;
+            int32_t type = 0;
+            if (valid) {
+                x = pos[off + k];
+                d = A.diam[off + k];
+                type = A.type[off + k];
+            }
+            const int key = valid ? batch_key<D>(PosStore<D>::load(x), G) : 0;
             unsigned long long eq = __ballot(valid);
 #pragma unroll
             for (int b = 0; b < kKeyBits; b++) {
@@ -255,44 +367,39 @@ __device__ __forceinline__ void sort_system(
             const int r = __popcll(eq & below);
             const bool lastk = valid && (eq >> lane) == 1ull;
             const int cntk = __popcll(eq);
+            int slot = 0;
             for (int w2 = 0; w2 < NT / kWave; w2++) {
                 if (wv == w2) {
-                    if (valid) cellidx[off + hist[key] + r] = off + k;
+                    if (valid) slot = hist[key] + r;
                     if (lastk) hist[key] += cntk;
                 }
                 __syncthreads();
             }
+            if (valid) place(slot, k, key, x, d, type);
         }
     }
-    // sorted copies of the positions and diameters, and xref = x (the
-    // reference stores lastlocs inside the rebuild loop)
-    for (int u = t; u < n; u += NT) {
-        const int i = cellidx[off + u];
-        xs[off + u] = pos[i];
-        dsort[off + u] = A.diam[i];
-    }
-    for (int k = t; k < n; k += NT) static_cast<PT *>(A.xref_w)[off + k] = pos[off + k];
     if (t == 0) {
         nent[s] = 0ull;
         if (count_rebuild) which[s] += 1u;
-        flags[s] = 0u;
     }
     // the next listed system reuses the LDS
     __syncthreads();
 }
 
+// wl_next: the worklist that the step's skin test fills, emptied here (its
+// last readers were the launches of the step before).
 template <int D>
 __global__ __launch_bounds__(kSortThreads) void k_batch_sort(
     BatchArrays A, const typename PosStore<D>::T *__restrict__ pos, int count_rebuild,
-    int32_t *__restrict__ keys, int32_t *__restrict__ cellidx, int32_t *__restrict__ cstart,
-    typename PosStore<D>::T *__restrict__ xs, double *__restrict__ dsort,
-    uint32_t *__restrict__ flags, uint32_t *__restrict__ which,
-    unsigned long long *__restrict__ nent, const int32_t *__restrict__ work) {
-    __shared__ int hist[kBatchMaxCells];
-    const int count = work[0];
+    int type_bits, SortOut<D> S, uint32_t *__restrict__ which,
+    unsigned long long *__restrict__ nent, const unsigned long long *__restrict__ wl,
+    unsigned long long *__restrict__ wl_next, const int32_t *__restrict__ work) {
+    __shared__ int hist[kBatchMaxCells + 1];
+    __shared__ int slots[kSortKeep * kSortThreads];
+    const int count = (int)(*wl >> 32);
+    if (wl_next && blockIdx.x == 0 && threadIdx.x == 0) *wl_next = 0ull;
     for (int q = blockIdx.x; q < count; q += gridDim.x)
-        sort_system<D>(work[1 + q], A, pos, count_rebuild, keys, cellidx, cstart, xs, dsort,
-                       flags, which, nent, hist);
+        sort_system<D>(work[q], A, pos, count_rebuild, type_bits, S, which, nent, hist, slots);
 }
 
 // G lanes per atom, U candidates per lane and round.  The build is bound by
@@ -308,15 +415,15 @@ __global__ __launch_bounds__(kBuildThreads) void k_batch_build(
     BatchArrays A, const typename PosStore<D>::T *__restrict__ alt, double skin,
     int type_bits, int tpa, int cap, int npad, uint32_t *__restrict__ nbr,
     int32_t *__restrict__ ncount, const int32_t *__restrict__ keys,
-    const int32_t *__restrict__ cellidx, const int32_t *__restrict__ cstart,
+    const uint32_t *__restrict__ ent, const int32_t *__restrict__ cstart,
     const typename PosStore<D>::T *__restrict__ xs, const double *__restrict__ dsort,
     unsigned long long *__restrict__ nent, uint32_t *__restrict__ gflag,
-    const int32_t *__restrict__ work, const int32_t *__restrict__ wslice) {
+    const unsigned long long *__restrict__ wl, const int32_t *__restrict__ work,
+    const int32_t *__restrict__ wslice) {
     constexpr int kSlice = kBuildThreads / G;  // atoms per slice
     constexpr int RPL = (9 + G - 1) / G;       // rows whose bounds a lane loads
     __shared__ unsigned long long red[kBuildThreads / kWave];
-    const int count = work[0];
-    const int total = wslice[count];
+    const int count = (int)(*wl >> 32), total = (int)(*wl & 0xffffffffull);
     const int t = threadIdx.x;
     const int sub = t % G, lane = t % kWave;
     const int gbase = lane - sub;  // first lane of this atom's group
@@ -331,17 +438,17 @@ __global__ __launch_bounds__(kBuildThreads) void k_batch_build(
             else
                 hi = mid;
         }
-        const int s = work[1 + lo];
+        const int s = work[lo];
         const BatchGeom G_ = A.geom[s];
         const int off = G_.off, n = G_.n, nc0 = G_.grid.nc[0], nc1 = G_.grid.nc[1],
                   nc2 = G_.grid.nc[2];
         const int u = (gs - wslice[lo]) * kSlice + t / G;
         unsigned long long mycnt = 0;
         if (u < n) {
-            const int i = cellidx[off + u];
+            const int i = (int)(ent[off + u] >> type_bits);
             const Vec<D> xi = PosStore<D>::load(xs[off + u]);
             const double di = dsort[off + u];
-            int key = keys[i];
+            int key = keys[off + u];
             const int c0 = key % nc0;
             key /= nc0;
             const int c1 = D >= 2 ? key % nc1 : 0;
@@ -394,12 +501,14 @@ __global__ __launch_bounds__(kBuildThreads) void k_batch_build(
                         // the range reads the atom's own (and is not tested)
                         Vec<D> xj[U];
                         double dj[U];
+                        uint32_t ej[U];
 #pragma unroll
                         for (int q = 0; q < U; q++) {
                             const int v = base + q * G + sub;
                             const int vv = v < b ? v : off + u;
                             xj[q] = PosStore<D>::load(xs[vv]);
                             dj[q] = dsort[vv];
+                            ej[q] = ent[vv];
                         }
 #pragma unroll
                         for (int q = 0; q < U; q++) {
@@ -428,11 +537,7 @@ __global__ __launch_bounds__(kBuildThreads) void k_batch_build(
                                 (__ballot(pass) >> gbase) & ((1ull << G) - 1ull);
                             if (pass) {
                                 const int w = cnt + __popcll(m & below);
-                                if (w < cap) {
-                                    const int j = cellidx[v];
-                                    nbr[untiled_entry(w, i, tpa, npad)] =
-                                        ((uint32_t)j << type_bits) | (uint32_t)A.type[j];
-                                }
+                                if (w < cap) nbr[untiled_entry(w, i, tpa, npad)] = ej[q];
                             }
                             cnt += __popcll(m);
                         }
@@ -463,6 +568,53 @@ __global__ __launch_bounds__(kBuildThreads) void k_batch_build(
             atomicAdd(&nent[s], tot);
         }
         __syncthreads();
+    }
+}
+
+// Every per-atom column in sorted order (slot k takes the slot in ent[k]):
+// FORWARD gathers into the scratch arrays, the other way copies back, so the
+// columns stay where they are (a captured run of steps holds their addresses).
+// The caller's order is none in space: with it, an atom's neighbours are
+// anywhere among its system's positions, each a cache line of its own for one
+// gather.  MEASURED_ORDER
+template <int D>
+struct OrderScratch {
+    typename PosStore<D>::T *pos;
+    double *v, *a, *m, *diam;  // v, a: D x ntot
+    int32_t *type, *orig;
+};
+
+template <int D, bool FORWARD>
+__global__ __launch_bounds__(kBlock) void k_batch_reorder(
+    BatchArrays A, typename PosStore<D>::T *__restrict__ pos, double *__restrict__ m,
+    double *__restrict__ diam, int32_t *__restrict__ type, int32_t *__restrict__ orig,
+    const uint32_t *__restrict__ ent, int type_bits, OrderScratch<D> S) {
+    const int k = blockIdx.x * kBlock + threadIdx.x;
+    const size_t n = (size_t)A.ntot;
+    if (k >= A.ntot) return;
+    if (FORWARD) {
+        const int i = (int)(ent[k] >> type_bits);
+        S.pos[k] = pos[i];
+#pragma unroll
+        for (int d = 0; d < D; d++) {
+            S.v[d * n + k] = A.v[d][i];
+            S.a[d * n + k] = A.a[d][i];
+        }
+        S.m[k] = m[i];
+        S.diam[k] = diam[i];
+        S.type[k] = type[i];
+        S.orig[k] = orig[i];
+    } else {
+        pos[k] = S.pos[k];
+#pragma unroll
+        for (int d = 0; d < D; d++) {
+            A.v[d][k] = S.v[d * n + k];
+            A.a[d][k] = S.a[d * n + k];
+        }
+        m[k] = S.m[k];
+        diam[k] = S.diam[k];
+        type[k] = S.type[k];
+        orig[k] = S.orig[k];
     }
 }
 
@@ -529,38 +681,31 @@ hipError_t launch_batch_force(int ndim, int precision, int stage, bool energy,
 }
 
 hipError_t launch_batch_drift(int ndim, bool damped, const BatchArrays &A,
-                              const StepCoef &c, hipStream_t s) {
+                              const StepCoef &c, unsigned long long *wl, hipStream_t s) {
     if (A.ntot <= 0) return hipSuccess;
     dim3 g(nblk1(A.ntot)), b(kBlock);
     if (ndim == 3) {
         if (damped)
-            hipLaunchKernelGGL((k_batch_drift<3, true>), g, b, 0, s, A, c);
+            hipLaunchKernelGGL((k_batch_drift<3, true>), g, b, 0, s, A, c, wl);
         else
-            hipLaunchKernelGGL((k_batch_drift<3, false>), g, b, 0, s, A, c);
+            hipLaunchKernelGGL((k_batch_drift<3, false>), g, b, 0, s, A, c, wl);
     } else {
         if (damped)
-            hipLaunchKernelGGL((k_batch_drift<2, true>), g, b, 0, s, A, c);
+            hipLaunchKernelGGL((k_batch_drift<2, true>), g, b, 0, s, A, c, wl);
         else
-            hipLaunchKernelGGL((k_batch_drift<2, false>), g, b, 0, s, A, c);
+            hipLaunchKernelGGL((k_batch_drift<2, false>), g, b, 0, s, A, c, wl);
     }
     return hipGetLastError();
 }
 
-hipError_t launch_batch_disp(int ndim, const BatchArrays &A, hipStream_t s) {
+hipError_t launch_batch_disp(int ndim, const BatchArrays &A, unsigned long long *wl,
+                             hipStream_t s) {
     if (A.ntot <= 0) return hipSuccess;
     dim3 g(nblk1(A.ntot)), b(kBlock);
     if (ndim == 3)
-        hipLaunchKernelGGL(k_batch_disp<3>, g, b, 0, s, A);
+        hipLaunchKernelGGL(k_batch_disp<3>, g, b, 0, s, A, wl);
     else
-        hipLaunchKernelGGL(k_batch_disp<2>, g, b, 0, s, A);
-    return hipGetLastError();
-}
-
-hipError_t launch_batch_skin(int nsys, const BatchArrays &A, double skin, uint32_t *flags,
-                             uint32_t *gflag, hipStream_t s) {
-    const int per = kBlock / kWave;
-    hipLaunchKernelGGL(k_batch_skin, dim3((nsys + per - 1) / per), dim3(kBlock), 0, s, nsys,
-                       A, skin, flags, gflag);
+        hipLaunchKernelGGL(k_batch_disp<2>, g, b, 0, s, A, wl);
     return hipGetLastError();
 }
 
@@ -573,40 +718,97 @@ hipError_t launch_batch_skin(int nsys, const BatchArrays &A, double skin, uint32
 constexpr int kBuildLanes = 8, kBuildAhead = 4;
 constexpr int kBuildLanesSparse = 4, kBuildAheadSparse = 2;
 
-hipError_t launch_batch_rebuild(int ndim, int nsys, const BatchArrays &A, const void *pos,
-                                const void *alt, int force, int count_rebuild, double skin,
-                                int type_bits, int tpa, int cap, int npad, uint32_t *nbr,
-                                int32_t *ncount, int32_t *keys, int32_t *cellidx,
-                                int32_t *cstart, void *xs, double *dsort, uint32_t *flags,
-                                uint32_t *which, unsigned long long *nent, uint32_t *gflag,
-                                int32_t *work, int32_t *wslice, int sort_grid, int build_grid,
-                                bool sparse, hipStream_t s) {
-    if (nsys <= 0) return hipSuccess;
-    // (see k_batch_build)
-    const int lanes = sparse ? kBuildLanesSparse : kBuildLanes;
-    hipLaunchKernelGGL(k_batch_worklist, dim3(1), dim3(kWorklistThreads), 0, s, nsys, flags,
-                       force, kBuildThreads / lanes, A.geom, work, wslice);
-    const int gs = sort_grid < nsys ? sort_grid : nsys;
-#define PARM_BB(DD, PT, GG, UU)                                                               \
-    hipLaunchKernelGGL((k_batch_build<DD, GG, UU>), dim3(build_grid), dim3(kBuildThreads), 0, \
-                       s, A, (const PT *)alt, skin, type_bits, tpa, cap, npad, nbr, ncount,   \
-                       keys, cellidx, cstart, (const PT *)xs, dsort, nent, gflag, work, wslice)
-#define PARM_BR(DD, PT)                                                                       \
-    hipLaunchKernelGGL(k_batch_sort<DD>, dim3(gs), dim3(kSortThreads), 0, s, A,               \
-                       (const PT *)pos, count_rebuild, keys, cellidx, cstart, (PT *)xs,       \
-                       dsort, flags, which, nent, work);                                      \
-    if (sparse)                                                                               \
-        PARM_BB(DD, PT, kBuildLanesSparse, kBuildAheadSparse);                                \
-    else                                                                                      \
-        PARM_BB(DD, PT, kBuildLanes, kBuildAhead)
-    if (ndim == 3) {
-        PARM_BR(3, double4);
-    } else {
-        PARM_BR(2, double2);
-    }
-#undef PARM_BR
+static inline int build_slice(bool sparse) {
+    return kBuildThreads / (sparse ? kBuildLanesSparse : kBuildLanes);
+}
+
+// One wavefront per system of up to kSkinWaveAtoms atoms on average (two
+// rounds of its loads), else a workgroup.
+constexpr long kSkinWaveAtoms = 2 * kSkinAhead * kWave;
+
+hipError_t launch_batch_skin(int nsys, const BatchArrays &A, double skin, bool sparse,
+                             unsigned long long *wl, int32_t *work, int32_t *wslice,
+                             uint32_t *gflag, hipStream_t s) {
+    constexpr int kWaves = kBlock / kWave;
+    if (A.ntot <= kSkinWaveAtoms * nsys)
+        hipLaunchKernelGGL(k_batch_skin<1>, dim3((nsys + kWaves - 1) / kWaves), dim3(kBlock), 0,
+                           s, nsys, A, skin, build_slice(sparse), wl, work, wslice, gflag);
+    else
+        hipLaunchKernelGGL(k_batch_skin<kWaves>, dim3(nsys), dim3(kBlock), 0, s, nsys, A, skin,
+                           build_slice(sparse), wl, work, wslice, gflag);
+    return hipGetLastError();
+}
+
+hipError_t launch_batch_all(int nsys, const BatchArrays &A, bool sparse, unsigned long long *wl,
+                            int32_t *work, int32_t *wslice, hipStream_t s) {
+    hipLaunchKernelGGL(k_batch_all, dim3(1), dim3(kAllThreads), 0, s, nsys, build_slice(sparse),
+                       A.geom, wl, work, wslice);
+    return hipGetLastError();
+}
+
+template <int D>
+static hipError_t batch_rebuild(const BatchArrays &A, const BatchLists &B, const void *pos,
+                                const void *alt, int count_rebuild, double skin,
+                                const unsigned long long *wl, unsigned long long *wl_next,
+                                uint32_t *gflag, hipStream_t s) {
+    using PT = typename PosStore<D>::T;
+    const SortOut<D> S{B.keys, B.ent, B.cstart, (PT *)B.xs, B.dsort};
+    hipLaunchKernelGGL(k_batch_sort<D>, dim3(B.sort_grid), dim3(kSortThreads), 0, s, A,
+                       (const PT *)pos, count_rebuild, B.type_bits, S, B.which, B.nent, wl,
+                       wl_next, B.work);
+    if (!B.nbr) return hipGetLastError();
+#define PARM_BB(GG, UU)                                                                       \
+    hipLaunchKernelGGL((k_batch_build<D, GG, UU>), dim3(B.build_grid), dim3(kBuildThreads),   \
+                       0, s, A, (const PT *)alt, skin, B.type_bits, B.tpa, B.cap, B.npad,     \
+                       B.nbr, B.ncount, B.keys, B.ent, B.cstart, (const PT *)B.xs, B.dsort,   \
+                       B.nent, gflag, wl, B.work, B.wslice)
+    if (B.sparse)
+        PARM_BB(kBuildLanesSparse, kBuildAheadSparse);
+    else
+        PARM_BB(kBuildLanes, kBuildAhead);
 #undef PARM_BB
     return hipGetLastError();
+}
+
+hipError_t launch_batch_rebuild(int ndim, const BatchArrays &A, const BatchLists &B,
+                                const void *pos, const void *alt, int count_rebuild,
+                                double skin, const unsigned long long *wl,
+                                unsigned long long *wl_next, uint32_t *gflag, hipStream_t s) {
+    return ndim == 3 ? batch_rebuild<3>(A, B, pos, alt, count_rebuild, skin, wl, wl_next, gflag,
+                                        s)
+                     : batch_rebuild<2>(A, B, pos, alt, count_rebuild, skin, wl, wl_next, gflag,
+                                        s);
+}
+
+template <int D>
+static hipError_t batch_reorder(const BatchArrays &A, const BatchLists &B, void *pos,
+                                void *pos_alt, double *m, double *diam, int32_t *type,
+                                int32_t *orig, double *stage, double *eatom, hipStream_t s) {
+    using PT = typename PosStore<D>::T;
+    const size_t n = (size_t)A.ntot;
+    // (the sorted positions in xs are free from here on; an atom's share of
+    // xs, at least two doubles, holds its diameter, type and index)
+    OrderScratch<D> S{};
+    S.pos = (PT *)pos_alt;
+    S.v = stage;
+    S.a = eatom;
+    S.m = eatom + 3 * n;
+    S.diam = (double *)B.xs;
+    S.type = (int32_t *)(S.diam + n);
+    S.orig = S.type + n;
+    const dim3 g(nblk1(A.ntot)), b(kBlock);
+    hipLaunchKernelGGL((k_batch_reorder<D, true>), g, b, 0, s, A, (PT *)pos, m, diam, type, orig,
+                       B.ent, B.type_bits, S);
+    hipLaunchKernelGGL((k_batch_reorder<D, false>), g, b, 0, s, A, (PT *)pos, m, diam, type,
+                       orig, B.ent, B.type_bits, S);
+    return hipGetLastError();
+}
+
+hipError_t launch_batch_reorder(int ndim, const BatchArrays &A, const BatchLists &B, void *pos,
+                                void *pos_alt, double *m, double *diam, int32_t *type,
+                                int32_t *orig, double *stage, double *eatom, hipStream_t s) {
+    return ndim == 3 ? batch_reorder<3>(A, B, pos, pos_alt, m, diam, type, orig, stage, eatom, s)
+                     : batch_reorder<2>(A, B, pos, pos_alt, m, diam, type, orig, stage, eatom, s);
 }
 
 hipError_t launch_batch_sys_sums(int nsys, const BatchArrays &A, const double *eatom,

@@ -77,16 +77,23 @@ struct parm_batch {
     double *v[3] = {}, *a[3] = {}, *f[3] = {};
     double *m = nullptr, *diam = nullptr, *disp = nullptr, *stage = nullptr;
     int32_t *type = nullptr, *sys = nullptr;
+    // the caller's index of the atom in each slot: parm_batch_initialize
+    // orders every system's slots by cell
+    int32_t *orig = nullptr;
 
     int cap = 0, tpa = 4, type_bits = 0, total_cells = 0;
     bool tuned = false, tpa_fixed = false, built = false;
     uint32_t *nbr = nullptr;
-    int32_t *ncount = nullptr, *keys = nullptr, *cellidx = nullptr, *cstart = nullptr;
+    int32_t *ncount = nullptr, *keys = nullptr, *cstart = nullptr;
+    uint32_t *ent = nullptr;
     void *xs = nullptr;        // positions in each system's cell order (rebuild scratch)
     double *dsort = nullptr;   // list diameters in the same order
-    uint32_t *flags = nullptr, *which = nullptr, *gflag = nullptr, *hgflag = nullptr;
-    int32_t *work = nullptr;   // worklist of systems to rebuild (count first)
-    int32_t *wslice = nullptr; // first build slice of each listed system, then the total
+    uint32_t *which = nullptr, *gflag = nullptr, *hgflag = nullptr;
+    // worklist counters (count, slices): two that the steps alternate between,
+    // one for a rebuild of every system
+    unsigned long long *wl = nullptr;
+    int32_t *work = nullptr;   // worklist of systems to rebuild
+    int32_t *wslice = nullptr; // first build slice of each listed system
     int sort_grid = 1;         // workgroups of the rebuild's sort launch
     int build_grid = 1;        // workgroups of the rebuild's list-build launch
     unsigned long long *nent = nullptr;  // list entries of each system (twice its pairs)
@@ -172,14 +179,15 @@ void bdestroy(parm_batch *b) {
     bfree(b->stage);
     bfree(b->type);
     bfree(b->sys);
+    bfree(b->orig);
     bfree(b->nbr);
     bfree(b->ncount);
     bfree(b->keys);
-    bfree(b->cellidx);
+    bfree(b->ent);
     bfree(b->xs);
     bfree(b->dsort);
     bfree(b->cstart);
-    bfree(b->flags);
+    bfree(b->wl);
     bfree(b->work);
     bfree(b->wslice);
     bfree(b->which);
@@ -208,42 +216,55 @@ __global__ void kb_sys_index(int nsys, const BatchGeom *__restrict__ geom,
     for (int k = threadIdx.x; k < geom[s].n; k += blockDim.x) sys[geom[s].off + k] = s;
 }
 
+__global__ void kb_iota(int n, int32_t *__restrict__ p) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i < n) p[i] = i;
+}
+
+// Slot i of dst takes the caller's value orig[i].
+template <typename T>
+__global__ void kb_gather(int n, const int32_t *__restrict__ orig, const T *__restrict__ src,
+                          T *__restrict__ dst) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i < n) dst[i] = src[orig[i]];
+}
+
 __global__ void kb_upload(int ntot, int ndim, int what, BatchArrays A,
-                          const double *__restrict__ src) {
+                          const int32_t *__restrict__ orig, const double *__restrict__ src) {
     const int i = blockIdx.x * 256 + threadIdx.x;
     if (i >= ntot) return;
+    const double *s = src + (size_t)ndim * orig[i];
     if (what == 0) {
         if (ndim == 3)
-            static_cast<double4 *>(A.pos_out)[i] =
-                double4{src[3 * (size_t)i], src[3 * (size_t)i + 1], src[3 * (size_t)i + 2], 0.0};
+            static_cast<double4 *>(A.pos_out)[i] = double4{s[0], s[1], s[2], 0.0};
         else
-            static_cast<double2 *>(A.pos_out)[i] =
-                double2{src[2 * (size_t)i], src[2 * (size_t)i + 1]};
+            static_cast<double2 *>(A.pos_out)[i] = double2{s[0], s[1]};
         return;
     }
     double *const *dst = what == 1 ? A.v : (what == 2 ? A.a : A.f);
-    for (int k = 0; k < ndim; k++) dst[k][i] = src[(size_t)ndim * i + k];
+    for (int k = 0; k < ndim; k++) dst[k][i] = s[k];
 }
 
 __global__ void kb_download(int ntot, int ndim, int what, BatchArrays A,
-                            double *__restrict__ dst) {
+                            const int32_t *__restrict__ orig, double *__restrict__ dst) {
     const int i = blockIdx.x * 256 + threadIdx.x;
     if (i >= ntot) return;
+    double *d = dst + (size_t)ndim * orig[i];
     if (what == 0) {
         if (ndim == 3) {
             const double4 p = static_cast<const double4 *>(A.pos_in)[i];
-            dst[3 * (size_t)i] = p.x;
-            dst[3 * (size_t)i + 1] = p.y;
-            dst[3 * (size_t)i + 2] = p.z;
+            d[0] = p.x;
+            d[1] = p.y;
+            d[2] = p.z;
         } else {
             const double2 p = static_cast<const double2 *>(A.pos_in)[i];
-            dst[2 * (size_t)i] = p.x;
-            dst[2 * (size_t)i + 1] = p.y;
+            d[0] = p.x;
+            d[1] = p.y;
         }
         return;
     }
     double *const *src = what == 1 ? A.v : (what == 2 ? A.a : A.f);
-    for (int k = 0; k < ndim; k++) dst[(size_t)ndim * i + k] = src[k][i];
+    for (int k = 0; k < ndim; k++) d[k] = src[k][i];
 }
 
 int nb256(long n) { return (int)((n + 255) / 256); }
@@ -253,7 +274,7 @@ int bupload(parm_batch *b, int what, const double *host) {
     if (bytes == 0) return PARM_OK;
     PB_HIP(hipMemcpyAsync(b->stage, host, bytes, hipMemcpyHostToDevice, b->stream));
     hipLaunchKernelGGL(kb_upload, dim3(nb256(b->ntot)), dim3(256), 0, b->stream, b->ntot,
-                       b->ndim, what, b->arrays(), b->stage);
+                       b->ndim, what, b->arrays(), b->orig, b->stage);
     PB_HIP(hipGetLastError());
     PB_HIP(hipStreamSynchronize(b->stream));
     return PARM_OK;
@@ -263,9 +284,22 @@ int bdownload(parm_batch *b, int what, double *host) {
     const size_t bytes = sizeof(double) * (size_t)b->ntot * b->ndim;
     if (bytes == 0) return PARM_OK;
     hipLaunchKernelGGL(kb_download, dim3(nb256(b->ntot)), dim3(256), 0, b->stream, b->ntot,
-                       b->ndim, what, b->arrays(), b->stage);
+                       b->ndim, what, b->arrays(), b->orig, b->stage);
     PB_HIP(hipGetLastError());
     PB_HIP(hipMemcpyAsync(host, b->stage, bytes, hipMemcpyDeviceToHost, b->stream));
+    PB_HIP(hipStreamSynchronize(b->stream));
+    return PARM_OK;
+}
+
+// A per-atom scalar in the caller's order -> slot order.
+template <typename T>
+int bupload_scalar(parm_batch *b, const T *host, T *dst) {
+    static_assert(sizeof(T) <= sizeof(double), "staged in a double per atom");
+    T *tmp = reinterpret_cast<T *>(b->stage);
+    PB_HIP(hipMemcpyAsync(tmp, host, sizeof(T) * b->ntot, hipMemcpyHostToDevice, b->stream));
+    hipLaunchKernelGGL(kb_gather<T>, dim3(nb256(b->ntot)), dim3(256), 0, b->stream, b->ntot,
+                       b->orig, tmp, dst);
+    PB_HIP(hipGetLastError());
     PB_HIP(hipStreamSynchronize(b->stream));
     return PARM_OK;
 }
@@ -278,17 +312,49 @@ int read_gflag(parm_batch *b, uint32_t *fl) {
     return PARM_OK;
 }
 
-// Rebuild every system (force) or those whose skin flag is set.
+BatchLists lists_of(const parm_batch *b) {
+    BatchLists B{};
+    B.type_bits = b->type_bits;
+    B.tpa = b->tpa;
+    B.cap = b->cap;
+    B.npad = b->npad;
+    B.nbr = b->nbr;
+    B.ncount = b->ncount;
+    B.keys = b->keys;
+    B.ent = b->ent;
+    B.xs = b->xs;
+    B.dsort = b->dsort;
+    B.cstart = b->cstart;
+    B.which = b->which;
+    B.nent = b->nent;
+    B.work = b->work;
+    B.wslice = b->wslice;
+    B.sort_grid = b->sort_grid;
+    B.build_grid = b->build_grid;
+    B.sparse = b->ntot * 3.0 <= 20.0 * b->total_cells;
+    return B;
+}
+
+constexpr int kListAll = 2;  // the worklist counter of a rebuild of every system
+
+int skin_test(parm_batch *b, int list) {
+    PB_HIP(launch_batch_skin(b->nsys, b->arrays(), b->skin, lists_of(b).sparse, b->wl + list,
+                             b->work, b->wslice, b->gflag, b->stream));
+    return PARM_OK;
+}
+
+// Rebuild the systems on worklist `list` (kListAll: every system).  The other
+// one of the steps' two is emptied for the step's skin test.
 // `alt`: positions one step ahead of `pos`; for a rebuilt system their
 // displacement from the new reference positions is recomputed.
-int brebuild(parm_batch *b, bool force, bool count, const void *pos,
-             const void *alt = nullptr) {
-    PB_HIP(launch_batch_rebuild(b->ndim, b->nsys, b->arrays(), pos, alt, force ? 1 : 0,
-                                count ? 1 : 0, b->skin, b->type_bits, b->tpa, b->cap,
-                                b->npad, b->nbr, b->ncount, b->keys, b->cellidx, b->cstart,
-                                b->xs, b->dsort, b->flags, b->which, b->nent, b->gflag,
-                                b->work, b->wslice, b->sort_grid, b->build_grid,
-                                b->ntot * 3.0 <= 20.0 * b->total_cells, b->stream));
+int brebuild(parm_batch *b, int list, bool count, const void *pos, const void *alt = nullptr) {
+    const BatchLists B = lists_of(b);
+    if (list == kListAll)
+        PB_HIP(launch_batch_all(b->nsys, b->arrays(), B.sparse, b->wl + list, b->work, b->wslice,
+                                b->stream));
+    PB_HIP(launch_batch_rebuild(b->ndim, b->arrays(), B, pos, alt, count ? 1 : 0, b->skin,
+                                b->wl + list, list == kListAll ? nullptr : b->wl + (1 - list),
+                                b->gflag, b->stream));
     return PARM_OK;
 }
 
@@ -300,12 +366,25 @@ int ensure_cap(parm_batch *b, int cap) {
     return PARM_OK;
 }
 
+// Every system's slots ordered by cell at the current positions.
+int order_slots(parm_batch *b) {
+    BatchLists B = lists_of(b);
+    B.nbr = nullptr;
+    PB_HIP(launch_batch_all(b->nsys, b->arrays(), B.sparse, b->wl + kListAll, b->work,
+                            b->wslice, b->stream));
+    PB_HIP(launch_batch_rebuild(b->ndim, b->arrays(), B, b->pos, nullptr, 0, b->skin,
+                                b->wl + kListAll, nullptr, b->gflag, b->stream));
+    PB_HIP(launch_batch_reorder(b->ndim, b->arrays(), B, b->pos, b->pos_alt, b->m, b->diam,
+                                b->type, b->orig, b->stage, b->eatom, b->stream));
+    return PARM_OK;
+}
+
 // First build of every system (NeighborList::update_list on a new list),
 // growing the list capacity until nothing overflows.
 int first_build(parm_batch *b) {
     for (int attempt = 0; attempt < 6; attempt++) {
         PB_HIP(hipMemsetAsync(b->gflag, 0, sizeof(uint32_t), b->stream));
-        PB_CHECK(brebuild(b, true, true, b->pos));
+        PB_CHECK(brebuild(b, kListAll, true, b->pos));
         uint32_t fl = 0;
         PB_CHECK(read_gflag(b, &fl));
         if (!(fl & kFlagOverflow)) {
@@ -337,7 +416,7 @@ int bautotune(parm_batch *b) {
     float best_ms = 1e30f;
     for (int tpa : {1, 2, 4, 8}) {
         b->tpa = tpa;
-        PB_CHECK(brebuild(b, true, false, b->xref));
+        PB_CHECK(brebuild(b, kListAll, false, b->xref));
         PB_HIP(launch_batch_force(b->ndim, b->prec, kStageForceOnly, false, b->arrays(),
                                   b->listview(), b->pairview(), c, b->eatom, b->stream));
         float tmin = 1e30f;
@@ -359,7 +438,7 @@ int bautotune(parm_batch *b) {
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
     b->tpa = best;
-    PB_CHECK(brebuild(b, true, false, b->xref));
+    PB_CHECK(brebuild(b, kListAll, false, b->xref));
     b->tuned = true;
     return PARM_OK;
 }
@@ -387,7 +466,8 @@ int prof_end(parm_batch *b, hipEvent_t *e,
     return PARM_OK;
 }
 
-int fused_step(parm_batch *b, bool damped, const StepCoef &c, void *cur, void *nxt) {
+// `list`: the worklist that the skin test at x_q filled.
+int fused_step(parm_batch *b, bool damped, const StepCoef &c, void *cur, void *nxt, int list) {
     BatchArrays A = b->arrays();
     A.pos_in = cur;
     A.pos_out = nxt;
@@ -398,10 +478,9 @@ int fused_step(parm_batch *b, bool damped, const StepCoef &c, void *cur, void *n
                               b->listview(), b->pairview(), c, b->eatom, b->stream));
     PB_CHECK(prof_end(b, ev, b->prof_force));
     PB_CHECK(prof_begin(b, ev));
-    PB_CHECK(brebuild(b, false, true, cur, nxt));
+    PB_CHECK(brebuild(b, list, true, cur, nxt));
     PB_CHECK(prof_end(b, ev, b->prof_rebuild));
-    PB_HIP(launch_batch_skin(b->nsys, b->arrays(), b->skin, b->flags, b->gflag, b->stream));
-    return PARM_OK;
+    return skin_test(b, 1 - list);
 }
 
 int run_batch(parm_batch *b, bool damped, const StepCoef &c, int64_t nsteps, bool graph) {
@@ -412,8 +491,8 @@ int run_batch(parm_batch *b, bool damped, const StepCoef &c, int64_t nsteps, boo
     hipStream_t st = b->stream;
     PB_HIP(hipMemsetAsync(b->gflag, 0, sizeof(uint32_t), st));
     // first half of step 0 and its skin test
-    PB_HIP(launch_batch_drift(b->ndim, damped, b->arrays(), c, st));
-    PB_HIP(launch_batch_skin(b->nsys, b->arrays(), b->skin, b->flags, b->gflag, st));
+    PB_HIP(launch_batch_drift(b->ndim, damped, b->arrays(), c, b->wl, st));
+    PB_CHECK(skin_test(b, 0));
     int64_t q = 0;
     const int64_t pairs = (nsteps - 1) / 2;
     if (graph && pairs > 0 && !b->prof) {
@@ -426,8 +505,8 @@ int run_batch(parm_batch *b, bool damped, const StepCoef &c, int64_t nsteps, boo
             }
             hipGraph_t g = nullptr;
             PB_HIP(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
-            int rc1 = fused_step(b, damped, c, b->pos, b->pos_alt);
-            int rc2 = rc1 == PARM_OK ? fused_step(b, damped, c, b->pos_alt, b->pos) : rc1;
+            int rc1 = fused_step(b, damped, c, b->pos, b->pos_alt, 0);
+            int rc2 = rc1 == PARM_OK ? fused_step(b, damped, c, b->pos_alt, b->pos, 1) : rc1;
             hipError_t ec = hipStreamEndCapture(st, &g);
             if (rc2 != PARM_OK) return rc2;
             if (ec != hipSuccess)
@@ -448,14 +527,14 @@ int run_batch(parm_batch *b, bool damped, const StepCoef &c, int64_t nsteps, boo
         q = 2 * pairs;
     }
     for (; q < nsteps - 1; q++) {
-        PB_CHECK(fused_step(b, damped, c, b->pos, b->pos_alt));
+        PB_CHECK(fused_step(b, damped, c, b->pos, b->pos_alt, (int)(q & 1)));
         std::swap(b->pos, b->pos_alt);
     }
     // last step: forces + closing kick, then update_trackers at x_n
     PB_HIP(launch_batch_force(b->ndim, b->prec, damped ? kStageDampedKick : kStageVerletKick,
                               false, b->arrays(), b->listview(), b->pairview(), c, b->eatom,
                               st));
-    PB_CHECK(brebuild(b, false, true, b->pos));
+    PB_CHECK(brebuild(b, (int)(q & 1), true, b->pos));
     uint32_t fl = 0;
     PB_CHECK(read_gflag(b, &fl));
     if (fl & kFlagNonFinite) return bfail(PARM_E_NONFINITE, "a position became non-finite");
@@ -524,7 +603,7 @@ int parm_batch_create(int ndim, int precision, int64_t nsys, const int64_t *nato
         return bail(bfail(PARM_E_DEVICE, "stream creation failed"));
     // rebuild launches: the sort one 1024-thread workgroup per CU, the list
     // build eight 256-thread workgroups per CU (both loop over their work)
-    b->sort_grid = std::max(1, prop.multiProcessorCount);
+    b->sort_grid = std::min(b->nsys, std::max(1, prop.multiProcessorCount));
     b->build_grid = 8 * std::max(1, prop.multiProcessorCount);
     const size_t n = (size_t)tot;
     int rc;
@@ -538,11 +617,11 @@ int parm_batch_create(int ndim, int precision, int64_t nsys, const int64_t *nato
             return bail(rc);
     if ((rc = balloc(&b->m, n)) || (rc = balloc(&b->diam, n)) || (rc = balloc(&b->disp, n)) ||
         (rc = balloc(&b->stage, n * ndim)) || (rc = balloc(&b->type, n)) ||
-        (rc = balloc(&b->sys, n)) || (rc = balloc(&b->ncount, (size_t)b->npad)) ||
-        (rc = balloc(&b->keys, n)) || (rc = balloc(&b->cellidx, n)) ||
+        (rc = balloc(&b->sys, n)) || (rc = balloc(&b->orig, n)) || (rc = balloc(&b->ncount, (size_t)b->npad)) ||
+        (rc = balloc(&b->keys, n)) || (rc = balloc(&b->ent, n)) ||
         (rc = balloc((char **)&b->xs, n * b->pos_bytes)) || (rc = balloc(&b->dsort, n)) ||
-        (rc = balloc(&b->flags, (size_t)nsys)) || (rc = balloc(&b->which, (size_t)nsys)) ||
-        (rc = balloc(&b->work, (size_t)nsys + 1)) || (rc = balloc(&b->wslice, (size_t)nsys + 1)) ||
+        (rc = balloc(&b->wl, 3)) || (rc = balloc(&b->which, (size_t)nsys)) ||
+        (rc = balloc(&b->work, (size_t)nsys)) || (rc = balloc(&b->wslice, (size_t)nsys)) ||
         (rc = balloc(&b->gflag, 1)) || (rc = balloc(&b->nent, (size_t)nsys)) ||
         (rc = balloc(&b->eatom, 4 * n)) || (rc = balloc(&b->sysout, 4 * (size_t)nsys)) ||
         (rc = balloc(&b->geom, (size_t)nsys)))
@@ -560,10 +639,12 @@ int parm_batch_create(int ndim, int precision, int64_t nsys, const int64_t *nato
     (void)hipMemsetAsync(b->xref, 0, n * b->pos_bytes, st);
     (void)hipMemsetAsync(b->disp, 0, n * sizeof(double), st);
     (void)hipMemsetAsync(b->type, 0, n * sizeof(int32_t), st);
-    (void)hipMemsetAsync(b->flags, 0, nsys * sizeof(uint32_t), st);
+    (void)hipMemsetAsync(b->wl, 0, 3 * sizeof(unsigned long long), st);
     (void)hipMemsetAsync(b->which, 0, nsys * sizeof(uint32_t), st);
     (void)hipMemsetAsync(b->nent, 0, nsys * sizeof(unsigned long long), st);
     (void)hipMemsetAsync(b->gflag, 0, sizeof(uint32_t), st);
+    hipLaunchKernelGGL(kb_iota, dim3(nb256(b->ntot)), dim3(256), 0, st, b->ntot, b->orig);
+    if (hipGetLastError() != hipSuccess) return bail(bfail(PARM_E_DEVICE, "initialisation failed"));
     std::vector<double> ones(n, 1.0);
     if (hipMemcpyAsync(b->m, ones.data(), n * sizeof(double), hipMemcpyHostToDevice, st) !=
             hipSuccess ||
@@ -589,8 +670,7 @@ int parm_batch_info(const parm_batch *b, int *ndim, int *nsys, int64_t *natoms_t
 int parm_batch_set_masses(parm_batch *b, const double *masses) {
     if (!b || !masses) return bfail(PARM_E_INVALID, "null argument");
     PB_HIP(hipSetDevice(b->device));
-    PB_HIP(hipMemcpy(b->m, masses, sizeof(double) * b->ntot, hipMemcpyHostToDevice));
-    return PARM_OK;
+    return bupload_scalar<double>(b, masses, b->m);
 }
 
 int parm_batch_set_state(parm_batch *b, const double *x, const double *v, const double *a) {
@@ -682,8 +762,8 @@ static int batch_pair(parm_batch *b, int kind, int ntypes, const double *eps,
     b->tab0 = tab[0];
     PB_HIP(hipMemcpy(b->geom, b->geom_h.data(), sizeof(BatchGeom) * b->nsys,
                      hipMemcpyHostToDevice));
-    PB_HIP(hipMemcpy(b->type, atype, sizeof(int32_t) * b->ntot, hipMemcpyHostToDevice));
-    PB_HIP(hipMemcpy(b->diam, dia.data(), sizeof(double) * b->ntot, hipMemcpyHostToDevice));
+    PB_CHECK(bupload_scalar<int32_t>(b, atype, b->type));
+    PB_CHECK(bupload_scalar<double>(b, dia.data(), b->diam));
     hipLaunchKernelGGL(kb_sys_index, dim3(b->nsys), dim3(256), 0, b->stream, b->nsys, b->geom,
                        b->sys);
     PB_HIP(hipGetLastError());
@@ -733,13 +813,15 @@ int parm_batch_initialize(parm_batch *b) {
     PB_HIP(hipSetDevice(b->device));
     // Collection::initialize: update_list(false) (a new list: rebuild),
     // set_forces(true), update_list(false)
+    b->built = false;  // until the lists of the new order stand
+    PB_CHECK(order_slots(b));
     PB_CHECK(first_build(b));
     StepCoef c{};
     PB_HIP(launch_batch_force(b->ndim, b->prec, kStageForceA, false, b->arrays(),
                               b->listview(), b->pairview(), c, b->eatom, b->stream));
-    PB_HIP(launch_batch_disp(b->ndim, b->arrays(), b->stream));
-    PB_HIP(launch_batch_skin(b->nsys, b->arrays(), b->skin, b->flags, b->gflag, b->stream));
-    PB_CHECK(brebuild(b, false, true, b->pos));
+    PB_HIP(launch_batch_disp(b->ndim, b->arrays(), b->wl, b->stream));
+    PB_CHECK(skin_test(b, 0));
+    PB_CHECK(brebuild(b, 0, true, b->pos));
     PB_HIP(hipStreamSynchronize(b->stream));
     return PARM_OK;
 }
@@ -868,31 +950,29 @@ int parm_batch_pairs(parm_batch *b, int64_t sysid, int64_t cap, int32_t *first,
     if (cap > 0 && (!first || !last)) return bfail(PARM_E_INVALID, "null output");
     PB_HIP(hipSetDevice(b->device));
     const int o = b->off[sysid], n = b->off[sysid + 1] - o;
-    std::vector<int32_t> cnt(n);
+    std::vector<int32_t> cnt(n), orig(n);
+    PB_HIP(hipMemcpyAsync(orig.data(), b->orig + o, sizeof(int32_t) * n, hipMemcpyDeviceToHost,
+                          b->stream));
     std::vector<uint32_t> nb((size_t)b->cap * b->npad);
     PB_HIP(hipMemcpyAsync(cnt.data(), b->ncount + o, sizeof(int32_t) * n,
                           hipMemcpyDeviceToHost, b->stream));
     PB_HIP(hipMemcpyAsync(nb.data(), b->nbr, sizeof(uint32_t) * nb.size(),
                           hipMemcpyDeviceToHost, b->stream));
     PB_HIP(hipStreamSynchronize(b->stream));
-    int64_t w = 0;
-    std::vector<int32_t> lower;
+    std::vector<std::pair<int32_t, int32_t>> pairs;  // the caller's indices
     for (int li = 0; li < n; li++) {
         const int i = o + li;
-        lower.clear();
         for (int q = 0; q < cnt[li]; q++) {
             const size_t idx = ((size_t)(q / b->tpa) * b->npad + i) * b->tpa + q % b->tpa;
-            const int j = (int)(nb[idx] >> b->type_bits) - o;
-            if (j < li) lower.push_back(j);
+            const int lj = (int)(nb[idx] >> b->type_bits) - o;
+            if (orig[lj] < orig[li]) pairs.emplace_back(orig[li] - o, orig[lj] - o);
         }
-        std::sort(lower.begin(), lower.end());
-        for (int32_t lj : lower) {
-            if (w < cap) {
-                first[w] = li;
-                last[w] = lj;
-            }
-            w++;
-        }
+    }
+    std::sort(pairs.begin(), pairs.end());
+    const int64_t w = (int64_t)pairs.size();
+    for (int64_t k = 0; k < std::min(cap, w); k++) {
+        first[k] = pairs[k].first;
+        last[k] = pairs[k].second;
     }
     if (npairs) *npairs = w;
     return PARM_OK;

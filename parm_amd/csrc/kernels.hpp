@@ -324,25 +324,49 @@ void batch_force_part(int stage, bool energy, const BatchArrays &A, const ListVi
 hipError_t launch_batch_force(int ndim, int precision, int stage, bool energy,
                               const BatchArrays &A, const ListView &Lv, const PairView &P,
                               const StepCoef &c, double *eatom, hipStream_t s);
+// A worklist (wl): the number of listed systems (high word) and of their build
+// slices (low word).  The drift and disp launches empty it, the skin test
+// fills it with the systems to rebuild, launch_batch_all with every system.
 hipError_t launch_batch_drift(int ndim, bool damped, const BatchArrays &A,
-                              const StepCoef &c, hipStream_t s);
-hipError_t launch_batch_disp(int ndim, const BatchArrays &A, hipStream_t s);
-hipError_t launch_batch_skin(int nsys, const BatchArrays &A, double skin, uint32_t *flags,
+                              const StepCoef &c, unsigned long long *wl, hipStream_t s);
+hipError_t launch_batch_disp(int ndim, const BatchArrays &A, unsigned long long *wl,
+                             hipStream_t s);
+hipError_t launch_batch_skin(int nsys, const BatchArrays &A, double skin, bool sparse,
+                             unsigned long long *wl, int32_t *work, int32_t *wslice,
                              uint32_t *gflag, hipStream_t s);
-// Rebuilds the systems whose skin flag is set (all with force): worklist,
-// sort, then the list build spread over slices of the listed systems.
-// work: nsys + 1 ints (count, then system ids); wslice: nsys + 1 ints (each
-// listed system's first build slice, then the total).  sparse: few atoms per
-// stencil row (the build's lanes per atom).  nent: per system the
-// list entries of its last build (twice its pairs).
-hipError_t launch_batch_rebuild(int ndim, int nsys, const BatchArrays &A, const void *pos,
-                                const void *alt, int force, int count_rebuild, double skin,
-                                int type_bits, int tpa, int cap, int npad, uint32_t *nbr,
-                                int32_t *ncount, int32_t *keys, int32_t *cellidx,
-                                int32_t *cstart, void *xs, double *dsort, uint32_t *flags,
-                                uint32_t *which, unsigned long long *nent, uint32_t *gflag,
-                                int32_t *work, int32_t *wslice, int sort_grid, int build_grid,
-                                bool sparse, hipStream_t s);
+hipError_t launch_batch_all(int nsys, const BatchArrays &A, bool sparse, unsigned long long *wl,
+                            int32_t *work, int32_t *wslice, hipStream_t s);
+// The batch's lists and what their build works on.
+struct BatchLists {
+    int type_bits, tpa, cap, npad;
+    uint32_t *nbr;        // null: sort only
+    int32_t *ncount;
+    int32_t *keys;        // sorted slots: cell,
+    uint32_t *ent;        // list word (index << type_bits | type),
+    void *xs;             // position
+    double *dsort;        // and diameter
+    int32_t *cstart;      // each cell's first sorted slot
+    uint32_t *which;      // rebuilds per system
+    unsigned long long *nent;  // list entries of its last build (twice its pairs)
+    int32_t *work, *wslice;    // nsys each: listed systems, their first build slice
+    int sort_grid, build_grid;
+    bool sparse;          // few atoms per stencil row (the build's lanes per atom)
+};
+// Rebuilds the systems listed in wl: sort, then the list build spread over
+// slices of the listed systems; empties wl_next (may be null).  alt: positions
+// one step ahead, whose displacements from the new reference positions are
+// stored.
+hipError_t launch_batch_rebuild(int ndim, const BatchArrays &A, const BatchLists &B,
+                                const void *pos, const void *alt, int count_rebuild,
+                                double skin, const unsigned long long *wl,
+                                unsigned long long *wl_next, uint32_t *gflag, hipStream_t s);
+// Every system's slots in the order of its last sort: pos, v, a, m, diam, type
+// and orig (the caller's index of each slot) permuted in place, through
+// scratch arrays of the batch (pos_alt, stage: ndim doubles per atom, eatom: 4,
+// B.xs).  f and the lists are void afterwards.
+hipError_t launch_batch_reorder(int ndim, const BatchArrays &A, const BatchLists &B, void *pos,
+                                void *pos_alt, double *m, double *diam, int32_t *type,
+                                int32_t *orig, double *stage, double *eatom, hipStream_t s);
 hipError_t launch_batch_sys_sums(int nsys, const BatchArrays &A, const double *eatom,
                                  double *out, hipStream_t s);
 constexpr int kBatchMaxCellsPerSystem = 4096;
