@@ -77,7 +77,8 @@ __global__ __launch_bounds__(kBlock) void k_batch_disp(BatchArrays A,
 // systems arrive in (their rebuilds are independent).
 // W wavefronts per system, each thread kSkinAhead loads at a time: the pass is
 // bound by the latency of its loads, not their 8 bytes per atom.  1024 systems
-// of 64 - 4096 atoms: SKIN_MEASURED
+// of 64 - 4096 atoms: 31 us per launch with one wavefront per
+// system and one load at a time, 6.7 us.
 constexpr int kSkinAhead = 4;
 
 template <int W>
@@ -196,7 +197,8 @@ __global__ __launch_bounds__(kAllThreads) void k_batch_all(
 // atom's arrival on its cell's counter, then its rank among the cell's atoms
 // by their indices (so the order is the stable one).  The general form
 // reloads the positions per chunk and takes its ranks from ballots, the
-// wavefronts in turn: 16 barriers per chunk.  SORT_MEASURED
+// wavefronts in turn: 16 barriers per chunk.  1024 systems of
+// 64 - 4096: 28 us per launch in the general form, 14 us.
 constexpr int kSortKeep = 4;
 constexpr int kRankMax = 64;
 
@@ -402,15 +404,16 @@ __global__ __launch_bounds__(kSortThreads) void k_batch_sort(
         sort_system<D>(work[q], A, pos, count_rebuild, type_bits, S, which, nent, hist, slots);
 }
 
-// G lanes per atom, U candidates per lane and round.  The build is bound by
-// the latency of its chain of dependent loads (cell bounds, then candidates),
-// not by arithmetic: at a step a few dozen systems rebuild.  A stencil row of
-// three x-adjacent cells is one contiguous range (two where it wraps), so an
-// atom takes 9 rows, not 27 cells; the group's lanes load all rows' bounds
-// together and test G * U candidates per round.  48 liquids of 300 - 1000 atoms:
-// 179 us per launch with one thread per atom, a step 210 -> 69 us; 1024
-// packings of 64 - 4096 (4 x 2 lanes): 200 steps 85.1 -> 80.0 ms.
-template <int D, int G, int U>
+// G lanes per atom.  The build is bound by the latency of its chain of
+// dependent loads (cell bounds, then candidates), not by arithmetic: at a step
+// a few systems rebuild.  A stencil row of three x-adjacent cells is one
+// contiguous range (two where it wraps), so an atom takes 9 rows, not 27
+// cells; the group's lanes load all rows' bounds together and test G
+// candidates per round.  48 liquids of 300 - 1000 atoms: 179 us per launch with
+// one thread per atom, 27 us with 8 lanes of four candidates.  (Loading the
+// next round's candidates before testing this one's is no faster: 200 liquids
+// 7.67 against 7.57 ms per 100 steps.)
+template <int D, int G>
 __global__ __launch_bounds__(kBuildThreads) void k_batch_build(
     BatchArrays A, const typename PosStore<D>::T *__restrict__ alt, double skin,
     int type_bits, int tpa, int cap, int npad, uint32_t *__restrict__ nbr,
@@ -484,63 +487,48 @@ __global__ __launch_bounds__(kBuildThreads) void k_batch_build(
             }
             int cnt = 0;
             for (int r = 0; r < nrows; r++) {
-                const int owner = gbase + (r % G);
                 int rb[4];
 #pragma unroll
                 for (int k = 0; k < 4; k++) {
                     int v = bnd[0][k];
 #pragma unroll
                     for (int q = 1; q < RPL; q++) v = r / G == q ? bnd[q][k] : v;
-                    rb[k] = __shfl(v, owner);
+                    rb[k] = __shfl(v, gbase + r % G);
                 }
 #pragma unroll
                 for (int h = 0; h < 2; h++) {
-                    const int a = rb[2 * h], b = rb[2 * h + 1];
-                    for (int base = a; base < b; base += G * U) {
-                        // the round's loads in flight together; a slot past
-                        // the range reads the atom's own (and is not tested)
-                        Vec<D> xj[U];
-                        double dj[U];
-                        uint32_t ej[U];
+                    for (int base = rb[2 * h]; base < rb[2 * h + 1]; base += G) {
+                        // (a lane past the range reads the atom's own slot,
+                        // which is not tested)
+                        const int v = base + sub < rb[2 * h + 1] ? base + sub : off + u;
+                        const Vec<D> xj = PosStore<D>::load(xs[v]);
+                        const double dj = dsort[v];
+                        const uint32_t ej = ent[v];
+                        bool pass = false;
+                        if (v != off + u) {
+                            // minimum image by rint: equal to the reference's
+                            // remainder up to rounding far inside the 1e-6
+                            // band, where the reference's predicate decides
+                            double d2 = 0.0;
 #pragma unroll
-                        for (int q = 0; q < U; q++) {
-                            const int v = base + q * G + sub;
-                            const int vv = v < b ? v : off + u;
-                            xj[q] = PosStore<D>::load(xs[vv]);
-                            dj[q] = dsort[vv];
-                            ej[q] = ent[vv];
-                        }
-#pragma unroll
-                        for (int q = 0; q < U; q++) {
-                            if (base + q * G >= b) break;  // uniform over the group
-                            const int v = base + q * G + sub;
-                            bool pass = false;
-                            if (v < b && v != off + u) {
-                                // minimum image by rint: equal to the
-                                // reference's remainder up to rounding far
-                                // inside the 1e-6 band, where the reference's
-                                // predicate decides
-                                double d2 = 0.0;
-#pragma unroll
-                                for (int k = 0; k < D; k++) {
-                                    double dk = xi.c[k] - xj[q].c[k];
-                                    dk -= G_.box.L[k] * rint(dk * G_.box.invL[k]);
-                                    d2 = fma(dk, dk, d2);
-                                }
-                                const double cut = (di + dj[q]) / 2 + skin;
-                                const double c2c = cut * cut;
-                                pass = d2 < c2c * (1.0 - 1e-6) ||
-                                       (d2 <= c2c * (1.0 + 1e-6) &&
-                                        in_list<D>(xi, xj[q], di, dj[q], G_.box, skin));
+                            for (int k = 0; k < D; k++) {
+                                double dk = xi.c[k] - xj.c[k];
+                                dk -= G_.box.L[k] * rint(dk * G_.box.invL[k]);
+                                d2 = fma(dk, dk, d2);
                             }
-                            const unsigned long long m =
-                                (__ballot(pass) >> gbase) & ((1ull << G) - 1ull);
-                            if (pass) {
-                                const int w = cnt + __popcll(m & below);
-                                if (w < cap) nbr[untiled_entry(w, i, tpa, npad)] = ej[q];
-                            }
-                            cnt += __popcll(m);
+                            const double cut = (di + dj) / 2 + skin;
+                            const double c2c = cut * cut;
+                            pass = d2 < c2c * (1.0 - 1e-6) ||
+                                   (d2 <= c2c * (1.0 + 1e-6) &&
+                                    in_list<D>(xi, xj, di, dj, G_.box, skin));
                         }
+                        const unsigned long long m =
+                            (__ballot(pass) >> gbase) & ((1ull << G) - 1ull);
+                        if (pass) {
+                            const int w = cnt + __popcll(m & below);
+                            if (w < cap) nbr[untiled_entry(w, i, tpa, npad)] = ej;
+                        }
+                        cnt += __popcll(m);
                     }
                 }
             }
@@ -576,7 +564,8 @@ __global__ __launch_bounds__(kBuildThreads) void k_batch_build(
 // columns stay where they are (a captured run of steps holds their addresses).
 // The caller's order is none in space: with it, an atom's neighbours are
 // anywhere among its system's positions, each a cache line of its own for one
-// gather.  MEASURED_ORDER
+// gather.  1024 packed systems of 64 - 4096 given in random order: the force
+// launch 208 -> 182 us.
 template <int D>
 struct OrderScratch {
     typename PosStore<D>::T *pos;
@@ -709,39 +698,40 @@ hipError_t launch_batch_disp(int ndim, const BatchArrays &A, unsigned long long 
     return hipGetLastError();
 }
 
-// Build lanes per atom and candidates per lane and round: a dense system (a
-// liquid: ~50 atoms in a stencil row) 8 x 4, a sparse one (packed spheres: ~8)
-// 4 x 2, whose round is a row (200 steps of 1024 packings: 80.0 ms, 87.1 ms with
-// 8 x 4; one thread per atom 85.1 ms).  The caller's line between them, 20
-// atoms to a row of three cells, lies where a row is two to three sparse
-// rounds and over half a dense one.
-constexpr int kBuildLanes = 8, kBuildAhead = 4;
-constexpr int kBuildLanesSparse = 4, kBuildAheadSparse = 2;
-
-static inline int build_slice(bool sparse) {
-    return kBuildThreads / (sparse ? kBuildLanesSparse : kBuildLanes);
+// Build lanes per atom: those whose round is a stencil row or more leave the
+// shortest chain, as long as the wavefronts that they make fit the chip.
+// A dense batch (a liquid: ~50 atoms to a row) takes 32: 48 / 200 / 800
+// liquids of 300 - 1000, passes of 100 steps with 8 x 4 (lanes x candidates
+// per lane and round), 16 x 2 and 32 x 1: 5.23 / 4.22 / 3.82, 9.03 / 7.87 /
+// 7.45, 20.6 / 19.6 / 19.8 ms.  A sparse one (packed spheres: ~8 to a row) of
+// 16 / 64 / 256 / 1024 systems of 64 - 4096, passes of 200 steps: 16 lanes
+// 5.8 / 9.6 / 19.6 / - , 8 lanes 6.2 / 9.8 / 18.6 / 61.4, 4 lanes 7.0 / 11.2 /
+// 19.7 / 59.4 ms.  The lines in between: 20 atoms to a row, 2^18 and 2^20 atoms.
+int batch_build_lanes(int ntot, int cells) {
+    if (3.0 * ntot > 20.0 * cells) return 32;
+    return ntot <= (1 << 18) ? 16 : (ntot <= (1 << 20) ? 8 : 4);
 }
 
 // One wavefront per system of up to kSkinWaveAtoms atoms on average (two
 // rounds of its loads), else a workgroup.
 constexpr long kSkinWaveAtoms = 2 * kSkinAhead * kWave;
 
-hipError_t launch_batch_skin(int nsys, const BatchArrays &A, double skin, bool sparse,
+hipError_t launch_batch_skin(int nsys, const BatchArrays &A, double skin, int lanes,
                              unsigned long long *wl, int32_t *work, int32_t *wslice,
                              uint32_t *gflag, hipStream_t s) {
     constexpr int kWaves = kBlock / kWave;
     if (A.ntot <= kSkinWaveAtoms * nsys)
         hipLaunchKernelGGL(k_batch_skin<1>, dim3((nsys + kWaves - 1) / kWaves), dim3(kBlock), 0,
-                           s, nsys, A, skin, build_slice(sparse), wl, work, wslice, gflag);
+                           s, nsys, A, skin, kBuildThreads / lanes, wl, work, wslice, gflag);
     else
         hipLaunchKernelGGL(k_batch_skin<kWaves>, dim3(nsys), dim3(kBlock), 0, s, nsys, A, skin,
-                           build_slice(sparse), wl, work, wslice, gflag);
+                           kBuildThreads / lanes, wl, work, wslice, gflag);
     return hipGetLastError();
 }
 
-hipError_t launch_batch_all(int nsys, const BatchArrays &A, bool sparse, unsigned long long *wl,
+hipError_t launch_batch_all(int nsys, const BatchArrays &A, int lanes, unsigned long long *wl,
                             int32_t *work, int32_t *wslice, hipStream_t s) {
-    hipLaunchKernelGGL(k_batch_all, dim3(1), dim3(kAllThreads), 0, s, nsys, build_slice(sparse),
+    hipLaunchKernelGGL(k_batch_all, dim3(1), dim3(kAllThreads), 0, s, nsys, kBuildThreads / lanes,
                        A.geom, wl, work, wslice);
     return hipGetLastError();
 }
@@ -757,15 +747,21 @@ static hipError_t batch_rebuild(const BatchArrays &A, const BatchLists &B, const
                        (const PT *)pos, count_rebuild, B.type_bits, S, B.which, B.nent, wl,
                        wl_next, B.work);
     if (!B.nbr) return hipGetLastError();
-#define PARM_BB(GG, UU)                                                                       \
-    hipLaunchKernelGGL((k_batch_build<D, GG, UU>), dim3(B.build_grid), dim3(kBuildThreads),   \
-                       0, s, A, (const PT *)alt, skin, B.type_bits, B.tpa, B.cap, B.npad,     \
-                       B.nbr, B.ncount, B.keys, B.ent, B.cstart, (const PT *)B.xs, B.dsort,   \
-                       B.nent, gflag, wl, B.work, B.wslice)
-    if (B.sparse)
-        PARM_BB(kBuildLanesSparse, kBuildAheadSparse);
-    else
-        PARM_BB(kBuildLanes, kBuildAhead);
+#define PARM_BB(GG)                                                                           \
+    case GG:                                                                                  \
+        hipLaunchKernelGGL((k_batch_build<D, GG>), dim3(B.build_grid), dim3(kBuildThreads),   \
+                           0, s, A, (const PT *)alt, skin, B.type_bits, B.tpa, B.cap, B.npad, \
+                           B.nbr, B.ncount, B.keys, B.ent, B.cstart, (const PT *)B.xs,        \
+                           B.dsort, B.nent, gflag, wl, B.work, B.wslice);                     \
+        break
+    switch (B.lanes) {
+        PARM_BB(4);
+        PARM_BB(8);
+        PARM_BB(16);
+        PARM_BB(32);
+        default:
+            return hipErrorInvalidValue;
+    }
 #undef PARM_BB
     return hipGetLastError();
 }

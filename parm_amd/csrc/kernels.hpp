@@ -331,11 +331,13 @@ hipError_t launch_batch_drift(int ndim, bool damped, const BatchArrays &A,
                               const StepCoef &c, unsigned long long *wl, hipStream_t s);
 hipError_t launch_batch_disp(int ndim, const BatchArrays &A, unsigned long long *wl,
                              hipStream_t s);
-hipError_t launch_batch_skin(int nsys, const BatchArrays &A, double skin, bool sparse,
+hipError_t launch_batch_skin(int nsys, const BatchArrays &A, double skin, int lanes,
                              unsigned long long *wl, int32_t *work, int32_t *wslice,
                              uint32_t *gflag, hipStream_t s);
-hipError_t launch_batch_all(int nsys, const BatchArrays &A, bool sparse, unsigned long long *wl,
+hipError_t launch_batch_all(int nsys, const BatchArrays &A, int lanes, unsigned long long *wl,
                             int32_t *work, int32_t *wslice, hipStream_t s);
+// Lanes per atom of the list build for a batch of ntot atoms in `cells` cells.
+int batch_build_lanes(int ntot, int cells);
 // The batch's lists and what their build works on.
 struct BatchLists {
     int type_bits, tpa, cap, npad;
@@ -350,7 +352,7 @@ struct BatchLists {
     unsigned long long *nent;  // list entries of its last build (twice its pairs)
     int32_t *work, *wslice;    // nsys each: listed systems, their first build slice
     int sort_grid, build_grid;
-    bool sparse;          // few atoms per stencil row (the build's lanes per atom)
+    int lanes;            // the build's lanes per atom (batch_build_lanes)
 };
 // Rebuilds the systems listed in wl: sort, then the list build spread over
 // slices of the listed systems; empties wl_next (may be null).  alt: positions

@@ -16,7 +16,7 @@ def _device_or_fail():
         pytest.fail("no GPU visible: the -m gpu tests need an MI355X")
 
 
-# build slices of 32 (dense) and 64 (sparse) atoms: one less, equal, one more
+# build slices of 8 and 16 atoms and their multiples: one less, equal, one more
 @pytest.mark.parametrize("ndim", [2, 3])
 @pytest.mark.parametrize("lj", [False, True])
 def test_batch_build_slice_edges(ndim, lj):
@@ -32,6 +32,46 @@ def test_batch_build_slice_edges(ndim, lj):
         fd, ld = b.pairs(s)
         fr, lr = r.pairs()
         assert np.array_equal(fd, fr) and np.array_equal(ld, lr), (s, sizes[s])
+    b.close()
+
+
+# the sort: from registers (up to 4096 atoms, 64 to a cell), by chunks (a cell of
+# more: boxes of fewer than three cells per edge; a system of more), and a
+# workgroup or a wavefront per system in the skin test; slices of 8 to 64 atoms
+# (32, 16, 8 and 4 build lanes); runs shorter and longer than a graph's eight steps
+@pytest.mark.parametrize("sizes,ndim,lj", [
+    ([4097, 1, 64, 65, 66, 130], 3, False), ([4096, 8200, 2], 2, False),
+    ([200, 3, 1000, 4500], 3, True), ([5] * 200 + [400], 3, True),
+    ([4000] * 67 + [70], 3, False), ([4000] * 263 + [70], 2, False)])
+def test_batch_sort_and_worklist(sizes, ndim, lj):
+    _device_or_fail()
+    print(f"batch sort {len(sizes)} systems ndim={ndim} lj={lj}", flush=True)
+    if lj:
+        systems = []
+        for k, n in enumerate(sizes):
+            x, L = S.jittered_lattice(n, 0.5, 3, seed=90 + k)
+            systems.append(dict(n=n, L=float(L[0]), x=x, v=np.zeros((n, 3)),
+                                types=np.zeros(n, np.int32), sig=np.ones(n)))
+    else:
+        systems = B.packings(sizes, 0.5, ndim, seed=31)
+    b = B.make_batch(systems, ndim, 0.3, lj=lj)
+    b.initialize()
+    look = sorted({0, len(sizes) // 2, len(sizes) - 2, len(sizes) - 1})
+    refs = dict(zip(look, B.oracle_systems([systems[k] for k in look], ndim, 0.3, lj=lj)))
+    for r in refs.values():
+        r.initialize()
+    for steps in (0, 1, 10, 19):
+        if steps:
+            b.damped(0.004, 1.0, steps)
+            for r in refs.values():
+                r.damped(0.004, 1.0, steps)
+        w, npairs = b.lists()
+        for s, r in refs.items():
+            fd, ld = b.pairs(s)
+            fr, lr = r.pairs()
+            assert np.array_equal(fd, fr) and np.array_equal(ld, lr), (s, steps)
+            assert w[s] == r.which() and npairs[s] == len(fr), (s, steps)
+    assert w.max() > 1
     b.close()
 
 
