@@ -129,7 +129,7 @@ struct parm_system {
     bool tpa_fixed = false, tuned = false;
     uint32_t *nbr = nullptr;       // untiled: uint32 entries; tiled: uint16 staged slots
     int32_t *ncount = nullptr;
-    uint16_t *lcount = nullptr;   // per-lane entry counts, npad x 8
+    uint16_t *lcount = nullptr;   // per-lane entry counts, npad x max_lanes(n)
     // tiled layout (tiles.hpp): the current list is tiled when `tiled`
     bool tiled = false, tile_ok = false;
     int layout_pref = 0;  // 0: tiled when possible, until tuned; 1: tiled; 2: untiled
@@ -257,7 +257,7 @@ struct parm_system {
     ReduceBuf redbuf(int flag_index) const {
         ReduceBuf R{};
         R.part = part;
-        R.pstride = force_blocks(std::max(n, 1), 8);
+        R.pstride = part_blocks(n);
         R.out = out;
         R.flag = dflag + flag_index;
         R.skin = skin;
@@ -332,13 +332,14 @@ int check_lane_counts(const parm_system *s) { return check_lane_counts(s->cap, s
 
 int ensure_list_capacity(parm_system *s, int cap) {
     if (cap <= s->cap && s->nbr) return PARM_OK;
+    const int round = max_lanes(s->n) - 1;
     // refused before the list is reallocated
-    PARM_CHECK(check_lane_counts(((int64_t)cap + 7) & ~(int64_t)7, s->tpa));
+    PARM_CHECK(check_lane_counts(((int64_t)cap + round) & ~(int64_t)round, s->tpa));
     free_list(s);
-    s->cap = (cap + 7) & ~7;
+    s->cap = (cap + round) & ~round;
     PARM_CHECK(dalloc(&s->nbr, (size_t)s->cap * s->npad));
     PARM_CHECK(dalloc(&s->ncount, (size_t)s->npad));
-    PARM_CHECK(dalloc(&s->lcount, (size_t)s->npad * 8));
+    PARM_CHECK(dalloc(&s->lcount, (size_t)s->npad * max_lanes(s->n)));
     return PARM_OK;
 }
 
@@ -440,7 +441,7 @@ void accept_tiles(parm_system *s, int nt, int smax, int bad) {
     s->tile_ok = true;
     s->ntiles = nt;
     s->smax = std::max(smax, 1);
-    s->tiled = s->layout_pref != 2 && tiled_force_fits(s);
+    s->tiled = s->layout_pref != 2 && s->tpa <= 8 && tiled_force_fits(s);
 }
 
 // The plan queued by launch_tile_plan, read back (one host round trip).
@@ -798,6 +799,11 @@ int autotune(parm_system *s, int stage, const StepCoef &c) {
             cands.emplace_back(lay, s->tpa);
         } else {
             for (int tpa : {1, 2, 4, 8}) cands.emplace_back(lay, tpa);
+            // (lanes past twice the mean row would find no entry)
+            for (int tpa = 16; lay == 0 && tpa <= max_lanes(s->n) &&
+                               (int64_t)tpa * s->n <= 4 * s->npairs;
+                 tpa *= 2)
+                cands.emplace_back(lay, tpa);
         }
     }
     // Mixed-precision repulsion of many atoms: only the candidates that add
@@ -1226,14 +1232,15 @@ int parm_system_create(int ndim, int precision, int64_t natoms, const double *ma
     s->npad = (int)((natoms + 63) / 64 * 64);
     if (s->npad == 0) s->npad = 64;
     s->pos_bytes = ndim == 3 ? sizeof(double4) : sizeof(double2);
+    if (const char *e = std::getenv("PARM_TILED")) s->layout_pref = std::atoi(e) == 0 ? 2 : 1;
     if (const char *e = std::getenv("PARM_TPA")) {
         int t = std::atoi(e);
-        if (t == 1 || t == 2 || t == 4 || t == 8) {
+        if (t == 1 || t == 2 || t == 4 || t == 8 ||
+            ((t == 16 || t == 32) && t <= max_lanes(s->n) && s->layout_pref == 2)) {
             s->tpa = t;
             s->tpa_fixed = true;
         }
     }
-    if (const char *e = std::getenv("PARM_TILED")) s->layout_pref = std::atoi(e) == 0 ? 2 : 1;
     int rc = PARM_OK;
     auto bail = [&](int r) {
         destroy(s);
@@ -1278,8 +1285,8 @@ int parm_system_create(int ndim, int precision, int64_t natoms, const double *ma
         (rc = dalloc(&s->hist, (size_t)256 * (radix_blocks((int)n) + 1))) ||
         (rc = dalloc(&s->stats, 2)) ||
         (rc = dalloc(&s->bpart, 2 * (size_t)build_blocks((int)n))) ||
-        (rc = dalloc(&s->part, (size_t)kRedWidth * force_blocks((int)n, 8))) ||
-        (rc = dalloc(&s->part2, (size_t)kRedWidth * force_blocks((int)n, 8))) ||
+        (rc = dalloc(&s->part, (size_t)kRedWidth * part_blocks((int)n))) ||
+        (rc = dalloc(&s->part2, (size_t)kRedWidth * part_blocks((int)n))) ||
         (rc = dalloc(&s->out, kRedWidth)) || (rc = dalloc(&s->fcnt, 1)) ||
         (rc = dalloc(&s->fgpart, 3 * kFinBlocks)) ||
         (rc = dalloc(&s->dflag, 2 * kFlagRing + 4)) || (rc = dalloc(&s->tinfo, 4)))
@@ -1633,7 +1640,7 @@ int parm_pair_sums(parm_system *s, double *U, double *W, double *S, uint64_t *co
 
 // ------------------------------------------- sums without allocation
 // Scratch of parm_pair_sums_noalloc: the per-workgroup partials of one force
-// launch (kRedWidth fields x force_blocks(n, 8) workgroups) and the reduced
+// launch (kRedWidth fields x part_blocks(n) workgroups) and the reduced
 // fields, for systems of at most kNoAllocMaxAtoms atoms.  Each GPU holds its
 // own copy for the life of the process; host code reaches it only through
 // the per-device address from hipGetSymbolAddress.
@@ -1690,7 +1697,7 @@ int parm_pair_sums_noalloc(parm_system *s, double *out) {
     PARM_CHECK(scratch_address(s->device, &scr));
     ReduceBuf R = s->redbuf(kSlotScratch);
     R.part = scr;
-    R.pstride = force_blocks(std::max(s->n, 1), 8);  // <= kNoAllocParts
+    R.pstride = part_blocks(s->n);  // <= kNoAllocParts
     R.out = scr + kRedWidth * kNoAllocParts;
     if (s->n > 0) {
         StepCoef c{};

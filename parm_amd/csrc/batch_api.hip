@@ -361,7 +361,8 @@ int brebuild(parm_batch *b, int list, bool count, const void *pos, const void *a
 int ensure_cap(parm_batch *b, int cap) {
     if (cap <= b->cap && b->nbr) return PARM_OK;
     bfree(b->nbr);
-    b->cap = (cap + 7) & ~7;
+    const int round = max_lanes(b->ntot) - 1;
+    b->cap = (cap + round) & ~round;
     PB_CHECK(balloc(&b->nbr, (size_t)b->cap * b->npad));
     return PARM_OK;
 }
@@ -414,7 +415,7 @@ int bautotune(parm_batch *b) {
     StepCoef c{};
     int best = b->tpa;
     float best_ms = 1e30f;
-    for (int tpa : {1, 2, 4, 8}) {
+    for (int tpa = 1; tpa <= max_lanes(b->ntot); tpa *= 2) {
         b->tpa = tpa;
         PB_CHECK(brebuild(b, kListAll, false, b->xref));
         PB_HIP(launch_batch_force(b->ndim, b->prec, kStageForceOnly, false, b->arrays(),
@@ -598,7 +599,7 @@ int parm_batch_create(int ndim, int precision, int64_t nsys, const int64_t *nato
     b->L.assign(L, L + nsys * ndim);
     if (const char *e = std::getenv("PARM_TPA")) {
         int t = std::atoi(e);
-        if (t == 1 || t == 2 || t == 4 || t == 8) {
+        if (t >= 1 && t <= max_lanes(b->ntot) && (t & (t - 1)) == 0) {
             b->tpa = t;
             b->tpa_fixed = true;
         }

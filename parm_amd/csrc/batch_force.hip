@@ -201,6 +201,12 @@ static void bforce_t(bool energy, const BatchArrays &A, const ListView &Lv,
     case 2:
         bforce_tt<D, KIND, PREC, SINGLE, HARM, STAGE, 2>(energy, A, Lv, P, c, eatom, s);
         break;
+    case 32:
+        bforce_tt<D, KIND, PREC, SINGLE, HARM, STAGE, 32>(energy, A, Lv, P, c, eatom, s);
+        break;
+    case 16:
+        bforce_tt<D, KIND, PREC, SINGLE, HARM, STAGE, 16>(energy, A, Lv, P, c, eatom, s);
+        break;
     case 8:
         bforce_tt<D, KIND, PREC, SINGLE, HARM, STAGE, 8>(energy, A, Lv, P, c, eatom, s);
         break;

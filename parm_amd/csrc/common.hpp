@@ -95,40 +95,48 @@ __device__ __forceinline__ double sqnorm(const Vec<D> &r) {
 // if |fma(-n, L, dx)| < L/2, n = n*.  Otherwise n* is the one of n-1, n,
 // n+1 whose result is below L/2, or, on an exact tie (two results of
 // magnitude L/2), the even one.
+__device__ __forceinline__ double min_image_near(double dx, double n, double L, double halfL) {
+    double best = fma(-n, L, dx);
+    bool found = false;
+    for (int d = -1; d <= 1; d++) {
+        const double m = n + (double)d;
+        const double rm = fma(-m, L, dx);
+        const double am = fabs(rm);
+        if (am < halfL) {
+            best = rm;
+            found = true;
+        } else if (!found && am == halfL && rint(m * 0.5) == m * 0.5) {
+            best = rm;
+        }
+    }
+    return best;
+}
+
 __device__ __forceinline__ double min_image1(double dx, double L, double invL,
                                              double halfL) {
     const double n = rint(dx * invL);
     double r = fma(-n, L, dx);
-    if (__builtin_expect(!(fabs(r) < halfL), 0)) {
-        double best = r, bestn = n;
-        bool found = false;
-        for (int d = -1; d <= 1; d++) {
-            const double m = n + (double)d;
-            const double rm = fma(-m, L, dx);
-            const double am = fabs(rm);
-            if (am < halfL) {
-                best = rm;
-                bestn = m;
-                found = true;
-            } else if (!found && am == halfL && rint(m * 0.5) == m * 0.5) {
-                best = rm;
-                bestn = m;
-            }
-        }
-        (void)bestn;
-        r = best;
-    }
+    if (__builtin_expect(!(fabs(r) < halfL), 0)) r = min_image_near(dx, n, L, halfL);
     return r;
 }
 
 template <int D>
 __device__ __forceinline__ Vec<D> diff(const Vec<D> &a, const Vec<D> &b,
                                        const Box &box) {
+    // (min_image1 of each component, with one branch for all of them)
     Vec<D> r;
+    bool near = true;
 #pragma unroll
-    for (int k = 0; k < D; k++)
-        r.c[k] = min_image1(a.c[k] - b.c[k], box.L[k], box.invL[k],
-                            box.halfL[k]);
+    for (int k = 0; k < D; k++) {
+        const double dx = a.c[k] - b.c[k];
+        r.c[k] = fma(-rint(dx * box.invL[k]), box.L[k], dx);
+        near &= fabs(r.c[k]) < box.halfL[k];
+    }
+    if (__builtin_expect(!near, 0)) {
+#pragma unroll
+        for (int k = 0; k < D; k++)
+            r.c[k] = min_image1(a.c[k] - b.c[k], box.L[k], box.invL[k], box.halfL[k]);
+    }
     return r;
 }
 

@@ -287,7 +287,18 @@ hipError_t launch_upload(int ndim, int what, const AtomArrays &A, const int32_t 
 hipError_t launch_download(int ndim, int what, const AtomArrays &A,
                            const int32_t *orig, double *dst, hipStream_t s);
 int reduce_blocks(int n);
+// Most lanes per atom of an untiled force launch over n atoms, of which the
+// autotuner takes as many as pay: up to 2^18 lanes make at most four wavefronts
+// per SIMD, which a launch of few atoms otherwise leaves empty while each lane
+// walks its chain of list words, gathers and pair forces.  1000 LJ atoms, 200
+// steps with 8 / 16 / 32 lanes: 2.13 / 1.69 / 1.47 ms; 10,007 (mixed), 100 steps
+// with 8 / 16: 1.48 / 1.27 ms.
+constexpr int kWideLanes = 1 << 18;
+constexpr int max_lanes(int n) {
+    return n <= kWideLanes / 32 ? 32 : (n <= kWideLanes / 16 ? 16 : 8);
+}
 int force_blocks(int n, int tpa);  // workgroups of a force launch (also partials)
+inline int part_blocks(int n) { return force_blocks(n > 1 ? n : 1, max_lanes(n)); }
 int force_partials(int n, const ListView &Lv);  // partials of a launch over this list
 
 // ---------------------------------------------------------------- batch.hip

@@ -71,6 +71,16 @@ template <int D, bool ENERGY>
 __device__ __forceinline__ void lj64(const PairParam &pp, const Vec<D> &r,
                                      double (&f)[D], PairAcc &acc) {
     const double d2 = sqnorm<D>(r);
+    if (!ENERGY) {
+        // (most entries of a list are in range, so hardly a wavefront skips
+        // an entry: the force of one out of range is computed as 0)
+        bool in = d2 < pp.lim_lo;
+        if (__builtin_expect(!in && !(d2 > pp.lim_hi), 0)) in = !(d2 / pp.sig2 > pp.cut2);
+        const double fs = lj64_force(pp.sig2, pp.p6, far_unless(in, d2));
+#pragma unroll
+        for (int k = 0; k < D; k++) f[k] = fma(fs, r.c[k], f[k]);
+        return;
+    }
     bool in = d2 < pp.lim_lo ||
               (!(d2 > pp.lim_hi) && !(d2 / pp.sig2 > pp.cut2));
     if (!in) return;

@@ -167,6 +167,52 @@ def test_tiled_lj_group_edges(monkeypatch, tpa, ntypes, n):
     s.close()
 
 
+# 16 and 32 lanes per atom: rows shorter than the lanes, rows of more than the
+# entries in flight per lane, both pair kinds, the largest system of either
+@pytest.mark.parametrize("lanes,n", [(16, 2), (16, 700), (16, 1 << 14), (32, 2), (32, 700),
+                                     (32, 1 << 13)])
+@pytest.mark.parametrize("lj", [True, False])
+def test_wide_untiled_lanes(monkeypatch, lanes, n, lj):
+    _device_or_fail()
+    print(f"wide lanes={lanes} n={n} lj={lj}", flush=True)
+    monkeypatch.setenv("PARM_TPA", str(lanes))
+    monkeypatch.setenv("PARM_TILED", "0")
+    x, L = S.jittered_lattice(n, 0.8, 3, seed=n) if n > 2 else (np.array([[0.1, 0, 0], [1.2, 0, 0]]),
+                                                               np.full(3, 6.0))
+    v = S.gaussian_velocities(n, 3, 0.5, seed=n)
+    s = capi.System(3, np.ones(n))
+    s.set_box(L)
+    if lj:
+        p = S.lj_params(n, sigcut=3.2 if n == 700 else 2.5)
+        t = O.PairTable(O.LJ_ATTRACT_REPULSE, p["eps"], p["sigma"], p["third"], p["types"])
+        s.nlist_set(0.3, p["diam"])
+        s.set_lj(p["eps"], p["sigma"], p["third"], p["types"])
+    else:
+        p = S.bidisperse_repulsion(n, n)
+        t = O.PairTable(O.REPULSION, p["eps"], p["sigma"], p["third"], p["types"])
+        s.nlist_set(0.3, p["diam"])
+        s.set_repulsion(p["eps"], p["sigma"], p["third"], p["types"])
+    s.set_state(x=x, v=v, a=np.zeros_like(x))
+    s.update_list(True)
+    s.set_forces(False)
+    assert s.list_info()["lanes"] == lanes
+    first, last = O.nlist(x, L, p["diam"], 0.3)
+    ref = O.forces(x, L, t, first, last)
+    S.assert_fp64_forces(s.forces(), ref, x, L, t, first, last)
+    fd, ld = s.pairs()
+    assert np.array_equal(fd, first) and np.array_equal(ld, last)
+    assert abs(s.pair_sums()["U"] - ref["U"]) <= 1e-12 * max(1.0, abs(ref["U"]))
+    r = O.System(np.ones(n), L, t, p["diam"], 0.3, ndim=3, brute=n < 1000)
+    r.set_state(x=x, v=v, a=np.zeros_like(x))
+    for q in (r, s):
+        q.initialize()
+        q.verlet(0.001, 5)
+    assert s.which() == r.which()
+    xr, xd = r.state()[0], s.state()[0]
+    assert np.abs(xd - xr).max() <= 1e-12 * max(1.0, np.abs(xr).max())
+    s.close()
+
+
 # the counted order and the tile plan: one and several scan tiles of cells,
 # several rows to a plan workgroup, crowded cells, empty rows, and a rebuild on
 # top of the order of the one before
