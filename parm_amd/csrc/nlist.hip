@@ -342,6 +342,65 @@ __global__ __launch_bounds__(kScanThreads) void k_cell_scan(int ncell, int n,
     if (blockIdx.x == 0 && threadIdx.x == 0) cstart[ncell] = n;
 }
 
+// The count, the scan and the scatter of a small system in one workgroup, its
+// counters in LDS and its atoms' cells in registers: each of the three launches
+// takes 2 to 3 us, mostly its start and end.  2,003 disks, 200 steps with 26
+// rebuilds: 2925 -> 2790 us; a minimiser's 4,001 spheres 1570 -> 1530 us.
+constexpr int kSmallThreads = 1024, kSmallPer = 8;
+constexpr int kSmallAtoms = kSmallThreads * kSmallPer;
+constexpr int kSmallCells = 8192;
+
+template <int D>
+__global__ __launch_bounds__(kSmallThreads) void k_cell_order_small(
+    int n, const typename PosStore<D>::T *__restrict__ pos, CellGrid g, Box box,
+    uint32_t *__restrict__ key, int32_t *__restrict__ cstart, int32_t *__restrict__ slot,
+    int *__restrict__ info) {
+    constexpr int kPer = kSmallCells / kSmallThreads;
+    __shared__ uint32_t count[kSmallCells];
+    const int t = threadIdx.x;
+    if (t < 3) info[t] = 0;  // the tile plan's totals (k_tile_plan)
+    typename PosStore<D>::T x[kSmallPer];
+    uint32_t c[kSmallPer], at[kSmallPer];
+#pragma unroll
+    for (int q = 0; q < kSmallPer; q++)
+        if (t + q * kSmallThreads < n) x[q] = pos[t + q * kSmallThreads];
+#pragma unroll
+    for (int q = 0; q < kPer; q++) count[t + q * kSmallThreads] = 0u;
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < kSmallPer; q++) {
+        const int i = t + q * kSmallThreads;
+        c[q] = at[q] = 0u;
+        if (i < n) {
+            Vec<D> w;
+            c[q] = cell_of<D>(PosStore<D>::load(x[q]), g, box, w);
+            key[i] = c[q];
+            at[q] = atomicAdd(&count[c[q]], 1u);
+        }
+    }
+    __syncthreads();
+    uint32_t v[kPer], sum = 0, all = 0;
+#pragma unroll
+    for (int q = 0; q < kPer; q++) {
+        v[q] = count[t * kPer + q];
+        sum += v[q];
+    }
+    uint32_t run = block_excl_scan_u32<kSmallThreads>(sum, all);
+#pragma unroll
+    for (int q = 0; q < kPer; q++) {
+        if (t * kPer + q < g.ncell) cstart[t * kPer + q] = (int32_t)run;
+        count[t * kPer + q] = run;
+        run += v[q];
+    }
+    if (t == 0) cstart[g.ncell] = n;
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < kSmallPer; q++) {
+        const int i = t + q * kSmallThreads;
+        if (i < n) slot[count[c[q]] + at[q]] = i;
+    }
+}
+
 // Thread p takes the atom i at place p of its cell's arrival order to its
 // place in the stable order: the cell's start plus the number of the cell's
 // atoms from smaller old slots (a cell's atoms are few, and the list build
@@ -1184,12 +1243,11 @@ __global__ __launch_bounds__(kWave *G) void k_build_tiled(
                 scan(std::true_type{});
             else
                 scan(std::false_type{});
+            const int cc = cnt < cap ? cnt : cap;
+            for (int l = sub; l < tpa; l += G)
+                lcount[(size_t)i * tpa + l] = (uint16_t)(cc > l ? (cc - l + tpa - 1) >> ts : 0);
             if (sub == 0) {
-                const int cc = cnt < cap ? cnt : cap;
                 ncount[i] = cc;
-                for (int l = 0; l < tpa; l++)
-                    lcount[(size_t)i * tpa + l] =
-                        (uint16_t)(cc > l ? (cc - l + tpa - 1) / tpa : 0);
                 if (cnt > cap) atomicOr(flag, kFlagOverflow);
                 mysum = (unsigned long long)cnt;
                 myreq = (unsigned long long)cnt;
@@ -1336,6 +1394,15 @@ hipError_t launch_cell_order(int ndim, int n, const void *pos, const CellGrid &g
                              const Box &box, uint32_t *ukeys, int32_t *arrival,
                              uint32_t *count, uint32_t *total, int32_t *cstart, int32_t *slot,
                              int *info, hipStream_t s) {
+    if (n <= kSmallAtoms && g.ncell <= kSmallCells) {
+        if (ndim == 3)
+            hipLaunchKernelGGL(k_cell_order_small<3>, dim3(1), dim3(kSmallThreads), 0, s, n,
+                               (const double4 *)pos, g, box, ukeys, cstart, slot, info);
+        else
+            hipLaunchKernelGGL(k_cell_order_small<2>, dim3(1), dim3(kSmallThreads), 0, s, n,
+                               (const double2 *)pos, g, box, ukeys, cstart, slot, info);
+        return hipGetLastError();
+    }
     if (ndim == 3)
         hipLaunchKernelGGL(k_cell_count<3>, dim3(nblk(n)), dim3(kBlock), 0, s, n,
                            (const double4 *)pos, g, box, ukeys, arrival, count, info);
@@ -1503,6 +1570,12 @@ constexpr int kTiledLanes = 4;   // lanes per atom in k_build_tiled
 // 1M atoms); a sparse one (packed discs / spheres: ~7-9 atoms) one round of
 // 4 x 2
 constexpr int kTiledUnroll = 16, kTiledUnrollSparse = 2;
+// A dense system of few tiles (at most one workgroup for each of the 256 CUs at
+// kTiledWideAtoms) takes 16 lanes of two candidates: 10,007 atoms (mixed), 100
+// steps with their rebuilds 1375 -> 1310 us.  (A sparse one does not gain: 20,011
+// spheres 3250 us, 3810 us with 16 x 1.)
+constexpr int kTiledLanesWide = 16, kTiledUnrollWide = 2;
+constexpr int kTiledWideAtoms = 1 << 14;
 
 size_t tiled_build_lds(int smax) {
     return (size_t)(smax + kBuildPad) * sizeof(float4) + (size_t)smax * sizeof(uint32_t);
@@ -1529,17 +1602,19 @@ hipError_t launch_build_tiled(int ndim, int n, int ntiles, int smax, const TileR
     const size_t esize = out32 ? 4 : 2;
     const size_t row = out32 ? ((size_t)npad << ts) : ((size_t)npad << (ts + 1));
     const int off24 = (size_t)cap * (size_t)npad * esize <= 0xffffffffull && row < (1u << 24);
-#define PARM_BT(DD, PT, O32, UU, UNR)                                                        \
-    hipLaunchKernelGGL((k_build_tiled<DD, kTiledLanes, UNR, O32, UU>), dim3(ntiles),          \
-                       dim3(kWave * kTiledLanes), lds, s, tiles, truns, smax, (const PT *)pos, \
+#define PARM_BT(DD, PT, O32, UU, GG, UNR)                                                    \
+    hipLaunchKernelGGL((k_build_tiled<DD, GG, UNR, O32, UU>), dim3(ntiles),                   \
+                       dim3(kWave * GG), lds, s, tiles, truns, smax, (const PT *)pos, \
                        (const PT *)xw, rank, diam, type, type_bits, keys, cstart, g, box,     \
                        skin, dmax, tpa, cap, npad, off24, nbr, ncount, lcount, (PT *)xref,    \
                        part, flag, spec, ex)
 #define PARM_BT_S(DD, PT, O32, UU)                       \
-    if (sparse) {                                       \
-        PARM_BT(DD, PT, O32, UU, kTiledUnrollSparse);   \
-    } else {                                            \
-        PARM_BT(DD, PT, O32, UU, kTiledUnroll);         \
+    if (sparse) {                                                    \
+        PARM_BT(DD, PT, O32, UU, kTiledLanes, kTiledUnrollSparse);   \
+    } else if (n <= kTiledWideAtoms) {                               \
+        PARM_BT(DD, PT, O32, UU, kTiledLanesWide, kTiledUnrollWide); \
+    } else {                                                         \
+        PARM_BT(DD, PT, O32, UU, kTiledLanes, kTiledUnroll);         \
     }
 #define PARM_BT_U(DD, PT, O32)        \
     if (uni) {                       \
