@@ -932,6 +932,12 @@ __global__ __launch_bounds__(kWave *G) void k_build_tiled(
     Slot *st_f = reinterpret_cast<Slot *>(st_raw);
     uint32_t *st_e = reinterpret_cast<uint32_t *>(st_f + smax + kBuildPad);  // OUT32 entries
     static_assert(G * U <= kBuildPad, "a round stays inside the padded stage");
+    // Candidate u of lane `sub` in a round is the slot first + cand(u).  Two
+    // lanes of four take theirs so that the passes come in the order in which
+    // four lanes of two leave them: an atom's list, and with it the order of its
+    // force's sum, is the same from either.
+    constexpr bool kAs4x2 = G == 2 && U == 4;
+    auto cand = [](int u) { return kAs4x2 ? (u >> 1) + 4 * (u & 1) : u * G; };
     static_assert(U <= 32, "a round's candidates are the bits of one word");
     constexpr int kBatch = U < 4 ? U : 4;  // slots read and tested together
     static_assert(U % kBatch == 0, "a round is whole batches");
@@ -1098,13 +1104,20 @@ __global__ __launch_bounds__(kWave *G) void k_build_tiled(
                     for (int h = 0; h < nh; h++) {
                         const int lo = h ? lo1 : lo0, hi = h ? hi1 : hi0;
                         for (int base = lo; base < hi; base += G * U) {
-                            // candidate u of this lane is slot base + u G + sub;
-                            // `valid`: the ones below hi that are not the atom
-                            // itself (one mask per round, not a test per slot)
-                            const int first = base + sub;
-                            const int nv = min(U, max(0, (hi - first + G - 1) / G));
-                            uint32_t valid = nv >= 32 ? ~0u : ((1u << nv) - 1u);
-                            {
+                            // `valid`: the candidates below hi that are not
+                            // the atom itself (one mask per round, not a test
+                            // per slot)
+                            const int first = base + (kAs4x2 ? 2 * sub : sub);
+                            uint32_t valid = 0u;
+                            if constexpr (kAs4x2) {
+#pragma unroll
+                                for (int u = 0; u < U; u++) {
+                                    const int s = first + cand(u);
+                                    valid |= s < hi && s != self ? 1u << u : 0u;
+                                }
+                            } else {
+                                const int nv = min(U, max(0, (hi - first + G - 1) / G));
+                                valid = nv >= 32 ? ~0u : ((1u << nv) - 1u);
                                 const int ds = self - first;
                                 if (ds >= 0 && (ds % G) == 0 && ds / G < U)
                                     valid &= ~(1u << (ds / G));
@@ -1128,7 +1141,7 @@ __global__ __launch_bounds__(kWave *G) void k_build_tiled(
                                 Slot pw[kBatch];
 #pragma unroll
                                 for (int u = 0; u < kBatch; u++)
-                                    pw[u] = st_f[first + (b * kBatch + u) * G];
+                                    pw[u] = st_f[first + cand(b * kBatch + u)];
 #pragma unroll
                                 for (int u = kBatch - 1; u >= 0; u--) {
                                     float d2 = 0.0f;
@@ -1161,7 +1174,7 @@ __global__ __launch_bounds__(kWave *G) void k_build_tiled(
                                 while (ubits) {
                                     const int u = __builtin_ctz(ubits);
                                     ubits &= ubits - 1u;
-                                    const int s = first + u * G;
+                                    const int s = first + cand(u);
                                     const int cj = slot_cell(L, s);
                                     const int j = L.g0[cj] + (s - L.off[cj]);
                                     if (in_list<D>(xi, PosStore<D>::load(pos[j]), di, diam[j], box,
@@ -1175,7 +1188,7 @@ __global__ __launch_bounds__(kWave *G) void k_build_tiled(
                                 while (b) {
                                     const int u = __builtin_ctz(b);
                                     b &= b - 1u;
-                                    const int s = first + u * G;
+                                    const int s = first + cand(u);
                                     const int cj = slot_cell(L, s);
                                     const int j = L.g0[cj] + (s - L.off[cj]);
                                     if (excluded(ex, oi, ex.orig[j])) pbits &= ~(1u << u);
@@ -1208,7 +1221,7 @@ __global__ __launch_bounds__(kWave *G) void k_build_tiled(
                                 const int u = __builtin_ctz(bits);
                                 bits &= bits - 1u;
                                 {
-                                    const int s = first + u * G;
+                                    const int s = first + cand(u);
                                     if (off24) {
                                         const uint32_t qq = (uint32_t)q;
                                         uint32_t e;
@@ -1570,6 +1583,13 @@ constexpr int kTiledLanes = 4;   // lanes per atom in k_build_tiled
 // 1M atoms); a sparse one (packed discs / spheres: ~7-9 atoms) one round of
 // 4 x 2
 constexpr int kTiledUnroll = 16, kTiledUnrollSparse = 2;
+// A sparse 2D system of many atoms is bound by the instructions each wavefront
+// spends beside its candidates (870 vector instructions for 16 atoms), so its
+// wavefronts take 32 atoms, two lanes of four candidates each: 120,000 /
+// 262,144 / 500,000 disks, 200 steps 4.33 / 5.93 / 10.28 -> 4.25 / 5.65 / 9.57 ms; 60,000
+// and below lose 4 % (too few wavefronts), and so do spheres (nine rows: 300,000,
+// 150 steps 10.68 -> 10.95 ms).
+constexpr int kTiledLanesFlat = 2, kTiledUnrollFlat = 4, kTiledFlatAtoms = 100000;
 // A dense system of few tiles (at most one workgroup for each of the 256 CUs at
 // kTiledWideAtoms) takes 16 lanes of two candidates: 10,007 atoms (mixed), 100
 // steps with their rebuilds 1375 -> 1310 us.  (A sparse one does not gain: 20,011
@@ -1609,7 +1629,9 @@ hipError_t launch_build_tiled(int ndim, int n, int ntiles, int smax, const TileR
                        skin, dmax, tpa, cap, npad, off24, nbr, ncount, lcount, (PT *)xref,    \
                        part, flag, spec, ex)
 #define PARM_BT_S(DD, PT, O32, UU)                       \
-    if (sparse) {                                                    \
+    if (DD == 2 && sparse && n >= kTiledFlatAtoms) {                 \
+        PARM_BT(DD, PT, O32, UU, kTiledLanesFlat, kTiledUnrollFlat); \
+    } else if (sparse) {                                             \
         PARM_BT(DD, PT, O32, UU, kTiledLanes, kTiledUnrollSparse);   \
     } else if (n <= kTiledWideAtoms) {                               \
         PARM_BT(DD, PT, O32, UU, kTiledLanesWide, kTiledUnrollWide); \

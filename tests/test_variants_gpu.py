@@ -215,12 +215,14 @@ def test_wide_untiled_lanes(monkeypatch, lanes, n, lj):
 
 # the counted order and the tile plan: one workgroup (up to 8192 atoms and cells)
 # and several launches, one and several scan tiles of cells,
-# several rows to a plan workgroup, crowded cells, empty rows, and a rebuild on
+# several rows to a plan workgroup, crowded cells, empty rows, the build lanes of a
+# large 2D system, and a rebuild on
 # top of the order of the one before
 @pytest.mark.parametrize("n,ndim,edge,clustered", [
     (1, 3, 9.0, False), (2, 2, 9.0, False), (63, 3, 4.0, False), (65, 2, 12.0, True),
     (1500, 3, 40.0, False), (1500, 3, 40.0, True), (3000, 2, 150.0, False),
-    (8192, 2, 60.0, False), (8192, 3, 20.0, False), (8193, 3, 20.0, False), (70000, 3, 84.0, False)])
+    (8192, 2, 60.0, False), (8192, 3, 20.0, False), (8193, 3, 20.0, False), (70000, 3, 84.0, False),
+    (99999, 2, 400.0, False), (100000, 2, 400.0, False)])
 def test_counted_order_and_tile_plan(n, ndim, edge, clustered):
     _device_or_fail()
     print(f"counted order n={n} ndim={ndim} edge={edge} clustered={clustered}", flush=True)
