@@ -64,7 +64,7 @@ HBM_PEAK_GBS = 8000.0
 # WRITE_SIZE by 1.0, the factors that make the same counters read 1 GiB for a
 # 1 GiB device copy (profiles/k_force_lj_1M_pmc.txt).
 TRAFFIC_BYTES_PER_ATOM = {  # (tiled list, lanes per atom) -> bytes per atom
-    (True, 1): 401.6, (True, 2): 401.0, (True, 4): 404.5, (True, 8): 416.0,
+    (True, 1): 389.7, (True, 2): 391.7, (True, 4): 398.1, (True, 8): 403.7,
     (False, 1): 559.3, (False, 2): 546.2, (False, 4): 563.3, (False, 8): 571.9,
 }
 

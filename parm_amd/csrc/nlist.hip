@@ -4,15 +4,16 @@
 // The reference rebuild is an O(N^2) double loop over members testing
 //   |diff(x_i, x_j)| < (d_i + d_j)/2 + skin.
 // Here the same predicate, evaluated bit-identically, runs over a periodic
-// cell grid (cell edge >= the largest list radius) after a stable LSD radix
-// sort of the atoms by cell.  The sort also renumbers the device slots, so
-// atoms that are close in space are close in memory for the force gathers.
+// cell grid (cell edge >= the largest list radius) after a stable ordering of
+// the atoms by cell.  The order also renumbers the device slots, so atoms that
+// are close in space are close in memory for the force gathers.
 //
 // Pipeline (one rebuild), every atom a list member:
 //   k_cell_count     cell of each atom, counted; the atom's arrival number
 //   k_cell_scan      counts -> first slot of each cell (two launches when
 //                    there are many cells)
 //   k_cell_scatter   the atoms of each cell, in arrival order
+//   (k_cell_order_small: these three in one launch for few atoms and cells)
 //   k_cell_permute   every per-slot array into the new order (each atom's place
 //                    in its cell from the number of the cell's atoms with a
 //                    smaller old slot: the stable order), the wrapped copies

@@ -227,9 +227,11 @@ __global__ __launch_bounds__(kFinThreads) void k_finalize_skin(int nparts, Reduc
     }
 }
 
-// below this many partials the one-workgroup k_finalize is the quicker (the
-// counter's fences and the second merge cost more than they save: +6 % per
-// step at 1000 atoms, +4 % at 32,768; -1.6 % at 1M atoms, 16,384 partials)
+// For skin tests on demand (the step loop reduces its own inside the next step
+// launch).  Below this many partials the one-workgroup k_finalize is the
+// quicker (the counter's fences and the second merge cost more than they save:
+// measured after every step, +6 % per step at 1000 atoms, +4 % at 32,768; -1.6 %
+// at 1M atoms, 16,384 partials)
 constexpr int kFinMultiMin = 8 * kFinal;
 
 static void launch_finalize(int nparts, const ReduceBuf &R, hipStream_t s) {

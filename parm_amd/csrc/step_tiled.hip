@@ -1,5 +1,5 @@
 // step_tiled.hip -- pair forces over the tiled list (tiles.hpp), fused with
-// the integrator stages exactly as k_force in step.hip.
+// the integrator stages exactly as k_force in force.hip.
 //
 // Reference behaviour restated (paths relative to the reference root):
 //   NListed<A,P>::set_forces / energy / pressure / stress

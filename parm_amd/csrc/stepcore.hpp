@@ -1,4 +1,4 @@
-// stepcore.hpp -- pieces shared by the force kernels of step.hip (untiled
+// stepcore.hpp -- pieces shared by the force kernels of force.hip (untiled
 // list) and step_tiled.hip (tiled list): per-workgroup reduction partials,
 // the skin test of one atom, and the per-atom epilogue that applies the
 // integrator stage fused into a force launch.
