@@ -56,7 +56,7 @@ __device__ __forceinline__ int xcd_block(int b, int nb) {
     return (x < r) ? x * (q + 1) + k : r * (q + 1) + (x - r) * q + k;
 }
 
-// log2 of the lanes per atom (a power of two: 1, 2, 4 or 8), so that list
+// log2 of the lanes per atom (a power of two), so that list
 // entry positions take shifts and masks instead of integer divisions.
 __device__ __forceinline__ int tpa_shift(int tpa) { return 31 - __clz(tpa); }
 
