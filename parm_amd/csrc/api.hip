@@ -80,7 +80,7 @@ void dfree(T *&p) {
 
 constexpr int kFlagRing = 4;
 // flag words: [0, kFlagRing) the step loop's skin tests (by step number), then the list-build overflow flag, a
-// scratch word for reductions that raise no flag, and the on-demand skin test
+// scratch word for reductions that raise no flag, the on-demand skin test, and the verdict on a list build
 // dynamic LDS of one tiled build workgroup, at most (the stencil's atoms)
 constexpr size_t kTiledLdsMax = 56 * 1024;
 constexpr int kMixedUntiledAtoms = 1 << 15, kMixedRepulsionFixed = 100000;  // autotune
@@ -88,7 +88,7 @@ constexpr int kMixedUntiledAtoms = 1 << 15, kMixedRepulsionFixed = 100000;  // a
 constexpr int kRunAhead = 2, kRunAheadAtoms = 1 << 15;
 static_assert(kRunAhead + 1 < kFlagRing, "a flag word is not reused while a launch may read it");
 constexpr int kSlotBuild = kFlagRing + 1, kSlotScratch = kFlagRing + 2,
-              kSlotSkin = kFlagRing + 3;
+              kSlotSkin = kFlagRing + 3, kSlotVerdict = kFlagRing + 4;
 
 struct parm_system {
     int device = 0;
@@ -132,6 +132,9 @@ struct parm_system {
     uint16_t *lcount = nullptr;   // per-lane entry counts, npad x max_lanes(n)
     // tiled layout (tiles.hpp): the current list is tiled when `tiled`
     bool tiled = false, tile_ok = false;
+    // a build whose report has not been read (settle_build), and whether the
+    // ordering left the wrapped positions
+    bool build_due = false, build_wrapped = false;
     int layout_pref = 0;  // 0: tiled when possible, until tuned; 1: tiled; 2: untiled
     int4 *tiles = nullptr;
     int2 *truns = nullptr;
@@ -472,7 +475,7 @@ int build_list(parm_system *s, const void *at, bool wrapped) {
                                     s->cap, s->npad, !s->tiled, s->nbr, s->ncount, s->lcount,
                                     s->xref, s->bpart, s->stats, s->dflag + kSlotBuild,
                                     nullptr, s->dmin == s->dmax, s->exview(), wrapped,
-                                    s->hrep_dev, ++s->build_seq, st));
+                                    s->hrep_dev, ++s->build_seq, nullptr, st));
     } else {
         PARM_HIP(launch_build_list(s->ndim, s->n, at, s->xwrap, s->rank, s->diam, s->type,
                                    s->keys, s->cstart, s->grid, s->box, s->skin, s->dmax,
@@ -528,6 +531,7 @@ int read_report(parm_system *s, BuildReport *r) {
     r->smax = h->smax;
     r->bad = h->bad;
     r->flag = h->flag;
+    r->ok = h->ok;
     return PARM_OK;
 }
 
@@ -552,13 +556,38 @@ int build_checked(parm_system *s, const void *at, bool wrapped = false) {
     return fail(PARM_E_DEVICE, "neighbour list build did not converge");
 }
 
+// Reads the report of the build that build_speculative queued; builds again if
+// it does not stand.
+int settle_build(parm_system *s, bool *stands) {
+    const bool tiled = s->tiled;
+    s->build_due = false;
+    BuildReport r{};
+    PARM_CHECK(read_report(s, &r));
+    accept_tiles(s, r.ntiles, r.smax, r.bad);
+    s->spec_smax = s->tile_ok ? s->smax : 0;
+    const bool fits = s->tile_ok && s->tiled == tiled && !(r.flag & kFlagReplan);
+    *stands = r.ok && fits;
+    if (*stands) {
+        s->npairs = (int64_t)(r.sum / 2);
+        return PARM_OK;
+    }
+    if (fits && r.max > (unsigned long long)s->cap)
+        PARM_CHECK(ensure_list_capacity(s, (int)(r.max + r.max / 8 + 8)));
+    return build_checked(s, s->pos, s->build_wrapped);
+}
+
 // Rebuild-time list build with one host round trip: the tiled build is
 // queued behind the tile plan before the host has read it, with the
 // previous plan's largest stencil (plus a margin) as its LDS bound and the
 // tile capacity as its grid.  The report then carries the plan: when the
 // plan fits the bounds (and the list its capacity) the build stands;
 // otherwise the plan is accepted as read and the list built again.
-int build_speculative(parm_system *s, bool wrapped) {
+//
+// defer (inside a step loop on a system settled on the untiled list, whose
+// launches do not depend on the plan): the report is left for settle_build, and
+// the caller queues its next launch behind the device's own verdict instead of
+// idling while the host reads the report and answers.  DEFER_MEASURED
+int build_speculative(parm_system *s, bool wrapped, bool defer) {
     PARM_CHECK(check_lane_counts(s));
     const int pstride = force_blocks(std::max(s->n, 1), 8);
     const int grid = std::min(s->tiles_cap, pstride);
@@ -575,19 +604,13 @@ int build_speculative(parm_system *s, bool wrapped) {
                                 s->box, s->skin, s->dmax, s->tpa, s->cap, s->npad, !tiled,
                                 s->nbr, s->ncount, s->lcount, s->xref, s->bpart, s->stats,
                                 s->dflag + kSlotBuild, s->tinfo, s->dmin == s->dmax,
-                                s->exview(), wrapped, s->hrep_dev, ++s->build_seq, s->stream));
-    BuildReport r{};
-    PARM_CHECK(read_report(s, &r));
-    accept_tiles(s, r.ntiles, r.smax, r.bad);
-    s->spec_smax = s->tile_ok ? s->smax : 0;
-    const bool fits = s->tile_ok && s->tiled == tiled && r.ntiles <= grid &&
-                      !(r.flag & kFlagReplan);
-    if (fits && r.max <= (unsigned long long)s->cap) {
-        s->npairs = (int64_t)(r.sum / 2);
-        return PARM_OK;
-    }
-    if (fits) PARM_CHECK(ensure_list_capacity(s, (int)(r.max + r.max / 8 + 8)));
-    return build_checked(s, s->pos, wrapped);
+                                s->exview(), wrapped, s->hrep_dev, ++s->build_seq,
+                                defer ? s->dflag + kSlotVerdict : nullptr, s->stream));
+    s->build_due = true;
+    s->build_wrapped = wrapped;
+    if (defer) return PARM_OK;
+    bool stands = false;
+    return settle_build(s, &stands);
 }
 
 // The exclusion CSR of s->excl on the device: for every atom (original
@@ -636,7 +659,9 @@ int upload_exclusions(parm_system *s) {
 // lastlocs = x, then the full pair list from the predicate.
 // skin (inside a step loop): where the skin test of pos_alt against the new
 // reference positions leaves its partials.
-int rebuild(parm_system *s, bool keep_af = true, const ReduceBuf *skin = nullptr) {
+// defer: the list build's report may be left due (build_due, settle_build).
+int rebuild(parm_system *s, bool keep_af = true, const ReduceBuf *skin = nullptr,
+            bool defer = false) {
     if (!s->list_cfg) return fail(PARM_E_STATE, "neighbour list not configured");
     PARM_CHECK(upload_exclusions(s));
     hipStream_t st = s->stream;
@@ -654,6 +679,7 @@ int rebuild(parm_system *s, bool keep_af = true, const ReduceBuf *skin = nullptr
     }
     // from here on the previous list no longer matches the atom order
     s->built = false;
+    s->build_due = false;
     const bool counted = n > 0 && s->nmem == n;
     if (counted) {
         if (!s->ccount_clear)
@@ -677,7 +703,8 @@ int rebuild(parm_system *s, bool keep_af = true, const ReduceBuf *skin = nullptr
     if (s->cap == 0) PARM_CHECK(ensure_list_capacity(s, initial_capacity(s)));
     PARM_CHECK(launch_tile_plan(s));
     if (n > 0 && s->spec_smax > 0) {
-        PARM_CHECK(build_speculative(s, counted));
+        PARM_CHECK(build_speculative(s, counted,
+                                     defer && counted && s->layout_pref == 2 && !s->tiled));
     } else {
         PARM_CHECK(plan_tiles(s));
         PARM_CHECK(build_checked(s, s->pos, counted));
@@ -938,9 +965,16 @@ int run_steps(parm_system *s, bool damped, const StepCoef &c, int64_t nsteps) {
     const int ahead = step_runahead(s);
     int64_t queued = 0;
     bool gated = false;  // launch `queued` checks the flag before it
-    for (int64_t q = 0; q < nsteps; q++) {
-        // queue launches up to q + ahead (none past q while a forced rebuild
-        // is due at its end)
+    // the launches queued past q did nothing: queue them again
+    auto requeue = [&](int64_t q) {
+        s->prof_seq -= std::max<int64_t>(0, std::min(queued, nsteps - 1) - (q + 1));
+        s->prof_step.resize(nprof[q % kFlagRing]);
+        queued = q + 1;
+        gated = false;
+    };
+    // queue launches up to q + ahead (none past q while a forced rebuild is due
+    // at its end)
+    auto queue = [&](int64_t q) -> int {
         while (queued < nsteps && queued < q + ahead && !(s->ignorechanged && queued > q)) {
             const bool last = (queued == nsteps - 1);
             const int cur = (int)(queued & 1), slot = (int)(queued % kFlagRing);
@@ -951,7 +985,9 @@ int run_steps(parm_system *s, bool damped, const StepCoef &c, int64_t nsteps) {
             R.part = pbuf[1 - cur];
             R.g.prev = pbuf[cur];
             R.g.nprev = npart[cur];
-            R.g.gate = gated ? s->dflag + (queued + kFlagRing - 1) % kFlagRing : nullptr;
+            R.g.gate = gated          ? s->dflag + (queued + kFlagRing - 1) % kFlagRing
+                       : s->build_due ? s->dflag + kSlotVerdict
+                                      : nullptr;
             R.g.flag = s->dflag + slot;
             R.g.hflag = s->hflag_dev + slot;
             R.g.seq = seq[slot] = ++s->step_seq;
@@ -970,6 +1006,20 @@ int run_steps(parm_system *s, bool damped, const StepCoef &c, int64_t nsteps) {
             gated = true;
             queued++;
         }
+        return PARM_OK;
+    };
+    for (int64_t q = 0; q < nsteps; q++) {
+        PARM_CHECK(queue(q));
+        if (s->build_due) {
+            // (the launches behind a build that does not stand did nothing)
+            bool stands = false;
+            PARM_CHECK(settle_build(s, &stands));
+            if (!stands) {
+                requeue(q - 1);
+                npart[q & 1] = reduce_blocks(s->n);  // the permutation's
+                PARM_CHECK(queue(q));
+            }
+        }
         // update_trackers at the end of step q: skin test of x_{q+1}
         const bool last = (q == nsteps - 1);
         const int cur = (int)(q & 1), slot = (int)(q % kFlagRing);
@@ -981,18 +1031,14 @@ int run_steps(parm_system *s, bool damped, const StepCoef &c, int64_t nsteps) {
             return fail(PARM_E_NONFINITE,
                         "position became non-finite at step " + std::to_string(q));
         if ((fl & kFlagRebuild) || s->ignorechanged) {
-            // the launches queued past q did nothing: queue them again
-            s->prof_seq -= std::max<int64_t>(0, std::min(queued, nsteps - 1) - (q + 1));
-            s->prof_step.resize(nprof[slot]);
-            queued = q + 1;
-            gated = false;
+            requeue(q);
             {
                 ProfScope ps(s, &s->prof_rebuild);
                 // before the last step's end the next launch rewrites a and
                 // f before anything reads them: they need no permutation
                 ReduceBuf R = s->redbuf(kSlotScratch);
                 R.part = pbuf[1 - cur];
-                PARM_CHECK(rebuild(s, last, last ? nullptr : &R));
+                PARM_CHECK(rebuild(s, last, last ? nullptr : &R, !last));
             }
             xb[cur] = s->pos;
             xb[1 - cur] = s->pos_alt;

@@ -69,6 +69,7 @@ struct BuildReport {
     unsigned long long sum, max;
     int ntiles, smax, bad;
     uint32_t flag;
+    int ok;        // the verdict of a build that a step launch waits for
     uint32_t seq;  // the launch's number, stored last
 };
 
@@ -111,7 +112,10 @@ size_t tiled_build_lds(int smax);
 // spec == null: ntiles and smax are the plan's.  spec == the plan's info
 // (launch_tiles, not yet read by the host): ntiles and smax are bounds;
 // tiles past info[0] do nothing, and a tile with more than smax staged slots
-// (or none that fit) sets kFlagReplan instead of building.  uni: every list
+// (or none that fit) sets kFlagReplan instead of building.  verdict (may be
+// null): 0 when the speculative build stands (the plan fits its bounds, the list
+// its capacity), else kFlagStopped: the gate of a step launch queued behind it.
+// uni: every list
 // member has the same diameter.
 hipError_t launch_build_tiled(int ndim, int n, int ntiles, int smax, const int4 *tiles,
                               const int2 *truns, const void *pos, void *xw, const int32_t *rank,
@@ -122,7 +126,8 @@ hipError_t launch_build_tiled(int ndim, int n, int ntiles, int smax, const int4 
                               uint16_t *lcount, void *xref, unsigned long long *part,
                               unsigned long long *stats, uint32_t *flag, const int *spec,
                               int uni, const ExclView &ex, bool wrapped,
-                              BuildReport *report, uint32_t seq, hipStream_t s);
+                              BuildReport *report, uint32_t seq, uint32_t *verdict,
+                              hipStream_t s);
 hipError_t launch_tiled_to_global(int ndim, int ntiles, const int4 *tiles,
                                   const uint32_t *keys, const int32_t *cstart,
                                   const CellGrid &g, const uint16_t *nb16,

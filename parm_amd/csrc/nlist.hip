@@ -1339,7 +1339,7 @@ __global__ __launch_bounds__(kStatsThreads) void k_build_stats(
     int nparts, const unsigned long long *__restrict__ part,
     unsigned long long *__restrict__ stats, uint32_t *__restrict__ flag,
     const TileRec *__restrict__ tiles, const int *__restrict__ info, BuildReport *report,
-    uint32_t seq) {
+    uint32_t seq, int cap, uint32_t *__restrict__ verdict) {
     __shared__ unsigned long long red[kStatsThreads / kWave][2];
     int smax = 0, bad = 0;
     if (info) tile_extremes(tiles, info[0], smax, bad);
@@ -1371,7 +1371,12 @@ __global__ __launch_bounds__(kStatsThreads) void k_build_stats(
         stats[1] = m2;
         const uint32_t fl = *flag;
         *flag = 0;
+        const bool ok = info && info[0] > 0 && info[0] <= nparts && !(info[2] | bad) &&
+                        fl == 0u && m2 <= (unsigned long long)cap;
+        if (verdict) *verdict = ok ? 0u : (uint32_t)kFlagStopped;
         if (report) {
+            __hip_atomic_store(&report->ok, ok ? 1 : 0, __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_SYSTEM);
             __hip_atomic_store(&report->sum, s2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
             __hip_atomic_store(&report->max, m2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
             __hip_atomic_store(&report->flag, fl, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
@@ -1552,7 +1557,8 @@ hipError_t launch_build_list(int ndim, int n, const void *pos, void *xw,
                            nbr, ncount, lcount, (double2 *)xref, part, flag, ex);
     }
     hipLaunchKernelGGL(k_build_stats, dim3(1), dim3(kStatsThreads), 0, s, nb, part, stats,
-                       flag, (const TileRec *)nullptr, (const int *)nullptr, report, seq);
+                       flag, (const TileRec *)nullptr, (const int *)nullptr, report, seq, cap,
+                       (uint32_t *)nullptr);
     return hipGetLastError();
 }
 
@@ -1611,7 +1617,8 @@ hipError_t launch_build_tiled(int ndim, int n, int ntiles, int smax, const TileR
                               uint16_t *lcount, void *xref, unsigned long long *part,
                               unsigned long long *stats, uint32_t *flag, const int *spec,
                               int uni, const ExclView &ex, bool wrapped,
-                              BuildReport *report, uint32_t seq, hipStream_t s) {
+                              BuildReport *report, uint32_t seq, uint32_t *verdict,
+                              hipStream_t s) {
     if (n <= 0 || ntiles <= 0) return hipSuccess;
     const size_t slot = (size_t)(uni ? ndim : ndim + 1) * sizeof(float);
     const size_t lds = (size_t)(smax + kBuildPad) * slot +
@@ -1668,7 +1675,7 @@ hipError_t launch_build_tiled(int ndim, int n, int ntiles, int smax, const TileR
 #undef PARM_BT_S
 #undef PARM_BT
     hipLaunchKernelGGL(k_build_stats, dim3(1), dim3(kStatsThreads), 0, s, ntiles, part, stats,
-                       flag, tiles, spec, report, seq);
+                       flag, tiles, spec, report, seq, cap, verdict);
     return hipGetLastError();
 }
 

@@ -131,6 +131,44 @@ def test_step_loop_stops_at_nonfinite():
     s.close()
 
 
+# atoms falling together: rebuilds inside a run whose rows outgrow the list's
+# capacity and whose stencils outgrow the build's bound, with step launches
+# already queued behind the build that does not stand
+@pytest.mark.parametrize("tiled", ["0", "1"])
+@pytest.mark.parametrize("n,ndim,steps", [(600, 3, 60), (600, 2, 15), (6000, 3, 40)])
+def test_rebuilds_outgrow_the_list_inside_a_run(monkeypatch, tiled, n, ndim, steps):
+    _device_or_fail()
+    print(f"outgrow tiled={tiled} n={n} ndim={ndim} steps={steps}", flush=True)
+    monkeypatch.setenv("PARM_TILED", tiled)
+    monkeypatch.setenv("PARM_TPA", "4")
+    rng = np.random.default_rng(n + ndim)
+    edge = 2.2 * n ** (1.0 / ndim)
+    L = np.full(ndim, edge)
+    x = rng.uniform(0, edge, (n, ndim))
+    v = -(x - edge / 2) * 0.85  # all but together at t = 1
+    t = O.PairTable(O.REPULSION, [1e-6], [1.0], [2.0], np.zeros(n, np.int32))
+    r = O.System(np.ones(n), L, t, np.ones(n), 0.4, ndim=ndim, brute=False)
+    s = capi.System(ndim, np.ones(n))
+    s.set_box(L)
+    s.nlist_set(0.4, np.ones(n))
+    s.set_repulsion([1e-6], [1.0], [2.0], np.zeros(n, np.int32))
+    for q in (r, s):
+        q.set_state(x=x, v=v, a=np.zeros_like(x))
+        q.initialize()
+    cap = s.list_info()["capacity"]
+    for _ in range(2):
+        for q in (r, s):
+            q.verlet(0.5 / steps, steps)
+        assert s.which() == r.which()
+        fd, ld = s.pairs()
+        fr, lr = r.pairs()
+        assert np.array_equal(fd, fr) and np.array_equal(ld, lr)
+        xr, xd = r.state()[0], s.state()[0]
+        assert np.abs(xd - xr).max() <= 1e-12 * np.abs(xr).max()
+    assert s.list_info()["capacity"] > cap and s.which() > 10
+    s.close()
+
+
 # the tiled LJ pair loop: several types (table and type bytes in LDS), counts
 # that are no multiple of a group, folded (small box) and plain offsets, and
 # pairs at the cutoff itself
