@@ -33,7 +33,10 @@ namespace parm {
 // With kAheadLanes lanes or more (few atoms: latency, not registers or
 // bandwidth, bounds them) a lane's first kAhead entries are all in flight
 // before the first is evaluated, instead of two at a time: 1000 LJ atoms at 8
-// lanes, 200 steps 2320 -> 2130 us (4 or 8 ahead: within 3 % of 6).
+// lanes, 200 steps 2320 -> 2130 us (4 or 8 ahead: within 3 % of 6).  A repulsion
+// with a general exponent takes two: its rows are short, and each entry
+// evaluated ahead is another copy of pow (2,003 disks, 200 steps: six 2615 us, two
+// 2540).
 constexpr int kAheadLanes = 8, kAhead = 6;
 
 template <int D, int KIND, int PREC, bool SINGLE, bool HARM, int STAGE, bool ENERGY,
@@ -61,7 +64,7 @@ __global__ __launch_bounds__(kBlock) void k_force(AtomArrays A, ListView Lv,
     // as two lanes do, so the result does not depend on which of them the
     // autotuner takes
     constexpr bool PAIRSUM = PREC != kFP64 && TPA == 1;
-    constexpr int AHEAD = TPA >= kAheadLanes ? kAhead : 0;
+    constexpr int AHEAD = TPA < kAheadLanes ? 0 : (KIND == kPairRepulsion && !HARM ? 2 : kAhead);
     float f32[D], f32o[D];
 #pragma unroll
     for (int k = 0; k < D; k++) {

@@ -1,7 +1,6 @@
 // pairs.hpp -- per-pair force / energy math and the per-atom integrator
-// updates shared by the single-system (force.hip, step_tiled.hip, step.hip) and batched
-// (batch_force.hip, batch.hip)
-// kernels.
+// updates shared by the single-system (force.hip, step_tiled.hip, step.hip)
+// and batched (batch_force.hip, batch.hip) kernels.
 //
 // Reference behaviour restated (paths relative to the reference root):
 //   LJAttractRepulsePair::forces/energy  src/interaction.hpp:1270-1298
