@@ -746,7 +746,8 @@ static hipError_t batch_rebuild(const BatchArrays &A, const BatchLists &B, const
     hipLaunchKernelGGL(k_batch_sort<D>, dim3(B.sort_grid), dim3(kSortThreads), 0, s, A,
                        (const PT *)pos, count_rebuild, B.type_bits, S, B.which, B.nent, wl,
                        wl_next, B.work);
-    if (!B.nbr) return hipGetLastError();
+    if (B.sort_only) return hipGetLastError();
+    if (!B.nbr) return hipErrorInvalidValue;
 #define PARM_BB(GG)                                                                           \
     case GG:                                                                                  \
         hipLaunchKernelGGL((k_batch_build<D, GG>), dim3(B.build_grid), dim3(kBuildThreads),   \

@@ -70,7 +70,6 @@ struct parm_batch {
     double skin = 0.0;
     std::vector<int> off;           // nsys + 1
     std::vector<double> L;          // nsys * ndim
-    std::vector<BatchGeom> geom_h;
     BatchGeom *geom = nullptr;
 
     void *pos = nullptr, *pos_alt = nullptr, *xref = nullptr;
@@ -81,7 +80,9 @@ struct parm_batch {
     // orders every system's slots by cell
     int32_t *orig = nullptr;
 
-    int cap = 0, tpa = 4, type_bits = 0, total_cells = 0;
+    // cap: entries per atom that nbr holds (0: no list array); cap_want: what was
+    // last asked for (an allocation refused is tried again at the next build)
+    int cap = 0, cap_want = 0, tpa = 4, type_bits = 0, total_cells = 0;
     bool tuned = false, tpa_fixed = false, built = false;
     uint32_t *nbr = nullptr;
     int32_t *ncount = nullptr, *keys = nullptr, *cstart = nullptr;
@@ -359,18 +360,20 @@ int brebuild(parm_batch *b, int list, bool count, const void *pos, const void *a
 }
 
 int ensure_cap(parm_batch *b, int cap) {
-    if (cap <= b->cap && b->nbr) return PARM_OK;
-    bfree(b->nbr);
+    if (cap <= b->cap) return PARM_OK;
     const int round = max_lanes(b->ntot) - 1;
-    b->cap = (cap + round) & ~round;
-    PB_CHECK(balloc(&b->nbr, (size_t)b->cap * b->npad));
+    b->cap_want = (cap + round) & ~round;
+    bfree(b->nbr);
+    b->cap = 0;
+    PB_CHECK(balloc(&b->nbr, (size_t)b->cap_want * b->npad));
+    b->cap = b->cap_want;
     return PARM_OK;
 }
 
 // Every system's slots ordered by cell at the current positions.
 int order_slots(parm_batch *b) {
     BatchLists B = lists_of(b);
-    B.nbr = nullptr;
+    B.sort_only = true;
     PB_HIP(launch_batch_all(b->nsys, b->arrays(), B.lanes, b->wl + kListAll, b->work,
                             b->wslice, b->stream));
     PB_HIP(launch_batch_rebuild(b->ndim, b->arrays(), B, b->pos, nullptr, 0, b->skin,
@@ -383,6 +386,7 @@ int order_slots(parm_batch *b) {
 // First build of every system (NeighborList::update_list on a new list),
 // growing the list capacity until nothing overflows.
 int first_build(parm_batch *b) {
+    PB_CHECK(ensure_cap(b, b->cap_want));
     for (int attempt = 0; attempt < 6; attempt++) {
         PB_HIP(hipMemsetAsync(b->gflag, 0, sizeof(uint32_t), b->stream));
         PB_CHECK(brebuild(b, kListAll, true, b->pos));
@@ -714,6 +718,10 @@ static int batch_pair(parm_batch *b, int kind, int ntypes, const double *eps,
     if (!asym.empty())
         return bfail(PARM_E_UNSUPPORTED,
                      asym + ": the device evaluates each pair from both of its atoms");
+    int bits = 0;
+    while ((1 << bits) < ntypes) bits++;
+    if (bits > 0 && (int64_t)b->ntot >= (int64_t(1) << (32 - bits)))
+        return bfail(PARM_E_UNSUPPORTED, "too many atoms for this many types");
     std::vector<PairParam> tab;
     bool harm = true;
     make_pair_table(kind, ntypes, eps, sigma, third, tab, harm);
@@ -724,7 +732,7 @@ static int batch_pair(parm_batch *b, int kind, int ntypes, const double *eps,
         dia[i] = type_diameter(kind, sigma, third, atype[i]);
         dmax = std::max(dmax, dia[i]);
     }
-    b->geom_h.resize(b->nsys);
+    std::vector<BatchGeom> geom(b->nsys);
     int cells = 0;
     for (int s = 0; s < b->nsys; s++) {
         BatchGeom G{};
@@ -759,18 +767,32 @@ static int batch_pair(parm_batch *b, int kind, int ntypes, const double *eps,
         G.n = b->off[s + 1] - b->off[s];
         G.cell_off = cells;
         cells += G.grid.ncell + 1;
-        b->geom_h[s] = G;
+        geom[s] = G;
     }
     PB_HIP(hipSetDevice(b->device));
+    int32_t *cstart = nullptr;
+    PairParam *dtab = nullptr;
+    PB_CHECK(balloc(&cstart, (size_t)cells));
+    if (const int rc = balloc(&dtab, tab.size())) {
+        bfree(cstart);
+        return rc;
+    }
+    // the interaction before is gone, and until the end of this call there is none
+    b->pair_kind = kPairNone;
+    b->built = false;
+    if (b->gexec) {
+        (void)hipGraphExecDestroy(b->gexec);
+        b->gexec = nullptr;
+    }
     bfree(b->cstart);
-    PB_CHECK(balloc(&b->cstart, (size_t)cells));
+    b->cstart = cstart;
     b->total_cells = cells;
     bfree(b->tab);
-    PB_CHECK(balloc(&b->tab, tab.size()));
+    b->tab = dtab;
     PB_HIP(hipMemcpy(b->tab, tab.data(), sizeof(PairParam) * tab.size(),
                      hipMemcpyHostToDevice));
     b->tab0 = tab[0];
-    PB_HIP(hipMemcpy(b->geom, b->geom_h.data(), sizeof(BatchGeom) * b->nsys,
+    PB_HIP(hipMemcpy(b->geom, geom.data(), sizeof(BatchGeom) * b->nsys,
                      hipMemcpyHostToDevice));
     PB_CHECK(bupload_scalar<int32_t>(b, atype, b->type));
     PB_CHECK(bupload_scalar<double>(b, dia.data(), b->diam));
@@ -778,16 +800,10 @@ static int batch_pair(parm_batch *b, int kind, int ntypes, const double *eps,
                        b->sys);
     PB_HIP(hipGetLastError());
     PB_HIP(hipStreamSynchronize(b->stream));
-    int bits = 0;
-    while ((1 << bits) < ntypes) bits++;
-    if (bits > 0 && (int64_t)b->ntot >= (int64_t(1) << (32 - bits)))
-        return bfail(PARM_E_UNSUPPORTED, "too many atoms for this many types");
     b->type_bits = bits;
     b->ntypes = ntypes;
     b->single = ntypes == 1 ? 1 : 0;
     b->harmonic = (kind == kPairRepulsion && harm) ? 1 : 0;
-    b->pair_kind = kind;
-    b->built = false;
     // initial list capacity from the densest system
     double dens = 0;
     for (int s = 0; s < b->nsys; s++) {
@@ -798,10 +814,7 @@ static int batch_pair(parm_batch *b, int kind, int ntypes, const double *eps,
     const double r = dmax + b->skin;
     const double ball = b->ndim == 3 ? 4.0 / 3.0 * kPi * r * r * r : kPi * r * r;
     PB_CHECK(ensure_cap(b, std::max(16, (int)(1.6 * dens * ball + 24))));
-    if (b->gexec) {
-        (void)hipGraphExecDestroy(b->gexec);
-        b->gexec = nullptr;
-    }
+    b->pair_kind = kind;
     return PARM_OK;
 }
 
@@ -959,6 +972,8 @@ int parm_batch_pairs(parm_batch *b, int64_t sysid, int64_t cap, int32_t *first,
     if (!b || sysid < 0 || sysid >= b->nsys) return bfail(PARM_E_INVALID, "bad system");
     if (cap > 0 && (!first || !last)) return bfail(PARM_E_INVALID, "null output");
     PB_HIP(hipSetDevice(b->device));
+    if (npairs) *npairs = 0;
+    if (!b->built) return PARM_OK;  // no lists
     const int o = b->off[sysid], n = b->off[sysid + 1] - o;
     std::vector<int32_t> cnt(n), orig(n);
     PB_HIP(hipMemcpyAsync(orig.data(), b->orig + o, sizeof(int32_t) * n, hipMemcpyDeviceToHost,

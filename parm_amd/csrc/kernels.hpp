@@ -357,7 +357,7 @@ int batch_build_lanes(int ntot, int cells);
 // The batch's lists and what their build works on.
 struct BatchLists {
     int type_bits, tpa, cap, npad;
-    uint32_t *nbr;        // null: sort only
+    uint32_t *nbr;
     int32_t *ncount;
     int32_t *keys;        // sorted slots: cell,
     uint32_t *ent;        // list word (index << type_bits | type),
@@ -369,6 +369,7 @@ struct BatchLists {
     int32_t *work, *wslice;    // nsys each: listed systems, their first build slice
     int sort_grid, build_grid;
     int lanes;            // the build's lanes per atom (batch_build_lanes)
+    bool sort_only;       // order the slots, build no list
 };
 // Rebuilds the systems listed in wl: sort, then the list build spread over
 // slices of the listed systems; empties wl_next (may be null).  alt: positions

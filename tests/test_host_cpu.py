@@ -1,0 +1,93 @@
+"""The library's host logic on a HIP runtime of host memory whose kernels do not
+run (host_hip.hip): allocations and launches that are refused, list builds that
+overflow or are refused.  Each case is a process of its own, in which that
+runtime is loaded before the library."""
+import ctypes as C
+import os
+import subprocess
+import sys
+
+import numpy as np
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+NOMEM, UNSUPPORTED, DEVICE = -3, -4, -2
+REBUILD = 1  # skin flag
+
+
+@pytest.fixture(scope="module")
+def runtime(tmp_path_factory):
+    d = tmp_path_factory.mktemp("host_hip")
+    obj, so = str(d / "host_hip.o"), str(d / "libhost_hip.so")
+    subprocess.run(["/opt/rocm/bin/hipcc", "-x", "hip", "--offload-host-only", "-std=c++17",
+                    "-O1", "-fPIC", "-c", os.path.join(ROOT, "tests", "host_hip.hip"), "-o", obj],
+                   check=True)
+    subprocess.run(["g++", "-shared", "-o", so, obj], check=True)
+    return so
+
+
+def _child(runtime, case, *args, **env):
+    r = subprocess.run([sys.executable, os.path.abspath(__file__), runtime, case,
+                        *map(str, args)], capture_output=True, text=True, timeout=120, cwd=ROOT,
+                       env={**os.environ, **env})
+    assert r.returncode == 0, r.stdout + r.stderr
+
+
+def _refused(code, f, *a):
+    from parm_amd import capi
+    try:
+        f(*a)
+    except (capi.ParmError, capi.ParmValueError) as e:
+        assert e.code == code, e
+    else:
+        raise AssertionError("not refused")
+
+
+# ------------------------------------------------------------------- batches
+def _batch(hh, n=300, nsys=2):
+    from parm_amd import capi
+    b = capi.Batch(3, [n] * nsys, [[9.0] * 3] * nsys, 0.2)
+    b.set_state(x=np.random.default_rng(0).uniform(0, 9, (n * nsys, 3)))
+    return b
+
+
+def _set_pair(b):
+    b.set_repulsion([1.0], [1.0], [2.0], np.zeros(b.n, np.int32))
+
+
+def case_batch_list_refused(hh, where):
+    b = _batch(hh)
+    if where == "set":      # the interaction's own list allocation
+        hh.hh_alloc_limit(16 * b.n * 4 - 1)
+        _refused(NOMEM, _set_pair, b)
+        hh.hh_reset()
+        _refused(-6, b.initialize)  # no interaction set
+        _set_pair(b)
+    else:                   # the growth of a list that overflowed
+        _set_pair(b)
+        hh.hh_overflows(1)
+        hh.hh_fail_at(1)
+        _refused(NOMEM, b.initialize)
+        assert len(b.pairs(0)[0]) == 0
+        hh.hh_reset()
+    b.initialize()
+    assert "k_batch_build" in hh.hh_log().decode()
+    b.damped(0.01, 1.0, 12)
+    assert hh.hh_bad() == 0
+    b.close()
+
+
+@pytest.mark.parametrize("where", ["set", "grow"])
+def test_batch_list_refused(runtime, where):
+    _child(runtime, "case_batch_list_refused", where)
+
+
+if __name__ == "__main__":
+    sys.path.insert(0, ROOT)
+    hh = C.CDLL(sys.argv[1], mode=C.RTLD_GLOBAL)
+    hh.hh_log.restype = C.c_char_p
+    hh.hh_alloc_limit.argtypes = [C.c_size_t]
+    hh.hh_row.argtypes = [C.c_ulonglong]
+    from parm_amd import capi
+    assert capi.device_count() == 1 and hh.hh_bad() == 0
+    globals()[sys.argv[2]](hh, *sys.argv[3:])
