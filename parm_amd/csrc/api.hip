@@ -340,11 +340,15 @@ int ensure_list_capacity(parm_system *s, int cap) {
     // refused before the list is reallocated
     PARM_CHECK(check_lane_counts(((int64_t)cap + round) & ~(int64_t)round, s->tpa));
     free_list(s);
-    s->cap = (cap + round) & ~round;
-    PARM_CHECK(dalloc(&s->nbr, (size_t)s->cap * s->npad));
-    PARM_CHECK(dalloc(&s->ncount, (size_t)s->npad));
-    PARM_CHECK(dalloc(&s->lcount, (size_t)s->npad * max_lanes(s->n)));
-    return PARM_OK;
+    cap = (cap + round) & ~round;
+    int rc = dalloc(&s->nbr, (size_t)cap * s->npad);
+    if (rc == PARM_OK) rc = dalloc(&s->ncount, (size_t)s->npad);
+    if (rc == PARM_OK) rc = dalloc(&s->lcount, (size_t)s->npad * max_lanes(s->n));
+    if (rc == PARM_OK)
+        s->cap = cap;
+    else
+        free_list(s);  // (a capacity stands for arrays that are there)
+    return rc;
 }
 
 int initial_capacity(const parm_system *s) {
@@ -417,9 +421,10 @@ int launch_tile_plan(parm_system *s) {
     if (need > s->tiles_cap) {
         dfree(s->tiles);
         dfree(s->truns);
-        s->tiles_cap = need;
+        s->tiles_cap = 0;  // until both are there
         PARM_CHECK(dalloc(&s->tiles, (size_t)need));
         PARM_CHECK(dalloc(&s->truns, (size_t)need * kTileRuns));
+        s->tiles_cap = need;
     }
     PARM_HIP(launch_tiles(s->ndim, s->n, s->grid, s->keys, s->cstart, s->tiles_cap, s->tiles,
                           s->truns, s->tinfo, s->stream));
@@ -650,8 +655,9 @@ int upload_exclusions(parm_system *s) {
     if (!s->ex_off) PARM_CHECK(dalloc(&s->ex_off, (size_t)n + 1));
     if (np > s->ex_part_cap) {
         dfree(s->ex_part);
+        s->ex_part_cap = 0;
+        PARM_CHECK(dalloc(&s->ex_part, (size_t)(np + np / 2 + 16)));
         s->ex_part_cap = np + np / 2 + 16;
-        PARM_CHECK(dalloc(&s->ex_part, (size_t)s->ex_part_cap));
     }
     if (np > 0) {
         PARM_HIP(hipMemcpyAsync(s->ex_off, off.data(), sizeof(int32_t) * off.size(),
@@ -677,19 +683,21 @@ int rebuild(parm_system *s, bool keep_af = true, const ReduceBuf *skin = nullptr
     hipStream_t st = s->stream;
     const int n = s->n;
     make_grid(s);
+    // from here on the previous list no longer matches the cells and the atom order
+    s->built = false;
+    s->build_due = false;
     if (s->grid.ncell + 1 > s->cstart_cap) {
         dfree(s->cstart);
         dfree(s->ccount);
         dfree(s->ctotal);
-        s->cstart_cap = s->grid.ncell + 1;
-        PARM_CHECK(dalloc(&s->cstart, (size_t)s->cstart_cap));
-        PARM_CHECK(dalloc(&s->ccount, (size_t)s->cstart_cap));
-        PARM_CHECK(dalloc(&s->ctotal, (size_t)scan_tiles(s->cstart_cap)));
+        s->cstart_cap = 0;  // until all three are there
         s->ccount_clear = false;
+        const int cells = s->grid.ncell + 1;
+        PARM_CHECK(dalloc(&s->cstart, (size_t)cells));
+        PARM_CHECK(dalloc(&s->ccount, (size_t)cells));
+        PARM_CHECK(dalloc(&s->ctotal, (size_t)scan_tiles(cells)));
+        s->cstart_cap = cells;
     }
-    // from here on the previous list no longer matches the atom order
-    s->built = false;
-    s->build_due = false;
     const bool counted = n > 0 && s->nmem == n;
     if (counted) {
         if (!s->ccount_clear)
@@ -1221,17 +1229,19 @@ int build_pair_table(parm_system *s, int form, int ntypes, const double *eps,
     std::vector<PairParam> tab;
     bool harm = true;
     make_pair_table(form, ntypes, eps, sigma, third, tab, harm);
-    PARM_CHECK(set_device(s));
-    dfree(s->tab);
-    PARM_CHECK(dalloc(&s->tab, tab.size()));
-    PARM_HIP(hipMemcpy(s->tab, tab.data(), sizeof(PairParam) * tab.size(),
-                       hipMemcpyHostToDevice));
-    s->tab0 = tab[0];
-    if (s->n > 0) PARM_CHECK(upload_scalar<int32_t>(s, atype, s->type));
     int bits = 0;
     while ((1 << bits) < ntypes) bits++;
     if (bits > 0 && (int64_t)s->n >= (int64_t(1) << (32 - bits)))
         return fail(PARM_E_UNSUPPORTED, "too many atoms for this many types");
+    PARM_CHECK(set_device(s));
+    PairParam *dtab = nullptr;
+    PARM_CHECK(dalloc(&dtab, tab.size()));
+    dfree(s->tab);
+    s->tab = dtab;
+    PARM_HIP(hipMemcpy(s->tab, tab.data(), sizeof(PairParam) * tab.size(),
+                       hipMemcpyHostToDevice));
+    s->tab0 = tab[0];
+    if (s->n > 0) PARM_CHECK(upload_scalar<int32_t>(s, atype, s->type));
     s->type_bits = bits;
     s->ntypes = ntypes;
     s->single = ntypes == 1 ? 1 : 0;
@@ -1934,8 +1944,10 @@ int parm_snapshot_begin(parm_system *s, int what, int64_t *ticket) {
     if (!q.dev) {
         PARM_CHECK(dalloc(&q.dev, 2 * std::max<size_t>(nv, 1)));
         if (hipHostMalloc((void **)&q.host, sizeof(double) * 2 * std::max<size_t>(nv, 1), 0) !=
-            hipSuccess)
+            hipSuccess) {
+            dfree(q.dev);
             return fail(PARM_E_NOMEM, "pinned snapshot allocation failed");
+        }
         PARM_HIP(hipEventCreateWithFlags(&q.ready, hipEventDisableTiming));
         PARM_HIP(hipEventCreateWithFlags(&q.done, hipEventDisableTiming));
     } else if (q.ticket >= 0) {

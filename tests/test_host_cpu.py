@@ -82,6 +82,56 @@ def test_batch_list_refused(runtime, where):
     _child(runtime, "case_batch_list_refused", where)
 
 
+# ------------------------------------------------------------- single systems
+def _system(n=20000, **kw):
+    from parm_amd import capi
+    s = capi.System(3, np.ones(n))
+    s.set_box([40.0] * 3)
+    s.nlist_set(0.3, np.ones(n))
+    s.set_repulsion([1.0], [1.0], [2.0], np.zeros(n, np.int32))
+    s.set_state(x=np.random.default_rng(0).uniform(0, 40, (n, 3)))
+    return s
+
+
+def _log(hh):
+    out = hh.hh_log().decode()
+    hh.hh_clear_log()
+    return out
+
+
+# every allocation of a first list build refused in turn, and of one with more
+# cells and tiles (a larger box): no launch goes through what is not there
+def case_list_allocations_refused(hh, edge):
+    refused = 0
+    for k in range(1, 40):
+        s = _system()
+        if float(edge) > 0:
+            s.update_list(True)
+            s.set_box([float(edge)] * 3)
+        hh.hh_fail_at(k)
+        try:
+            s.update_list(True)
+            done = True
+        except RuntimeError as e:
+            assert e.code == NOMEM
+            done = False
+            refused += 1
+        hh.hh_fail_at(0)
+        s.update_list(True)
+        s.set_forces()
+        s.verlet(0.001, 5)
+        assert hh.hh_bad() == 0, k
+        s.close()
+        if done:
+            break
+    assert refused >= (8 if float(edge) == 0 else 5), refused
+
+
+@pytest.mark.parametrize("edge", [0, 60])
+def test_list_allocations_refused(runtime, edge):
+    _child(runtime, "case_list_allocations_refused", edge)
+
+
 if __name__ == "__main__":
     sys.path.insert(0, ROOT)
     hh = C.CDLL(sys.argv[1], mode=C.RTLD_GLOBAL)
