@@ -123,7 +123,9 @@ struct parm_system {
     bool ignorechanged = true;
     uint32_t which = 0;
     int64_t npairs = 0;
-    bool built = false;
+    // list_lost: a build failed (refused capacity, allocation) with no list left;
+    // whatever needs one builds it first (need_list)
+    bool built = false, list_lost = false;
     CellGrid grid{};
     int cap = 0, npad = 0, type_bits = 0;
     int tpa = 4;            // lanes per atom in the force kernel (autotuned)
@@ -289,6 +291,13 @@ void free_list(parm_system *s) {
     dfree(s->ncount);
     dfree(s->lcount);
     s->cap = 0;
+}
+
+// The current list is void: until a build stands, calls that need one rebuild.
+void lose_list(parm_system *s) {
+    s->built = false;
+    s->build_due = false;
+    s->list_lost = true;
 }
 
 // Cell grid for the current box / diameters / skin: edge >= largest list
@@ -580,12 +589,13 @@ int settle_build(parm_system *s, bool *stands) {
     // until it is built anew there is no list (and a deferred build has been
     // counted already)
     const bool counted = s->built;
-    s->built = false;
+    lose_list(s);
     if (counted) s->which--;
     if (fits && r.max > (unsigned long long)s->cap)
         PARM_CHECK(ensure_list_capacity(s, (int)(r.max + r.max / 8 + 8)));
     PARM_CHECK(build_checked(s, s->pos, s->build_wrapped));
     s->built = counted;
+    s->list_lost = !counted;  // (else rebuild, which is under way, says so)
     if (counted) s->which++;
     return PARM_OK;
 }
@@ -684,8 +694,7 @@ int rebuild(parm_system *s, bool keep_af = true, const ReduceBuf *skin = nullptr
     const int n = s->n;
     make_grid(s);
     // from here on the previous list no longer matches the cells and the atom order
-    s->built = false;
-    s->build_due = false;
+    lose_list(s);
     if (s->grid.ncell + 1 > s->cstart_cap) {
         dfree(s->cstart);
         dfree(s->ccount);
@@ -734,15 +743,21 @@ int rebuild(parm_system *s, bool keep_af = true, const ReduceBuf *skin = nullptr
         PARM_HIP(launch_skin(s->ndim, A, *skin, false, st));
     }
     s->built = true;
+    s->list_lost = false;
     s->which++;
     s->ignorechanged = false;
     return PARM_OK;
 }
 
+// A list in place of one that a failed build left behind (NeighborList has none
+// to lose: its update cannot fail).  A list never built is another matter: until
+// its first update there are no pairs.
+int need_list(parm_system *s) { return s->list_lost ? rebuild(s) : PARM_OK; }
+
 int update_list(parm_system *s, bool force, int *rebuilt) {
     if (rebuilt) *rebuilt = 0;
     if (!s->list_cfg) return fail(PARM_E_STATE, "neighbour list not configured");
-    if (!force && !s->ignorechanged) {
+    if (!force && !s->ignorechanged && !s->list_lost) {
         ReduceBuf R = s->redbuf(kSlotSkin);
         R.g.seq = ++s->step_seq;
         PARM_HIP(launch_skin(s->ndim, s->arrays(), R, true, s->stream));
@@ -766,6 +781,7 @@ int require_ready(parm_system *s) {
 }
 
 int set_forces(parm_system *s, bool and_a) {
+    PARM_CHECK(need_list(s));
     StepCoef c{};
     PARM_HIP(launch_force(s->ndim, s->prec, and_a ? kStageForceA : kStageForceOnly, false,
                           s->arrays(), s->listview(), s->pairview(), s->box, c,
@@ -816,8 +832,9 @@ struct ProfScope {
 int relayout(parm_system *s) {
     if (!s->built || s->n == 0) return PARM_OK;
     if (s->tiled && !(s->tile_ok && tiled_force_fits(s))) s->tiled = false;
-    PARM_CHECK(build_checked(s, s->xref));
-    return PARM_OK;
+    const int rc = build_checked(s, s->xref);
+    if (rc != PARM_OK) lose_list(s);
+    return rc;
 }
 
 // Autotuner of the step kernel: list layout (tiled / untiled, tiles.hpp) x
@@ -958,6 +975,14 @@ int step_runahead(const parm_system *s) { return s->n <= kRunAheadAtoms ? kRunAh
 int run_steps(parm_system *s, bool damped, const StepCoef &c, int64_t nsteps) {
     PARM_CHECK(require_ready(s));
     if (nsteps <= 0) return PARM_OK;
+    PARM_CHECK(need_list(s));
+    // a run that ends in an error leaves no build whose report nobody reads
+    struct Settled {
+        parm_system *s;
+        ~Settled() {
+            if (s->build_due) lose_list(s);
+        }
+    } settled{s};
     const int kick = damped ? kStageDampedKick : kStageVerletKick;
     const int kick_drift = damped ? kStageDampedKickDrift : kStageVerletKickDrift;
     if (nsteps >= 16) PARM_CHECK(autotune(s, kick_drift, c));
@@ -1493,7 +1518,7 @@ int parm_nlist_set(parm_system *s, double skin, int64_t nmembers, const int32_t 
     // a new NeighborList has an empty PairList
     s->excl.clear();
     s->excl_dirty = true;
-    s->built = false;
+    s->built = s->list_lost = false;
     s->npairs = 0;
     free_list(s);
     return PARM_OK;
@@ -1676,6 +1701,7 @@ int parm_add_pair_forces(parm_system *s) {
     PARM_CHECK(check_sys(s));
     PARM_CHECK(require_ready(s));
     PARM_CHECK(set_device(s));
+    PARM_CHECK(need_list(s));
     StepCoef c{};
     PARM_HIP(launch_force(s->ndim, s->prec, kStageForceAdd, false, s->arrays(),
                           s->listview(), s->pairview(), s->box, c, s->redbuf(kSlotScratch),
@@ -1688,6 +1714,7 @@ int parm_pair_sums(parm_system *s, double *U, double *W, double *S, uint64_t *co
     PARM_CHECK(check_sys(s));
     PARM_CHECK(require_ready(s));
     PARM_CHECK(set_device(s));
+    PARM_CHECK(need_list(s));
     StepCoef c{};
     PARM_HIP(launch_force(s->ndim, s->prec, kStageSums, true, s->arrays(), s->listview(),
                           s->pairview(), s->box, c, sumbuf(s), s->stream));
@@ -1758,6 +1785,9 @@ int parm_pair_sums_noalloc(parm_system *s, double *out) {
                     "parm_pair_sums_noalloc: at most " + std::to_string(kNoAllocMaxAtoms) +
                         " atoms (its scratch is a fixed device array)");
     PARM_CHECK(require_ready(s));
+    // (a rebuild allocates)
+    if (s->list_lost)
+        return fail(PARM_E_STATE, "the last list build failed: call parm_nlist_update first");
     PARM_CHECK(set_device(s));
     double *scr = nullptr;
     PARM_CHECK(scratch_address(s->device, &scr));
@@ -2128,6 +2158,7 @@ int nlcg_set_forces(parm_nlcg *c, bool constraints_and_a, bool setV) {
     parm_system *s = c->s;
     const double V = box_V(s);
     if (setV) {
+        PARM_CHECK(need_list(s));
         StepCoef cf{};
         PARM_HIP(launch_force(s->ndim, s->prec, kStageNlcg, false, s->arrays(), s->listview(),
                               s->pairview(), s->box, cf, sumbuf(s), s->stream));

@@ -132,6 +132,68 @@ def test_list_allocations_refused(runtime, edge):
     _child(runtime, "case_list_allocations_refused", edge)
 
 
+# a rebuild inside a run, queued with step launches behind it or not, and the
+# relaying of a list, whose row no lane could hold: the list is gone, and the
+# next call that needs it builds one or is refused again
+def case_refused_list_comes_back(hh, call):
+    s = _system()
+    s.update_list(True)
+    s.update_list(True)  # (with the plan of the one before: built speculatively)
+    built = s.which()
+    assert built == 2
+    if call == "set_pair":
+        hh.hh_row(10 ** 7)
+        _refused(UNSUPPORTED, s.set_repulsion, [1.0], [1.0], [2.0], np.zeros(s.n, np.int32))
+    else:
+        s.ignore([0], [1])  # an update that is due
+        hh.hh_row(10 ** 7)
+        _refused(UNSUPPORTED, s.verlet, 0.001, 6)
+    assert s.which() == built and s.numpairs() == 0
+    _log(hh)
+    calls = dict(forces=s.set_forces, add=s.add_pair_forces, sums=s.pair_sums,
+                 verlet=lambda: s.verlet(0.001, 4), damped=lambda: s.damped(0.001, 0.1, 4),
+                 update=lambda: s.update_list(False), init=s.initialize,
+                 tune=lambda: s.autotune(0.001), set_pair=s.set_forces)
+    hh.hh_row(10 ** 7)
+    _refused(UNSUPPORTED, calls[call])
+    assert "k_force" not in _log(hh)
+    calls[call]()
+    first = [k for k in _log(hh).split() if "k_build" in k or "k_force" in k][0]
+    assert "k_build" in first
+    assert s.which() == built + 1 and s.numpairs() == 1
+    s.update_list(False)
+    assert s.which() == built + 1 and hh.hh_bad() == 0
+    s.close()
+
+
+@pytest.mark.parametrize("tiled", ["0", "1"])
+@pytest.mark.parametrize("call", ["forces", "add", "sums", "verlet", "damped", "update", "init",
+                                  "tune", "set_pair"])
+def test_refused_list_comes_back(runtime, call, tiled):
+    _child(runtime, "case_refused_list_comes_back", call, PARM_TILED=tiled, PARM_TPA="4")
+
+
+# the minimiser's force launches, and the sums that may not allocate
+def case_refused_list_nlcg(hh):
+    from parm_amd import capi
+    s = _system()
+    c = capi.NLCG(s, 0.1, 1e-3)
+    hh.hh_row(10 ** 7)
+    _refused(UNSUPPORTED, s.update_list, True)
+    out = C.c_void_p()
+    assert capi.lib().parm_pair_sums_noalloc(s.h, C.byref(out)) == -6  # no list, by rule
+    hh.hh_row(10 ** 7)
+    _refused(UNSUPPORTED, c.timestep)
+    _log(hh)
+    c.timestep(1)
+    assert "k_build" in [k for k in _log(hh).split() if "k_build" in k or "k_force" in k][0]
+    assert hh.hh_bad() == 0
+
+
+def test_refused_list_nlcg(runtime):
+    _child(runtime, "case_refused_list_nlcg")
+
+
 if __name__ == "__main__":
     sys.path.insert(0, ROOT)
     hh = C.CDLL(sys.argv[1], mode=C.RTLD_GLOBAL)
