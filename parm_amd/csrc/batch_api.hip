@@ -113,7 +113,6 @@ struct parm_batch {
     StepCoef g_coef{};
     void *g_pos = nullptr;
     int g_tpa = 0;
-    const uint32_t *g_nbr = nullptr;
 
     BatchArrays arrays(bool alt_out = false) const {
         BatchArrays A{};
@@ -359,8 +358,17 @@ int brebuild(parm_batch *b, int list, bool count, const void *pos, const void *a
     return PARM_OK;
 }
 
+// A captured run of steps holds the lists' address and capacity, the pair
+// parameters and the cells: it goes with any of them (the address alone does
+// not tell: a longer list may get the place of the one before).
+void drop_graph(parm_batch *b) {
+    if (b->gexec) (void)hipGraphExecDestroy(b->gexec);
+    b->gexec = nullptr;
+}
+
 int ensure_cap(parm_batch *b, int cap) {
     if (cap <= b->cap) return PARM_OK;
+    drop_graph(b);
     const int round = max_lanes(b->ntot) - 1;
     b->cap_want = (cap + round) & ~round;
     bfree(b->nbr);
@@ -509,12 +517,9 @@ int run_batch(parm_batch *b, bool damped, const StepCoef &c, int64_t nsteps, boo
     const int64_t runs = (nsteps - 1) / kGraphSteps;
     if (graph && runs > 0 && !b->prof) {
         const bool same = b->gexec && b->g_damped == damped && b->g_pos == b->pos &&
-                          b->g_tpa == b->tpa && b->g_nbr == b->nbr && std::memcmp(&b->g_coef, &c, sizeof c) == 0;
+                          b->g_tpa == b->tpa && std::memcmp(&b->g_coef, &c, sizeof c) == 0;
         if (!same) {
-            if (b->gexec) {
-                (void)hipGraphExecDestroy(b->gexec);
-                b->gexec = nullptr;
-            }
+            drop_graph(b);
             hipGraph_t g = nullptr;
             PB_HIP(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
             int rc = PARM_OK;
@@ -534,7 +539,6 @@ int run_batch(parm_batch *b, bool damped, const StepCoef &c, int64_t nsteps, boo
             b->g_damped = damped;
             b->g_pos = b->pos;
             b->g_tpa = b->tpa;
-            b->g_nbr = b->nbr;
             b->g_coef = c;
         }
         for (int64_t r = 0; r < runs; r++) PB_HIP(hipGraphLaunch(b->gexec, st));
@@ -780,10 +784,7 @@ static int batch_pair(parm_batch *b, int kind, int ntypes, const double *eps,
     // the interaction before is gone, and until the end of this call there is none
     b->pair_kind = kPairNone;
     b->built = false;
-    if (b->gexec) {
-        (void)hipGraphExecDestroy(b->gexec);
-        b->gexec = nullptr;
-    }
+    drop_graph(b);
     bfree(b->cstart);
     b->cstart = cstart;
     b->total_cells = cells;

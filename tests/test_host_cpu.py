@@ -82,6 +82,26 @@ def test_batch_list_refused(runtime, where):
     _child(runtime, "case_batch_list_refused", where)
 
 
+# a list that grew in place (the freed block's address given out again): the
+# captured run of steps holds the capacity that was
+def case_graph_follows_the_list(hh):
+    b = _batch(hh)
+    _set_pair(b)
+    b.initialize()
+    b.damped(0.01, 1.0, 17)  # 16 steps in graphs, then the last
+    b.damped(0.01, 1.0, 17)
+    assert hh.hh_graphs() == 1
+    hh.hh_overflows(1)
+    b.initialize()
+    b.damped(0.01, 1.0, 17)
+    assert hh.hh_graphs() == 2 and hh.hh_bad() == 0
+    b.close()
+
+
+def test_graph_follows_the_list(runtime):
+    _child(runtime, "case_graph_follows_the_list", PARM_TPA="4")
+
+
 # ------------------------------------------------------------- single systems
 def _system(n=20000, **kw):
     from parm_amd import capi
