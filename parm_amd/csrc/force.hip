@@ -158,9 +158,9 @@ __global__ __launch_bounds__(kBlock) void k_force(AtomArrays A, ListView Lv,
 }
 
 template <int D, int KIND, int PREC, bool SINGLE, bool HARM, int STAGE, int TPA>
-static void launch_force_tt(bool energy, const AtomArrays &A, const ListView &Lv,
-                            const PairView &P, const Box &box, const StepCoef &c,
-                            const ReduceBuf &R, hipStream_t s) {
+static hipError_t launch_force_tt(bool energy, const AtomArrays &A, const ListView &Lv,
+                                  const PairView &P, const Box &box, const StepCoef &c,
+                                  const ReduceBuf &R, hipStream_t s) {
     constexpr bool DRIFT =
         (STAGE == kStageVerletKickDrift || STAGE == kStageDampedKickDrift);
     // energies and virials are accumulated by these stages only
@@ -171,52 +171,48 @@ static void launch_force_tt(bool energy, const AtomArrays &A, const ListView &Lv
     dim3 g(nb + (STEP && R.g.nprev > 0 ? 1 : 0)), b(kBlock);
     hipLaunchKernelGGL((k_force<D, KIND, PREC, SINGLE, HARM, STAGE, ENERGY, TPA>), g, b, 0,
                        s, A, Lv, P, box, c, R);
+    // (before any other call: the next one's outcome would take its place)
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
     if (R.done) (void)hipEventRecord(R.done, s);
-    if (ENERGY) (void)launch_finalize_sums(false, nb, R, s);
+    return ENERGY ? launch_finalize_sums(false, nb, R, s) : hipSuccess;
 }
 
 template <int D, int KIND, int PREC, bool SINGLE, bool HARM, int STAGE>
-static void launch_force_t(bool energy, const AtomArrays &A, const ListView &Lv,
-                           const PairView &P, const Box &box, const StepCoef &c,
-                           const ReduceBuf &R, hipStream_t s) {
+static hipError_t launch_force_t(bool energy, const AtomArrays &A, const ListView &Lv,
+                                 const PairView &P, const Box &box, const StepCoef &c,
+                                 const ReduceBuf &R, hipStream_t s) {
     switch (Lv.tpa) {
     case 1:
-        launch_force_tt<D, KIND, PREC, SINGLE, HARM, STAGE, 1>(energy, A, Lv, P, box, c,
-                                                               R, s);
-        break;
+        return launch_force_tt<D, KIND, PREC, SINGLE, HARM, STAGE, 1>(energy, A, Lv, P, box, c,
+                                                                      R, s);
     case 2:
-        launch_force_tt<D, KIND, PREC, SINGLE, HARM, STAGE, 2>(energy, A, Lv, P, box, c,
-                                                               R, s);
-        break;
+        return launch_force_tt<D, KIND, PREC, SINGLE, HARM, STAGE, 2>(energy, A, Lv, P, box, c,
+                                                                      R, s);
     case 32:
-        launch_force_tt<D, KIND, PREC, SINGLE, HARM, STAGE, 32>(energy, A, Lv, P, box, c,
-                                                                R, s);
-        break;
+        return launch_force_tt<D, KIND, PREC, SINGLE, HARM, STAGE, 32>(energy, A, Lv, P, box, c,
+                                                                      R, s);
     case 16:
-        launch_force_tt<D, KIND, PREC, SINGLE, HARM, STAGE, 16>(energy, A, Lv, P, box, c,
-                                                                R, s);
-        break;
+        return launch_force_tt<D, KIND, PREC, SINGLE, HARM, STAGE, 16>(energy, A, Lv, P, box, c,
+                                                                      R, s);
     case 8:
-        launch_force_tt<D, KIND, PREC, SINGLE, HARM, STAGE, 8>(energy, A, Lv, P, box, c,
-                                                               R, s);
-        break;
+        return launch_force_tt<D, KIND, PREC, SINGLE, HARM, STAGE, 8>(energy, A, Lv, P, box, c,
+                                                                      R, s);
     default:
-        launch_force_tt<D, KIND, PREC, SINGLE, HARM, STAGE, 4>(energy, A, Lv, P, box, c,
-                                                               R, s);
-        break;
+        return launch_force_tt<D, KIND, PREC, SINGLE, HARM, STAGE, 4>(energy, A, Lv, P, box, c,
+                                                                      R, s);
     }
 }
 
 template <int D, int KIND, int PREC, bool SINGLE, bool HARM>
-static void launch_force_s(int stage, bool energy, const AtomArrays &A,
-                           const ListView &Lv, const PairView &P, const Box &box,
-                           const StepCoef &c, const ReduceBuf &R, hipStream_t s) {
+static hipError_t launch_force_s(int stage, bool energy, const AtomArrays &A,
+                                 const ListView &Lv, const PairView &P, const Box &box,
+                                 const StepCoef &c, const ReduceBuf &R, hipStream_t s) {
     switch (stage) {
-#define PARM_STAGE(S)                                                          \
-    case S:                                                                    \
-        launch_force_t<D, KIND, PREC, SINGLE, HARM, S>(energy, A, Lv, P, box,  \
-                                                       c, R, s);               \
-        break;
+#define PARM_STAGE(S)                                                                 \
+    case S:                                                                           \
+        return launch_force_t<D, KIND, PREC, SINGLE, HARM, S>(energy, A, Lv, P, box,  \
+                                                              c, R, s);
         PARM_STAGE(kStageForceOnly)
         PARM_STAGE(kStageForceA)
         PARM_STAGE(kStageVerletKick)
@@ -228,40 +224,34 @@ static void launch_force_s(int stage, bool energy, const AtomArrays &A,
         PARM_STAGE(kStageNlcg)
 #undef PARM_STAGE
     }
+    return hipErrorInvalidValue;
 }
 
 template <int D, int KIND, int PREC>
-static void launch_force_k(int stage, bool energy, const AtomArrays &A,
-                           const ListView &Lv, const PairView &P, const Box &box,
-                           const StepCoef &c, const ReduceBuf &R, hipStream_t s) {
+static hipError_t launch_force_k(int stage, bool energy, const AtomArrays &A,
+                                 const ListView &Lv, const PairView &P, const Box &box,
+                                 const StepCoef &c, const ReduceBuf &R, hipStream_t s) {
     if constexpr (KIND == kPairRepulsion) {
         if (P.harmonic) {
-            if (P.single)
-                launch_force_s<D, KIND, PREC, true, true>(stage, energy, A, Lv, P, box,
-                                                          c, R, s);
-            else
-                launch_force_s<D, KIND, PREC, false, true>(stage, energy, A, Lv, P, box,
-                                                           c, R, s);
-            return;
+            return P.single ? launch_force_s<D, KIND, PREC, true, true>(stage, energy, A, Lv,
+                                                                        P, box, c, R, s)
+                            : launch_force_s<D, KIND, PREC, false, true>(stage, energy, A, Lv,
+                                                                         P, box, c, R, s);
         }
     }
-    {
-        if (P.single)
-            launch_force_s<D, KIND, PREC, true, false>(stage, energy, A, Lv, P, box,
-                                                       c, R, s);
-        else
-            launch_force_s<D, KIND, PREC, false, false>(stage, energy, A, Lv, P, box,
-                                                        c, R, s);
-    }
+    return P.single ? launch_force_s<D, KIND, PREC, true, false>(stage, energy, A, Lv, P, box,
+                                                                 c, R, s)
+                    : launch_force_s<D, KIND, PREC, false, false>(stage, energy, A, Lv, P, box,
+                                                                  c, R, s);
 }
 
 template <int D, int KIND, int PREC>
-void force_part(int stage, bool energy, const AtomArrays &A, const ListView &Lv,
-                const PairView &P, const Box &box, const StepCoef &c, const ReduceBuf &R,
-                hipStream_t s) {
-    launch_force_k<D, KIND, PREC>(stage, energy, A, Lv, P, box, c, R, s);
+hipError_t force_part(int stage, bool energy, const AtomArrays &A, const ListView &Lv,
+                      const PairView &P, const Box &box, const StepCoef &c,
+                      const ReduceBuf &R, hipStream_t s) {
+    return launch_force_k<D, KIND, PREC>(stage, energy, A, Lv, P, box, c, R, s);
 }
-template void force_part<PARM_PART_D, PARM_PART_KIND, PARM_PART_PREC>(
+template hipError_t force_part<PARM_PART_D, PARM_PART_KIND, PARM_PART_PREC>(
     int, bool, const AtomArrays &, const ListView &, const PairView &, const Box &,
     const StepCoef &, const ReduceBuf &, hipStream_t);
 

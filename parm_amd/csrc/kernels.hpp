@@ -266,12 +266,13 @@ size_t tiled_force_lds(int ndim, int prec, int kind, int ntypes, int smax);
 // The force launches of one dimension, pair kind and precision: over the
 // untiled list (force.hip) and the tiled one (step_tiled.hip).
 template <int D, int KIND, int PREC>
-void force_part(int stage, bool energy, const AtomArrays &A, const ListView &Lv,
-                const PairView &P, const Box &box, const StepCoef &c, const ReduceBuf &R,
-                hipStream_t s);
+hipError_t force_part(int stage, bool energy, const AtomArrays &A, const ListView &Lv,
+                      const PairView &P, const Box &box, const StepCoef &c,
+                      const ReduceBuf &R, hipStream_t s);
 template <int D, int KIND, int PREC>
-void force_tiled_part(int stage, const AtomArrays &A, const ListView &Lv, const PairView &P,
-                      const Box &box, const StepCoef &c, const ReduceBuf &R, hipStream_t s);
+hipError_t force_tiled_part(int stage, const AtomArrays &A, const ListView &Lv,
+                            const PairView &P, const Box &box, const StepCoef &c,
+                            const ReduceBuf &R, hipStream_t s);
 // The sums over nparts workgroup partials (and with top the top-2 fields).
 hipError_t launch_finalize_sums(bool top, int nparts, const ReduceBuf &R, hipStream_t s);
 // The drift leaves its skin-test partials (reduce_blocks(n) of them) to the

@@ -430,15 +430,14 @@ hipError_t launch_force(int ndim, int precision, int stage, bool energy,
     if (A.n <= 0) return hipSuccess;
     if (Lv.tiled && Lv.built) {
         if (Lv.ntiles <= 0) return hipSuccess;
-#define PARM_F(D, K, Q) force_tiled_part<D, K, Q>(stage, A, Lv, P, box, c, R, s)
+#define PARM_F(D, K, Q) return force_tiled_part<D, K, Q>(stage, A, Lv, P, box, c, R, s)
         PARM_DISPATCH(PARM_F);
 #undef PARM_F
     } else {
-#define PARM_F(D, K, Q) force_part<D, K, Q>(stage, energy, A, Lv, P, box, c, R, s)
+#define PARM_F(D, K, Q) return force_part<D, K, Q>(stage, energy, A, Lv, P, box, c, R, s)
         PARM_DISPATCH(PARM_F);
 #undef PARM_F
     }
-    return hipGetLastError();
 }
 
 hipError_t launch_drift(int ndim, int stage, const AtomArrays &A, const StepCoef &c,

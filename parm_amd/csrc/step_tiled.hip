@@ -688,8 +688,8 @@ __global__ __launch_bounds__(kWave *TPA) void k_force_tiled(AtomArrays A, ListVi
 namespace {
 
 template <int D, int KIND, int PREC, bool SINGLE, bool HARM, int STAGE, int TPA>
-void tiled_tt(const AtomArrays &A, const ListView &Lv, const PairView &P, const Box &box,
-              const StepCoef &c, const ReduceBuf &R, hipStream_t s) {
+hipError_t tiled_tt(const AtomArrays &A, const ListView &Lv, const PairView &P,
+                    const Box &box, const StepCoef &c, const ReduceBuf &R, hipStream_t s) {
     constexpr bool DRIFT =
         (STAGE == kStageVerletKickDrift || STAGE == kStageDampedKickDrift);
     constexpr bool ENERGY = STAGE == kStageSums || STAGE == kStageNlcg;
@@ -698,37 +698,35 @@ void tiled_tt(const AtomArrays &A, const ListView &Lv, const PairView &P, const 
     const int nb = Lv.ntiles + (STEP && R.g.nprev > 0 ? 1 : 0);
     hipLaunchKernelGGL((k_force_tiled<D, KIND, PREC, SINGLE, HARM, STAGE, TPA>),
                        dim3(nb), dim3(kWave * TPA), lds, s, A, Lv, P, box, c, R);
+    // (before any other call: the next one's outcome would take its place)
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
     if (R.done) (void)hipEventRecord(R.done, s);
-    if (ENERGY) (void)launch_finalize_sums(false, Lv.ntiles, R, s);
+    return ENERGY ? launch_finalize_sums(false, Lv.ntiles, R, s) : hipSuccess;
 }
 
 template <int D, int KIND, int PREC, bool SINGLE, bool HARM, int STAGE>
-void tiled_t(const AtomArrays &A, const ListView &Lv, const PairView &P, const Box &box,
-             const StepCoef &c, const ReduceBuf &R, hipStream_t s) {
+hipError_t tiled_t(const AtomArrays &A, const ListView &Lv, const PairView &P, const Box &box,
+                   const StepCoef &c, const ReduceBuf &R, hipStream_t s) {
     switch (Lv.tpa) {
     case 1:
-        tiled_tt<D, KIND, PREC, SINGLE, HARM, STAGE, 1>(A, Lv, P, box, c, R, s);
-        break;
+        return tiled_tt<D, KIND, PREC, SINGLE, HARM, STAGE, 1>(A, Lv, P, box, c, R, s);
     case 2:
-        tiled_tt<D, KIND, PREC, SINGLE, HARM, STAGE, 2>(A, Lv, P, box, c, R, s);
-        break;
+        return tiled_tt<D, KIND, PREC, SINGLE, HARM, STAGE, 2>(A, Lv, P, box, c, R, s);
     case 8:
-        tiled_tt<D, KIND, PREC, SINGLE, HARM, STAGE, 8>(A, Lv, P, box, c, R, s);
-        break;
+        return tiled_tt<D, KIND, PREC, SINGLE, HARM, STAGE, 8>(A, Lv, P, box, c, R, s);
     default:
-        tiled_tt<D, KIND, PREC, SINGLE, HARM, STAGE, 4>(A, Lv, P, box, c, R, s);
-        break;
+        return tiled_tt<D, KIND, PREC, SINGLE, HARM, STAGE, 4>(A, Lv, P, box, c, R, s);
     }
 }
 
 template <int D, int KIND, int PREC, bool SINGLE, bool HARM>
-void tiled_s(int stage, const AtomArrays &A, const ListView &Lv, const PairView &P,
-             const Box &box, const StepCoef &c, const ReduceBuf &R, hipStream_t s) {
+hipError_t tiled_s(int stage, const AtomArrays &A, const ListView &Lv, const PairView &P,
+                   const Box &box, const StepCoef &c, const ReduceBuf &R, hipStream_t s) {
     switch (stage) {
-#define PARM_TSTAGE(S)                                                    \
-    case S:                                                               \
-        tiled_t<D, KIND, PREC, SINGLE, HARM, S>(A, Lv, P, box, c, R, s); \
-        break;
+#define PARM_TSTAGE(S) \
+    case S:            \
+        return tiled_t<D, KIND, PREC, SINGLE, HARM, S>(A, Lv, P, box, c, R, s);
         PARM_TSTAGE(kStageForceOnly)
         PARM_TSTAGE(kStageForceA)
         PARM_TSTAGE(kStageVerletKick)
@@ -740,24 +738,20 @@ void tiled_s(int stage, const AtomArrays &A, const ListView &Lv, const PairView 
         PARM_TSTAGE(kStageNlcg)
 #undef PARM_TSTAGE
     }
+    return hipErrorInvalidValue;
 }
 
 template <int D, int KIND, int PREC>
-void tiled_k(int stage, const AtomArrays &A, const ListView &Lv, const PairView &P,
-             const Box &box, const StepCoef &c, const ReduceBuf &R, hipStream_t s) {
+hipError_t tiled_k(int stage, const AtomArrays &A, const ListView &Lv, const PairView &P,
+                   const Box &box, const StepCoef &c, const ReduceBuf &R, hipStream_t s) {
     if constexpr (KIND == kPairRepulsion) {
         if (P.harmonic) {
-            if (P.single)
-                tiled_s<D, KIND, PREC, true, true>(stage, A, Lv, P, box, c, R, s);
-            else
-                tiled_s<D, KIND, PREC, false, true>(stage, A, Lv, P, box, c, R, s);
-            return;
+            return P.single ? tiled_s<D, KIND, PREC, true, true>(stage, A, Lv, P, box, c, R, s)
+                            : tiled_s<D, KIND, PREC, false, true>(stage, A, Lv, P, box, c, R, s);
         }
     }
-    if (P.single)
-        tiled_s<D, KIND, PREC, true, false>(stage, A, Lv, P, box, c, R, s);
-    else
-        tiled_s<D, KIND, PREC, false, false>(stage, A, Lv, P, box, c, R, s);
+    return P.single ? tiled_s<D, KIND, PREC, true, false>(stage, A, Lv, P, box, c, R, s)
+                    : tiled_s<D, KIND, PREC, false, false>(stage, A, Lv, P, box, c, R, s);
 }
 
 }  // namespace
@@ -765,11 +759,12 @@ void tiled_k(int stage, const AtomArrays &A, const ListView &Lv, const PairView 
 // One dimension, pair kind and precision per object file (PARM_PART, set by
 // the Makefile), so that the instantiations compile side by side.
 template <int D, int KIND, int PREC>
-void force_tiled_part(int stage, const AtomArrays &A, const ListView &Lv, const PairView &P,
-                      const Box &box, const StepCoef &c, const ReduceBuf &R, hipStream_t s) {
-    tiled_k<D, KIND, PREC>(stage, A, Lv, P, box, c, R, s);
+hipError_t force_tiled_part(int stage, const AtomArrays &A, const ListView &Lv,
+                            const PairView &P, const Box &box, const StepCoef &c,
+                            const ReduceBuf &R, hipStream_t s) {
+    return tiled_k<D, KIND, PREC>(stage, A, Lv, P, box, c, R, s);
 }
-template void force_tiled_part<PARM_PART_D, PARM_PART_KIND, PARM_PART_PREC>(
+template hipError_t force_tiled_part<PARM_PART_D, PARM_PART_KIND, PARM_PART_PREC>(
     int, const AtomArrays &, const ListView &, const PairView &, const Box &, const StepCoef &,
     const ReduceBuf &, hipStream_t);
 

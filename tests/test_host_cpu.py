@@ -214,6 +214,27 @@ def test_refused_list_nlcg(runtime):
     _child(runtime, "case_refused_list_nlcg")
 
 
+# a refused launch whose sums the host would read: the error of the force kernel is
+# not lost in the launch of its reduction
+def case_refused_sums_launch(hh, what):
+    from parm_amd import capi
+    s = _system()
+    s.update_list(True)
+    s.set_forces()
+    c = capi.NLCG(s, 0.1, 1e-3) if what == "nlcg" else None
+    hh.hh_refuse("7k_force" if os.environ["PARM_TILED"] == "0" else "k_force_tiled")
+    _refused(DEVICE, s.pair_sums if what == "sums" else c.timestep)
+    hh.hh_refuse("")
+    (s.pair_sums if what == "sums" else c.timestep)()
+    s.close()
+
+
+@pytest.mark.parametrize("tiled", ["0", "1"])
+@pytest.mark.parametrize("what", ["sums", "nlcg"])
+def test_refused_sums_launch(runtime, what, tiled):
+    _child(runtime, "case_refused_sums_launch", what, PARM_TILED=tiled, PARM_TPA="4")
+
+
 if __name__ == "__main__":
     sys.path.insert(0, ROOT)
     hh = C.CDLL(sys.argv[1], mode=C.RTLD_GLOBAL)
