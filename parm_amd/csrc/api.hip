@@ -235,6 +235,7 @@ struct parm_system {
         L.ntiles = ntiles;
         L.smax = smax;
         L.wcap = tpa > 0 ? cap / tpa : 0;
+        L.lds_max = lds_max;
         L.tiles = tiles;
         L.truns = truns;
         L.keys = keys;

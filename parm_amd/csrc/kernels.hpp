@@ -179,6 +179,7 @@ struct ListView {
     int ntiles;            // tiles = workgroups of a tiled force launch
     int smax;              // largest staged stencil of any tile
     int wcap;              // 32-bit words per lane the list array holds (cap / tpa)
+    size_t lds_max;        // dynamic LDS that a tiled launch may take
     const int4 *tiles;
     const int2 *truns;     // kTileRuns runs per tile (tiles.hpp)
     const uint32_t *keys;  // sorted cell keys of the last rebuild
@@ -259,9 +260,9 @@ hipError_t launch_force(int ndim, int precision, int stage, bool energy,
                         const AtomArrays &A, const ListView &Lv, const PairView &P,
                         const Box &box, const StepCoef &c, const ReduceBuf &R,
                         hipStream_t s);
-// Dynamic LDS of the tiled force kernel for a stencil of smax staged slots
-// (dimension, precision, pair kind, pair types; no pair kind yet gets the
-// largest staging).
+// Dynamic LDS that the tiled force kernel cannot do without for a stencil of
+// smax staged slots (dimension, precision, pair kind, pair types; no pair kind
+// yet gets the largest staging).  A pair table in LDS comes on top where it fits.
 size_t tiled_force_lds(int ndim, int prec, int kind, int ntypes, int smax);
 // The force launches of one dimension, pair kind and precision: over the
 // untiled list (force.hip) and the tiled one (step_tiled.hip).

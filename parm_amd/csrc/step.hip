@@ -393,11 +393,10 @@ size_t tiled_force_lds(int ndim, int prec, int kind, int ntypes, int smax) {
     const bool raw = prec == kFP64 && kind == kPairRepulsion;
     if (raw) return (size_t)smax * sizeof(double4);
     if (kind == kPairLJ) {
-        // (lj_slots_bytes in step_tiled.hip) + table + type bytes
+        // (lj_slots_bytes in step_tiled.hip) + type bytes
         const size_t real = prec == kFP64 ? sizeof(double) : sizeof(float);
-        size_t b = ((size_t)(smax + 1) * ndim * real + 15) & ~(size_t)15;
-        if (ntypes > 1) b += (size_t)ntypes * ntypes * 4 * real + (size_t)smax + 1;
-        return b;
+        const size_t b = ((size_t)(smax + 1) * ndim * real + 15) & ~(size_t)15;
+        return ntypes > 1 ? b + (size_t)smax + 1 : b;
     }
     if (ntypes == 1 && kind != kPairNone) return (size_t)smax * ndim * sizeof(double);
     return (size_t)smax * (sizeof(double4) + sizeof(int32_t));

@@ -128,7 +128,7 @@ constexpr int kChunkWords = 4;
 constexpr int kGroup = 4;
 static_assert(kChunkWords % (kGroup / 2) == 0, "groups tile a chunk");
 
-// One row of the LJ pair table in LDS (several types).
+// One row of the LJ pair table (several types).
 template <int PREC>
 struct LjRow;
 template <>
@@ -148,13 +148,21 @@ struct LjRow<kMixed> {
 
 // Dynamic LDS of the LJ staging, in this order: smax + 1 slots of D offsets
 // (the last one a stand-in for entries past a lane's count: see the pair
-// loop), then with several types the pair table and a type byte per slot.
+// loop), then with several types the pair table (TABLDS) and a type byte per
+// slot.
 template <int D, int PREC>
 __host__ __device__ constexpr size_t lj_slots_bytes(int smax) {
     return (((size_t)(smax + 1) * D * (PREC == kFP64 ? 8 : 4)) + 15) & ~(size_t)15;
 }
 
-template <int D, int KIND, int PREC, bool SINGLE, bool HARM, int STAGE, int TPA>
+// TABLDS (LJ of several types, force stages): the pair table is copied to LDS;
+// otherwise a pair's row comes from memory.  LDS is the faster as long as it has
+// room for the table beside the stencil (up to about 24 types in FP64, 45 in
+// FP32), and at that size both take the same: 262,144 atoms of 8 / 20 / 24 types
+// in FP64 68.7 / 73.3 / 90.7 us per launch from LDS, 75.0 / 85.8 / 90.1 from
+// memory; 28 / 32 / 64 types from memory 98 / 103 / 132, where the untiled list
+// takes 168 / 173 / 201.
+template <int D, int KIND, int PREC, bool SINGLE, bool HARM, int STAGE, int TPA, bool TABLDS>
 __global__ __launch_bounds__(kWave *TPA) void k_force_tiled(AtomArrays A, ListView Lv,
                                                             PairView P, Box box, StepCoef c,
                                                             ReduceBuf R) {
@@ -180,7 +188,8 @@ __global__ __launch_bounds__(kWave *TPA) void k_force_tiled(AtomArrays A, ListVi
     Real *stc = reinterpret_cast<Real *>(st64);
     LjRow<PREC> *ljtab = reinterpret_cast<LjRow<PREC> *>(reinterpret_cast<char *>(st64) +
                                                          lj_slots_bytes<D, PREC>(Lv.smax));
-    uint8_t *ljtype = reinterpret_cast<uint8_t *>(ljtab + (size_t)P.ntypes * P.ntypes);
+    uint8_t *ljtype = reinterpret_cast<uint8_t *>(
+        ljtab + (TABLDS ? (size_t)P.ntypes * P.ntypes : (size_t)0));
     int32_t *stj = REL32 ? reinterpret_cast<int32_t *>(st32 + Lv.smax)
                          : reinterpret_cast<int32_t *>(st64 + Lv.smax);
 
@@ -240,8 +249,9 @@ __global__ __launch_bounds__(kWave *TPA) void k_force_tiled(AtomArrays A, ListVi
         if (threadIdx.x < D) stc[(size_t)Lv.smax * D + threadIdx.x] = (Real)(REL32 ? 1e18 : 1e150);
         if constexpr (!SINGLE) {
             if (threadIdx.x == 0) ljtype[Lv.smax] = 0;
-            for (int q = threadIdx.x; q < P.ntypes * P.ntypes; q += NT)
-                ljtab[q] = LjRow<PREC>::make(P.tab[q]);
+            if constexpr (TABLDS)
+                for (int q = threadIdx.x; q < P.ntypes * P.ntypes; q += NT)
+                    ljtab[q] = LjRow<PREC>::make(P.tab[q]);
         }
     }
     // the tile origin, its middle atom (offsets half as large, and rounded
@@ -517,8 +527,10 @@ __global__ __launch_bounds__(kWave *TPA) void k_force_tiled(AtomArrays A, ListVi
         auto ljrow = [&](int s) {
             if constexpr (SINGLE)
                 return LjRow<PREC>::make(p0);
-            else
+            else if constexpr (TABLDS)
                 return ljtab[ti + ljtype[s]];
+            else
+                return LjRow<PREC>::make(prow[ljtype[s]]);
         };
         auto ljfs = [&](const LjRow<PREC> &q, Real d2) {
             if constexpr (PREC == kFP64) {
@@ -693,11 +705,20 @@ hipError_t tiled_tt(const AtomArrays &A, const ListView &Lv, const PairView &P,
     constexpr bool DRIFT =
         (STAGE == kStageVerletKickDrift || STAGE == kStageDampedKickDrift);
     constexpr bool ENERGY = STAGE == kStageSums || STAGE == kStageNlcg;
-    const size_t lds = tiled_force_lds(D, PREC, KIND, P.ntypes, Lv.smax);
     constexpr bool STEP = DRIFT || STAGE == kStageVerletKick || STAGE == kStageDampedKick;
-    const int nb = Lv.ntiles + (STEP && R.g.nprev > 0 ? 1 : 0);
-    hipLaunchKernelGGL((k_force_tiled<D, KIND, PREC, SINGLE, HARM, STAGE, TPA>),
-                       dim3(nb), dim3(kWave * TPA), lds, s, A, Lv, P, box, c, R);
+    const size_t lds = tiled_force_lds(D, PREC, KIND, P.ntypes, Lv.smax);
+    const dim3 g(Lv.ntiles + (STEP && R.g.nprev > 0 ? 1 : 0)), b(kWave * TPA);
+    bool tab = false;
+    if constexpr (KIND == kPairLJ && !SINGLE && !ENERGY) {
+        const size_t bytes = (size_t)P.ntypes * P.ntypes * sizeof(LjRow<PREC>);
+        tab = lds + bytes <= Lv.lds_max;
+        if (tab)
+            hipLaunchKernelGGL((k_force_tiled<D, KIND, PREC, SINGLE, HARM, STAGE, TPA, true>), g,
+                               b, lds + bytes, s, A, Lv, P, box, c, R);
+    }
+    if (!tab)
+        hipLaunchKernelGGL((k_force_tiled<D, KIND, PREC, SINGLE, HARM, STAGE, TPA, false>), g, b,
+                           lds, s, A, Lv, P, box, c, R);
     // (before any other call: the next one's outcome would take its place)
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;

@@ -205,6 +205,56 @@ def test_tiled_lj_group_edges(monkeypatch, tpa, ntypes, n):
     s.close()
 
 
+# LJ of so many types that LDS has no room for their table beside the stencil
+# (FP64: from about 25 on, mixed: 45): the tiled list all the same, rows from memory
+@pytest.mark.parametrize("prec", [capi.FP64, capi.MIXED])
+@pytest.mark.parametrize("ndim,n,tpa", [(3, 500, 4), (3, 6000, 8), (2, 3000, 1)])
+@pytest.mark.parametrize("ntypes", [20, 33, 64])
+def test_tiled_lj_many_types(monkeypatch, ntypes, ndim, n, tpa, prec):
+    _device_or_fail()
+    print(f"tiled lj ntypes={ntypes} ndim={ndim} n={n} tpa={tpa} prec={prec}", flush=True)
+    monkeypatch.setenv("PARM_TPA", str(tpa))
+    monkeypatch.setenv("PARM_TILED", "1")
+    x, L = S.jittered_lattice(n, 0.75, ndim, seed=n + ntypes)
+    rng = np.random.default_rng(ntypes)
+    types = rng.integers(0, ntypes, n).astype(np.int32)
+    types[:ntypes] = np.arange(ntypes)
+    eps = rng.uniform(0.5, 1.5, (ntypes, ntypes))
+    eps = (eps + eps.T) / 2
+    sigma = rng.uniform(0.8, 1.0, ntypes)
+    cut = rng.uniform(1.5, 2.2, ntypes)
+    diam = (sigma * cut)[types]
+    t = O.PairTable(O.LJ_ATTRACT_REPULSE, eps, sigma, cut, types)
+    v = S.gaussian_velocities(n, ndim, 0.5, seed=n)
+    s = capi.System(ndim, np.ones(n), prec)
+    s.set_box(L)
+    s.nlist_set(0.3, diam)
+    s.set_lj(eps, sigma, cut, types)
+    s.set_state(x=x, v=v, a=np.zeros_like(x))
+    s.update_list(True)
+    s.set_forces(False)
+    assert s.list_info()["tiled"]
+    first, last = O.nlist(x, L, diam, 0.3)
+    ref = O.forces(x, L, t, first, last)
+    u = s.pair_sums()["U"]
+    if prec == capi.FP64:
+        S.assert_fp64_forces(s.forces(), ref, x, L, t, first, last)
+        assert abs(u - ref["U"]) <= 1e-12 * max(1.0, abs(ref["U"]))
+        r = O.System(np.ones(n), L, t, diam, 0.3, ndim=ndim, brute=False)
+        r.set_state(x=x, v=v, a=np.zeros_like(x))
+        for q in (r, s):
+            q.initialize()
+            q.verlet(0.001, 5)
+        assert np.abs(s.positions() - r.state()[0]).max() <= 1e-12 * max(1.0, np.abs(x).max())
+    else:
+        # two offsets of up to ~10 sigma rounded to FP32 (half an ulp: 5e-7 each)
+        # move a pair force by 14 |dr| / r = 1.6e-5 of its terms; three times that
+        scale = S.pair_term_scale(x, L, t, first, last)
+        d = np.sqrt(((s.forces() - ref["f"]) ** 2).sum(1))
+        assert np.all(d <= 5e-5 * scale + 1e-12)
+    s.close()
+
+
 # 16 and 32 lanes per atom: rows shorter than the lanes, rows of more than the
 # entries in flight per lane, both pair kinds, the largest system of either
 @pytest.mark.parametrize("lanes,n", [(16, 2), (16, 700), (16, 1 << 14), (32, 2), (32, 700),
