@@ -886,6 +886,7 @@ int autotune(parm_system *s, int stage, const StepCoef &c) {
             s->tpa = cands[0].second;
             PARM_CHECK(relayout(s));
         }
+        if (coarse) s->layout_pref = 2;  // for the rebuilds to come as well
         s->tuned = true;
         return PARM_OK;
     }

@@ -235,6 +235,30 @@ def test_refused_sums_launch(runtime, what, tiled):
     _child(runtime, "case_refused_sums_launch", what, PARM_TILED=tiled, PARM_TPA="4")
 
 
+# lanes given, layout by rule (mixed LJ of few atoms: untiled): the rule holds for
+# the rebuilds after the tuning too
+def case_tuned_layout_stays(hh):
+    from parm_amd import capi
+    n = 2000
+    s = capi.System(3, np.ones(n), capi.MIXED)
+    s.set_box([14.0] * 3)
+    s.nlist_set(0.3, np.full(n, 2.5))
+    s.set_lj([[1.0]], [1.0], [2.5], np.zeros(n, np.int32))
+    s.set_state(x=np.random.default_rng(0).uniform(0, 14, (n, 3)))
+    s.update_list(True)
+    assert s.list_info()["tiled"]
+    s.verlet(0.001, 16)
+    assert not s.list_info()["tiled"]
+    s.update_list(True)
+    assert not s.list_info()["tiled"]
+    s.close()
+
+
+@pytest.mark.parametrize("tpa", ["", "4"])
+def test_tuned_layout_stays(runtime, tpa):
+    _child(runtime, "case_tuned_layout_stays", PARM_TPA=tpa)
+
+
 if __name__ == "__main__":
     sys.path.insert(0, ROOT)
     hh = C.CDLL(sys.argv[1], mode=C.RTLD_GLOBAL)
