@@ -84,7 +84,9 @@ constexpr int kFlagRing = 4;
 // flag, the on-demand skin test, and the verdict on a list build
 // dynamic LDS of one tiled build workgroup, at most (the stencil's atoms)
 constexpr size_t kTiledLdsMax = 56 * 1024;
-constexpr int kMixedUntiledAtoms = 1 << 15, kMixedRepulsionFixed = 100000;  // autotune
+// limits of the autotuner's rules (autotune)
+constexpr int kMixedUntiledAtoms = 1 << 15;
+constexpr int kMixedRepulsionFixed = 100000, kMixedRepulsionRow = 16;
 // run-ahead of the step loop (step_runahead)
 constexpr int kRunAhead = 2, kRunAheadAtoms = 1 << 15;
 static_assert(kRunAhead + 1 < kFlagRing, "a flag word is not reused while a launch may read it");
@@ -850,9 +852,12 @@ int autotune(parm_system *s, int stage, const StepCoef &c) {
     std::vector<std::pair<int, int>> cands;  // (tiled, tpa)
     std::vector<int> layouts;
     const bool tiled_ok = s->tile_ok && tiled_force_fits(s);
-    // (mixed-precision LJ: the tiled list's FP32 offsets cost precision, the
-    // error of a 10,007-atom trajectory is 4.6e-7 against 1e-7 untiled, and
-    // at such sizes gain nothing: 1685 against 1706 us per 100 steps)
+    // Mixed-precision LJ of few atoms keeps the untiled list for its precision: the
+    // tiled one's FP32 offsets cost some (the error of a 10,007-atom trajectory is
+    // 4.6e-7 against 1e-7).  Up to 16,000 atoms that costs no time (step launch
+    // untiled / tiled at 4,000, 8,000, 16,000 atoms: 8.4 / 11.0, 9.4 / 11.2, 11.7 /
+    // 12.8 us), to the limit up to a sixth (24,000: 14.2 / 13.0, 32,000: 16.6 /
+    // 14.2), beyond it more (48,000: 20.5 / 15.9).
     const bool coarse = s->prec == kMixed && s->pair_kind == kPairLJ && s->layout_pref == 0 &&
                         s->n <= kMixedUntiledAtoms;
     if (tiled_ok && s->layout_pref != 2 && !coarse) layouts.push_back(1);
@@ -869,14 +874,19 @@ int autotune(parm_system *s, int stage, const StepCoef &c) {
                 cands.emplace_back(lay, tpa);
         }
     }
-    // Mixed-precision repulsion of many atoms: only the candidates that add
-    // an atom's pair forces in the same order (one lane untiled keeps a lane
-    // pair's two sums: force.hip).  They are the fastest there and race within
-    // a few per cent, so the pick differs from run to run, and a relaxation
-    // from random positions amplifies another order of the FP32 sums (1e-3 in
-    // single velocities after 200 steps of 262,144 disks).
+    // Mixed-precision repulsion of many atoms in short rows: only the candidates
+    // that add an atom's pair forces in the same order (one lane untiled keeps a
+    // lane pair's two sums: force.hip).  They are the fastest there and race
+    // within a few per cent, so the pick differs from run to run, and a
+    // relaxation from random positions amplifies another order of the FP32 sums
+    // (1e-3 in single velocities after 200 steps of 262,144 disks).  The step
+    // launch with the best of them / of all, 100,000 - 600,000 disks and spheres:
+    // equal for rows of 4 to 11 entries (at most 18.4 / 18.0 us), 39.6 / 38.3 at
+    // 23; at 29 31.2 / 27.1 (100,000 spheres) and 60.5 / 56.9 (262,144), at 90
+    // 67.0 / 53.1 and 131 / 126: long rows have the whole choice.
     if (s->prec == kMixed && s->pair_kind == kPairRepulsion && s->n >= kMixedRepulsionFixed &&
-        s->layout_pref == 0 && !s->tpa_fixed) {
+        2 * s->npairs <= (int64_t)kMixedRepulsionRow * s->n && s->layout_pref == 0 &&
+        !s->tpa_fixed) {
         cands = {{0, 1}, {0, 2}};
         if (tiled_ok) cands.emplace_back(1, 2);
     }

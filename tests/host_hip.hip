@@ -32,6 +32,7 @@ bool g_capturing = false;
 hipError_t g_last = hipSuccess;
 std::deque<uint32_t> g_flags;         // of the next skin tests
 std::deque<unsigned long long> g_max; // fullest rows of the next list builds
+unsigned long long g_entries = 2;     // entries of every list built
 
 struct Config {
     dim3 grid, block;
@@ -94,7 +95,7 @@ void run(const std::string &name, void **a) {
             g_max.pop_front();
         }
         if (r) {
-            r->sum = 2;
+            r->sum = g_entries;
             r->max = mx;
             r->flag = 0;
             r->ntiles = arg<const int *>(a, 5) ? 1 : 0;
@@ -155,6 +156,7 @@ void hh_reset() {
     g_refuse.clear();
     g_graphs = g_bad = g_overflows = g_fail_in = 0;
     g_last = hipSuccess;
+    g_entries = 2;
     g_flags.clear();
     g_max.clear();
 }
@@ -163,6 +165,7 @@ void hh_fail_at(int k) { g_fail_in = k; }  // the k-th allocation from here
 void hh_refuse(const char *kernel) { g_refuse = kernel; }
 void hh_flag(uint32_t f) { g_flags.push_back(f); }
 void hh_row(unsigned long long m) { g_max.push_back(m); }
+void hh_entries(unsigned long long m) { g_entries = m; }
 void hh_overflows(int n) { g_overflows = n; }
 int hh_graphs() { return g_graphs; }
 int hh_bad() { return g_bad; }

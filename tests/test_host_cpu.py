@@ -259,12 +259,37 @@ def test_tuned_layout_stays(runtime, tpa):
     _child(runtime, "case_tuned_layout_stays", PARM_TPA=tpa)
 
 
+# mixed repulsion of many atoms: the candidates that add up alike, unless rows
+# are long, where more lanes are the faster
+def case_repulsion_candidates(hh, row):
+    from parm_amd import capi
+    n = 100000
+    s = capi.System(3, np.ones(n), capi.MIXED)
+    s.set_box([60.0] * 3)
+    s.nlist_set(0.3, np.ones(n))
+    s.set_repulsion([1.0], [1.0], [2.0], np.zeros(n, np.int32))
+    s.set_state(x=np.random.default_rng(0).uniform(0, 60, (n, 3)))
+    hh.hh_entries(int(row) * n)
+    s.update_list(True)
+    _log(hh)
+    s.autotune(0.001)
+    lanes = {int(k.split("EEEv")[0].split("ELi")[-1]) for k in _log(hh).split()
+             if "7k_forceI" in k}
+    assert lanes == ({1, 2} if int(row) <= 16 else {1, 2, 4, 8}), lanes
+    s.close()
+
+
+@pytest.mark.parametrize("row", [6, 16, 17, 90])
+def test_repulsion_candidates(runtime, row):
+    _child(runtime, "case_repulsion_candidates", row)
+
+
 if __name__ == "__main__":
     sys.path.insert(0, ROOT)
     hh = C.CDLL(sys.argv[1], mode=C.RTLD_GLOBAL)
     hh.hh_log.restype = C.c_char_p
     hh.hh_alloc_limit.argtypes = [C.c_size_t]
-    hh.hh_row.argtypes = [C.c_ulonglong]
+    hh.hh_row.argtypes = hh.hh_entries.argtypes = [C.c_ulonglong]
     from parm_amd import capi
     assert capi.device_count() == 1 and hh.hh_bad() == 0
     globals()[sys.argv[2]](hh, *sys.argv[3:])
