@@ -724,8 +724,12 @@ __global__ __launch_bounds__(kBlock) void k_build_list(
 // of dependent loads bounds it, so a workgroup takes one row until there are
 // more than kPlanGroups of them (1,521 rows at 1M atoms: eight rows each 32
 // us, one 10 us; as two launches, one workgroup laying out the rows and a
-// thread per tile, 26 us).
-constexpr int kPlanMaxRows = 64, kPlanGroups = 2048, kPlanLanes = 32;
+// thread per tile, 26 us).  Past kPlanManyRows (slabs of short rows) the counting
+// of the rows before, which grows with the square of the rows over `per`, is the
+// larger part: there are fewer workgroups then, of up to kBlock rows (a rebuild of
+// 1M spheres in a slab of 175,000 rows: 64 rows each 1450 us, 85 1393, 256 1348).
+constexpr int kPlanMaxRows = kBlock, kPlanGroups = 2048, kPlanLanes = 32;
+constexpr int kPlanManyRows = 64 * kPlanGroups, kPlanFewGroups = 512;
 static_assert(kPlanLanes >= kTileRuns, "a lane per run");
 
 __device__ __forceinline__ int row_tiles(const int32_t *cstart, int r, int nc0) {
@@ -746,21 +750,16 @@ __global__ __launch_bounds__(kBlock) void k_tile_plan(
     (void)block_excl_scan_u32<kBlock>(v, base);
     const int m0 = cstart[g.ncell];
     const int ntail = lastb ? (n - m0 + kTileAtoms - 1) / kTileAtoms : 0;
-    if ((int)threadIdx.x < per)
-        first[threadIdx.x] =
-            r0 + (int)threadIdx.x < r1 ? row_tiles(cstart, r0 + (int)threadIdx.x, nc0) : 0;
-    __syncthreads();
+    const int mine = r0 + (int)threadIdx.x < r1;  // a row per thread (per <= kBlock)
+    uint32_t t = 0;
+    const uint32_t at0 = block_excl_scan_u32<kBlock>(
+        mine ? (uint32_t)row_tiles(cstart, r0 + (int)threadIdx.x, nc0) : 0u, t);
+    if ((int)threadIdx.x < per) first[threadIdx.x] = (int)at0;
     if (threadIdx.x == 0) {
-        int t = 0;
-        for (int q = 0; q < per; q++) {
-            const int c = first[q];
-            first[q] = t;
-            t += c;
-        }
-        first[per] = t;
-        first[per + 1] = t + ntail;
+        first[per] = (int)t;
+        first[per + 1] = (int)t + ntail;
         if (lastb) {
-            const int nt = (int)base + t + ntail;
+            const int nt = (int)(base + t) + ntail;
             info[0] = nt <= cap_tiles ? nt : 0;
             if (nt > cap_tiles) info[2] = 1;
         }
@@ -774,8 +773,15 @@ __global__ __launch_bounds__(kBlock) void k_tile_plan(
         TileRec T;
         int g0 = 0, len = 0, wide = 0;
         if (q < rowt) {
-            int r = r0;
-            while (first[r - r0 + 1] <= q) r++;
+            int lo = 0, hi = per;  // the last row whose first tile is <= q
+            while (hi - lo > 1) {
+                const int mid = (lo + hi) >> 1;
+                if (first[mid] <= q)
+                    lo = mid;
+                else
+                    hi = mid;
+            }
+            const int r = r0 + lo;
             const int a = cstart[r * nc0], cnt = cstart[(r + 1) * nc0] - a;
             const int at = (q - first[r - r0]) * kTileAtoms;
             T = TileRec{a + at, min(kTileAtoms, cnt - at), r, 0};
@@ -1572,7 +1578,8 @@ hipError_t launch_tiles(int ndim, int n, const CellGrid &g, const uint32_t *keys
                         const int32_t *cstart, int cap_tiles, TileRec *tiles, int2 *truns,
                         int *info, hipStream_t s) {
     const int nrows = g.ncell / g.nc[0];
-    const int per = std::min(kPlanMaxRows, std::max(1, nrows / kPlanGroups));
+    const int per = nrows <= kPlanManyRows ? std::max(1, nrows / kPlanGroups)
+                                           : std::min(kPlanMaxRows, nrows / kPlanFewGroups);
     const int nb = (nrows + per - 1) / per;
     if (ndim == 3)
         hipLaunchKernelGGL(k_tile_plan<3>, dim3(nb), dim3(kBlock), 0, s, n, nrows, per, g, keys,

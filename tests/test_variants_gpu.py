@@ -337,6 +337,30 @@ def test_counted_order_and_tile_plan(n, ndim, edge, clustered):
     s.close()
 
 
+# a slab of more than 131,072 short rows (up to 256 to a plan workgroup): a cubic
+# lattice in random order, whose atoms all have 32 neighbours within the list
+# radius and no net force
+def test_tile_plan_of_many_rows(monkeypatch):
+    _device_or_fail()
+    print("tile plan of many rows", flush=True)
+    monkeypatch.setenv("PARM_TILED", "1")
+    m, a = (7, 812, 812), 1.08
+    n = m[0] * m[1] * m[2]
+    rng = np.random.default_rng(5)
+    x = np.stack(np.unravel_index(rng.permutation(n), m), -1) * a + rng.uniform(-9, 9, 3)
+    s = capi.System(3, np.ones(n))
+    s.set_box(np.array(m) * a)
+    s.nlist_set(0.3, np.full(n, 2.1))
+    s.set_lj([[1.0]], [1.0], [2.1], np.zeros(n, np.int32))
+    s.set_state(x=x)
+    for _ in range(2):
+        s.update_list(True)
+        assert s.list_info()["tiled"] and s.numpairs() == 16 * n
+    s.set_forces(False)
+    assert np.abs(s.forces()).max() <= 1e-10
+    s.close()
+
+
 # the minimiser's sums out of the force launch: fixed atoms (no dot products,
 # a = 0), both list layouts, workgroup edges
 @pytest.mark.parametrize("tiled", ["0", "1"])
