@@ -284,6 +284,24 @@ def test_repulsion_candidates(runtime, row):
     _child(runtime, "case_repulsion_candidates", row)
 
 
+# the most lanes per atom on both sides of the sizes where they change (lanes asked
+# for beyond them leave the default of four)
+def case_most_lanes(hh, n, lanes):
+    s = _system(int(n))
+    s.update_list(True)
+    assert s.list_info()["lanes"] == int(lanes)
+    s.set_forces()
+    s.verlet(0.001, 3)
+    assert hh.hh_bad() == 0
+    s.close()
+
+
+@pytest.mark.parametrize("n,ask,lanes", [(8192, 32, 32), (8193, 32, 4), (8193, 16, 16),
+                                         (16384, 16, 16), (16385, 16, 4), (16385, 8, 8)])
+def test_most_lanes(runtime, n, ask, lanes):
+    _child(runtime, "case_most_lanes", n, lanes, PARM_TPA=str(ask), PARM_TILED="0")
+
+
 if __name__ == "__main__":
     sys.path.insert(0, ROOT)
     hh = C.CDLL(sys.argv[1], mode=C.RTLD_GLOBAL)

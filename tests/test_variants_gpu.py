@@ -301,6 +301,189 @@ def test_wide_untiled_lanes(monkeypatch, lanes, n, lj):
     s.close()
 
 
+# mixed precision with a lane's first entries in flight ahead of the loop (8 lanes
+# and more)
+@pytest.mark.parametrize("lanes,n", [(8, 2), (8, 701), (16, 2), (16, 701), (32, 2), (32, 701),
+                                     (32, 1 << 13)])
+@pytest.mark.parametrize("form", ["lj", "harmonic", "hertz"])
+def test_wide_untiled_lanes_mixed(monkeypatch, lanes, n, form):
+    _device_or_fail()
+    print(f"wide mixed lanes={lanes} n={n} {form}", flush=True)
+    monkeypatch.setenv("PARM_TPA", str(lanes))
+    monkeypatch.setenv("PARM_TILED", "0")
+    x, L = S.jittered_lattice(n, 0.8, 3, seed=n) if n > 2 else (np.array([[0.1, 0, 0], [1.2, 0, 0]]),
+                                                               np.full(3, 6.0))
+    s = capi.System(3, np.ones(n), capi.MIXED)
+    s.set_box(L)
+    if form == "lj":
+        p = S.lj_params(n, sigcut=3.2 if n == 701 else 2.5)
+        t = O.PairTable(O.LJ_ATTRACT_REPULSE, p["eps"], p["sigma"], p["third"], p["types"])
+        s.nlist_set(0.3, p["diam"])
+        s.set_lj(p["eps"], p["sigma"], p["third"], p["types"])
+    else:
+        e = 2.0 if form == "harmonic" else 2.5
+        p = S.bidisperse_repulsion(n, n, exponent=(e, e))
+        t = O.PairTable(O.REPULSION, p["eps"], p["sigma"], p["third"], p["types"])
+        s.nlist_set(0.3, p["diam"])
+        s.set_repulsion(p["eps"], p["sigma"], p["third"], p["types"])
+    s.set_state(x=x)
+    s.update_list(True)
+    s.set_forces(False)
+    assert s.list_info()["lanes"] == lanes
+    first, last = O.nlist(x, L, p["diam"], 0.3)
+    ref = O.forces(x, L, t, first, last)
+    d = np.sqrt(((s.forces() - ref["f"]) ** 2).sum(1))
+    assert np.all(d <= 2e-5 * ref["fabs"] + 1e-6), np.max(d - 2e-5 * ref["fabs"])
+    s.close()
+
+
+# the autotuner's candidates for mixed repulsion of many atoms differ in time only:
+# one lane adds the even and the odd entries apart, as two lanes do
+@pytest.mark.parametrize("ndim,n", [(2, 63), (2, 3001), (3, 2), (3, 1500)])
+@pytest.mark.parametrize("exponent", [2.0, 2.5])
+def test_mixed_repulsion_one_lane_adds_as_two(monkeypatch, ndim, n, exponent):
+    _device_or_fail()
+    print(f"one lane as two ndim={ndim} n={n} exponent={exponent}", flush=True)
+    monkeypatch.setenv("PARM_TILED", "0")
+    rng = np.random.default_rng(n)
+    p = S.bidisperse_repulsion(n, n, exponent=(exponent, exponent))
+    L = np.full(ndim, max(4.5, (0.9 * n) ** (1 / ndim)))
+    x = rng.uniform(0, 1, (n, ndim)) * L
+    v = rng.normal(size=(n, ndim)) * 0.1
+    out = []
+    for tpa in ("1", "2"):
+        monkeypatch.setenv("PARM_TPA", tpa)
+        s = capi.System(ndim, np.ones(n), capi.MIXED)
+        s.set_box(L)
+        s.nlist_set(0.3, p["diam"])
+        s.set_repulsion(p["eps"], p["sigma"], p["third"], p["types"])
+        s.set_state(x=x, v=v, a=np.zeros_like(x))
+        s.initialize()
+        f = s.forces()
+        s.damped(0.02, 0.5, 12)
+        assert s.list_info()["lanes"] == int(tpa)
+        out.append((f, *s.state()))
+        s.close()
+    assert n < 10 or np.abs(out[0][0]).max() > 0
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)
+
+
+# 16 and 32 lanes per atom in a batch: systems smaller than a group, odd sizes
+@pytest.mark.parametrize("prec", [capi.FP64, capi.MIXED])
+@pytest.mark.parametrize("lj", [False, True])
+@pytest.mark.parametrize("lanes", [16, 32])
+def test_batch_wide_lanes(monkeypatch, lanes, lj, prec):
+    _device_or_fail()
+    print(f"batch lanes={lanes} lj={lj} prec={prec}", flush=True)
+    monkeypatch.setenv("PARM_TPA", str(lanes))
+    if lj:
+        systems = []
+        for k, n in enumerate([3, 33, 300, 701]):
+            x, L = S.jittered_lattice(n, 0.5, 3, seed=70 + k)
+            systems.append(dict(n=n, L=float(L[0]), x=x, v=S.gaussian_velocities(n, 3, 0.5, seed=k),
+                                types=np.zeros(n, np.int32), sig=np.ones(n)))
+    else:
+        systems = B.packings([1, 2, 31, 33, 300, 701], 0.64, 3, seed=8)
+    b = B.make_batch(systems, 3, 0.25, prec=prec, lj=lj)
+    refs = B.oracle_systems(systems, 3, 0.25, lj=lj)
+    b.initialize()
+    for s, r in enumerate(refs):
+        r.initialize()
+        fd, ld = b.pairs(s)
+        fr, lr = r.pairs()
+        assert np.array_equal(fd, fr) and np.array_equal(ld, lr), s
+    if prec == capi.FP64:
+        B._compare(b, refs, systems, 1e-12, 0)
+        for q in (b, *refs):
+            q.damped(0.004, 0.5, 10)
+        B._compare(b, refs, systems, 1e-12, 10)
+    else:
+        f, off = b.state()[3], b.offsets
+        for s, (q, r) in enumerate(zip(systems, refs)):
+            t = (O.PairTable(O.LJ_ATTRACT_REPULSE, [[1.0, 1.0], [1.0, 1.0]], [1.0, 1.4],
+                             [2.5, 2.5], q["types"]) if lj else
+                 O.PairTable(O.REPULSION, B.REP["eps"], B.REP["sigma"], B.REP["third"], q["types"]))
+            ref = O.forces(q["x"], [q["L"]] * 3, t, *r.pairs())
+            d = np.sqrt(((f[off[s]:off[s + 1]] - ref["f"]) ** 2).sum(1))
+            assert np.all(d <= 2e-5 * ref["fabs"] + 1e-6), s
+    b.close()
+
+
+# the build of a large sparse 2D system (two lanes of four candidates) with one
+# diameter, and with ignored pairs, for either list
+@pytest.mark.parametrize("tiled", ["0", "1"])
+@pytest.mark.parametrize("one_diameter,ignored", [(True, 0), (True, 3000), (False, 3000)])
+def test_flat_build_variants(monkeypatch, tiled, one_diameter, ignored):
+    _device_or_fail()
+    print(f"flat build tiled={tiled} one={one_diameter} ignored={ignored}", flush=True)
+    monkeypatch.setenv("PARM_TILED", tiled)
+    n, edge = 100003, 270.0  # (dense enough that no tile is wider than its limit)
+    rng = np.random.default_rng(ignored + one_diameter)
+    L = np.full(2, edge)
+    x = rng.uniform(0, edge, (n, 2))
+    x[::2000] += rng.integers(-2, 3, (len(x[::2000]), 2)) * edge
+    diam = np.ones(n) if one_diameter else rng.uniform(0.8, 1.0, n)
+    first, last = O.nlist(x, L, diam, 0.3)
+    pick = rng.permutation(len(first))[:ignored]
+    ex = np.stack([first[pick], last[pick]], -1).astype(np.int32)
+    s = capi.System(2, np.ones(n))
+    s.set_box(L)
+    s.nlist_set(0.3, diam)
+    if ignored:
+        s.ignore(ex[:, 0], ex[:, 1])
+        keep = np.ones(len(first), bool)
+        keep[pick] = False
+        first, last = first[keep], last[keep]
+    s.set_repulsion([1.0], [1.0], [2.0], np.zeros(n, np.int32))
+    s.set_state(x=x)
+    for _ in range(2):
+        s.update_list(True)
+        fd, ld = s.pairs()
+        assert np.array_equal(fd, first) and np.array_equal(ld, last)
+    assert s.list_info()["tiled"] == (tiled == "1")
+    s.close()
+
+
+# rebuilds inside a run on the untiled list, step launches queued behind them, with
+# ignored pairs and with an ignore between two runs
+def test_rebuilds_inside_a_run_with_ignored_pairs(monkeypatch):
+    _device_or_fail()
+    print("deferred rebuilds, ignored pairs", flush=True)
+    monkeypatch.setenv("PARM_TILED", "0")
+    monkeypatch.setenv("PARM_TPA", "4")
+    n = 6000
+    x, L = S.jittered_lattice(n, 0.7, 3, seed=3)
+    v = S.gaussian_velocities(n, 3, 1.0, seed=3)
+    p = S.lj_params(n)
+    t = O.PairTable(O.LJ_ATTRACT_REPULSE, p["eps"], p["sigma"], p["third"], p["types"])
+    r = O.System(np.ones(n), L, t, p["diam"], 0.05, ndim=3, brute=False)
+    s = capi.System(3, np.ones(n))
+    s.set_box(L)
+    s.nlist_set(0.05, p["diam"])
+    s.set_lj(p["eps"], p["sigma"], p["third"], p["types"])
+    first, last = O.nlist(x, L, p["diam"], 0.05)
+    pick = np.random.default_rng(1).permutation(len(first))[:800]
+    for q in (r, s):
+        q.set_state(x=x, v=v, a=np.zeros_like(x))
+    for part in (pick[:400], pick[400:]):
+        s.ignore(first[part], last[part])
+        for k in part:
+            r.ignore(first[k], last[k])
+        for q in (r, s):
+            if part[0] == pick[0]:
+                q.initialize()
+            q.verlet(0.002, 14)
+        assert s.which() == r.which()
+        fd, ld = s.pairs()
+        fr, lr = r.pairs()
+        assert np.array_equal(fd, fr) and np.array_equal(ld, lr)
+        xr, xd = r.state()[0], s.state()[0]
+        assert np.abs(xd - xr).max() <= 1e-11 * max(1.0, np.abs(xr).max())
+    assert s.which() > 6
+    s.close()
+
+
 # the counted order and the tile plan: one workgroup (up to 8192 atoms and cells)
 # and several launches, one and several scan tiles of cells,
 # several rows to a plan workgroup, crowded cells, empty rows, the build lanes of a
