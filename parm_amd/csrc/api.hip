@@ -78,10 +78,6 @@ void dfree(T *&p) {
 
 }  // namespace
 
-constexpr int kFlagRing = 4;
-// flag words: [0, kFlagRing) the step loop's skin tests (by step number), then
-// the list-build overflow flag, a scratch word for reductions that raise no
-// flag, the on-demand skin test, and the verdict on a list build
 // dynamic LDS of one tiled build workgroup, at most (the stencil's atoms)
 constexpr size_t kTiledLdsMax = 56 * 1024;
 // limits of the autotuner's rules (autotune)
@@ -89,6 +85,10 @@ constexpr int kMixedUntiledAtoms = 1 << 15;
 constexpr int kMixedRepulsionFixed = 100000, kMixedRepulsionRow = 16;
 // run-ahead of the step loop (step_runahead)
 constexpr int kRunAhead = 2, kRunAheadAtoms = 1 << 15;
+// flag words: [0, kFlagRing) the step loop's skin tests (by step number), then
+// the list-build overflow flag, a scratch word for reductions that raise no
+// flag, the on-demand skin test, and the verdict on a list build
+constexpr int kFlagRing = 4;
 static_assert(kRunAhead + 1 < kFlagRing, "a flag word is not reused while a launch may read it");
 constexpr int kSlotBuild = kFlagRing + 1, kSlotScratch = kFlagRing + 2,
               kSlotSkin = kFlagRing + 3, kSlotVerdict = kFlagRing + 4;
@@ -715,7 +715,7 @@ int rebuild(parm_system *s, bool keep_af = true, const ReduceBuf *skin = nullptr
         if (!s->ccount_clear)
             PARM_HIP(hipMemsetAsync(s->ccount, 0, sizeof(uint32_t) * s->cstart_cap, st));
         s->ccount_clear = false;
-        PARM_HIP(launch_cell_order(s->ndim, n, s->pos, s->grid, s->box, s->tkeys, s->tvals,
+        PARM_HIP(launch_cell_order(s->ndim, n, s->pos, s->grid, s->tkeys, s->tvals,
                                    s->ccount, s->ctotal, s->cstart, s->vals, s->tinfo, st));
         s->ccount_clear = true;
         PARM_CHECK(permute_all(s, keep_af, true, skin));
@@ -803,7 +803,7 @@ hipEvent_t pool_event(parm_system *s) {
 
 // Brackets a launch with timing events when instrumentation is on.  A force
 // launch given end() as its ReduceBuf::done records the end itself, right
-// after the force kernel (its k_finalize then falls outside the bracket).
+// after the force kernel (a reduction of its sums then falls outside the bracket).
 struct ProfScope {
     parm_system *s;
     std::vector<std::pair<hipEvent_t, hipEvent_t>> *dst;

@@ -16,6 +16,7 @@
 //            k_batch_skin     top-2 of |x - xref| per system -> the list of
 //                             systems for the next rebuild
 // parm_batch_initialize orders every system's slots by cell (k_batch_reorder).
+#include "cells.hpp"
 #include "common.hpp"
 #include "kernels.hpp"
 #include "pairs.hpp"
@@ -202,20 +203,6 @@ __global__ __launch_bounds__(kAllThreads) void k_batch_all(
 constexpr int kSortKeep = 4;
 constexpr int kRankMax = 64;
 
-template <int D>
-__device__ __forceinline__ int batch_key(const Vec<D> &x, const BatchGeom &G) {
-    int key = 0;
-#pragma unroll
-    for (int d = D - 1; d >= 0; d--) {
-        double sv = x.c[d] * G.grid.invL[d];
-        sv -= floor(sv);
-        int cd = (int)(sv * (double)G.grid.nc[d]);
-        cd = cd < 0 ? 0 : (cd >= G.grid.nc[d] ? G.grid.nc[d] - 1 : cd);
-        key = key * G.grid.nc[d] + cd;
-    }
-    return key;
-}
-
 // The per-slot outputs of the sort.
 template <int D>
 struct SortOut {
@@ -262,7 +249,7 @@ __device__ __forceinline__ void sort_system(const int s, const BatchArrays &A,
             const int k = t + q * NT;
             kk[q] = ak[q] = 0;
             if (k < n) {
-                kk[q] = batch_key<D>(PosStore<D>::load(xk[q]), G);
+                kk[q] = (int)cell_of<D>(PosStore<D>::load(xk[q]), G.grid);
                 ak[q] = atomicAdd(&hist[kk[q]], 1);
                 xref[off + k] = xk[q];
             }
@@ -270,7 +257,7 @@ __device__ __forceinline__ void sort_system(const int s, const BatchArrays &A,
     } else {
         for (int k = t; k < n; k += NT) {
             const PT x = pos[off + k];
-            atomicAdd(&hist[batch_key<D>(PosStore<D>::load(x), G)], 1);
+            atomicAdd(&hist[(int)cell_of<D>(PosStore<D>::load(x), G.grid)], 1);
             xref[off + k] = x;
         }
     }
@@ -358,7 +345,7 @@ __device__ __forceinline__ void sort_system(const int s, const BatchArrays &A,
                 d = A.diam[off + k];
                 type = A.type[off + k];
             }
-            const int key = valid ? batch_key<D>(PosStore<D>::load(x), G) : 0;
+            const int key = valid ? (int)cell_of<D>(PosStore<D>::load(x), G.grid) : 0;
             unsigned long long eq = __ballot(valid);
 #pragma unroll
             for (int b = 0; b < kKeyBits; b++) {

@@ -52,9 +52,9 @@ hipError_t launch_permute(int ndim, int n, const int32_t *perm, const PermuteSet
 int scan_tiles(int ncell);
 struct ReduceBuf;
 hipError_t launch_cell_order(int ndim, int n, const void *pos, const CellGrid &g,
-                             const Box &box, uint32_t *ukeys, int32_t *arrival,
-                             uint32_t *count, uint32_t *total, int32_t *cstart, int32_t *slot,
-                             int *info, hipStream_t s);
+                             uint32_t *ukeys, int32_t *arrival, uint32_t *count,
+                             uint32_t *total, int32_t *cstart, int32_t *slot, int *info,
+                             hipStream_t s);
 hipError_t launch_cell_permute(int ndim, int n, const int32_t *slot, const uint32_t *ukeys,
                                const int32_t *cstart, const CellGrid &g, const Box &box,
                                uint32_t *keys, void *xw, const PermuteSet &P,
@@ -242,9 +242,9 @@ struct ReduceBuf {
     double *out;                  // kRedWidth doubles (final sums)
     uint32_t *flag;               // flag word
     double skin;                  // skin test threshold
-    uint32_t *hflag;              // device-visible pinned host copy of the flag word, or null
+    uint32_t *hflag;              // device-visible pinned host copy of the flag word
     hipEvent_t done;              // host side, or null: recorded on the launch stream right
-                                  // after the force kernel, before its k_finalize (timing)
+                                  // after the force kernel, before its sums' reduction (timing)
     uint32_t *cnt;                // or null: the skin-test reduction over several
     double *gpart;                // workgroups (counter, kFinBlocks x 3 results)
     StepGate g;

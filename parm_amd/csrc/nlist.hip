@@ -35,30 +35,13 @@
 #include <type_traits>
 #include <utility>
 
+#include "cells.hpp"
 #include "common.hpp"
 #include "kernels.hpp"
 #include "stepcore.hpp"
 #include "tiles.hpp"
 
 namespace parm {
-
-// ------------------------------------------------------------ cell keys
-// Cell of x, and x wrapped into [0, L) per component with the same floor.
-template <int D>
-__device__ __forceinline__ uint32_t cell_of(const Vec<D> &x, const CellGrid &g, const Box &box,
-                                            Vec<D> &w) {
-    uint32_t key = 0;
-#pragma unroll
-    for (int k = D - 1; k >= 0; k--) {
-        double s = x.c[k] * g.invL[k];
-        s -= floor(s);
-        w.c[k] = s * box.L[k];
-        int c = (int)(s * (double)g.nc[k]);
-        c = c < 0 ? 0 : (c >= g.nc[k] ? g.nc[k] - 1 : c);
-        key = key * (uint32_t)g.nc[k] + (uint32_t)c;
-    }
-    return key;
-}
 
 // ---------------------------------------------------- order by cell, counted
 // A rebuild is a chain of short launches, bound by their number and latency
@@ -73,7 +56,7 @@ __device__ __forceinline__ uint32_t cell_of(const Vec<D> &x, const CellGrid &g, 
 // 262,144 disks 7.91 -> 6.04, 50 of 1M atoms 11.46 -> 11.34.
 template <int D>
 __global__ __launch_bounds__(kBlock) void k_cell_count(
-    int n, const typename PosStore<D>::T *__restrict__ pos, CellGrid g, Box box,
+    int n, const typename PosStore<D>::T *__restrict__ pos, CellGrid g,
     uint32_t *__restrict__ key, int32_t *__restrict__ arrival, uint32_t *__restrict__ count,
     int *__restrict__ info) {
     const int i = blockIdx.x * kBlock + threadIdx.x;
@@ -81,8 +64,7 @@ __global__ __launch_bounds__(kBlock) void k_cell_count(
     const bool act = i < n;
     uint32_t c = 0xffffffffu;
     if (act) {
-        Vec<D> w;
-        c = cell_of<D>(PosStore<D>::load(pos[i]), g, box, w);
+        c = cell_of<D>(PosStore<D>::load(pos[i]), g);
         key[i] = c;
     }
     // neighbouring slots mostly share a cell (the order of the last rebuild):
@@ -121,17 +103,7 @@ __global__ __launch_bounds__(kBlock) void k_cell_keys(
         keys[i] = (uint32_t)g.ncell;
         return;
     }
-    Vec<D> x = PosStore<D>::load(pos[i]);
-    uint32_t key = 0;
-#pragma unroll
-    for (int k = D - 1; k >= 0; k--) {
-        double s = x.c[k] * g.invL[k];
-        s -= floor(s);
-        int c = (int)(s * (double)g.nc[k]);
-        c = c < 0 ? 0 : (c >= g.nc[k] ? g.nc[k] - 1 : c);
-        key = key * (uint32_t)g.nc[k] + (uint32_t)c;
-    }
-    keys[i] = key;
+    keys[i] = cell_of<D>(PosStore<D>::load(pos[i]), g);
 }
 
 // ------------------------------------------------------------ radix sort
@@ -353,7 +325,7 @@ constexpr int kSmallCells = 8192;
 
 template <int D>
 __global__ __launch_bounds__(kSmallThreads) void k_cell_order_small(
-    int n, const typename PosStore<D>::T *__restrict__ pos, CellGrid g, Box box,
+    int n, const typename PosStore<D>::T *__restrict__ pos, CellGrid g,
     uint32_t *__restrict__ key, int32_t *__restrict__ cstart, int32_t *__restrict__ slot,
     int *__restrict__ info) {
     constexpr int kPer = kSmallCells / kSmallThreads;
@@ -373,8 +345,7 @@ __global__ __launch_bounds__(kSmallThreads) void k_cell_order_small(
         const int i = t + q * kSmallThreads;
         c[q] = at[q] = 0u;
         if (i < n) {
-            Vec<D> w;
-            c[q] = cell_of<D>(PosStore<D>::load(x[q]), g, box, w);
+            c[q] = cell_of<D>(PosStore<D>::load(x[q]), g);
             key[i] = c[q];
             at[q] = atomicAdd(&count[c[q]], 1u);
         }
@@ -438,10 +409,8 @@ __global__ __launch_bounds__(kBlock) void k_cell_permute(
         int to = s0;
 #pragma unroll 8
         for (int k = s0; k < s1; k++) to += slot[k] < i ? 1 : 0;
-        Vec<D> w;
-        (void)cell_of<D>(PosStore<D>::load(x0), g, box, w);
         keys[to] = c;
-        xw[to] = PosStore<D>::make(w);
+        xw[to] = PosStore<D>::make(wrapped<D>(PosStore<D>::load(x0), g, box));
         static_cast<PT *>(P.pos_dst[0])[to] = x0;
         static_cast<PT *>(P.pos_dst[1])[to] = x1;
 #pragma unroll
@@ -1326,8 +1295,7 @@ __global__ __launch_bounds__(kBlock) void k_tiled_to_global(
     }
 }
 
-// Wrapped copy of the positions, frac(x / L) * L per component, computed
-// with the same floor as the cell keys: the list build's prefilter uses it.
+// Wrapped copy of the positions, which the list build's prefilter uses.
 template <int D>
 __global__ __launch_bounds__(kBlock) void k_wrap(int n,
                                                  const typename PosStore<D>::T *__restrict__ pos,
@@ -1335,14 +1303,7 @@ __global__ __launch_bounds__(kBlock) void k_wrap(int n,
                                                  typename PosStore<D>::T *__restrict__ xw) {
     const int i = blockIdx.x * kBlock + threadIdx.x;
     if (i >= n) return;
-    Vec<D> x = PosStore<D>::load(pos[i]);
-#pragma unroll
-    for (int k = 0; k < D; k++) {
-        double s = x.c[k] * g.invL[k];
-        s -= floor(s);
-        x.c[k] = s * box.L[k];
-    }
-    xw[i] = PosStore<D>::make(x);
+    xw[i] = PosStore<D>::make(wrapped<D>(PosStore<D>::load(pos[i]), g, box));
 }
 
 __global__ __launch_bounds__(kStatsThreads) void k_build_stats(
@@ -1420,24 +1381,24 @@ hipError_t launch_cell_keys(int ndim, int n, const void *pos, const int32_t *ran
 int scan_tiles(int ncell) { return (ncell + kScanTile - 1) / kScanTile; }
 
 hipError_t launch_cell_order(int ndim, int n, const void *pos, const CellGrid &g,
-                             const Box &box, uint32_t *ukeys, int32_t *arrival,
-                             uint32_t *count, uint32_t *total, int32_t *cstart, int32_t *slot,
-                             int *info, hipStream_t s) {
+                             uint32_t *ukeys, int32_t *arrival, uint32_t *count,
+                             uint32_t *total, int32_t *cstart, int32_t *slot, int *info,
+                             hipStream_t s) {
     if (n <= kSmallAtoms && g.ncell <= kSmallCells) {
         if (ndim == 3)
             hipLaunchKernelGGL(k_cell_order_small<3>, dim3(1), dim3(kSmallThreads), 0, s, n,
-                               (const double4 *)pos, g, box, ukeys, cstart, slot, info);
+                               (const double4 *)pos, g, ukeys, cstart, slot, info);
         else
             hipLaunchKernelGGL(k_cell_order_small<2>, dim3(1), dim3(kSmallThreads), 0, s, n,
-                               (const double2 *)pos, g, box, ukeys, cstart, slot, info);
+                               (const double2 *)pos, g, ukeys, cstart, slot, info);
         return hipGetLastError();
     }
     if (ndim == 3)
         hipLaunchKernelGGL(k_cell_count<3>, dim3(nblk(n)), dim3(kBlock), 0, s, n,
-                           (const double4 *)pos, g, box, ukeys, arrival, count, info);
+                           (const double4 *)pos, g, ukeys, arrival, count, info);
     else
         hipLaunchKernelGGL(k_cell_count<2>, dim3(nblk(n)), dim3(kBlock), 0, s, n,
-                           (const double2 *)pos, g, box, ukeys, arrival, count, info);
+                           (const double2 *)pos, g, ukeys, arrival, count, info);
     const int nt = scan_tiles(g.ncell);
     if (nt > 1)
         hipLaunchKernelGGL(k_cell_total, dim3(nt), dim3(kScanThreads), 0, s, g.ncell, count,

@@ -182,7 +182,6 @@ __global__ __launch_bounds__(kWave *TPA) void k_force_tiled(AtomArrays A, ListVi
     extern __shared__ double4 st64[];
     __shared__ int2 runs[kRunSlots];  // run_entry form (tiles.hpp)
     __shared__ int wides[TPA];
-    float4 *st32 = reinterpret_cast<float4 *>(st64);
     double *stc64 = reinterpret_cast<double *>(st64);
     float *stc32 = reinterpret_cast<float *>(st64);
     Real *stc = reinterpret_cast<Real *>(st64);
@@ -190,8 +189,7 @@ __global__ __launch_bounds__(kWave *TPA) void k_force_tiled(AtomArrays A, ListVi
                                                          lj_slots_bytes<D, PREC>(Lv.smax));
     uint8_t *ljtype = reinterpret_cast<uint8_t *>(
         ljtab + (TABLDS ? (size_t)P.ntypes * P.ntypes : (size_t)0));
-    int32_t *stj = REL32 ? reinterpret_cast<int32_t *>(st32 + Lv.smax)
-                         : reinterpret_cast<int32_t *>(st64 + Lv.smax);
+    int32_t *stj = reinterpret_cast<int32_t *>(st64 + Lv.smax);  // unless COMPACT or RAW
 
     constexpr bool STEP = STAGE == kStageVerletKickDrift || STAGE == kStageDampedKickDrift ||
                           STAGE == kStageVerletKick || STAGE == kStageDampedKick;
@@ -341,13 +339,6 @@ __global__ __launch_bounds__(kWave *TPA) void k_force_tiled(AtomArrays A, ListVi
                     stc64[s * D + k] = v.c[k];
             }
             if constexpr (LJ && !SINGLE) ljtype[s] = (uint8_t)tj;
-        } else if (REL32) {
-            float4 q;
-            q.x = (float)v.c[0];
-            q.y = (float)v.c[1];
-            q.z = D == 3 ? (float)v.c[2] : 0.0f;
-            q.w = __int_as_float(tj);
-            st32[s] = q;
         } else {
             double4 q;
             q.x = v.c[0];
@@ -431,23 +422,12 @@ __global__ __launch_bounds__(kWave *TPA) void k_force_tiled(AtomArrays A, ListVi
                 const Vec<D> r = diff<D>(xi, xj, box);
                 visit<D, KIND, PREC, ENERGY, HARM>(SINGLE ? p0 : prow[tj], r, fi, f32, acc);
             } else if constexpr (REL32) {
-                float qc[3] = {0.0f, 0.0f, 0.0f};
                 int tj = 0;
-                if constexpr (COMPACT) {
-#pragma unroll
-                    for (int k = 0; k < D; k++) qc[k] = stc32[s * D + k];
-                    if constexpr (!SINGLE) tj = ljtype[s];
-                } else {
-                    const float4 q = st32[s];
-                    qc[0] = q.x;
-                    qc[1] = q.y;
-                    qc[2] = q.z;
-                    tj = __float_as_int(q.w);
-                }
+                if constexpr (!SINGLE) tj = ljtype[s];
                 float rf[D];
 #pragma unroll
                 for (int k = 0; k < D; k++) {
-                    float d = ri[k] - qc[k];
+                    float d = ri[k] - stc32[s * D + k];
                     if (FOLD) d = d > hLf[k] ? d - Lf[k] : (d < -hLf[k] ? d + Lf[k] : d);
                     rf[k] = d;
                 }
