@@ -228,11 +228,12 @@ __global__ __launch_bounds__(kFinThreads) void k_finalize_skin(int nparts, Reduc
 }
 
 // For skin tests on demand (the step loop reduces its own inside the next step
-// launch).  Below this many partials the one-workgroup k_finalize is the
-// quicker (the counter's fences and the second merge cost more than they save:
-// measured after every step, +6 % per step at 1000 atoms, +4 % at 32,768; -1.6 %
-// at 1M atoms, 16,384 partials)
-constexpr int kFinMultiMin = 8 * kFinal;
+// launch).  From about this many partials (1M atoms) on several workgroups are
+// the quicker; below, the counter's fences and the second merge cost more than
+// they save.  parm_nlist_update with nothing to rebuild, one workgroup / several:
+// 32,768 atoms 12.5 / 13.5 us, 262,144 13.7 / 14.6, 1M 24.1 / 23.5, 2M 34.9 / 32.4,
+// 4M 61 / 51, 16M 221 / 192.
+constexpr int kFinMultiMin = 4 * kFinal;
 
 static void launch_finalize(int nparts, const ReduceBuf &R, hipStream_t s) {
     if (R.cnt && R.gpart && nparts >= kFinMultiMin) {
