@@ -336,8 +336,9 @@ void make_grid(parm_system *s) {
 
 // Per-lane entry counts are 16-bit (lcount): a list whose capacity could
 // give one lane more than 65535 entries is refused, not wrapped.
+constexpr int kLaneEntries = 65535;
 int check_lane_counts(int64_t cap, int tpa) {
-    if (cap > (int64_t)65535 * tpa)
+    if (cap > (int64_t)kLaneEntries * tpa)
         return fail(PARM_E_UNSUPPORTED,
                     "more than 65535 list entries per lane (capacity " + std::to_string(cap) +
                         " at " + std::to_string(tpa) +
@@ -890,6 +891,12 @@ int autotune(parm_system *s, int stage, const StepCoef &c) {
         cands = {{0, 1}, {0, 2}};
         if (tiled_ok) cands.emplace_back(1, 2);
     }
+    // (lanes whose counts could not hold the list's capacity)
+    cands.erase(std::remove_if(cands.begin(), cands.end(),
+                               [&](const std::pair<int, int> &q) {
+                                   return s->cap > (int64_t)kLaneEntries * q.second;
+                               }),
+                cands.end());
     if (cands.size() <= 1) {
         if (!cands.empty() && (cands[0].first != (int)s->tiled || cands[0].second != s->tpa)) {
             s->tiled = cands[0].first != 0;
@@ -920,6 +927,8 @@ int autotune(parm_system *s, int stage, const StepCoef &c) {
     }
     hipEvent_t e0 = pool_event(s), e1 = pool_event(s);
     if (rc == PARM_OK && (!e0 || !e1)) rc = fail(PARM_E_DEVICE, "event creation failed");
+    const bool was_tiled = s->tiled;
+    const int was_tpa = s->tpa;
     size_t best = 0;
     float best_ms = 1e30f;
     for (size_t q = 0; q < cands.size() && rc == PARM_OK; q++) {
@@ -950,7 +959,13 @@ int autotune(parm_system *s, int stage, const StepCoef &c) {
     if (e0 && e1) s->ev_used -= 2;
     (void)hipStreamSynchronize(st);
     dfree(sc);
-    if (rc != PARM_OK) return rc;
+    if (rc != PARM_OK) {
+        // the system as it was, its list to be built anew
+        s->tiled = was_tiled;
+        s->tpa = was_tpa;
+        lose_list(s);
+        return rc;
+    }
     s->tiled = cands[best].first != 0;
     s->tpa = cands[best].second;
     s->layout_pref = s->tiled ? 1 : 2;

@@ -302,6 +302,34 @@ def test_most_lanes(runtime, n, ask, lanes):
     _child(runtime, "case_most_lanes", n, lanes, PARM_TPA=str(ask), PARM_TILED="0")
 
 
+# rows that one lane's 16-bit count cannot hold: fewer lanes are no candidate; and
+# a candidate whose layout is refused leaves the lanes and the layout as they were
+def case_tuning_long_rows(hh, refused):
+    s = _system()
+    if refused == "no":
+        hh.hh_row(80000)
+        s.update_list(True)
+        assert s.list_info()["capacity"] >= 80000
+        s.verlet(0.001, 16)
+        assert s.list_info()["lanes"] > 1
+    else:
+        s.update_list(True)
+        was = s.list_info()
+        hh.hh_row(10 ** 7)
+        _refused(UNSUPPORTED, s.verlet, 0.001, 16)
+        assert s.list_info() == was
+        s.verlet(0.001, 8)
+        assert s.which() == 2  # (the list that was lost)
+    assert hh.hh_bad() == 0
+    s.close()
+
+
+@pytest.mark.parametrize("refused", ["no", "yes"])
+@pytest.mark.parametrize("tiled", ["", "0"])
+def test_tuning_long_rows(runtime, tiled, refused):
+    _child(runtime, "case_tuning_long_rows", refused, **({"PARM_TILED": tiled} if tiled else {}))
+
+
 if __name__ == "__main__":
     sys.path.insert(0, ROOT)
     hh = C.CDLL(sys.argv[1], mode=C.RTLD_GLOBAL)
