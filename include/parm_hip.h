@@ -113,7 +113,9 @@ int parm_nlist_set(parm_system *sys, double skin, int64_t nmembers,
 /* NeighborList::update_list(force) (src/trackers.cpp:19-85): the O(N) skin
  * test (two largest displacements since the last rebuild sum to >= skin),
  * then, if needed or forced, a rebuild.  *rebuilt (may be NULL) is 1 if the
- * list was rebuilt. */
+ * list was rebuilt.  A rebuild that fails, here or inside a run, leaves no list
+ * (the pair count is 0): the next update, force, sum, step or minimiser call
+ * rebuilds before anything else, or fails the same way. */
 int parm_nlist_update(parm_system *sys, int force, int *rebuilt);
 
 /* NeighborList::ignore(a[k], b[k]) for k = 0..npairs-1 (src/trackers.hpp:
@@ -226,7 +228,8 @@ int parm_pair_sums(parm_system *sys, double *U, double *W, double *S,
  * workgroup partials live in a fixed device array of the library (about
  * 8 MiB per GPU, held until the process ends), so systems of at most
  * 2^21 atoms (larger: PARM_E_UNSUPPORTED), and calls that overlap on one GPU
- * race (order them on one stream, or synchronise between them). */
+ * race (order them on one stream, or synchronise between them).  After a
+ * rebuild that failed: PARM_E_STATE (a rebuild allocates). */
 int parm_pair_sums_noalloc(parm_system *sys, double *out);
 
 /* AtomGroup::kinetic_energy(originv) (box.cpp:401-411), momentum()
@@ -410,7 +413,7 @@ int parm_batch_profile_read(parm_batch *b, int reset, double *force_ms,
 int parm_batch_lists(parm_batch *b, uint32_t *which, int64_t *npairs);
 /* The pairs of system sysid's list as (first, last) atom indices within the
  * system, first > last, sorted by first then last.  Writes min(cap, n) pairs
- * and the total n. */
+ * and the total n (0 while there are no lists). */
 int parm_batch_pairs(parm_batch *b, int64_t sysid, int64_t cap, int32_t *first,
                      int32_t *last, int64_t *npairs);
 
